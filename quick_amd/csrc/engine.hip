@@ -99,6 +99,109 @@ struct HostBlock {
 };
 
 // --------------------------------------------------------------------------
+// Side streams.  The class launches of a build are independent (they only
+// add into G with atomics), and most of them cannot fill the GPU: a launch
+// of a small molecule is one wave's latency long, a launch of a large one
+// ends in a tail of few waves.  A build therefore forks from the caller's
+// stream onto kSide more streams of default priority and joins them again
+// before G is summed, all by events, so the caller's stream order (and a
+// capture of it) covers everything.  Four streams in all, the hardware
+// queues a process has.  One stream -> four, ms per build: water 6-31G*
+// (host call) 0.35 -> 0.21, glycine 6-31G** 1.51 -> 0.95, (H2O)8 cc-pVDZ
+// 2.73 -> 1.48, ethane def2-TZVP 4.47 -> 2.79, (H2O)8+ open shell 3.71 ->
+// 1.54, (H2O)32 6-31G* 13.9 -> 11.6, (Gly)10 mixed 33.4 -> 30.7.
+//
+// A set belongs to one engine or batch while that lives (a set that takes
+// part in a capture cannot serve another thread's builds); at most kKeep
+// sets per device are kept when their owners have gone.
+// --------------------------------------------------------------------------
+constexpr int kSide = 3;
+
+struct SideStreams {
+    int device = -1;
+    hipStream_t s[kSide] = {};
+    hipEvent_t fork = nullptr, done[kSide] = {};
+
+    bool create(int dev)
+    {
+        device = dev;
+        bool ok = hipEventCreateWithFlags(&fork, hipEventDisableTiming) == hipSuccess;
+        for (int k = 0; ok && k < kSide; ++k)
+            ok = hipStreamCreateWithFlags(&s[k], hipStreamNonBlocking) == hipSuccess &&
+                 hipEventCreateWithFlags(&done[k], hipEventDisableTiming) == hipSuccess;
+        return ok;
+    }
+    ~SideStreams()
+    {
+        if (fork) (void)hipEventDestroy(fork);
+        for (int k = 0; k < kSide; ++k) {
+            if (s[k]) (void)hipStreamDestroy(s[k]);
+            if (done[k]) (void)hipEventDestroy(done[k]);
+        }
+    }
+};
+
+class SidePool {
+public:
+    static SidePool& get()
+    {
+        // never destroyed: the streams it keeps must not outlive the HIP runtime
+        static SidePool* pool = new SidePool();
+        return *pool;
+    }
+    SideStreams* take(int device)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            for (size_t k = 0; k < free_.size(); ++k)
+                if (free_[k]->device == device) {
+                    SideStreams* ss = free_[k];
+                    free_.erase(free_.begin() + k);
+                    return ss;
+                }
+        }
+        SideStreams* ss = new SideStreams();
+        if (ss->create(device)) return ss;
+        delete ss;
+        return nullptr;   // the caller runs on its own stream alone
+    }
+    void give(SideStreams* ss)
+    {
+        if (!ss) return;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            int same = 0;
+            for (auto* x : free_) same += x->device == ss->device;
+            if (same < kKeep) {
+                free_.push_back(ss);
+                return;
+            }
+        }
+        delete ss;
+    }
+
+private:
+    static constexpr int kKeep = 8;
+    std::mutex mu_;
+    std::vector<SideStreams*> free_;
+};
+
+// Makes sure `side` has its streams, unless s is being captured (creating
+// streams is no work for a capture; without them everything runs on s).
+bool side_ready(SideStreams*& side, int device, hipStream_t s)
+{
+    if (side) return true;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (st != hipStreamCaptureStatusNone) return false;
+    side = SidePool::get().take(device);
+    return side != nullptr;
+}
+
+// --------------------------------------------------------------------------
 // Device helper kernels
 // --------------------------------------------------------------------------
 __global__ void k_cutmat(const double* __restrict__ P, int n, int nshell, const int* __restrict__ f0,
@@ -285,6 +388,8 @@ struct qf_engine {
         int os_lean;     // ... or, on the tile kernel, in the fused lean form
     };
     std::vector<Launch> launches;
+    std::vector<std::pair<int, int>> order;   // issue order: (launch index, stream 0..kSide)
+    SideStreams* side = nullptr;              // taken at the first build
     bool prepared = false;
     unsigned long long generation = 0;   // bumped by every prepare(): batches check it
     bool built = false;                  // a build has run since the last prepare()
@@ -321,6 +426,7 @@ struct qf_engine {
     ~qf_engine()
     {
         for (hipEvent_t ev : ev_pool) (void)hipEventDestroy(ev);
+        SidePool::get().give(side);
     }
 
     int set_device() { return hipSetDevice(device) == hipSuccess ? QF_OK : fail(QF_ERR_BADDEVICE, "hipSetDevice"); }
@@ -584,6 +690,46 @@ int prefix_count(const std::vector<qf::PairInfo>& kets, double yi, double thr, b
             hi = mid;
     }
     return lo;
+}
+
+// Issue order of class launches and the stream of each: longest first, each
+// to the stream with the least time so far.  The time of a launch is taken
+// as one wave's latency plus its algorithmic FLOPs (every quartet of the
+// windows) at the rate its kernel reaches.  Classes whose node programs keep
+// their slots in the shared global buffer stay on one stream (0).
+std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launch>& launches,
+                                              const std::vector<qf::Task>& tasks)
+{
+    constexpr double kLatency = 1e-5, kRateCoop = 1.2e12, kRateLane = 6e12;
+    const int n = (int)launches.size();
+    std::vector<double> t(n);
+    for (int l = 0; l < n; ++l) {
+        const auto& L = launches[l];
+        double nq = 0.0, np = 0.0;
+        for (int x = L.offset; x < L.offset + L.count; ++x) {
+            const qf::Task& k = tasks[x];
+            const double q = (double)(k.ke - k.kb) * k.ket_count;
+            if (k.pb == 0 && k.qb == 0) nq += q;
+            np += q * (k.pe - k.pb) * (k.qe - k.qb);
+        }
+        t[l] = kLatency + qf::class_flops(L.cb, L.ck, (unsigned long long)nq, (unsigned long long)np) /
+                              (L.tile == 2 ? kRateCoop : kRateLane);
+    }
+    std::vector<int> ord(n);
+    std::iota(ord.begin(), ord.end(), 0);
+    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return t[x] > t[y]; });
+    double load[kSide + 1] = {};
+    std::vector<std::pair<int, int>> out;
+    for (int l : ord) {
+        const auto& L = launches[l];
+        int to = 0;
+        if (!(L.tile == 2 && qf::coop_global_doubles(L.cb, L.ck) > 0))
+            for (int k = 1; k <= kSide; ++k)
+                if (load[k] < load[to]) to = k;
+        load[to] += t[l];
+        out.push_back({l, to});
+    }
+    return out;
 }
 
 int prepare(qf_engine* e)
@@ -940,6 +1086,7 @@ int prepare(qf_engine* e)
     }
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
+    e->order = stream_order(e->launches, e->tasks);
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
     size_t gdoubles = 0;
@@ -1027,8 +1174,43 @@ struct GBufs {
     int replicas;
     double* Gs;
     bool timing;   // per-launch HIP events (never in the no-alloc path: it creates events)
+    bool fork;     // spread the class launches over side streams (not in the no-alloc path)
     double* Gt2 = nullptr;   // open-shell pass: accumulators of the second exchange density
 };
+
+// Issues the launches of `order` with issue(launch index, stream): forked
+// from s over the side streams and joined again, or all on s where there are
+// none.  After a failed launch the streams are joined all the same, so that a
+// capture of s stays whole.
+template <class F>
+int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<int, int>>& order, F&& issue)
+{
+    int rc = QF_OK;
+    if (!side) {
+        for (const auto& o : order)
+            if ((rc = issue(o.first, s))) return rc;
+        return rc;
+    }
+    bool used[kSide] = {};
+    QF_HIP(hipEventRecord(side->fork, s));
+    for (const auto& o : order) {
+        hipStream_t q = s;
+        if (o.second > 0) {
+            q = side->s[o.second - 1];
+            if (!used[o.second - 1]) {
+                QF_HIP(hipStreamWaitEvent(q, side->fork, 0));
+                used[o.second - 1] = true;
+            }
+        }
+        if ((rc = issue(o.first, q))) break;
+    }
+    for (int k = 0; k < kSide; ++k)
+        if (used[k]) {
+            QF_HIP(hipEventRecord(side->done[k], side->s[k]));
+            QF_HIP(hipStreamWaitEvent(s, side->done[k], 0));
+        }
+    return rc;
+}
 
 // dP2 != nullptr: the open-shell pass.  Every integral is digested with dP
 // (Coulomb and exchange, into Gt) and with dP2 (exchange only, into gb.Gt2);
@@ -1073,51 +1255,53 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     }
     hipLaunchKernelGGL(k_zero, dim3(1024), dim3(256), 0, s, gb.Gt, (size_t)n * n * gb.replicas);
     if (os) hipLaunchKernelGGL(k_zero, dim3(1024), dim3(256), 0, s, gb.Gt2, (size_t)n * n * gb.replicas);
-    for (size_t li = 0; li < e->launches.size(); ++li) {
-        const auto& L = e->launches[li];
-        hipEvent_t ea = nullptr, eb = nullptr;
-        if (gb.timing) {
+    // one class launch with descriptor m on stream q; los: its open-shell form
+    auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, hipStream_t q) -> int {
+        if (L.tile == 2) {
+            qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
+            if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
+            fc(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p, q);
+        } else if (L.tile) {
+            qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
+            if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
+            // open shell: a second exchange tile where two fit, else its terms go to Gt2
+            const int tos = !los ? 0 : L.lds_os ? 1 : 2;
+            ft(e->d_groups.p + L.goffset, L.gcount, e->d_tasks.p, e->d_blocks.p, m, L.fp32,
+               tos | (los && L.os_lean ? 4 : 0), L.waves, tos == 1 ? L.lds_os : L.lds, e->persist, q);
+        } else {
+            qf::FockLaunch f = qf::fock_launcher(L.cb, L.ck);
+            if (!f) return fail(QF_ERR_ARG, "no per-lane kernel for class");
+            if (f(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, L.fp32, los, e->persist, q))
+                return fail(QF_ERR_ARG, kDirectFp32Refused);
+        }
+        return QF_OK;
+    };
+    auto class_launch = [&](const qf_engine::Launch& L, hipStream_t q) -> int {
+        if (!(os && L.os_split)) return launch(L, dmol, os, q);
+        const int rc = launch(L, dmol, 0, q);
+        return rc ? rc : launch(L, dmol_x, 0, q);
+    };
+    if (gb.timing) {
+        // timed launches run one after another on s
+        for (size_t li = 0; li < e->launches.size(); ++li) {
             while (e->ev_pool.size() < e->ev_used + 2) {
                 hipEvent_t ev;
                 QF_HIP(hipEventCreate(&ev));
                 e->ev_pool.push_back(ev);
             }
-            ea = e->ev_pool[e->ev_used];
-            eb = e->ev_pool[e->ev_used + 1];
+            hipEvent_t ea = e->ev_pool[e->ev_used], eb = e->ev_pool[e->ev_used + 1];
             e->ev_used += 2;
             e->ev_launch.push_back((int)li);
             QF_HIP(hipEventRecord(ea, s));
+            const int rc = class_launch(e->launches[li], s);
+            if (rc) return rc;
+            QF_HIP(hipEventRecord(eb, s));
         }
-        // one class launch with descriptor m; los: its open-shell form
-        auto launch = [&](qf::MolDesc* m, int los) -> int {
-            if (L.tile == 2) {
-                qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
-                if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
-                fc(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p, s);
-            } else if (L.tile) {
-                qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
-                if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
-                // open shell: a second exchange tile where two fit, else its terms go to Gt2
-                const int tos = !los ? 0 : L.lds_os ? 1 : 2;
-                ft(e->d_groups.p + L.goffset, L.gcount, e->d_tasks.p, e->d_blocks.p, m, L.fp32,
-                   tos | (los && L.os_lean ? 4 : 0), L.waves, tos == 1 ? L.lds_os : L.lds, e->persist, s);
-            } else {
-                qf::FockLaunch f = qf::fock_launcher(L.cb, L.ck);
-                if (!f) return fail(QF_ERR_ARG, "no per-lane kernel for class");
-                if (f(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, L.fp32, los, e->persist, s))
-                    return fail(QF_ERR_ARG, kDirectFp32Refused);
-            }
-            return QF_OK;
-        };
-        int rc = QF_OK;
-        if (os && L.os_split) {
-            rc = launch(dmol, 0);
-            if (rc == QF_OK) rc = launch(dmol_x, 0);
-        } else {
-            rc = launch(dmol, os);
-        }
+    } else {
+        const bool forked = gb.fork && e->order.size() > 1 && side_ready(e->side, e->device, s);
+        const int rc = issue_forked(forked ? e->side : nullptr, s, e->order,
+                                    [&](int li, hipStream_t q) { return class_launch(e->launches[li], q); });
         if (rc) return rc;
-        if (gb.timing) QF_HIP(hipEventRecord(eb, s));
     }
     if (os)
         hipLaunchKernelGGL(k_finalize_os, dim3((n * n + 255) / 256), dim3(256), 0, s, gb.Gt, gb.Gt2, gb.replicas,
@@ -1139,7 +1323,7 @@ int build(qf_engine* e, const double* dP, double* dF, const double* dcm, hipStre
                            e->d_f1.p, e->d_cm.p);
         dcm = e->d_cm.p;
     }
-    const int rc = build_pass(e, dP, dcm, dF, 0, s, GBufs{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing});
+    const int rc = build_pass(e, dP, dcm, dF, 0, s, GBufs{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing, true});
     if (rc == QF_OK) {
         e->built = true;
         e->count_cm_own = (dcm == e->d_cm.p);
@@ -1175,7 +1359,7 @@ int build_os(qf_engine* e, const double* dPa, const double* dPb, double* dFa, do
         QF_HIP(e->d_zero.resize(n2));
         hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, s, e->d_zero.p, (size_t)n2);
     }
-    GBufs gb{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing};
+    GBufs gb{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing, true};
     gb.Gt2 = e->d_Gt2.p;
     const int rc = build_pass(e, e->d_Pt.p, dcm, dFa, 0, s, gb, e->d_Ps.p, dFb);
     if (rc == QF_OK) {
@@ -1368,7 +1552,7 @@ int qf_fock_build_device_noalloc(qf_engine* e, const double* d_P, double* d_F, c
                            e->d_f1.p, cm);
         d_cutmat = cm;
     }
-    return build_pass(e, d_P, d_cutmat, d_F, 2, s, GBufs{Gt, 1, Gs, false});
+    return build_pass(e, d_P, d_cutmat, d_F, 2, s, GBufs{Gt, 1, Gs, false, false});
 }
 
 // Two-electron gradient (QUICK's gpu_get_cshell_eri_grad_ -> getGrad,
@@ -1883,11 +2067,14 @@ struct qf_batch {
     std::vector<hipEvent_t> ev_pool;
     size_t ev_used = 0;
     std::vector<int> ev_launch;
+    std::vector<std::pair<int, int>> order;   // issue order: (launch index, stream 0..kSide)
+    SideStreams* side = nullptr;
     ~qf_batch()
     {
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
         if (cap_stream) (void)hipStreamDestroy(cap_stream);
+        SidePool::get().give(side);
         for (hipEvent_t ev : ev_pool) (void)hipEventDestroy(ev);
     }
 };
@@ -1899,37 +2086,43 @@ int batch_issue(qf_batch* b, hipStream_t s)
     const int nm = (int)b->mols.size();
     hipLaunchKernelGGL(k_cutmat_batch, dim3((b->max_ns2 + 255) / 256, nm), dim3(256), 0, s, b->d_bm.p);
     hipLaunchKernelGGL(k_zero, dim3(1024), dim3(256), 0, s, b->d_Gt.p, b->gt_total);
-    for (size_t li = 0; li < b->launches.size(); ++li) {
-        const auto& L = b->launches[li];
-        hipEvent_t ea = nullptr, eb = nullptr;
-        if (b->timing) {
+    auto class_launch = [&](const qf_engine::Launch& L, hipStream_t q) -> int {
+        if (L.tile == 2) {
+            qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
+            if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
+            fc(b->d_tasks.p + L.offset, L.count, b->d_blocks.p, b->d_moldesc.p, 0, b->persist, b->d_cscratch.p, q);
+        } else if (L.tile) {
+            qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
+            if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
+            ft(b->d_groups.p + L.goffset, L.gcount, b->d_tasks.p, b->d_blocks.p, b->d_moldesc.p, L.fp32, 0, L.waves,
+               L.lds, b->persist, q);
+        } else {
+            qf::FockLaunch f = qf::fock_launcher(L.cb, L.ck);
+            if (!f) return fail(QF_ERR_ARG, "no per-lane kernel for class");
+            if (f(b->d_tasks.p + L.offset, L.count, b->d_blocks.p, b->d_moldesc.p, L.fp32, 0, b->persist, q))
+                return fail(QF_ERR_ARG, kDirectFp32Refused);
+        }
+        return QF_OK;
+    };
+    if (b->timing) {
+        for (size_t li = 0; li < b->launches.size(); ++li) {
             while (b->ev_pool.size() < b->ev_used + 2) {
                 hipEvent_t ev;
                 QF_HIP(hipEventCreate(&ev));
                 b->ev_pool.push_back(ev);
             }
-            ea = b->ev_pool[b->ev_used];
-            eb = b->ev_pool[b->ev_used + 1];
+            hipEvent_t ea = b->ev_pool[b->ev_used], eb = b->ev_pool[b->ev_used + 1];
             b->ev_used += 2;
             b->ev_launch.push_back((int)li);
             QF_HIP(hipEventRecord(ea, s));
+            const int rc = class_launch(b->launches[li], s);
+            if (rc) return rc;
+            QF_HIP(hipEventRecord(eb, s));
         }
-        if (L.tile == 2) {
-            qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
-            if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
-            fc(b->d_tasks.p + L.offset, L.count, b->d_blocks.p, b->d_moldesc.p, 0, b->persist, b->d_cscratch.p, s);
-        } else if (L.tile) {
-            qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
-            if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
-            ft(b->d_groups.p + L.goffset, L.gcount, b->d_tasks.p, b->d_blocks.p, b->d_moldesc.p, L.fp32, 0, L.waves,
-               L.lds, b->persist, s);
-        } else {
-            qf::FockLaunch f = qf::fock_launcher(L.cb, L.ck);
-            if (!f) return fail(QF_ERR_ARG, "no per-lane kernel for class");
-            if (f(b->d_tasks.p + L.offset, L.count, b->d_blocks.p, b->d_moldesc.p, L.fp32, 0, b->persist, s))
-                return fail(QF_ERR_ARG, kDirectFp32Refused);
-        }
-        if (b->timing) QF_HIP(hipEventRecord(eb, s));
+    } else {
+        const int rc = issue_forked(b->order.size() > 1 ? b->side : nullptr, s, b->order,
+                                    [&](int li, hipStream_t q) { return class_launch(b->launches[li], q); });
+        if (rc) return rc;
     }
     hipLaunchKernelGGL(k_finalize_batch, dim3((b->max_n2 + 255) / 256, nm), dim3(256), 0, s, b->d_bm.p,
                        b->replicas);
@@ -2092,6 +2285,8 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
         b->d_groups.upload(groups) != hipSuccess || b->d_moldesc.upload(md) != hipSuccess ||
         b->d_bm.upload(b->mols) != hipSuccess)
         return bail(fail(QF_ERR_HIP, "batch table upload"));
+    b->order = stream_order(b->launches, tasks);
+    b->side = SidePool::get().take(b->device);   // null: the batch runs on the caller's stream alone
     *out = b;
     return QF_OK;
 }
