@@ -682,8 +682,9 @@ def launcher_source(name, diag, coop=False, lane=True):
         out += ["void launch_schwarz_%s(PairBlock blk, double* out, double* gscratch, hipStream_t s)" % name, "{",
                 "    if (blk.n <= 0) return;"]
         if lane:
-            out += ["    hipLaunchKernelGGL((schwarz_kernel<%s>), dim3((blk.n + WAVE - 1) / WAVE), dim3(WAVE), 0, s,"
-                    " blk, out);" % name]
+            out += ["    const int G = schwarz_lanes(blk.K), per = WAVE / G;",
+                    "    hipLaunchKernelGGL((schwarz_kernel<%s>), dim3((blk.n + per - 1) / per), dim3(WAVE), 0, s,"
+                    " blk, out, G);" % name]
         else:
             out += ["    using D = %sCoop;" % name,
                     "    const int grid = D::GLOBAL_SLOTS && blk.n > COOP_GLOBAL_SLICES ? COOP_GLOBAL_SLICES : blk.n;",

@@ -44,7 +44,8 @@ void launch_fock_tile_C1010(const TileGroup* g, int ng, const Task* t, const Pai
 void launch_schwarz_C1010(PairBlock blk, double* out, double* gscratch, hipStream_t s)
 {
     if (blk.n <= 0) return;
-    hipLaunchKernelGGL((schwarz_kernel<C1010>), dim3((blk.n + WAVE - 1) / WAVE), dim3(WAVE), 0, s, blk, out);
+    const int G = schwarz_lanes(blk.K), per = WAVE / G;
+    hipLaunchKernelGGL((schwarz_kernel<C1010>), dim3((blk.n + per - 1) / per), dim3(WAVE), 0, s, blk, out, G);
 }
 
 }  // namespace qf

@@ -952,25 +952,42 @@ void fock_tile_kernel(const TileGroup* __restrict__ groups, int ngroups, const T
 }
 
 // ---------------------------------------------------------------------------
-// Schwarz kernel for a diagonal class (La Lb | La Lb): one lane per pair,
-// out[j] = max over components |(ab|ab)| with no screening
+// Schwarz kernel for a diagonal class (La Lb | La Lb): G lanes per pair (a
+// power of two <= 64), out[j] = max over components |(ab|ab)| with no screening
 // (shellcutoff / classcutoff, quick_cutoff_module.f90:91-424).  Used with
 // contracted pairs (Ycutoff) and with single-primitive pairs (cutprim).
+//
+// Each lane of a pair sums the bra primitives [g K/G, (g+1) K/G) against all
+// ket primitives; the contracted accumulators are then summed over the G
+// lanes.  The kernel is bound by one lane's serial chain of K x K primitive
+// quartets (1296 for an O 1s pair of 6-31G): glycine 6-31G**, all (ss|ss)
+// blocks, 0.80 -> 0.10 ms with G = the largest power of two <= K.
 // ---------------------------------------------------------------------------
+inline int schwarz_lanes(int K)
+{
+    int g = 1;
+    while (2 * g <= K && g < WAVE) g *= 2;
+    return g;
+}
+
 template <class C>
-__global__ __launch_bounds__(WAVE) void schwarz_kernel(PairBlock blk, double* __restrict__ out)
+__global__ __launch_bounds__(WAVE) void schwarz_kernel(PairBlock blk, double* __restrict__ out, int G)
 {
     constexpr int na = ncart(C::La), nb = ncart(C::Lb);
     QF_BOYS_LDS_DECL;
     QF_BOYS_LDS_FILL();
-    const int j = blockIdx.x * WAVE + threadIdx.x;
-    if (j >= blk.n) return;
+    const int per = WAVE / G, g = threadIdx.x % G;
+    const int jt = blockIdx.x * per + threadIdx.x / G;
+    const int j = jt < blk.n ? jt : blk.n - 1;   // spare lanes repeat the last pair (every lane joins the sums)
     const PairInfo pi = blk.info[j];
     double acc[C::NACC];
 #pragma unroll
     for (int k = 0; k < C::NACC; ++k) acc[k] = 0.0;
-    contract<C, double, false>(blk, j, pi, blk, j, pi, 0.0, 0.0, false, 2 * pi.qfs, acc, QF_BOYS_LDS_PTR, 0, blk.K, 0,
-                               blk.K);
+    contract<C, double, false>(blk, j, pi, blk, j, pi, 0.0, 0.0, false, 2 * pi.qfs, acc, QF_BOYS_LDS_PTR,
+                               blk.K * g / G, blk.K * (g + 1) / G, 0, blk.K);
+    for (int o = G / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < C::NACC; ++k) acc[k] += __shfl_xor(acc[k], o, WAVE);
     double I[C::NI];
     const double AB[3] = {pi.AB[0], pi.AB[1], pi.AB[2]};
     C::template hrr<double>(acc, AB, AB, I);
@@ -982,7 +999,7 @@ __global__ __launch_bounds__(WAVE) void schwarz_kernel(PairBlock blk, double* __
             const double cons = kCons[C::La][a] * kCons[C::Lb][b];
             m = fmax(m, fabs(I[((a * nb + b) * na + a) * nb + b] * cons * cons));
         }
-    out[j] = m;
+    if (g == 0 && jt < blk.n) out[j] = m;
 }
 
 }  // namespace qf
