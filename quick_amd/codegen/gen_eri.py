@@ -269,14 +269,18 @@ def quartet_classes():
 
 # Classes that get a wave-per-quartet kernel (fock_coop_kernel): the VRR and
 # HRR run as level-scheduled node programs over LDS, so a quartet's
-# intermediates never leave the chip.  Every class with an f shell has only
-# this kernel.
+# intermediates never leave the chip.  Every class with an f shell has one;
+# the f classes above LANE_LSUM_MAX have only this kernel.
 COOP_CLASSES = [(1, 1, 1, 1), (2, 0, 1, 1), (2, 0, 2, 0), (2, 1, 1, 1), (2, 1, 2, 0), (2, 1, 2, 1), (2, 2, 0, 0),
                 (2, 2, 1, 0), (2, 2, 1, 1), (2, 2, 2, 0), (2, 2, 2, 1), (2, 2, 2, 2)]
 COOP_CLASSES += [c for c in quartet_classes() if max(c) == 3]
 
 
-# Classes with La+Lb+Lc+Ld above this get no per-lane kernels: their per-lane
+# Classes with La+Lb+Lc+Ld above this get no per-lane kernels.  The f classes up
+# to it have both forms: one quartet per wave leaves most of its lanes idle
+# where a quartet is small (ethane def2-TZVP, wave per quartet -> per lane:
+# (fs|ss) 0.205 -> 0.11 ms beside the other launches, the build 2.79 -> 2.48).
+# Above it their per-lane
 # forms need several KB of scratch per lane (a (dd|dd) quartet holds 961
 # contracted accumulators), and provisioning that private segment for a
 # full-occupancy launch is what the runtime cannot always do.  Every launch of
@@ -285,7 +289,13 @@ LANE_LSUM_MAX = 5
 
 
 def has_lane_kernels(La, Lb, Lc, Ld):
-    return La + Lb + Lc + Ld <= LANE_LSUM_MAX and max(La, Lb, Lc, Ld) <= 2
+    return La + Lb + Lc + Ld <= LANE_LSUM_MAX
+
+
+def has_fp32_kernels(La, Lb, Lc, Ld):
+    """The classes that mixed builds may split: an f class runs every quartet
+    in FP64."""
+    return has_lane_kernels(La, Lb, Lc, Ld) and max(La, Lb, Lc, Ld) <= 2
 
 
 # Per-workgroup LDS the wave-per-quartet kernel may use; classes whose node
@@ -611,7 +621,7 @@ def gen_class(La, Lb, Lc, Ld):
                                              vrr_flop=vflops, hrr_flop=hflops, nodes=len(vrr.nodes))
 
 
-def launcher_source(name, diag, coop=False, lane=True):
+def launcher_source(name, diag, coop=False, lane=True, fp32=True):
     """Launchers of one class.  ``lane``: the class has per-lane kernels
     (direct FP64 and LDS-tile FP64/FP32); without them every launch of the
     class goes to the wave-per-quartet kernel and its Schwarz diagonal to the
@@ -645,14 +655,17 @@ def launcher_source(name, diag, coop=False, lane=True):
                 "    if (grid <= 0 || grid > ng) grid = ng;",
                 "    const bool lean = (os & 4) != 0;",
                 "    os &= 3;",
-                "    const int k2 = os == 1;",
-                "    if (fp32 && os)",
-                "        hipLaunchKernelGGL((fock_tile_kernel<%s, float, true>), dim3(grid), dim3(waves * WAVE), lds, s,"
-                " g, ng, t, b, m, k2);" % name,
-                "    else if (fp32)",
-                "        hipLaunchKernelGGL((fock_tile_kernel<%s, float>), dim3(grid), dim3(waves * WAVE), lds, s,"
-                " g, ng, t, b, m, 0);" % name,
-                "    else if (os && lean)",
+                "    const int k2 = os == 1;"]
+        out += (["    if (fp32 && os)",
+                 "        hipLaunchKernelGGL((fock_tile_kernel<%s, float, true>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                 " g, ng, t, b, m, k2);" % name,
+                 "    else if (fp32)",
+                 "        hipLaunchKernelGGL((fock_tile_kernel<%s, float>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                 " g, ng, t, b, m, 0);" % name,
+                 "    else if (os && lean)"] if fp32 else
+                ["    (void)fp32;   // f classes are never split",
+                 "    if (os && lean)"])
+        out += [
                 "        hipLaunchKernelGGL((fock_tile_kernel<%s, double, true, true>), dim3(grid), dim3(waves * WAVE), lds,"
                 " s, g, ng, t, b, m, k2);" % name,
                 "    else if (os)",
@@ -724,7 +737,8 @@ def main():
                    "#include \"../qf_coop.h\"\nnamespace qf {\n" + csrc + "}  // namespace qf\n")
         lane = has_lane_kernels(La, Lb, Lc, Ld)
         assert lane or coop, "a class needs per-lane or wave-per-quartet kernels"
-        _write(os.path.join(OUT, "eri_" + name + ".hip"), launcher_source(name, diag, coop, lane))
+        _write(os.path.join(OUT, "eri_" + name + ".hip"), launcher_source(name, diag, coop, lane,
+                                                                           has_fp32_kernels(La, Lb, Lc, Ld)))
         names.append((name, La, Lb, Lc, Ld, diag))
         info["boys_setup_flop"] = boys_setup_flop(La + Lb + Lc + Ld)
         info["prim_flop"] = info["vrr_flop"] + info["boys_setup_flop"]

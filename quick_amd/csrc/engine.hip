@@ -895,7 +895,8 @@ int prepare(qf_engine* e)
                 // to pay (256 batched molecules: 1389 builds/s splitting all,
                 // FP64 1432).
                 const int lmin = e->split_lmin >= 0 ? e->split_lmin : e->nbasis <= 256 ? 5 : 0;
-                const bool split_class = e->prec == QF_PREC_MIXED && mfit >= 1 && lane_class &&
+                const bool f_class = std::max(kClassL[cb][0], kClassL[ck][0]) == 3;   // f classes stay FP64
+                const bool split_class = e->prec == QF_PREC_MIXED && mfit >= 1 && lane_class && !f_class &&
                                          (ct.split >= 0 ? ct.split == 1 : Lsum_s >= lmin);
                 if (fp32 && !split_class) continue;
                 // wave-per-quartet kernel (FP64 launches of classes that have one)

@@ -1,7 +1,43 @@
 // Generated by quick_amd/codegen/gen_eri.py - do not edit.
+#include "C3110.h"
 #include "coop_C3110.h"
 
 namespace qf {
+
+// Direct-atomic launch; FP64 only.  The FP32 instantiation of the direct
+// kernel is not built (it gave wrong Fock matrices on gfx950, cause not
+// found): a request for it is refused with a nonzero return.
+// os: 1 = the fused open-shell pass (second exchange density)
+int launch_fock_C3110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int fp32, int os, int grid, hipStream_t s)
+{
+    if (fp32) return 1;
+    if (nt <= 0) return 0;
+    if (grid <= 0 || grid > nt) grid = nt;
+    if (os)
+        hipLaunchKernelGGL((fock_kernel<C3110, double, true>), dim3(grid), dim3(WAVE), 0, s, t, nt, b, m);
+    else
+        hipLaunchKernelGGL((fock_kernel<C3110, double>), dim3(grid), dim3(WAVE), 0, s, t, nt, b, m);
+    return 0;
+}
+
+// os & 3: 0 closed shell, 1 open shell with a second LDS tile, 2 open
+// shell with the second exchange terms straight to G2; os & 4: the lean
+// open-shell form (FP64; FP32 launches take the register form)
+void launch_fock_tile_C3110(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)
+{
+    if (ng <= 0) return;
+    if (grid <= 0 || grid > ng) grid = ng;
+    const bool lean = (os & 4) != 0;
+    os &= 3;
+    const int k2 = os == 1;
+    (void)fp32;   // f classes are never split
+    if (os && lean)
+        hipLaunchKernelGGL((fock_tile_kernel<C3110, double, true, true>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, k2);
+    else if (os)
+        hipLaunchKernelGGL((fock_tile_kernel<C3110, double, true>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, k2);
+    else
+        hipLaunchKernelGGL((fock_tile_kernel<C3110, double>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, 0);
+}
 
 // gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its
 // slots in global memory (the grid is then capped to that many workgroups)

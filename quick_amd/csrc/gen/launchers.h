@@ -64,15 +64,27 @@ void launch_fock_coop_C2220(const Task*, int, const PairBlock*, const MolDesc*, 
 void launch_fock_coop_C2221(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C2222(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_schwarz_C2222(PairBlock, double*, double*, hipStream_t);
+int launch_fock_C3000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3000(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3010(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3011(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3011(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3011(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3020(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3020(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3020(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3021(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3022(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3030(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_schwarz_C3030(PairBlock, double*, double*, hipStream_t);
+int launch_fock_C3100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3100(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3110(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3120(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
@@ -81,6 +93,8 @@ void launch_fock_coop_C3122(const Task*, int, const PairBlock*, const MolDesc*, 
 void launch_fock_coop_C3130(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3131(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_schwarz_C3131(PairBlock, double*, double*, hipStream_t);
+int launch_fock_C3200(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
+void launch_fock_tile_C3200(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C3200(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3210(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C3211(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
@@ -185,6 +199,13 @@ inline FockLaunch fock_launcher(int cb, int ck)
     if (cb == 4 && ck == 3) return launch_fock_C2120;
     if (cb == 5 && ck == 0) return launch_fock_C2200;
     if (cb == 5 && ck == 1) return launch_fock_C2210;
+    if (cb == 6 && ck == 0) return launch_fock_C3000;
+    if (cb == 6 && ck == 1) return launch_fock_C3010;
+    if (cb == 6 && ck == 2) return launch_fock_C3011;
+    if (cb == 6 && ck == 3) return launch_fock_C3020;
+    if (cb == 7 && ck == 0) return launch_fock_C3100;
+    if (cb == 7 && ck == 1) return launch_fock_C3110;
+    if (cb == 8 && ck == 0) return launch_fock_C3200;
     return nullptr;
 }
 
@@ -206,6 +227,13 @@ inline FockTileLaunch fock_tile_launcher(int cb, int ck)
     if (cb == 4 && ck == 3) return launch_fock_tile_C2120;
     if (cb == 5 && ck == 0) return launch_fock_tile_C2200;
     if (cb == 5 && ck == 1) return launch_fock_tile_C2210;
+    if (cb == 6 && ck == 0) return launch_fock_tile_C3000;
+    if (cb == 6 && ck == 1) return launch_fock_tile_C3010;
+    if (cb == 6 && ck == 2) return launch_fock_tile_C3011;
+    if (cb == 6 && ck == 3) return launch_fock_tile_C3020;
+    if (cb == 7 && ck == 0) return launch_fock_tile_C3100;
+    if (cb == 7 && ck == 1) return launch_fock_tile_C3110;
+    if (cb == 8 && ck == 0) return launch_fock_tile_C3200;
     return nullptr;
 }
 
