@@ -204,46 +204,62 @@ bool side_ready(SideStreams*& side, int device, hipStream_t s)
 // --------------------------------------------------------------------------
 // Device helper kernels
 // --------------------------------------------------------------------------
-__global__ void k_cutmat(const double* __restrict__ P, int n, int nshell, const int* __restrict__ f0,
-                         const int* __restrict__ f1, double* __restrict__ cm)
-{
-    // QUICK's cshell_density_cutoff (cutoff.fh:65-92): max |P_ij| over the
-    // functions of the two original shells.
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nshell * nshell) return;
-    const int I = idx / nshell, J = idx % nshell;
-    double m = 0.0;
-    for (int i = f0[I]; i <= f1[I]; ++i)
-        for (int j = f0[J]; j <= f1[J]; ++j) m = fmax(m, fabs(P[i * n + j]));
-    cm[idx] = m;
-}
+// Opening kernel of a build, in one launch: the descriptors the class kernels
+// read (from the kernel arguments, so a captured build keeps its own), zeroed
+// G accumulators, the density screen matrix and, for an open-shell build, the
+// total and spin densities.  Before, two copies and up to four kernels.
+//
+// Screen matrix: QUICK's cshell_density_cutoff (cutoff.fh:65-92), max |P_ij|
+// over the functions of the two original shells, or, with Pb,
+// oshell_density_cutoff (cutoff.fh:16-89), max of max(|Pa+Pb|, |Pa|, |Pb|).
+struct OpenArgs {
+    qf::MolDesc md, mx;              // descriptors, written to *dmd and *dmx where not null
+    qf::MolDesc *dmd, *dmx;
+    const double *Pa, *Pb;           // densities (Pb null: closed shell)
+    double *Pt, *Ps;                 // open shell: Pa + Pb and Pa - Pb
+    double *G, *G2;                  // ng doubles each to zero (null: none)
+    size_t ng;
+    double* cm;                      // screen matrix to compute (null: the caller's is used)
+    const int *f0, *f1;              // first and last function of every shell
+    int n, nshell;
+};
 
-// QUICK's oshell_density_cutoff (cutoff.fh:16-89): max over the block of
-// max(|Pa+Pb|, |Pa|, |Pb|).
-__global__ void k_cutmat_os(const double* __restrict__ Pa, const double* __restrict__ Pb, int n, int nshell,
-                            const int* __restrict__ f0, const int* __restrict__ f1, double* __restrict__ cm)
+__global__ __launch_bounds__(256) void k_open(const OpenArgs a)
 {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= nshell * nshell) return;
-    const int I = idx / nshell, J = idx % nshell;
-    double m = 0.0;
-    for (int i = f0[I]; i <= f1[I]; ++i)
-        for (int j = f0[J]; j <= f1[J]; ++j) {
-            const double a = Pa[i * n + j], b = Pb[i * n + j];
-            m = fmax(m, fmax(fabs(a + b), fmax(fabs(a), fabs(b))));
+    const size_t first = blockIdx.x * (size_t)blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+    if (first == 0) {
+        if (a.dmd) *a.dmd = a.md;
+        if (a.dmx) *a.dmx = a.mx;
+    }
+    if (a.cm)
+        for (size_t idx = first; idx < (size_t)a.nshell * a.nshell; idx += step) {
+            const int I = (int)(idx / a.nshell), J = (int)(idx % a.nshell);
+            double m = 0.0;
+            for (int i = a.f0[I]; i <= a.f1[I]; ++i)
+                for (int j = a.f0[J]; j <= a.f1[J]; ++j) {
+                    const double p = a.Pa[(size_t)i * a.n + j], q = a.Pb ? a.Pb[(size_t)i * a.n + j] : 0.0;
+                    m = fmax(m, fmax(fabs(p + q), fmax(fabs(p), fabs(q))));
+                }
+            a.cm[idx] = m;
         }
-    cm[idx] = m;
+    if (a.Pt)
+        for (size_t idx = first; idx < (size_t)a.n * a.n; idx += step) {
+            const double p = a.Pa[idx], q = a.Pb[idx];
+            a.Pt[idx] = p + q;
+            a.Ps[idx] = p - q;
+        }
+    if (a.G)
+        for (size_t i = first; i < a.ng; i += step) a.G[i] = 0.0;
+    if (a.G2)
+        for (size_t i = first; i < a.ng; i += step) a.G2[i] = 0.0;
 }
 
-// Total and spin densities of the open-shell build: Pt = Pa + Pb, Ps = Pa - Pb.
-__global__ void k_spin(const double* __restrict__ Pa, const double* __restrict__ Pb, double* __restrict__ Pt,
-                       double* __restrict__ Ps, int n2)
+int open_build(const OpenArgs& a, hipStream_t s)
 {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n2) return;
-    const double a = Pa[idx], b = Pb[idx];
-    Pt[idx] = a + b;
-    Ps[idx] = a - b;
+    const size_t work = std::max((size_t)a.n * a.n, a.G ? a.ng : (size_t)0);
+    const int grid = (int)std::min<size_t>(2048, (work + 255) / 256);
+    hipLaunchKernelGGL(k_open, dim3(grid), dim3(256), 0, s, a);
+    return hipGetLastError() == hipSuccess ? QF_OK : fail(QF_ERR_HIP, "k_open");
 }
 
 __global__ void k_zero(double* __restrict__ p, size_t count)
@@ -386,6 +402,7 @@ struct qf_engine {
         size_t lds_os;   // open-shell pass with a second exchange tile (0: it does not fit)
         int os_split;    // open-shell builds run this class as two closed-shell passes
         int os_lean;     // ... or, on the tile kernel, in the fused lean form
+        size_t gslot;    // first double of its region of the global slot buffer (classes that need one)
     };
     std::vector<Launch> launches;
     std::vector<std::pair<int, int>> order;   // issue order: (launch index, stream 0..kSide)
@@ -417,7 +434,6 @@ struct qf_engine {
     DevBuf<double> d_grad;       // gradient of the host entry point (on first use)
     bool grad_built = false;     // a gradient has run since the last prepare() (counts need it) ...
     bool grad_cm_own = false;    // ... screened with the engine's own Cutmatrix
-    qf::MolDesc mol[4]{};   // slot 0: the build (or open-shell pass 1), slot 1: open-shell pass 2, slot 2: no-alloc build, slot 3: gradient
     // per-launch timing (HIP events on the build stream)
     bool timing = false;
     std::vector<hipEvent_t> ev_pool;
@@ -692,28 +708,45 @@ int prefix_count(const std::vector<qf::PairInfo>& kets, double yi, double thr, b
     return lo;
 }
 
+// Regions of the global slot buffer, one per launch whose node programs keep
+// their slots there (launches on different streams run at the same time), of
+// one slice per workgroup of its grid.  Returns the doubles needed in all.
+size_t place_slots(std::vector<qf_engine::Launch>& launches)
+{
+    size_t total = 0;
+    for (auto& L : launches) {
+        L.gslot = total;
+        if (L.tile == 2)
+            total += (size_t)qf::coop_global_doubles(L.cb, L.ck) * std::min(L.count, qf::COOP_GLOBAL_SLICES);
+    }
+    return total;
+}
+
 // Issue order of class launches and the stream of each: longest first, each
-// to the stream with the least time so far.  The time of a launch is taken
-// as one wave's latency plus its algorithmic FLOPs (every quartet of the
-// windows) at the rate its kernel reaches.  Classes whose node programs keep
-// their slots in the shared global buffer stay on one stream (0).
+// to the stream with the least time so far.  The time of a launch is taken as
+// the larger of its longest task alone and all of its work spread over the
+// GPU, plus a launch: algorithmic FLOPs of every quartet of the windows, at
+// 1.3 GFLOP/s for a wave that works through quartets one by one ((dd|dd)
+// 39 kFLOP in 34 us, (ff|ff) 340 kFLOP in 476 us) and 0.2 GFLOP/s for a lane
+// of the per-lane kernels, and at the 1.2 and 6 TFLOP/s that whole launches
+// reach.
 std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launch>& launches,
                                               const std::vector<qf::Task>& tasks)
 {
-    constexpr double kLatency = 1e-5, kRateCoop = 1.2e12, kRateLane = 6e12;
     const int n = (int)launches.size();
     std::vector<double> t(n);
     for (int l = 0; l < n; ++l) {
         const auto& L = launches[l];
-        double nq = 0.0, np = 0.0;
+        const bool wave = L.tile == 2;
+        double all = 0.0, longest = 0.0;
         for (int x = L.offset; x < L.offset + L.count; ++x) {
             const qf::Task& k = tasks[x];
-            const double q = (double)(k.ke - k.kb) * k.ket_count;
-            if (k.pb == 0 && k.qb == 0) nq += q;
-            np += q * (k.pe - k.pb) * (k.qe - k.qb);
+            const int bras = k.ke - k.kb;
+            const double one = qf::class_flops(L.cb, L.ck, 1, (unsigned long long)(k.pe - k.pb) * (k.qe - k.qb));
+            all += one * bras * k.ket_count;
+            longest = std::max(longest, one * bras * (wave ? k.ket_count : 1));
         }
-        t[l] = kLatency + qf::class_flops(L.cb, L.ck, (unsigned long long)nq, (unsigned long long)np) /
-                              (L.tile == 2 ? kRateCoop : kRateLane);
+        t[l] = 5e-6 + std::max(longest / (wave ? 1.3e9 : 0.2e9), all / (wave ? 1.2e12 : 6e12));
     }
     std::vector<int> ord(n);
     std::iota(ord.begin(), ord.end(), 0);
@@ -721,11 +754,9 @@ std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launc
     double load[kSide + 1] = {};
     std::vector<std::pair<int, int>> out;
     for (int l : ord) {
-        const auto& L = launches[l];
         int to = 0;
-        if (!(L.tile == 2 && qf::coop_global_doubles(L.cb, L.ck) > 0))
-            for (int k = 1; k <= kSide; ++k)
-                if (load[k] < load[to]) to = k;
+        for (int k = 1; k <= kSide; ++k)
+            if (load[k] < load[to]) to = k;
         load[to] += t[l];
         out.push_back({l, to});
     }
@@ -1090,10 +1121,8 @@ int prepare(qf_engine* e)
     e->order = stream_order(e->launches, e->tasks);
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
-    size_t gdoubles = 0;
-    for (const auto& L : e->launches)
-        if (L.tile == 2) gdoubles = std::max<size_t>(gdoubles, (size_t)qf::coop_global_doubles(L.cb, L.ck));
-    if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles * qf::COOP_GLOBAL_SLICES));
+    const size_t gdoubles = place_slots(e->launches);
+    if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles));
 
     // ---- per-build buffers -------------------------------------------------
     const size_t n2 = (size_t)e->nbasis * e->nbasis;
@@ -1213,16 +1242,22 @@ int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<i
     return rc;
 }
 
-// dP2 != nullptr: the open-shell pass.  Every integral is digested with dP
-// (Coulomb and exchange, into Gt) and with dP2 (exchange only, into gb.Gt2);
+// cm_out: where the opening kernel puts the density screen matrix (null: dcm
+// is the caller's).  dPb != nullptr: the open-shell pass.  Every integral is
+// digested with dP (Coulomb and exchange, into Gt) and with the spin density
+// dP2 (exchange only, into gb.Gt2);
 // then dF += A + B and dF2 += A - B (k_finalize_os).  A class with os_split
 // runs as two closed-shell launches instead of the fused one: dP into Gt,
 // then dP2 with a zero Coulomb density (e->d_zero) into Gt2 (descriptor slot
 // 1).
 int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, int slot, hipStream_t s,
-               const GBufs& gb, const double* dP2 = nullptr, double* dF2 = nullptr)
+               const GBufs& gb, double* cm_out, const double* dPa = nullptr, const double* dPb = nullptr,
+               double* dF2 = nullptr)
 {
-    const int os = dP2 != nullptr;
+    // open shell: dPa and dPb are the caller's densities, dP the engine's total
+    // density and e->d_Ps its spin density, both computed by the opening kernel
+    const int os = dPb != nullptr;
+    const double* dP2 = os ? e->d_Ps.p : nullptr;
     if (os && (!gb.Gt2 || !dF || !dF2 || !e->d_zero.p)) return fail(QF_ERR_ARG, "open-shell pass without its buffers");
     const int n = e->nbasis, ns = e->nshell;
     qf::MolDesc md{};
@@ -1239,29 +1274,40 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     md.split = (e->prec == QF_PREC_MIXED) ? e->split_thr : 0.0;
     md.P2 = dP2;
     md.G2 = gb.Gt2;
-    e->mol[slot] = md;
     qf::MolDesc* dmol = e->d_mol.p + slot;
-    QF_HIP(hipMemcpyAsync(dmol, &e->mol[slot], sizeof(md), hipMemcpyHostToDevice, s));
     qf::MolDesc* dmol_x = nullptr;   // exchange-only pass of the two-pass open-shell classes
+    OpenArgs oa{};
+    oa.md = md;
+    oa.dmd = dmol;
     if (os) {
-        qf::MolDesc mx = md;
-        mx.P = dP2;
-        mx.PJ = e->d_zero.p;
-        mx.G = gb.Gt2;
-        mx.P2 = nullptr;
-        mx.G2 = nullptr;
-        e->mol[1] = mx;
-        dmol_x = e->d_mol.p + 1;
-        QF_HIP(hipMemcpyAsync(dmol_x, &e->mol[1], sizeof(mx), hipMemcpyHostToDevice, s));
+        oa.mx = md;
+        oa.mx.P = dP2;
+        oa.mx.PJ = e->d_zero.p;
+        oa.mx.G = gb.Gt2;
+        oa.mx.P2 = nullptr;
+        oa.mx.G2 = nullptr;
+        oa.dmx = dmol_x = e->d_mol.p + 1;
+        oa.Pt = e->d_Pt.p;
+        oa.Ps = e->d_Ps.p;
     }
-    hipLaunchKernelGGL(k_zero, dim3(1024), dim3(256), 0, s, gb.Gt, (size_t)n * n * gb.replicas);
-    if (os) hipLaunchKernelGGL(k_zero, dim3(1024), dim3(256), 0, s, gb.Gt2, (size_t)n * n * gb.replicas);
+    oa.Pa = os ? dPa : dP;
+    oa.Pb = dPb;
+    oa.G = gb.Gt;
+    oa.G2 = os ? gb.Gt2 : nullptr;
+    oa.ng = (size_t)n * n * gb.replicas;
+    oa.cm = cm_out;
+    oa.f0 = e->d_f0.p;
+    oa.f1 = e->d_f1.p;
+    oa.n = n;
+    oa.nshell = ns;
+    const int orc = open_build(oa, s);
+    if (orc) return orc;
     // one class launch with descriptor m on stream q; los: its open-shell form
     auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, hipStream_t q) -> int {
         if (L.tile == 2) {
             qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
             if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
-            fc(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p, q);
+            fc(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p + L.gslot, q);
         } else if (L.tile) {
             qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
             if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
@@ -1317,14 +1363,9 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
 int build(qf_engine* e, const double* dP, double* dF, const double* dcm, hipStream_t s)
 {
     if (!e->prepared) return fail(QF_ERR_STATE, "qf_prepare has not been called");
-    const int n = e->nbasis, ns = e->nshell;
-    if (!dcm) {
-        const int nthr = 256, tot = ns * ns;
-        hipLaunchKernelGGL(k_cutmat, dim3((tot + nthr - 1) / nthr), dim3(nthr), 0, s, dP, n, ns, e->d_f0.p,
-                           e->d_f1.p, e->d_cm.p);
-        dcm = e->d_cm.p;
-    }
-    const int rc = build_pass(e, dP, dcm, dF, 0, s, GBufs{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing, true});
+    double* cm_out = dcm ? nullptr : e->d_cm.p;
+    if (!dcm) dcm = cm_out;
+    const int rc = build_pass(e, dP, dcm, dF, 0, s, GBufs{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing, true}, cm_out);
     if (rc == QF_OK) {
         e->built = true;
         e->count_cm_own = (dcm == e->d_cm.p);
@@ -1345,16 +1386,11 @@ int build_os(qf_engine* e, const double* dPa, const double* dPb, double* dFa, do
              hipStream_t s)
 {
     if (!e->prepared) return fail(QF_ERR_STATE, "qf_prepare has not been called");
-    const int n = e->nbasis, ns = e->nshell, n2 = n * n;
+    const int n2 = e->nbasis * e->nbasis;
     QF_HIP(e->d_Pt.resize(n2));
     QF_HIP(e->d_Ps.resize(n2));
-    hipLaunchKernelGGL(k_spin, dim3((n2 + 255) / 256), dim3(256), 0, s, dPa, dPb, e->d_Pt.p, e->d_Ps.p, n2);
-    if (!dcm) {
-        const int nthr = 256, tot = ns * ns;
-        hipLaunchKernelGGL(k_cutmat_os, dim3((tot + nthr - 1) / nthr), dim3(nthr), 0, s, dPa, dPb, n, ns, e->d_f0.p,
-                           e->d_f1.p, e->d_cm.p);
-        dcm = e->d_cm.p;
-    }
+    double* cm_out = dcm ? nullptr : e->d_cm.p;
+    if (!dcm) dcm = cm_out;
     QF_HIP(e->d_Gt2.resize((size_t)n2 * e->replicas));
     if (e->d_zero.n < (size_t)n2) {
         QF_HIP(e->d_zero.resize(n2));
@@ -1362,7 +1398,7 @@ int build_os(qf_engine* e, const double* dPa, const double* dPb, double* dFa, do
     }
     GBufs gb{e->d_Gt.p, e->replicas, e->d_Gs.p, e->timing, true};
     gb.Gt2 = e->d_Gt2.p;
-    const int rc = build_pass(e, e->d_Pt.p, dcm, dFa, 0, s, gb, e->d_Ps.p, dFb);
+    const int rc = build_pass(e, e->d_Pt.p, dcm, dFa, 0, s, gb, cm_out, dPa, dPb, dFb);
     if (rc == QF_OK) {
         e->built = true;
         e->count_cm_own = (dcm == e->d_cm.p);
@@ -1542,18 +1578,12 @@ int qf_fock_build_device_noalloc(qf_engine* e, const double* d_P, double* d_F, c
         if (L.tile == 2 && qf::coop_global_doubles(L.cb, L.ck) > 0)
             return fail(QF_ERR_ARG, "no-alloc build: a class keeps its node-program slots in global memory");
     const hipStream_t s = (hipStream_t)stream;
-    const int n = e->nbasis, ns = e->nshell;
     // scratch layout: [G partials n^2 | symmetrised G n^2 | Cutmatrix nshell^2]
     double* Gt = base;
     double* Gs = base + n2;
-    if (!d_cutmat) {
-        double* cm = base + 2 * n2;
-        const int nthr = 256, tot = ns * ns;
-        hipLaunchKernelGGL(k_cutmat, dim3((tot + nthr - 1) / nthr), dim3(nthr), 0, s, d_P, n, ns, e->d_f0.p,
-                           e->d_f1.p, cm);
-        d_cutmat = cm;
-    }
-    return build_pass(e, d_P, d_cutmat, d_F, 2, s, GBufs{Gt, 1, Gs, false, false});
+    double* cm_out = d_cutmat ? nullptr : base + 2 * n2;
+    if (!d_cutmat) d_cutmat = cm_out;
+    return build_pass(e, d_P, d_cutmat, d_F, 2, s, GBufs{Gt, 1, Gs, false, false}, cm_out);
 }
 
 // Two-electron gradient (QUICK's gpu_get_cshell_eri_grad_ -> getGrad,
@@ -1563,7 +1593,7 @@ int qf_fock_build_device_noalloc(qf_engine* e, const double* d_P, double* d_F, c
 namespace {
 constexpr size_t kGradLdsMax = 64 * 1024;   // dynamic LDS of one gradient workgroup
 
-int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* dgrad, hipStream_t s)
+int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out, double* dgrad, hipStream_t s)
 {
     // every class needs a gradient kernel: check before launching anything
     size_t gdoubles = 0;
@@ -1589,9 +1619,18 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* dgrad, 
     md.natom = e->natom;
     md.shell_atom = e->d_shell_atom.p;
     md.grad = dgrad;
-    e->mol[3] = md;
     qf::MolDesc* dmol = e->d_mol.p + 3;
-    QF_HIP(hipMemcpyAsync(dmol, &e->mol[3], sizeof(md), hipMemcpyHostToDevice, s));
+    OpenArgs oa{};
+    oa.md = md;
+    oa.dmd = dmol;
+    oa.Pa = dP;
+    oa.cm = cm_out;
+    oa.f0 = e->d_f0.p;
+    oa.f1 = e->d_f1.p;
+    oa.n = e->nbasis;
+    oa.nshell = e->nshell;
+    const int orc = open_build(oa, s);
+    if (orc) return orc;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
     for (size_t li = 0; li < e->launches.size(); ++li) {
         const auto& L = e->launches[li];
@@ -1656,14 +1695,9 @@ int qf_eri_grad_device(qf_engine* e, const double* d_P, double* d_grad, const do
     if (rc) return rc;
     if (!e->prepared) return fail(QF_ERR_STATE, "qf_prepare has not been called");
     const hipStream_t s = (hipStream_t)stream;
-    const double* dcm = d_cutmat;
-    if (!dcm) {
-        const int nthr = 256, tot = e->nshell * e->nshell;
-        hipLaunchKernelGGL(k_cutmat, dim3((tot + nthr - 1) / nthr), dim3(nthr), 0, s, d_P, e->nbasis, e->nshell,
-                           e->d_f0.p, e->d_f1.p, e->d_cm.p);
-        dcm = e->d_cm.p;
-    }
-    rc = grad_pass(e, d_P, dcm, d_grad, s);
+    double* cm_out = d_cutmat ? nullptr : e->d_cm.p;
+    const double* dcm = d_cutmat ? d_cutmat : cm_out;
+    rc = grad_pass(e, d_P, dcm, cm_out, d_grad, s);
     if (rc == QF_OK) {
         e->grad_built = true;
         e->grad_cm_own = (dcm == e->d_cm.p);
@@ -2091,7 +2125,7 @@ int batch_issue(qf_batch* b, hipStream_t s)
         if (L.tile == 2) {
             qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
             if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
-            fc(b->d_tasks.p + L.offset, L.count, b->d_blocks.p, b->d_moldesc.p, 0, b->persist, b->d_cscratch.p, q);
+            fc(b->d_tasks.p + L.offset, L.count, b->d_blocks.p, b->d_moldesc.p, 0, b->persist, b->d_cscratch.p + L.gslot, q);
         } else if (L.tile) {
             qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
             if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
@@ -2277,10 +2311,8 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
                     }
                     b->launches.push_back(C);
                 }
-    size_t gdoubles = 0;
-    for (const auto& L : b->launches)
-        if (L.tile == 2) gdoubles = std::max<size_t>(gdoubles, (size_t)qf::coop_global_doubles(L.cb, L.ck));
-    if (gdoubles && b->d_cscratch.resize(gdoubles * qf::COOP_GLOBAL_SLICES) != hipSuccess)
+    const size_t gdoubles = place_slots(b->launches);
+    if (gdoubles && b->d_cscratch.resize(gdoubles) != hipSuccess)
         return bail(fail(QF_ERR_MEMORY, "batch global slot buffer"));
     if (b->d_blocks.upload(blocks) != hipSuccess || b->d_tasks.upload(tasks) != hipSuccess ||
         b->d_groups.upload(groups) != hipSuccess || b->d_moldesc.upload(md) != hipSuccess ||
