@@ -763,6 +763,284 @@ std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launc
     return out;
 }
 
+// Wave tasks, tile groups and launches of one engine, per quartet class and
+// precision.  `size` stands for the number of basis functions in the rules
+// that choose launch shapes: the engine's own, or for an engine in a batch
+// that of the molecule whose build holds as much work (the precision split
+// goes by the engine's own size).  Index ranges are those of the output vectors.
+int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::vector<qf::TileGroup>& groups,
+               std::vector<qf_engine::Launch>& launches, qf_stats* stats)
+{
+    const double thr_hi = e->split_thr;
+    tasks.clear();
+    groups.clear();
+    launches.clear();
+    // Primitive pieces: a wave's lanes each run the whole primitive loop of
+    // one quartet, so the most contracted quartets set the tail of a launch
+    // (and, for small molecules with few waves, its whole time).  The
+    // primitive pairs of a task are cut into pieces of at most 1 up to 96
+    // functions, 2 up to 128, 4 up to 256 and 12 above (e.g. 36 -> 3 x 12).
+    // Measured on (H2O)32 6-31G(d): no split 17.0 ms, pieces of 6 / 12 / 18:
+    // 15.8 / 15.4 / 15.9 ms; on QUICK's 69 regression inputs (12-210
+    // functions), geometric mean of the build times up to 32 functions with
+    // pieces of 1 / 2: 0.39 / 0.55 ms, 33-64: 0.93 / 1.23 ms, 79 functions
+    // 2.20 / 2.49 ms, 114: 2.02 / 1.50 ms, 210 (pieces of 1 / 4): 5.53 /
+    // 4.57 ms.  A small molecule has too few quartets to fill the GPU, and
+    // one primitive quartet per lane gives it the most waves.
+    const int piece = e->prim_piece > 0   ? e->prim_piece
+                      : e->prim_piece < 0 ? 1 << 20
+                      : size <= 96   ? 1
+                      : size <= 128  ? 2
+                      : size <= 256  ? 4
+                                          : 12;
+    for (int cb = 0; cb < kNPC; ++cb)
+        for (int ck = 0; ck <= cb; ++ck)
+            for (int fp32 = 0; fp32 < 2; ++fp32) {
+                const int offset = (int)tasks.size();
+                const int goffset = (int)groups.size();
+                const int na = ncart(kClassL[cb][0]), nb = ncart(kClassL[cb][1]);
+                // bras per task: long loops for cheap classes (more register
+                // accumulation, fewer atomics), short ones for expensive classes
+                // (enough waves to fill 256 CUs)
+                const int ni = na * nb * ncart(kClassL[ck][0]) * ncart(kClassL[ck][1]);
+                const qf_engine::ClassTune& ct = e->ctune[cb][ck];
+                int mmax = ni <= 10 ? 16 : ni <= 36 ? 8 : ni <= 108 ? 4 : ni <= 324 ? 2 : 1;
+                // up to 32 functions at most 2 bras per task: more, shorter
+                // tasks for launches that hold few (QUICK's regression inputs
+                // up to 32 functions, geometric mean 16.3x -> 17.8x QUICK's
+                // saved build times; no gain above)
+                if (size <= 32) mmax = std::min(mmax, 2);
+                if (ct.mmax > 0) mmax = ct.mmax;
+                // tasks per tile workgroup: few for molecules up to 256
+                // functions, whose launches hold few tasks (QUICK's 69
+                // regression inputs, light classes with 1 / 2 / 4 / 8 / 16
+                // tasks per group: 15.7x / 16.5x / 16.5x / 13.9x / 10.4x
+                // QUICK's saved build times, geometric mean)
+                const int tile_tasks = ct.tpg > 0        ? ct.tpg
+                                       : e->tile_tasks > 0 ? e->tile_tasks
+                                       : size <= 256  ? 4
+                                                           : 16;
+                const int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
+                // LDS tile: (na + m*nb) x ncol exchange terms + m*na*nb Coulomb terms
+                int maxcol = 0;
+                for (const auto& Kb : e->blocks)
+                    if (Kb.cls == ck) maxcol = std::max(maxcol, (int)Kb.colf.size());
+                const long long room = e->lds_budget / 8 - (long long)na * maxcol;
+                const long long mfit = room > 0 ? room / ((long long)nb * maxcol + na * nb) : 0;
+                // Mixed precision splits a class only where its FP32 half can run
+                // through the LDS-tile kernel: the direct-atomic FP32 kernels of
+                // (dp|dp) gave wrong Fock matrices on gfx950 and the (dd|dp) one
+                // non-finite values, while CPU builds of the same code are right.
+                // (dd|dp) and (dd|dd) stay FP64 (their FP32 forms spill several KB
+                // per lane: little to gain).
+                // classes without per-lane kernels (La+Lb+Lc+Ld >= 6) run every
+                // quartet in FP64 on the wave-per-quartet kernel
+                const bool lane_class = qf::fock_launcher(cb, ck) != nullptr;
+                // Classes with La+Lb+Lc+Ld >= split_lmin are split (qf_set_split_classes).
+                // FP32 quartets compute their Boys function, exponents and
+                // recursions in FP32, which shortens the primitive loop (the
+                // FP64 Boys function is most of a light class's work) and halves
+                // the registers of the spilling d classes.
+                const int Lsum_s = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
+                // By default every class above 256 functions, and only the
+                // classes with La+Lb+Lc+Ld >= 5 below: a small molecule's
+                // light classes hold too few quartets for the second launch
+                // to pay (256 batched molecules: 1389 builds/s splitting all,
+                // FP64 1432).
+                const int lmin = e->split_lmin >= 0 ? e->split_lmin : e->nbasis <= 256 ? 5 : 0;
+                const bool f_class = std::max(kClassL[cb][0], kClassL[ck][0]) == 3;   // f classes stay FP64
+                const bool split_class = e->prec == QF_PREC_MIXED && mfit >= 1 && lane_class && !f_class &&
+                                         (ct.split >= 0 ? ct.split == 1 : Lsum_s >= lmin);
+                if (fp32 && !split_class) continue;
+                // wave-per-quartet kernel (FP64 launches of classes that have one)
+                // wave-per-quartet kernel: where the class tuning asks for it, and by
+                // default (unless qf_set_tile turned the shared-memory kernels off)
+                // for the d-heavy classes (La+Lb+Lc+Ld >= 6; >= 5 up to 128 functions and >= 4 up to 48,
+                // where few waves run and latency decides), whose per-lane
+                // kernels spill several KB per lane: one such quartet alone on a
+                // lane costs milliseconds, which dominates the build of a small
+                // molecule
+                const int Lsum = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
+                // (QUICK's regression inputs of 49-128 functions run their
+                // La+Lb+Lc+Ld = 4 classes faster on the tile kernel: PO4 6-31G*
+                // 15.8x -> 18.0x, PSB5 6-31G 26x -> 34x QUICK's build times;
+                // up to 48 functions and at 5 the wave-per-quartet kernel wins)
+                const int coop_lmin = size <= 48 ? 4 : size <= 128 ? 5 : 6;
+                const bool want_coop = !lane_class || ct.tile == 2 || (ct.tile < 0 && e->tile != 0 && Lsum >= coop_lmin);
+                const bool coop = !fp32 && want_coop && qf::fock_coop_launcher(cb, ck) != nullptr;
+                if (!coop && !lane_class) return fail(QF_ERR_STATE, "class has neither per-lane nor wave-per-quartet kernels");
+                const bool tile = !coop && (fp32 || (ct.tile >= 0 ? ct.tile != 0 : e->tile != 0)) && mfit >= 1;
+                if (tile) mmax = (int)std::min<long long>(mmax, mfit);
+                // kets per task: a full wave for the per-lane kernels; for the
+                // wave-per-quartet kernel a window (the class tuning's
+                // tasks_per_group): small windows give more workgroups to
+                // classes with few quartets
+                const int coop_win = size <= 256 ? 1 : kCoopWindow;
+                const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_win) : qf::WAVE;
+                size_t lds = 0, lds_os = 0;
+                long long group_tasks = 0;
+                for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
+                    const HostBlock& B = e->blocks[bbk];
+                    if (B.cls != cb) continue;
+                    for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
+                        const HostBlock& Kb = e->blocks[kbk];
+                        if (Kb.cls != ck) continue;
+                        if (cb == ck && kbk > bbk) continue;
+                        const bool same = (cb == ck && kbk == bbk);
+                        std::vector<std::pair<int, int>> chunks;
+                        for (const auto& g : B.groups)
+                            for (int c0 = g.first; c0 < g.second; c0 += mmax)
+                                chunks.push_back({c0, std::min(g.second, c0 + mmax)});
+                        for (const auto& g : chunks) {
+                            // per bra of the group: ket range [lo, hi) of this precision
+                            const int M = g.second - g.first;
+                            std::vector<int> lo(M), hi(M);
+                            int nmax = 0;
+                            for (int k = 0; k < M; ++k) {
+                                const int i = B.bperm[g.first + k];
+                                const double yi = B.info[i].ycut;
+                                int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
+                                if (same) n = std::min(n, i + 1);
+                                if (!fp32 && stats) stats->n_quartets_bound += n;
+                                int n64 = n;
+                                if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
+                                lo[k] = fp32 ? n64 : 0;
+                                hi[k] = fp32 ? n : n64;
+                                nmax = std::max(nmax, hi[k]);
+                            }
+                            const int chunk_first = (int)tasks.size();
+                            for (int s0 = 0; s0 < nmax; s0 += win) {
+                                int kb = -1, ke = -1;
+                                for (int k = 0; k < M; ++k)
+                                    if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
+                                        if (kb < 0) kb = k;
+                                        ke = k + 1;
+                                    }
+                                if (kb < 0) continue;
+                                qf::Task t{};
+                                t.bra_block = (int)bbk;
+                                t.kb = g.first + kb;
+                                t.ke = g.first + ke;
+                                t.ket_block = (int)kbk;
+                                t.ket_start = s0;
+                                t.ket_count = std::min(win, nmax - s0);
+                                t.same_block = same ? 1 : 0;
+                                t.all_fp64 = split_class ? 0 : 1;
+                                // highly contracted pairs: spread the primitive
+                                // pairs of the window over several tasks
+                                const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
+                                const int nbp = (B.K + cpiece - 1) / cpiece, nkp = (Kb.K + cpiece - 1) / cpiece;
+                                const int sb = (B.K + nbp - 1) / nbp, sk = (Kb.K + nkp - 1) / nkp;
+                                for (int pbi = 0; pbi < B.K; pbi += sb)
+                                    for (int qbi = 0; qbi < Kb.K; qbi += sk) {
+                                        t.pb = pbi;
+                                        t.pe = std::min(B.K, pbi + sb);
+                                        t.qb = qbi;
+                                        t.qe = std::min(Kb.K, qbi + sk);
+                                        tasks.push_back(t);
+                                    }
+                            }
+                            if (!tile) continue;
+                            // workgroups of the chunk: consecutive runs of its tasks
+                            const int chunk_end = (int)tasks.size();
+                            for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
+                                qf::TileGroup tg{};
+                                tg.task_begin = t0;
+                                tg.task_end = std::min(chunk_end, t0 + tile_tasks);
+                                tg.chunk_kb = g.first;
+                                tg.nbra = M;
+                                groups.push_back(tg);
+                                group_tasks += tg.task_end - tg.task_begin;
+                            }
+                            if (chunk_end > chunk_first) {
+                                const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
+                                lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
+                                lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
+                            }
+                        }
+                    }
+                }
+                const int count = (int)tasks.size() - offset;
+                const int gcount = (int)groups.size() - goffset;
+                // work of a task: bras x kets x primitive pairs (bra and ket);
+                // without the primitive factor the longest-first order misjudges
+                // the contracted classes (13 % of the (H2O)32 build)
+                auto cost = [](const qf::Task& x) {
+                    return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
+                };
+                if (tile && gcount > 0) {
+                    // longest workgroups first so the launch ends evenly
+                    std::vector<long long> gc(gcount, 0);
+                    for (int q = 0; q < gcount; ++q) {
+                        const auto& tg = groups[goffset + q];
+                        for (int x = tg.task_begin; x < tg.task_end; ++x) gc[q] += cost(tasks[x]);
+                    }
+                    std::vector<int> ord(gcount);
+                    std::iota(ord.begin(), ord.end(), 0);
+                    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return gc[x] > gc[y]; });
+                    std::vector<qf::TileGroup> sorted(gcount);
+                    for (int q = 0; q < gcount; ++q) sorted[q] = groups[goffset + ord[q]];
+                    std::copy(sorted.begin(), sorted.end(), groups.begin() + goffset);
+                } else if (e->shuffle && count > 1) {
+                    // deterministic permutation (concurrent waves then hit different
+                    // kets), then longest tasks first so the launch ends evenly
+                    uint64_t st = 0x9E3779B97F4A7C15ull ^ (uint64_t)(cb * 12 + ck * 2 + fp32);
+                    for (int q = count - 1; q > 0; --q) {
+                        st ^= st << 13;
+                        st ^= st >> 7;
+                        st ^= st << 17;
+                        const int r = (int)(st % (uint64_t)(q + 1));
+                        std::swap(tasks[offset + q], tasks[offset + r]);
+                    }
+                    std::stable_sort(tasks.begin() + offset, tasks.end(),
+                                     [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
+                }
+                if (count > 0) {
+                    qf_engine::Launch L{};
+                    L.cb = cb;
+                    L.ck = ck;
+                    L.fp32 = fp32;
+                    L.offset = offset;
+                    L.count = count;
+                    L.tile = coop ? 2 : (tile && gcount > 0) ? 1 : 0;
+                    L.goffset = goffset;
+                    L.gcount = gcount;
+                    L.waves = gcount > 0 ? (int)std::min<long long>(tile_waves,
+                                                                  std::max<long long>(1, (group_tasks + gcount - 1) / gcount))
+                                         : 1;
+                    L.lds = lds;
+                    L.lds_os = lds_os <= kMaxTileLds ? lds_os : 0;
+                    L.os_split = ct.os == 1;
+                    L.os_lean = ct.os == 2 || ct.os < 0;
+                    launches.push_back(L);
+                }
+                if (stats) (fp32 ? stats->n_tasks_fp32 : stats->n_tasks_fp64) += count;
+            }
+    // every tile workgroup must stay inside its chunk and its LDS allocation
+    for (const auto& L : launches) {
+        if (L.tile != 1) continue;
+        const int na = ncart(kClassL[L.cb][0]), nb = ncart(kClassL[L.cb][1]);
+        for (int q = L.goffset; q < L.goffset + L.gcount; ++q) {
+            const qf::TileGroup& g = groups[q];
+            if (g.task_begin < L.offset || g.task_end > L.offset + L.count || g.task_begin >= g.task_end)
+                return fail(QF_ERR_STATE, "tile group outside its launch");
+            const qf::Task& t0 = tasks[g.task_begin];
+            const size_t need = sizeof(double) * ((size_t)(na + g.nbra * nb) * e->blocks[t0.ket_block].colf.size() +
+                                                  (size_t)g.nbra * na * nb);
+            if (need > L.lds) return fail(QF_ERR_STATE, "tile group exceeds its LDS allocation");
+            if (L.lds_os && 2 * need - sizeof(double) * (size_t)g.nbra * na * nb > L.lds_os)
+                return fail(QF_ERR_STATE, "tile group exceeds its open-shell LDS allocation");
+            for (int x = g.task_begin; x < g.task_end; ++x) {
+                const qf::Task& t = tasks[x];
+                if (t.bra_block != t0.bra_block || t.ket_block != t0.ket_block || t.kb < g.chunk_kb ||
+                    t.ke > g.chunk_kb + g.nbra || t.kb >= t.ke)
+                    return fail(QF_ERR_STATE, "tile group mixes chunks");
+            }
+        }
+    }
+    return QF_OK;
+}
+
 int prepare(qf_engine* e)
 {
     if (e->prepared) return QF_OK;   // idempotent: setters clear the flag
@@ -846,276 +1124,11 @@ int prepare(qf_engine* e)
     QF_HIP(e->d_blocks.upload(e->hblocks));
 
     // ---- wave tasks per quartet class and precision ------------------------
-    const double thr_hi = e->split * ymax * ymax;
-    e->split_thr = thr_hi;
-    e->tasks.clear();
-    e->groups.clear();
-    e->launches.clear();
+    e->split_thr = e->split * ymax * ymax;
     e->stats = qf_stats{};
     for (auto& b : e->blocks) e->stats.n_pairs += (long long)b.info.size();
-    // Primitive pieces: a wave's lanes each run the whole primitive loop of
-    // one quartet, so the most contracted quartets set the tail of a launch
-    // (and, for small molecules with few waves, its whole time).  The
-    // primitive pairs of a task are cut into pieces of at most 1 up to 96
-    // functions, 2 up to 128, 4 up to 256 and 12 above (e.g. 36 -> 3 x 12).
-    // Measured on (H2O)32 6-31G(d): no split 17.0 ms, pieces of 6 / 12 / 18:
-    // 15.8 / 15.4 / 15.9 ms; on QUICK's 69 regression inputs (12-210
-    // functions), geometric mean of the build times up to 32 functions with
-    // pieces of 1 / 2: 0.39 / 0.55 ms, 33-64: 0.93 / 1.23 ms, 79 functions
-    // 2.20 / 2.49 ms, 114: 2.02 / 1.50 ms, 210 (pieces of 1 / 4): 5.53 /
-    // 4.57 ms.  A small molecule has too few quartets to fill the GPU, and
-    // one primitive quartet per lane gives it the most waves.
-    const int piece = e->prim_piece > 0   ? e->prim_piece
-                      : e->prim_piece < 0 ? 1 << 20
-                      : e->nbasis <= 96   ? 1
-                      : e->nbasis <= 128  ? 2
-                      : e->nbasis <= 256  ? 4
-                                          : 12;
-    for (int cb = 0; cb < kNPC; ++cb)
-        for (int ck = 0; ck <= cb; ++ck)
-            for (int fp32 = 0; fp32 < 2; ++fp32) {
-                const int offset = (int)e->tasks.size();
-                const int goffset = (int)e->groups.size();
-                const int na = ncart(kClassL[cb][0]), nb = ncart(kClassL[cb][1]);
-                // bras per task: long loops for cheap classes (more register
-                // accumulation, fewer atomics), short ones for expensive classes
-                // (enough waves to fill 256 CUs)
-                const int ni = na * nb * ncart(kClassL[ck][0]) * ncart(kClassL[ck][1]);
-                const qf_engine::ClassTune& ct = e->ctune[cb][ck];
-                int mmax = ni <= 10 ? 16 : ni <= 36 ? 8 : ni <= 108 ? 4 : ni <= 324 ? 2 : 1;
-                // up to 32 functions at most 2 bras per task: more, shorter
-                // tasks for launches that hold few (QUICK's regression inputs
-                // up to 32 functions, geometric mean 16.3x -> 17.8x QUICK's
-                // saved build times; no gain above)
-                if (e->nbasis <= 32) mmax = std::min(mmax, 2);
-                if (ct.mmax > 0) mmax = ct.mmax;
-                // tasks per tile workgroup: few for molecules up to 256
-                // functions, whose launches hold few tasks (QUICK's 69
-                // regression inputs, light classes with 1 / 2 / 4 / 8 / 16
-                // tasks per group: 15.7x / 16.5x / 16.5x / 13.9x / 10.4x
-                // QUICK's saved build times, geometric mean)
-                const int tile_tasks = ct.tpg > 0        ? ct.tpg
-                                       : e->tile_tasks > 0 ? e->tile_tasks
-                                       : e->nbasis <= 256  ? 4
-                                                           : 16;
-                const int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
-                // LDS tile: (na + m*nb) x ncol exchange terms + m*na*nb Coulomb terms
-                int maxcol = 0;
-                for (const auto& Kb : e->blocks)
-                    if (Kb.cls == ck) maxcol = std::max(maxcol, (int)Kb.colf.size());
-                const long long room = e->lds_budget / 8 - (long long)na * maxcol;
-                const long long mfit = room > 0 ? room / ((long long)nb * maxcol + na * nb) : 0;
-                // Mixed precision splits a class only where its FP32 half can run
-                // through the LDS-tile kernel: the direct-atomic FP32 kernels of
-                // (dp|dp) gave wrong Fock matrices on gfx950 and the (dd|dp) one
-                // non-finite values, while CPU builds of the same code are right.
-                // (dd|dp) and (dd|dd) stay FP64 (their FP32 forms spill several KB
-                // per lane: little to gain).
-                // classes without per-lane kernels (La+Lb+Lc+Ld >= 6) run every
-                // quartet in FP64 on the wave-per-quartet kernel
-                const bool lane_class = qf::fock_launcher(cb, ck) != nullptr;
-                // Classes with La+Lb+Lc+Ld >= split_lmin are split (qf_set_split_classes).
-                // FP32 quartets compute their Boys function, exponents and
-                // recursions in FP32, which shortens the primitive loop (the
-                // FP64 Boys function is most of a light class's work) and halves
-                // the registers of the spilling d classes.
-                const int Lsum_s = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
-                // By default every class above 256 functions, and only the
-                // classes with La+Lb+Lc+Ld >= 5 below: a small molecule's
-                // light classes hold too few quartets for the second launch
-                // to pay (256 batched molecules: 1389 builds/s splitting all,
-                // FP64 1432).
-                const int lmin = e->split_lmin >= 0 ? e->split_lmin : e->nbasis <= 256 ? 5 : 0;
-                const bool f_class = std::max(kClassL[cb][0], kClassL[ck][0]) == 3;   // f classes stay FP64
-                const bool split_class = e->prec == QF_PREC_MIXED && mfit >= 1 && lane_class && !f_class &&
-                                         (ct.split >= 0 ? ct.split == 1 : Lsum_s >= lmin);
-                if (fp32 && !split_class) continue;
-                // wave-per-quartet kernel (FP64 launches of classes that have one)
-                // wave-per-quartet kernel: where the class tuning asks for it, and by
-                // default (unless qf_set_tile turned the shared-memory kernels off)
-                // for the d-heavy classes (La+Lb+Lc+Ld >= 6; >= 5 up to 128 functions and >= 4 up to 48,
-                // where few waves run and latency decides), whose per-lane
-                // kernels spill several KB per lane: one such quartet alone on a
-                // lane costs milliseconds, which dominates the build of a small
-                // molecule
-                const int Lsum = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
-                // (QUICK's regression inputs of 49-128 functions run their
-                // La+Lb+Lc+Ld = 4 classes faster on the tile kernel: PO4 6-31G*
-                // 15.8x -> 18.0x, PSB5 6-31G 26x -> 34x QUICK's build times;
-                // up to 48 functions and at 5 the wave-per-quartet kernel wins)
-                const int coop_lmin = e->nbasis <= 48 ? 4 : e->nbasis <= 128 ? 5 : 6;
-                const bool want_coop = !lane_class || ct.tile == 2 || (ct.tile < 0 && e->tile != 0 && Lsum >= coop_lmin);
-                const bool coop = !fp32 && want_coop && qf::fock_coop_launcher(cb, ck) != nullptr;
-                if (!coop && !lane_class) return fail(QF_ERR_STATE, "class has neither per-lane nor wave-per-quartet kernels");
-                const bool tile = !coop && (fp32 || (ct.tile >= 0 ? ct.tile != 0 : e->tile != 0)) && mfit >= 1;
-                if (tile) mmax = (int)std::min<long long>(mmax, mfit);
-                // kets per task: a full wave for the per-lane kernels; for the
-                // wave-per-quartet kernel a window (the class tuning's
-                // tasks_per_group): small windows give more workgroups to
-                // classes with few quartets
-                const int coop_win = e->nbasis <= 256 ? 1 : kCoopWindow;
-                const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_win) : qf::WAVE;
-                size_t lds = 0, lds_os = 0;
-                long long group_tasks = 0;
-                for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
-                    const HostBlock& B = e->blocks[bbk];
-                    if (B.cls != cb) continue;
-                    for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
-                        const HostBlock& Kb = e->blocks[kbk];
-                        if (Kb.cls != ck) continue;
-                        if (cb == ck && kbk > bbk) continue;
-                        const bool same = (cb == ck && kbk == bbk);
-                        std::vector<std::pair<int, int>> chunks;
-                        for (const auto& g : B.groups)
-                            for (int c0 = g.first; c0 < g.second; c0 += mmax)
-                                chunks.push_back({c0, std::min(g.second, c0 + mmax)});
-                        for (const auto& g : chunks) {
-                            // per bra of the group: ket range [lo, hi) of this precision
-                            const int M = g.second - g.first;
-                            std::vector<int> lo(M), hi(M);
-                            int nmax = 0;
-                            for (int k = 0; k < M; ++k) {
-                                const int i = B.bperm[g.first + k];
-                                const double yi = B.info[i].ycut;
-                                int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
-                                if (same) n = std::min(n, i + 1);
-                                if (!fp32) e->stats.n_quartets_bound += n;
-                                int n64 = n;
-                                if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
-                                lo[k] = fp32 ? n64 : 0;
-                                hi[k] = fp32 ? n : n64;
-                                nmax = std::max(nmax, hi[k]);
-                            }
-                            const int chunk_first = (int)e->tasks.size();
-                            for (int s0 = 0; s0 < nmax; s0 += win) {
-                                int kb = -1, ke = -1;
-                                for (int k = 0; k < M; ++k)
-                                    if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
-                                        if (kb < 0) kb = k;
-                                        ke = k + 1;
-                                    }
-                                if (kb < 0) continue;
-                                qf::Task t{};
-                                t.bra_block = (int)bbk;
-                                t.kb = g.first + kb;
-                                t.ke = g.first + ke;
-                                t.ket_block = (int)kbk;
-                                t.ket_start = s0;
-                                t.ket_count = std::min(win, nmax - s0);
-                                t.same_block = same ? 1 : 0;
-                                t.all_fp64 = split_class ? 0 : 1;
-                                // highly contracted pairs: spread the primitive
-                                // pairs of the window over several tasks
-                                const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
-                                const int nbp = (B.K + cpiece - 1) / cpiece, nkp = (Kb.K + cpiece - 1) / cpiece;
-                                const int sb = (B.K + nbp - 1) / nbp, sk = (Kb.K + nkp - 1) / nkp;
-                                for (int pbi = 0; pbi < B.K; pbi += sb)
-                                    for (int qbi = 0; qbi < Kb.K; qbi += sk) {
-                                        t.pb = pbi;
-                                        t.pe = std::min(B.K, pbi + sb);
-                                        t.qb = qbi;
-                                        t.qe = std::min(Kb.K, qbi + sk);
-                                        e->tasks.push_back(t);
-                                    }
-                            }
-                            if (!tile) continue;
-                            // workgroups of the chunk: consecutive runs of its tasks
-                            const int chunk_end = (int)e->tasks.size();
-                            for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
-                                qf::TileGroup tg{};
-                                tg.task_begin = t0;
-                                tg.task_end = std::min(chunk_end, t0 + tile_tasks);
-                                tg.chunk_kb = g.first;
-                                tg.nbra = M;
-                                e->groups.push_back(tg);
-                                group_tasks += tg.task_end - tg.task_begin;
-                            }
-                            if (chunk_end > chunk_first) {
-                                const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
-                                lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
-                                lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
-                            }
-                        }
-                    }
-                }
-                const int count = (int)e->tasks.size() - offset;
-                const int gcount = (int)e->groups.size() - goffset;
-                // work of a task: bras x kets x primitive pairs (bra and ket);
-                // without the primitive factor the longest-first order misjudges
-                // the contracted classes (13 % of the (H2O)32 build)
-                auto cost = [](const qf::Task& x) {
-                    return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
-                };
-                if (tile && gcount > 0) {
-                    // longest workgroups first so the launch ends evenly
-                    std::vector<long long> gc(gcount, 0);
-                    for (int q = 0; q < gcount; ++q) {
-                        const auto& tg = e->groups[goffset + q];
-                        for (int x = tg.task_begin; x < tg.task_end; ++x) gc[q] += cost(e->tasks[x]);
-                    }
-                    std::vector<int> ord(gcount);
-                    std::iota(ord.begin(), ord.end(), 0);
-                    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return gc[x] > gc[y]; });
-                    std::vector<qf::TileGroup> sorted(gcount);
-                    for (int q = 0; q < gcount; ++q) sorted[q] = e->groups[goffset + ord[q]];
-                    std::copy(sorted.begin(), sorted.end(), e->groups.begin() + goffset);
-                } else if (e->shuffle && count > 1) {
-                    // deterministic permutation (concurrent waves then hit different
-                    // kets), then longest tasks first so the launch ends evenly
-                    uint64_t st = 0x9E3779B97F4A7C15ull ^ (uint64_t)(cb * 12 + ck * 2 + fp32);
-                    for (int q = count - 1; q > 0; --q) {
-                        st ^= st << 13;
-                        st ^= st >> 7;
-                        st ^= st << 17;
-                        const int r = (int)(st % (uint64_t)(q + 1));
-                        std::swap(e->tasks[offset + q], e->tasks[offset + r]);
-                    }
-                    std::stable_sort(e->tasks.begin() + offset, e->tasks.end(),
-                                     [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
-                }
-                if (count > 0) {
-                    qf_engine::Launch L{};
-                    L.cb = cb;
-                    L.ck = ck;
-                    L.fp32 = fp32;
-                    L.offset = offset;
-                    L.count = count;
-                    L.tile = coop ? 2 : (tile && gcount > 0) ? 1 : 0;
-                    L.goffset = goffset;
-                    L.gcount = gcount;
-                    L.waves = gcount > 0 ? (int)std::min<long long>(tile_waves,
-                                                                  std::max<long long>(1, (group_tasks + gcount - 1) / gcount))
-                                         : 1;
-                    L.lds = lds;
-                    L.lds_os = lds_os <= kMaxTileLds ? lds_os : 0;
-                    L.os_split = ct.os == 1;
-                    L.os_lean = ct.os == 2 || ct.os < 0;
-                    e->launches.push_back(L);
-                }
-                if (fp32) e->stats.n_tasks_fp32 += count; else e->stats.n_tasks_fp64 += count;
-            }
-    // every tile workgroup must stay inside its chunk and its LDS allocation
-    for (const auto& L : e->launches) {
-        if (L.tile != 1) continue;
-        const int na = ncart(kClassL[L.cb][0]), nb = ncart(kClassL[L.cb][1]);
-        for (int q = L.goffset; q < L.goffset + L.gcount; ++q) {
-            const qf::TileGroup& g = e->groups[q];
-            if (g.task_begin < L.offset || g.task_end > L.offset + L.count || g.task_begin >= g.task_end)
-                return fail(QF_ERR_STATE, "tile group outside its launch");
-            const qf::Task& t0 = e->tasks[g.task_begin];
-            const size_t need = sizeof(double) * ((size_t)(na + g.nbra * nb) * e->blocks[t0.ket_block].colf.size() +
-                                                  (size_t)g.nbra * na * nb);
-            if (need > L.lds) return fail(QF_ERR_STATE, "tile group exceeds its LDS allocation");
-            if (L.lds_os && 2 * need - sizeof(double) * (size_t)g.nbra * na * nb > L.lds_os)
-                return fail(QF_ERR_STATE, "tile group exceeds its open-shell LDS allocation");
-            for (int x = g.task_begin; x < g.task_end; ++x) {
-                const qf::Task& t = e->tasks[x];
-                if (t.bra_block != t0.bra_block || t.ket_block != t0.ket_block || t.kb < g.chunk_kb ||
-                    t.ke > g.chunk_kb + g.nbra || t.kb >= t.ke)
-                    return fail(QF_ERR_STATE, "tile group mixes chunks");
-            }
-        }
-    }
+    rc = make_tasks(e, e->nbasis, e->tasks, e->groups, e->launches, &e->stats);
+    if (rc) return rc;
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
     e->order = stream_order(e->launches, e->tasks);
@@ -2054,6 +2067,13 @@ __global__ void k_cutmat_batch(const BatchMol* __restrict__ bm)
     m.cm[idx] = v;
 }
 
+__global__ void k_clear_batch(const BatchMol* __restrict__ bm)
+{
+    const BatchMol m = bm[blockIdx.y];
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx < m.n * m.n) m.F[idx] = 0.0;
+}
+
 __global__ void k_add(double* __restrict__ y, const double* __restrict__ x, int count)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2258,6 +2278,24 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
     auto cost = [](const qf::Task& x) {
         return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
     };
+    // The molecules of a batch fill the GPU together, so their launch shapes are
+    // those of the one molecule with as much work: quartets grow about as the
+    // cube of the functions.  (With each molecule's own shapes, primitive pieces
+    // of one pair and four tasks a workgroup for the small ones, 48 molecules of
+    // 19-200 functions took 24.7 ms a build, with these 16.0.)
+    double cube = 0.0;
+    for (const qf_engine* e : b->engs) cube += std::pow((double)e->nbasis, 3.0);
+    const int size = (int)std::cbrt(cube);
+    struct EngineTasks {
+        std::vector<qf::Task> tasks;
+        std::vector<qf::TileGroup> groups;
+        std::vector<qf_engine::Launch> launches;
+    };
+    std::vector<EngineTasks> et(count);
+    for (int i = 0; i < count; ++i) {
+        rc = make_tasks(b->engs[i], size, et[i].tasks, et[i].groups, et[i].launches, nullptr);
+        if (rc) return bail(rc);
+    }
     for (int cb = 0; cb < kNPC; ++cb)
         for (int ck = 0; ck <= cb; ++ck)
             for (int fp32 = 0; fp32 < 2; ++fp32)
@@ -2271,7 +2309,7 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
                     C.goffset = (int)groups.size();
                     C.waves = 1;
                     for (int i = 0; i < count; ++i) {
-                        const qf_engine* e = b->engs[i];
+                        const EngineTasks* e = &et[i];
                         for (const auto& L : e->launches) {
                             if (L.cb != cb || L.ck != ck || L.fp32 != fp32 || L.tile != tile) continue;
                             const int tbase = (int)tasks.size();
@@ -2447,8 +2485,8 @@ int qf_batch_clear_fock(qf_batch* b, void* stream)
 {
     if (!b) return fail(QF_ERR_ARG, "NULL");
     QF_HIP(hipSetDevice(b->device));
-    for (const auto& m : b->mols)
-        hipLaunchKernelGGL(k_zero, dim3(64), dim3(256), 0, (hipStream_t)stream, m.F, (size_t)m.n * m.n);
+    hipLaunchKernelGGL(k_clear_batch, dim3((b->max_n2 + 255) / 256, (unsigned)b->mols.size()), dim3(256), 0,
+                       (hipStream_t)stream, b->d_bm.p);
     QF_HIP(hipGetLastError());
     return QF_OK;
 }
