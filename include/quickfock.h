@@ -234,7 +234,7 @@ int qf_set_tuning(qf_engine *e, int replicas, int shuffle);
  * enable = 1 accumulates J_ab and all exchange terms of a bra chunk in a
  * workgroup-shared tile and adds it to G once, instead of one FP64 atomic
  * per quartet.  waves: waves per workgroup (1..4); tasks_per_group: tasks
- * one workgroup takes (0, the default: 4 up to 256 basis functions, 16
+ * one workgroup takes (0, the default: 2 up to 200 basis functions, 4 up to 400, 16
  * above); lds_bytes: tile budget (1 KiB..64 KiB).  Classes
  * whose tile does not fit fall back to direct atomics.  With enable = 1 the
  * d-heavy classes (La+Lb+Lc+Ld >= 6; >= 5 up to 128 basis functions, >= 4 up to 48)
@@ -248,7 +248,7 @@ int qf_set_tile(qf_engine *e, int enable, int waves, int tasks_per_group, int ld
  * with ck <= cb: tile (-1 engine default, 0 direct atomics, 1 LDS tile, 2
  * one quartet per wave with the recursions in LDS - d-heavy classes; others
  * use the tile), waves per tile workgroup, tasks per tile workgroup (with
- * tile = 2: kets per task, 1..64, default 1 up to 256 basis functions and 8
+ * tile = 2: kets per task, 1..64, default 1 up to 256 basis functions and 2
  * above) and bras per task (0: default). */
 int qf_set_class_tuning(qf_engine *e, int cb, int ck, int tile, int waves, int tasks_per_group,
                         int bras_per_task);
@@ -260,7 +260,7 @@ int qf_set_persistent(qf_engine *e, int max_workgroups);
  * sums at most `piece` bra and `piece` ket primitive pairs of its quartets, so
  * the most contracted quartets of a small molecule are spread over several
  * waves; the pieces add up to the same Fock matrix.  piece = 0: automatic (1
- * up to 96 basis functions, 2 up to 128, 4 up to 256, 12 above); piece < 0:
+ * up to 48 basis functions, 2 up to 96, 3 up to 160, 4 up to 256, 6 up to 400, 12 above); piece < 0:
  * never split. */
 int qf_set_prim_split(qf_engine *e, int piece);
 /* Per-class primitive piece size (class indices as qf_set_class_tuning):

@@ -49,7 +49,7 @@ inline int pair_class(int La, int Lb) { return La * (La + 1) / 2 + Lb; }
 const char* const kDirectFp32Refused =
     "the direct-atomic kernels run FP64 only (their FP32 form gave wrong Fock matrices on gfx950 and is not "
     "built); FP32 halves run on the LDS-tile kernel";
-constexpr int kCoopWindow = 8;   // kets per task of the wave-per-quartet kernels
+constexpr int kCoopWindow = 2;   // kets per task of the wave-per-quartet kernels
 constexpr int kNPC = 10;   // pair classes (La >= Lb) for s, p, d, f
 constexpr size_t kMaxTileLds = 64 * 1024;   // dynamic LDS of one tile workgroup
 const int kClassL[kNPC][2] = {{0, 0}, {1, 0}, {1, 1}, {2, 0}, {2, 1}, {2, 2}, {3, 0}, {3, 1}, {3, 2}, {3, 3}};
@@ -378,7 +378,7 @@ struct qf_engine {
     int shuffle = 1;         // permute tasks inside a launch (decorrelates atomic targets)
     int tile = 1;            // accumulate exchange terms in LDS tiles (fock_tile_kernel)
     int tile_waves = 4;      // max waves per tile workgroup
-    int tile_tasks = 0;      // max tasks per tile workgroup (0: 4 up to 256 functions, 16 above)
+    int tile_tasks = 0;      // max tasks per tile workgroup (0: 2 up to 200 functions, 4 up to 400, 16 above)
     int lds_budget = 64 * 1024;
     int persist = 0;         // grid cap of the class launches (0: one workgroup per task / group)
     int prim_piece = 0;      // primitive pairs per task piece: 0 auto, < 0 never split
@@ -778,20 +778,24 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
     // Primitive pieces: a wave's lanes each run the whole primitive loop of
     // one quartet, so the most contracted quartets set the tail of a launch
     // (and, for small molecules with few waves, its whole time).  The
-    // primitive pairs of a task are cut into pieces of at most 1 up to 96
-    // functions, 2 up to 128, 4 up to 256 and 12 above (e.g. 36 -> 3 x 12).
-    // Measured on (H2O)32 6-31G(d): no split 17.0 ms, pieces of 6 / 12 / 18:
-    // 15.8 / 15.4 / 15.9 ms; on QUICK's 69 regression inputs (12-210
-    // functions), geometric mean of the build times up to 32 functions with
-    // pieces of 1 / 2: 0.39 / 0.55 ms, 33-64: 0.93 / 1.23 ms, 79 functions
-    // 2.20 / 2.49 ms, 114: 2.02 / 1.50 ms, 210 (pieces of 1 / 4): 5.53 /
-    // 4.57 ms.  A small molecule has too few quartets to fill the GPU, and
-    // one primitive quartet per lane gives it the most waves.
+    // primitive pairs of a task are therefore cut into pieces: a small molecule
+    // has too few quartets to fill the GPU and takes one primitive pair per
+    // piece, a large one only cuts the longest loops (e.g. 36 -> 3 x 12), since
+    // every piece repeats the screen, the HRR and the digestion.  Builds in us
+    // with pieces of 1 / 2 / 3 / 4 / 6 / 12, launches over four streams:
+    // water 6-31G* (19 functions) 143 / 184 / 284 / 291 / 396 / 731, butane 6-31G* (80)
+    // 835 / 521 / 776 / 805 / 1361 / 1793, glycine 6-31G** (100, two tasks a
+    // workgroup) 1710 / 824 / 614 / 589 / 616 / 989, (H2O)8 6-31G* (152) 1808 /
+    // 881 / 788 / 857 / 1015 / 1479, (Gly)2 6-31G** (175) 4526 / 2258 / 1483 /
+    // 1442 / 1560 / 2021, (H2O)16 6-31G* (304) 10064 / 4669 / 2909 / 2823 / 2599 /
+    // 2931, (H2O)32 (608) 34806 / 17910 / 11420 / 11298 / 10712 / 10692.
     const int piece = e->prim_piece > 0   ? e->prim_piece
                       : e->prim_piece < 0 ? 1 << 20
-                      : size <= 96   ? 1
-                      : size <= 128  ? 2
-                      : size <= 256  ? 4
+                      : size <= 48        ? 1
+                      : size <= 96        ? 2
+                      : size <= 160       ? 3
+                      : size <= 256       ? 4
+                      : size <= 400       ? 6
                                           : 12;
     for (int cb = 0; cb < kNPC; ++cb)
         for (int ck = 0; ck <= cb; ++ck)
@@ -811,14 +815,17 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // saved build times; no gain above)
                 if (size <= 32) mmax = std::min(mmax, 2);
                 if (ct.mmax > 0) mmax = ct.mmax;
-                // tasks per tile workgroup: few for molecules up to 256
-                // functions, whose launches hold few tasks (QUICK's 69
-                // regression inputs, light classes with 1 / 2 / 4 / 8 / 16
-                // tasks per group: 15.7x / 16.5x / 16.5x / 13.9x / 10.4x
-                // QUICK's saved build times, geometric mean)
+                // tasks per tile workgroup: few for small molecules, whose launches
+                // hold few tasks (builds in us with 1 / 2 / 4 / 8 / 16: glycine
+                // 6-31G** 633 / 633 / 814 / 992 / 992, (H2O)8 6-31G* 924 / 885 / 975 /
+                // 928 / 1180, (H2O)8 cc-pVDZ (200 functions) 1077 / 1129 / 1202 / 1242 /
+                // 1447, C20H42 3-21G (264) 1825 / 1105 / 912 / 897 / 994, (H2O)16
+                // 3703 / 2940 / 3133 / 3171 / 3142, (H2O)32 25512 / 14599 / 12000 / 11245 /
+                // 10973)
                 const int tile_tasks = ct.tpg > 0        ? ct.tpg
                                        : e->tile_tasks > 0 ? e->tile_tasks
-                                       : size <= 256  ? 4
+                                       : size <= 200       ? 2
+                                       : size <= 400       ? 4
                                                            : 16;
                 const int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
                 // LDS tile: (na + m*nb) x ncol exchange terms + m*na*nb Coulomb terms
@@ -875,6 +882,9 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // wave-per-quartet kernel a window (the class tuning's
                 // tasks_per_group): small windows give more workgroups to
                 // classes with few quartets
+                // (builds in us with windows of 1 / 2 / 4 / 8 / 16: (H2O)16 2828 / 2846 /
+                // 2853 / 2953 / 2987, (H2O)32 10701 / 10658 / 10663 / 11389 / 11136, (Gly)6
+                // 6-31G** 11829 / 11813 / 12198 / 12191 / 13524)
                 const int coop_win = size <= 256 ? 1 : kCoopWindow;
                 const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_win) : qf::WAVE;
                 size_t lds = 0, lds_os = 0;
@@ -2282,7 +2292,7 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
     // those of the one molecule with as much work: quartets grow about as the
     // cube of the functions.  (With each molecule's own shapes, primitive pieces
     // of one pair and four tasks a workgroup for the small ones, 48 molecules of
-    // 19-200 functions took 24.7 ms a build, with these 16.0.)
+    // 19-156 functions took 24.7 ms a build, with these 16.0.)
     double cube = 0.0;
     for (const qf_engine* e : b->engs) cube += std::pow((double)e->nbasis, 3.0);
     const int size = (int)std::cbrt(cube);
