@@ -27,6 +27,7 @@ from __future__ import annotations
 
 from .gen_eri import (COOP_LDS_CAP, COOP_NT, PAIR_CLASSES, Hrr, SlotPool, Vrr, Z, _allocate, add, am,
                       boys_setup_flop, comps, ncart, sub)
+from .gen_md import md_grad_source
 
 # derivative blocks: (name, accumulator set, (dLa, dLb, dLc))
 BLOCKS = [("AP", 1, (1, 0, 0)), ("AM", 0, (-1, 0, 0)), ("BP", 2, (0, 1, 0)), ("BM", 0, (0, -1, 0)),
@@ -255,121 +256,15 @@ def grad_tables(La, Lb, Lc, Ld):
                 prim_flop=boys_setup_flop(L) + vflops + 2 * len(accs), quartet_flop=hflops + ni * (10 + 9 * 4))
 
 
-# Classes with La+Lb+Lc+Ld up to this also get a per-lane gradient kernel
-# (one quartet per lane, recursions in registers); the wave-per-quartet
-# kernel serves the rest.  At 4 and 5 the per-lane kernels spill 1.3-10 KB
-# per lane and are still faster than the wave-per-quartet ones ((H2O)32
-# 6-31G(d) gradient: 192 ms with 3, 134 ms with 4, 123 ms with 5).
+# Classes with La+Lb+Lc+Ld up to this also get a per-lane gradient kernel (one
+# quartet per lane, gen_md.py); the wave-per-quartet kernel serves the rest:
+# one step up, (dp|dp), the straight-line code of a primitive quartet is 128 KB,
+# twice the instruction cache.
 LANE_GRAD_LSUM_MAX = 5
 
 
 def has_lane_grad(La, Lb, Lc, Ld):
     return La + Lb + Lc + Ld <= LANE_GRAD_LSUM_MAX
-
-
-def _hrr_lines(prefix, cls, accexpr):
-    """Straight-line HRR of one block; returns (lines, {output (a,b,c,d): expression})."""
-    A_, B_, C_, D_ = cls
-    h = Hrr(A_, B_, C_, D_)
-    outs = []
-    for a in comps(A_):
-        for b in comps(B_):
-            for c in comps(C_):
-                for d in comps(D_):
-                    h.need_bra(a, b, c, d)
-                    outs.append((a, b, c, d))
-    tg = lambda t: "%d%d%d" % t
-
-    def kv(e, c, d):
-        return accexpr(e, c) if d == Z else "%sk%s_%s_%s" % (prefix, tg(e), tg(c), tg(d))
-
-    def bv(a, b, c, d):
-        return kv(a, c, d) if b == Z else "%sb%s_%s_%s_%s" % (prefix, tg(a), tg(b), tg(c), tg(d))
-
-    lines = []
-    for (e, c, d) in h.order_k:
-        i = h.ket[(e, c, d)]
-        lines.append("const double %s = %s + CD[%d] * %s;" % (kv(e, c, d), kv(e, add(c, i), sub(d, i)), i,
-                                                           kv(e, c, sub(d, i))))
-    for (a, b, c, d) in h.order_b:
-        i = h.bra[(a, b, c, d)]
-        lines.append("const double %s = %s + AB[%d] * %s;" % (bv(a, b, c, d), bv(add(a, i), sub(b, i), c, d), i,
-                                                           bv(a, sub(b, i), c, d)))
-    return lines, {o: bv(*o) for o in outs}
-
-
-def lane_grad_source(name, La, Lb, Lc, Ld):
-    """Per-lane gradient recursions of one class: ``vrr`` adds one primitive
-    quartet into the four weighted sets, ``digest`` runs the six HRR blocks
-    and contracts the derivative integrals with the density blocks into
-    g[9] = dE/dA, dE/dB, dE/dC (without the degeneracy weight)."""
-    sets = grad_sets(La, Lb, Lc, Ld)
-    L = La + Lb + Lc + Ld + 1
-    acc = {}
-    for si, st in enumerate(sets):
-        for t in st:
-            acc[(si, t)] = len(acc)
-    targets, seen = [], set()
-    for st in sets:
-        for t in st:
-            if t not in seen:
-                seen.add(t)
-                targets.append(t)
-    v = VrrTargets(targets, L)
-    vlines, _ = v.emit({t: 0 for t in targets})
-    vlines = vlines[:-len(targets)]
-    for (si, t), x in sorted(acc.items(), key=lambda kv: kv[1]):
-        vlines.append("acc[%d] += w[%d] * %s;" % (x, si, v.var((t[0], t[1], 0))))
-    vlines = [l.replace("const R ", "const double ").replace("R(", "double(") for l in vlines]
-    na, nb, nc, nd = (ncart(x) for x in (La, Lb, Lc, Ld))
-    dlines, outs = [], {}
-    for bname, si, (da, db, dc) in BLOCKS:
-        cls = (La + da, Lb + db, Lc + dc, Ld)
-        if min(cls) < 0:
-            continue
-        lines, o = _hrr_lines(bname.lower() + "_", cls, lambda e, c, _s=si: "acc[%d]" % acc[(_s, (e, c))])
-        dlines += lines
-        outs[bname] = o
-    ca, cb_, cc, cd = comps(La), comps(Lb), comps(Lc), comps(Ld)
-    for ia, a in enumerate(ca):
-        for ib, b in enumerate(cb_):
-            for ic, c in enumerate(cc):
-                for id_, d in enumerate(cd):
-                    dlines.append("{")
-                    dlines.append("  const double gm = kCons[%d][%d] * kCons[%d][%d] * kCons[%d][%d] * kCons[%d][%d] * "
-                                  "(2.0 * Dab[%d] * Dcd[%d] - hh * (Dac[%d] * Dbd[%d] + Dad[%d] * Dbc[%d]));"
-                                  % (La, ia, Lb, ib, Lc, ic, Ld, id_, ia * nb + ib, ic * nd + id_, ia * nc + ic,
-                                     ib * nd + id_, ia * nd + id_, ib * nc + ic))
-                    for x in range(3):
-                        tA = outs["AP"][(add(a, x), b, c, d)]
-                        if a[x] > 0:
-                            tA = "(%s - %d.0 * %s)" % (tA, a[x], outs["AM"][(sub(a, x), b, c, d)])
-                        tB = outs["BP"][(a, add(b, x), c, d)]
-                        if b[x] > 0:
-                            tB = "(%s - %d.0 * %s)" % (tB, b[x], outs["BM"][(a, sub(b, x), c, d)])
-                        tC = outs["CP"][(a, b, add(c, x), d)]
-                        if c[x] > 0:
-                            tC = "(%s - %d.0 * %s)" % (tC, c[x], outs["CM"][(a, b, sub(c, x), d)])
-                        dlines.append("  g[%d] += gm * %s;" % (x, tA))
-                        dlines.append("  g[%d] += gm * %s;" % (3 + x, tB))
-                        dlines.append("  g[%d] += gm * %s;" % (6 + x, tC))
-                    dlines.append("}")
-    g = name + "GradLane"
-    src = ["struct %s {" % g,
-           "  static constexpr int La = %d, Lb = %d, Lc = %d, Ld = %d, L = %d;" % (La, Lb, Lc, Ld, L),
-           "  static constexpr int NACC = %d;" % len(acc),
-           "  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC",
-           "  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p,"
-           " const double (&w)[4], double (&acc)[NACC]) {"]
-    src += ["    " + l for l in vlines]
-    src += ["  }",
-            "  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3],"
-            " const double (&CD)[3], const double (&Dab)[%d], const double (&Dcd)[%d], const double (&Dac)[%d],"
-            " const double (&Dad)[%d], const double (&Dbc)[%d], const double (&Dbd)[%d], double hh, double (&g)[9]) {"
-            % (na * nb, nc * nd, na * nc, na * nd, nb * nc, nb * nd)]
-    src += ["    " + l for l in dlines]
-    src += ["  }", "};"]
-    return g, "\n".join(src) + "\n"
 
 
 def grad_source(name, La, Lb, Lc, Ld):
@@ -442,7 +337,7 @@ def launcher_source(name, g, lane):
             "    (void)gscratch;",
             "    if (nt <= 0) return;",
             "    if (grid <= 0 || grid > nt) grid = nt;",
-            "    hipLaunchKernelGGL((grad_lane_kernel<%sGradLane>), dim3(grid), dim3(WAVE), grad_tile, s, t, nt, b, m,"
+            "    hipLaunchKernelGGL((grad_md_kernel<%sGradMd>), dim3(grid), dim3(WAVE), grad_tile, s, t, nt, b, m,"
             " (int)(grad_tile / sizeof(double)), fp32);" % name,
             "}", ""]
     return "\n".join([
@@ -472,7 +367,7 @@ def main(outdir, write):
         g, src, t = grad_source(name, La, Lb, Lc, Ld)
         lane = has_lane_grad(La, Lb, Lc, Ld)
         if lane:
-            src += lane_grad_source(name, La, Lb, Lc, Ld)[1]
+            src += md_grad_source(name, La, Lb, Lc, Ld)[1]
         write("grad_%s.h" % name, "// Generated by quick_amd/codegen/gen_grad.py - do not edit.\n#pragma once\n"
               "#include \"../qf_grad.h\"\nnamespace qf {\n" + src + "}  // namespace qf\n")
         write("egrad_%s.hip" % name, launcher_source(name, g, lane))

@@ -1619,14 +1619,20 @@ constexpr size_t kGradLdsMax = 64 * 1024;   // dynamic LDS of one gradient workg
 int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out, double* dgrad, hipStream_t s)
 {
     // every class needs a gradient kernel: check before launching anything
+    auto lane_kernel = [&](const qf_engine::Launch& L) -> qf::GradLaunch {
+        const int gm = e->ctune[L.cb][L.ck].grad;
+        return (gm >= 0 ? gm == 1 : e->grad_lane) ? qf::grad_lane_launcher(L.cb, L.ck) : nullptr;
+    };
     size_t gdoubles = 0;
+    std::vector<size_t> gslot;   // per launch: its region of the global slot buffer
     for (const auto& L : e->launches) {
         if (!qf::grad_launcher(L.cb, L.ck))
             return fail(QF_ERR_ARG, "ERI gradients cover shells up to d; this basis has f shells");
-        gdoubles = std::max<size_t>(gdoubles, (size_t)qf::grad_global_doubles(L.cb, L.ck));
+        gslot.push_back(gdoubles);
+        if (!lane_kernel(L))
+            gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) * std::min(L.count, qf::COOP_GLOBAL_SLICES);
     }
-    if (gdoubles && e->d_gscratch.n < gdoubles * qf::COOP_GLOBAL_SLICES)
-        QF_HIP(e->d_gscratch.resize(gdoubles * qf::COOP_GLOBAL_SLICES));
+    if (gdoubles && e->d_gscratch.n < gdoubles) QF_HIP(e->d_gscratch.resize(gdoubles));
     qf::MolDesc md{};
     md.P = dP;
     md.PJ = dP;
@@ -1655,31 +1661,36 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     const int orc = open_build(oa, s);
     if (orc) return orc;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
-    for (size_t li = 0; li < e->launches.size(); ++li) {
+    auto launch = [&](int li, hipStream_t q) -> int {
         const auto& L = e->launches[li];
-        const int gm = e->ctune[L.cb][L.ck].grad;
-        const bool want_lane = gm >= 0 ? gm == 1 : e->grad_lane;
-        const qf::GradLaunch lane = want_lane ? qf::grad_lane_launcher(L.cb, L.ck) : nullptr;
+        const qf::GradLaunch lane = lane_kernel(L);
         const size_t slots = lane ? 0 : (size_t)qf::grad_lds_doubles(L.cb, L.ck) * sizeof(double);
         const size_t tile = slots + tile_bytes <= kGradLdsMax ? tile_bytes : 0;
         // one workgroup per task unless the engine caps the grid (qf_set_persistent):
         // the hardware then hands out tasks as workgroups finish
         const int grid = e->persist > 0 ? std::min(L.count, e->persist) : L.count;
-        hipEvent_t eb = nullptr;
-        if (e->timing) {
+        (lane ? lane : qf::grad_launcher(L.cb, L.ck))(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, dmol, grid,
+                                                      tile, e->d_gscratch.p + gslot[li], L.fp32, q);
+        return QF_OK;
+    };
+    if (e->timing) {
+        for (size_t li = 0; li < e->launches.size(); ++li) {
             while (e->ev_pool.size() < e->ev_used + 2) {
                 hipEvent_t ev;
                 QF_HIP(hipEventCreate(&ev));
                 e->ev_pool.push_back(ev);
             }
-            eb = e->ev_pool[e->ev_used + 1];
-            QF_HIP(hipEventRecord(e->ev_pool[e->ev_used], s));
+            hipEvent_t ea = e->ev_pool[e->ev_used], eb = e->ev_pool[e->ev_used + 1];
             e->ev_used += 2;
             e->ev_launch.push_back((int)li);
+            QF_HIP(hipEventRecord(ea, s));
+            launch((int)li, s);
+            QF_HIP(hipEventRecord(eb, s));
         }
-        (lane ? lane : qf::grad_launcher(L.cb, L.ck))(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, dmol, grid,
-                                                      tile, e->d_gscratch.p, L.fp32, s);
-        if (eb) QF_HIP(hipEventRecord(eb, s));
+    } else {
+        const bool forked = e->order.size() > 1 && side_ready(e->side, e->device, s);
+        const int rc = issue_forked(forked ? e->side : nullptr, s, e->order, launch);
+        if (rc) return rc;
     }
     QF_HIP(hipGetLastError());
     return QF_OK;

@@ -22,7 +22,7 @@ void launch_grad_lane_C2111(const Task* t, int nt, const PairBlock* b, const Mol
     (void)gscratch;
     if (nt <= 0) return;
     if (grid <= 0 || grid > nt) grid = nt;
-    hipLaunchKernelGGL((grad_lane_kernel<C2111GradLane>), dim3(grid), dim3(WAVE), grad_tile, s, t, nt, b, m, (int)(grad_tile / sizeof(double)), fp32);
+    hipLaunchKernelGGL((grad_md_kernel<C2111GradMd>), dim3(grid), dim3(WAVE), grad_tile, s, t, nt, b, m, (int)(grad_tile / sizeof(double)), fp32);
 }
 
 }  // namespace qf

@@ -28,46 +28,53 @@ __device__ inline const int* C0000Grad::vlev() { return kC0000Grad_vlev; }
 __device__ inline const GradAcc* C0000Grad::acc() { return kC0000Grad_acc; }
 __device__ inline const CoopHNode* C0000Grad::hrr() { return kC0000Grad_hrr; }
 __device__ inline const int* C0000Grad::hlev() { return kC0000Grad_hlev; }
-struct C0000GradLane {
+// (ss|ss): 4 Hermite Coulomb integrals, 0 bra products
+struct C0000GradMd {
   static constexpr int La = 0, Lb = 0, Lc = 0, Ld = 0, L = 1;
-  static constexpr int NACC = 10;
-  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC
-  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p, const double (&w)[4], double (&acc)[NACC]) {
-    const double v000_000_1 = F[1];
-    const double v000_000_0 = F[0];
-    const double v001_000_0 = p.PA[2] * v000_000_0 + p.WP[2] * v000_000_1;
-    const double v010_000_0 = p.PA[1] * v000_000_0 + p.WP[1] * v000_000_1;
-    const double v100_000_0 = p.PA[0] * v000_000_0 + p.WP[0] * v000_000_1;
-    const double v000_001_0 = p.QC[2] * v000_000_0 + p.WQ[2] * v000_000_1;
-    const double v000_010_0 = p.QC[1] * v000_000_0 + p.WQ[1] * v000_000_1;
-    const double v000_100_0 = p.QC[0] * v000_000_0 + p.WQ[0] * v000_000_1;
-    acc[0] += w[1] * v100_000_0;
-    acc[1] += w[1] * v010_000_0;
-    acc[2] += w[1] * v001_000_0;
-    acc[3] += w[2] * v000_000_0;
-    acc[4] += w[2] * v100_000_0;
-    acc[5] += w[2] * v010_000_0;
-    acc[6] += w[2] * v001_000_0;
-    acc[7] += w[3] * v000_100_0;
-    acc[8] += w[3] * v000_010_0;
-    acc[9] += w[3] * v000_001_0;
+  static constexpr int N1 = 1, NE = 0;   // 1D entries per direction, product table
+  static constexpr int MIN_WAVES = 3;      // waves per SIMD the register budget targets
+  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16
+  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p, rx = -beta/p, ry = alpha/p
+  template <class T>
+  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, double rx, double ry, T out) {
+    out[0] = 1.0;
   }
-  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3], const double (&CD)[3], const double (&Dab)[1], const double (&Dcd)[1], const double (&Dac)[1], const double (&Dad)[1], const double (&Dbc)[1], const double (&Dbd)[1], double hh, double (&g)[9]) {
-    const double bp_b000_100_000_000 = acc[4] + AB[0] * acc[3];
-    const double bp_b000_010_000_000 = acc[5] + AB[1] * acc[3];
-    const double bp_b000_001_000_000 = acc[6] + AB[2] * acc[3];
+  // Dcd with 2 cons, Dbc and Dbd with hyb/2 cons; oc, od: first elements of the a-c and a-d blocks of P
+  template <class ET, class PT, class PU>
+  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a, const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, double rc, double rd, const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[1], const double (&Dbc)[1], const double (&Dbd)[1], double& W, double (&gP)[3], double (&gR)[3], double (&gS)[3]) {
+    double am = pref;
+    const double r000_0 = F[0] * am;
+    am *= m2a;
+    const double r000_1 = F[1] * am;
+    const double r100_0 = PQ[0] * r000_1;
+    const double r010_0 = PQ[1] * r000_1;
+    const double r001_0 = PQ[2] * r000_1;
+    double w = 0.0, px = 0.0, py = 0.0, pz = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
     {
-      const double gm = kCons[0][0] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[0] * Dcd[0] - hh * (Dac[0] * Dbd[0] + Dad[0] * Dbc[0]));
-      g[0] += gm * acc[0];
-      g[3] += gm * bp_b000_100_000_000;
-      g[6] += gm * acc[7];
-      g[1] += gm * acc[1];
-      g[4] += gm * bp_b000_010_000_000;
-      g[7] += gm * acc[8];
-      g[2] += gm * acc[2];
-      g[5] += gm * bp_b000_001_000_000;
-      g[8] += gm * acc[9];
+      const double ac0 = P[oc + 0 * n + 0] * (kCons[0][0] * kCons[0][0]);
+      const double ad0 = P[od + 0 * n + 0] * (kCons[0][0] * kCons[0][0]);
+      {
+        const double ab = Pab[0 * n + 0] * (kCons[0][0] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        w = t000 + w;
+        px = t100 + px;
+        py = t010 + py;
+        pz = t001 + pz;
+      }
     }
+    W = w;
+    gP[0] = px; gP[1] = py; gP[2] = pz;
+    gR[0] = sx; gR[1] = sy; gR[2] = sz;
+    gS[0] = 0.0;
+    gS[1] = 0.0;
+    gS[2] = 0.0;
   }
 };
+__device__ const unsigned kC0000GradMd_index[1] = {0};
+__device__ inline const unsigned* C0000GradMd::index() { return kC0000GradMd_index; }
 }  // namespace qf

@@ -28,107 +28,122 @@ __device__ inline const int* C1000Grad::vlev() { return kC1000Grad_vlev; }
 __device__ inline const GradAcc* C1000Grad::acc() { return kC1000Grad_acc; }
 __device__ inline const CoopHNode* C1000Grad::hrr() { return kC1000Grad_hrr; }
 __device__ inline const int* C1000Grad::hlev() { return kC1000Grad_hlev; }
-struct C1000GradLane {
+// (ps|ss): 10 Hermite Coulomb integrals, 9 bra products
+struct C1000GradMd {
   static constexpr int La = 1, Lb = 0, Lc = 0, Ld = 0, L = 2;
-  static constexpr int NACC = 25;
-  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC
-  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p, const double (&w)[4], double (&acc)[NACC]) {
-    const double v000_000_2 = F[2];
-    const double v000_000_1 = F[1];
-    const double v000_000_0 = F[0];
-    const double v001_000_1 = p.PA[2] * v000_000_1 + p.WP[2] * v000_000_2;
-    const double v010_000_1 = p.PA[1] * v000_000_1 + p.WP[1] * v000_000_2;
-    const double v100_000_1 = p.PA[0] * v000_000_1 + p.WP[0] * v000_000_2;
-    const double v001_000_0 = p.PA[2] * v000_000_0 + p.WP[2] * v000_000_1;
-    const double v010_000_0 = p.PA[1] * v000_000_0 + p.WP[1] * v000_000_1;
-    const double v100_000_0 = p.PA[0] * v000_000_0 + p.WP[0] * v000_000_1;
-    const double v002_000_0 = p.PA[2] * v001_000_0 + p.WP[2] * v001_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v011_000_0 = p.PA[1] * v001_000_0 + p.WP[1] * v001_000_1;
-    const double v020_000_0 = p.PA[1] * v010_000_0 + p.WP[1] * v010_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v101_000_0 = p.PA[0] * v001_000_0 + p.WP[0] * v001_000_1;
-    const double v110_000_0 = p.PA[0] * v010_000_0 + p.WP[0] * v010_000_1;
-    const double v200_000_0 = p.PA[0] * v100_000_0 + p.WP[0] * v100_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v001_001_0 = p.QC[2] * v001_000_0 + p.WQ[2] * v001_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v001_010_0 = p.QC[1] * v001_000_0 + p.WQ[1] * v001_000_1;
-    const double v001_100_0 = p.QC[0] * v001_000_0 + p.WQ[0] * v001_000_1;
-    const double v010_001_0 = p.QC[2] * v010_000_0 + p.WQ[2] * v010_000_1;
-    const double v010_010_0 = p.QC[1] * v010_000_0 + p.WQ[1] * v010_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v010_100_0 = p.QC[0] * v010_000_0 + p.WQ[0] * v010_000_1;
-    const double v100_001_0 = p.QC[2] * v100_000_0 + p.WQ[2] * v100_000_1;
-    const double v100_010_0 = p.QC[1] * v100_000_0 + p.WQ[1] * v100_000_1;
-    const double v100_100_0 = p.QC[0] * v100_000_0 + p.WQ[0] * v100_000_1 + double(1) * p.oo2zn * v000_000_1;
-    acc[0] += w[0] * v000_000_0;
-    acc[1] += w[1] * v200_000_0;
-    acc[2] += w[1] * v110_000_0;
-    acc[3] += w[1] * v020_000_0;
-    acc[4] += w[1] * v101_000_0;
-    acc[5] += w[1] * v011_000_0;
-    acc[6] += w[1] * v002_000_0;
-    acc[7] += w[2] * v100_000_0;
-    acc[8] += w[2] * v010_000_0;
-    acc[9] += w[2] * v001_000_0;
-    acc[10] += w[2] * v200_000_0;
-    acc[11] += w[2] * v110_000_0;
-    acc[12] += w[2] * v020_000_0;
-    acc[13] += w[2] * v101_000_0;
-    acc[14] += w[2] * v011_000_0;
-    acc[15] += w[2] * v002_000_0;
-    acc[16] += w[3] * v100_100_0;
-    acc[17] += w[3] * v100_010_0;
-    acc[18] += w[3] * v100_001_0;
-    acc[19] += w[3] * v010_100_0;
-    acc[20] += w[3] * v010_010_0;
-    acc[21] += w[3] * v010_001_0;
-    acc[22] += w[3] * v001_100_0;
-    acc[23] += w[3] * v001_010_0;
-    acc[24] += w[3] * v001_001_0;
+  static constexpr int N1 = 4, NE = 9;   // 1D entries per direction, product table
+  static constexpr int MIN_WAVES = 3;      // waves per SIMD the register budget targets
+  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16
+  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p, rx = -beta/p, ry = alpha/p
+  template <class T>
+  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, double rx, double ry, T out) {
+    const double be100 = X;
+    const double be101 = h;
+    const double bd100 = rx;
+    out[0] = 1.0;
+    out[1] = be100;
+    out[2] = be101;
+    out[3] = bd100;
   }
-  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3], const double (&CD)[3], const double (&Dab)[3], const double (&Dcd)[1], const double (&Dac)[3], const double (&Dad)[3], const double (&Dbc)[1], const double (&Dbd)[1], double hh, double (&g)[9]) {
-    const double bp_b100_100_000_000 = acc[10] + AB[0] * acc[7];
-    const double bp_b100_010_000_000 = acc[11] + AB[1] * acc[7];
-    const double bp_b100_001_000_000 = acc[13] + AB[2] * acc[7];
-    const double bp_b010_100_000_000 = acc[11] + AB[0] * acc[8];
-    const double bp_b010_010_000_000 = acc[12] + AB[1] * acc[8];
-    const double bp_b010_001_000_000 = acc[14] + AB[2] * acc[8];
-    const double bp_b001_100_000_000 = acc[13] + AB[0] * acc[9];
-    const double bp_b001_010_000_000 = acc[14] + AB[1] * acc[9];
-    const double bp_b001_001_000_000 = acc[15] + AB[2] * acc[9];
+  // Dcd with 2 cons, Dbc and Dbd with hyb/2 cons; oc, od: first elements of the a-c and a-d blocks of P
+  template <class ET, class PT, class PU>
+  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a, const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, double rc, double rd, const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[1], const double (&Dbc)[1], const double (&Dbd)[1], double& W, double (&gP)[3], double (&gR)[3], double (&gS)[3]) {
+    double am = pref;
+    const double r000_0 = F[0] * am;
+    am *= m2a;
+    const double r000_1 = F[1] * am;
+    am *= m2a;
+    const double r000_2 = F[2] * am;
+    const double r100_1 = PQ[0] * r000_2;
+    const double r010_1 = PQ[1] * r000_2;
+    const double r001_1 = PQ[2] * r000_2;
+    const double r100_0 = PQ[0] * r000_1;
+    const double r010_0 = PQ[1] * r000_1;
+    const double r001_0 = PQ[2] * r000_1;
+    const double r200_0 = fma(1.0, r000_1, PQ[0] * r100_1);
+    const double r110_0 = PQ[0] * r010_1;
+    const double r101_0 = PQ[0] * r001_1;
+    const double r020_0 = fma(1.0, r000_1, PQ[1] * r010_1);
+    const double r011_0 = PQ[1] * r001_1;
+    const double r002_0 = fma(1.0, r000_1, PQ[2] * r001_1);
+    double w = 0.0, px = 0.0, py = 0.0, pz = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
     {
-      const double gm = kCons[1][0] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[0] * Dcd[0] - hh * (Dac[0] * Dbd[0] + Dad[0] * Dbc[0]));
-      g[0] += gm * (acc[1] - 1.0 * acc[0]);
-      g[3] += gm * bp_b100_100_000_000;
-      g[6] += gm * acc[16];
-      g[1] += gm * acc[2];
-      g[4] += gm * bp_b100_010_000_000;
-      g[7] += gm * acc[17];
-      g[2] += gm * acc[4];
-      g[5] += gm * bp_b100_001_000_000;
-      g[8] += gm * acc[18];
+      const double ac0 = P[oc + 0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+      const double ad0 = P[od + 0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+      {
+        const double ab = Pab[0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double e0 = E[0];
+        const double e1 = E[1];
+        w = fma(e1, t100, fma(e0, t000, w));
+        px = fma(e1, t200, fma(e0, t100, px));
+        py = fma(e1, t110, fma(e0, t010, py));
+        pz = fma(e1, t101, fma(e0, t001, pz));
+        sx = fma(E[2], t000, sx);
+      }
     }
     {
-      const double gm = kCons[1][1] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[1] * Dcd[0] - hh * (Dac[1] * Dbd[0] + Dad[1] * Dbc[0]));
-      g[0] += gm * acc[2];
-      g[3] += gm * bp_b010_100_000_000;
-      g[6] += gm * acc[19];
-      g[1] += gm * (acc[3] - 1.0 * acc[0]);
-      g[4] += gm * bp_b010_010_000_000;
-      g[7] += gm * acc[20];
-      g[2] += gm * acc[5];
-      g[5] += gm * bp_b010_001_000_000;
-      g[8] += gm * acc[21];
+      const double ac0 = P[oc + 1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+      const double ad0 = P[od + 1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+      {
+        const double ab = Pab[1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t110 = y000 * r110_0;
+        const double e0 = E[3];
+        const double e1 = E[4];
+        w = fma(e1, t010, fma(e0, t000, w));
+        px = fma(e1, t110, fma(e0, t100, px));
+        py = fma(e1, t020, fma(e0, t010, py));
+        pz = fma(e1, t011, fma(e0, t001, pz));
+        sy = fma(E[5], t000, sy);
+      }
     }
     {
-      const double gm = kCons[1][2] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[2] * Dcd[0] - hh * (Dac[2] * Dbd[0] + Dad[2] * Dbc[0]));
-      g[0] += gm * acc[4];
-      g[3] += gm * bp_b001_100_000_000;
-      g[6] += gm * acc[22];
-      g[1] += gm * acc[5];
-      g[4] += gm * bp_b001_010_000_000;
-      g[7] += gm * acc[23];
-      g[2] += gm * (acc[6] - 1.0 * acc[0]);
-      g[5] += gm * bp_b001_001_000_000;
-      g[8] += gm * acc[24];
+      const double ac0 = P[oc + 2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+      const double ad0 = P[od + 2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+      {
+        const double ab = Pab[2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t101 = y000 * r101_0;
+        const double e0 = E[6];
+        const double e1 = E[7];
+        w = fma(e1, t001, fma(e0, t000, w));
+        px = fma(e1, t101, fma(e0, t100, px));
+        py = fma(e1, t011, fma(e0, t010, py));
+        pz = fma(e1, t002, fma(e0, t001, pz));
+        sz = fma(E[8], t000, sz);
+      }
     }
+    W = w;
+    gP[0] = px; gP[1] = py; gP[2] = pz;
+    gR[0] = sx; gR[1] = sy; gR[2] = sz;
+    gS[0] = 0.0;
+    gS[1] = 0.0;
+    gS[2] = 0.0;
   }
 };
+__device__ const unsigned kC1000GradMd_index[9] = {1,2,3,256,512,768,65536,131072,196608};
+__device__ inline const unsigned* C1000GradMd::index() { return kC1000GradMd_index; }
 }  // namespace qf

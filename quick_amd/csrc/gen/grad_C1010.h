@@ -28,302 +28,194 @@ __device__ inline const int* C1010Grad::vlev() { return kC1010Grad_vlev; }
 __device__ inline const GradAcc* C1010Grad::acc() { return kC1010Grad_acc; }
 __device__ inline const CoopHNode* C1010Grad::hrr() { return kC1010Grad_hrr; }
 __device__ inline const int* C1010Grad::hlev() { return kC1010Grad_hlev; }
-struct C1010GradLane {
+// (ps|ps): 20 Hermite Coulomb integrals, 9 bra products
+struct C1010GradMd {
   static constexpr int La = 1, Lb = 0, Lc = 1, Ld = 0, L = 3;
-  static constexpr int NACC = 69;
-  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC
-  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p, const double (&w)[4], double (&acc)[NACC]) {
-    const double v000_000_3 = F[3];
-    const double v000_000_2 = F[2];
-    const double v000_000_1 = F[1];
-    const double v000_000_0 = F[0];
-    const double v001_000_2 = p.PA[2] * v000_000_2 + p.WP[2] * v000_000_3;
-    const double v010_000_2 = p.PA[1] * v000_000_2 + p.WP[1] * v000_000_3;
-    const double v100_000_2 = p.PA[0] * v000_000_2 + p.WP[0] * v000_000_3;
-    const double v001_000_1 = p.PA[2] * v000_000_1 + p.WP[2] * v000_000_2;
-    const double v010_000_1 = p.PA[1] * v000_000_1 + p.WP[1] * v000_000_2;
-    const double v100_000_1 = p.PA[0] * v000_000_1 + p.WP[0] * v000_000_2;
-    const double v001_000_0 = p.PA[2] * v000_000_0 + p.WP[2] * v000_000_1;
-    const double v010_000_0 = p.PA[1] * v000_000_0 + p.WP[1] * v000_000_1;
-    const double v100_000_0 = p.PA[0] * v000_000_0 + p.WP[0] * v000_000_1;
-    const double v000_001_1 = p.QC[2] * v000_000_1 + p.WQ[2] * v000_000_2;
-    const double v000_010_1 = p.QC[1] * v000_000_1 + p.WQ[1] * v000_000_2;
-    const double v000_100_1 = p.QC[0] * v000_000_1 + p.WQ[0] * v000_000_2;
-    const double v000_001_0 = p.QC[2] * v000_000_0 + p.WQ[2] * v000_000_1;
-    const double v000_010_0 = p.QC[1] * v000_000_0 + p.WQ[1] * v000_000_1;
-    const double v000_100_0 = p.QC[0] * v000_000_0 + p.WQ[0] * v000_000_1;
-    const double v002_000_1 = p.PA[2] * v001_000_1 + p.WP[2] * v001_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v011_000_1 = p.PA[1] * v001_000_1 + p.WP[1] * v001_000_2;
-    const double v020_000_1 = p.PA[1] * v010_000_1 + p.WP[1] * v010_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v101_000_1 = p.PA[0] * v001_000_1 + p.WP[0] * v001_000_2;
-    const double v110_000_1 = p.PA[0] * v010_000_1 + p.WP[0] * v010_000_2;
-    const double v200_000_1 = p.PA[0] * v100_000_1 + p.WP[0] * v100_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v002_000_0 = p.PA[2] * v001_000_0 + p.WP[2] * v001_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v011_000_0 = p.PA[1] * v001_000_0 + p.WP[1] * v001_000_1;
-    const double v020_000_0 = p.PA[1] * v010_000_0 + p.WP[1] * v010_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v101_000_0 = p.PA[0] * v001_000_0 + p.WP[0] * v001_000_1;
-    const double v110_000_0 = p.PA[0] * v010_000_0 + p.WP[0] * v010_000_1;
-    const double v200_000_0 = p.PA[0] * v100_000_0 + p.WP[0] * v100_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v001_001_1 = p.QC[2] * v001_000_1 + p.WQ[2] * v001_000_2 + double(1) * p.oo2zn * v000_000_2;
-    const double v001_010_1 = p.QC[1] * v001_000_1 + p.WQ[1] * v001_000_2;
-    const double v001_100_1 = p.QC[0] * v001_000_1 + p.WQ[0] * v001_000_2;
-    const double v010_001_1 = p.QC[2] * v010_000_1 + p.WQ[2] * v010_000_2;
-    const double v010_010_1 = p.QC[1] * v010_000_1 + p.WQ[1] * v010_000_2 + double(1) * p.oo2zn * v000_000_2;
-    const double v010_100_1 = p.QC[0] * v010_000_1 + p.WQ[0] * v010_000_2;
-    const double v100_001_1 = p.QC[2] * v100_000_1 + p.WQ[2] * v100_000_2;
-    const double v100_010_1 = p.QC[1] * v100_000_1 + p.WQ[1] * v100_000_2;
-    const double v100_100_1 = p.QC[0] * v100_000_1 + p.WQ[0] * v100_000_2 + double(1) * p.oo2zn * v000_000_2;
-    const double v001_001_0 = p.QC[2] * v001_000_0 + p.WQ[2] * v001_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v001_010_0 = p.QC[1] * v001_000_0 + p.WQ[1] * v001_000_1;
-    const double v001_100_0 = p.QC[0] * v001_000_0 + p.WQ[0] * v001_000_1;
-    const double v010_001_0 = p.QC[2] * v010_000_0 + p.WQ[2] * v010_000_1;
-    const double v010_010_0 = p.QC[1] * v010_000_0 + p.WQ[1] * v010_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v010_100_0 = p.QC[0] * v010_000_0 + p.WQ[0] * v010_000_1;
-    const double v100_001_0 = p.QC[2] * v100_000_0 + p.WQ[2] * v100_000_1;
-    const double v100_010_0 = p.QC[1] * v100_000_0 + p.WQ[1] * v100_000_1;
-    const double v100_100_0 = p.QC[0] * v100_000_0 + p.WQ[0] * v100_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v002_001_0 = p.QC[2] * v002_000_0 + p.WQ[2] * v002_000_1 + double(2) * p.oo2zn * v001_000_1;
-    const double v002_010_0 = p.QC[1] * v002_000_0 + p.WQ[1] * v002_000_1;
-    const double v002_100_0 = p.QC[0] * v002_000_0 + p.WQ[0] * v002_000_1;
-    const double v011_001_0 = p.QC[2] * v011_000_0 + p.WQ[2] * v011_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v011_010_0 = p.QC[1] * v011_000_0 + p.WQ[1] * v011_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v011_100_0 = p.QC[0] * v011_000_0 + p.WQ[0] * v011_000_1;
-    const double v020_001_0 = p.QC[2] * v020_000_0 + p.WQ[2] * v020_000_1;
-    const double v020_010_0 = p.QC[1] * v020_000_0 + p.WQ[1] * v020_000_1 + double(2) * p.oo2zn * v010_000_1;
-    const double v020_100_0 = p.QC[0] * v020_000_0 + p.WQ[0] * v020_000_1;
-    const double v101_001_0 = p.QC[2] * v101_000_0 + p.WQ[2] * v101_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v101_010_0 = p.QC[1] * v101_000_0 + p.WQ[1] * v101_000_1;
-    const double v101_100_0 = p.QC[0] * v101_000_0 + p.WQ[0] * v101_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v110_001_0 = p.QC[2] * v110_000_0 + p.WQ[2] * v110_000_1;
-    const double v110_010_0 = p.QC[1] * v110_000_0 + p.WQ[1] * v110_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v110_100_0 = p.QC[0] * v110_000_0 + p.WQ[0] * v110_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v200_001_0 = p.QC[2] * v200_000_0 + p.WQ[2] * v200_000_1;
-    const double v200_010_0 = p.QC[1] * v200_000_0 + p.WQ[1] * v200_000_1;
-    const double v200_100_0 = p.QC[0] * v200_000_0 + p.WQ[0] * v200_000_1 + double(2) * p.oo2zn * v100_000_1;
-    const double v001_002_0 = p.QC[2] * v001_001_0 + p.WQ[2] * v001_001_1 + double(1) * p.oo2n * (v001_000_0 - p.rn * v001_000_1) + double(1) * p.oo2zn * v000_001_1;
-    const double v001_011_0 = p.QC[1] * v001_001_0 + p.WQ[1] * v001_001_1;
-    const double v001_020_0 = p.QC[1] * v001_010_0 + p.WQ[1] * v001_010_1 + double(1) * p.oo2n * (v001_000_0 - p.rn * v001_000_1);
-    const double v001_101_0 = p.QC[0] * v001_001_0 + p.WQ[0] * v001_001_1;
-    const double v001_110_0 = p.QC[0] * v001_010_0 + p.WQ[0] * v001_010_1;
-    const double v001_200_0 = p.QC[0] * v001_100_0 + p.WQ[0] * v001_100_1 + double(1) * p.oo2n * (v001_000_0 - p.rn * v001_000_1);
-    const double v010_002_0 = p.QC[2] * v010_001_0 + p.WQ[2] * v010_001_1 + double(1) * p.oo2n * (v010_000_0 - p.rn * v010_000_1);
-    const double v010_011_0 = p.QC[2] * v010_010_0 + p.WQ[2] * v010_010_1;
-    const double v010_020_0 = p.QC[1] * v010_010_0 + p.WQ[1] * v010_010_1 + double(1) * p.oo2n * (v010_000_0 - p.rn * v010_000_1) + double(1) * p.oo2zn * v000_010_1;
-    const double v010_101_0 = p.QC[0] * v010_001_0 + p.WQ[0] * v010_001_1;
-    const double v010_110_0 = p.QC[0] * v010_010_0 + p.WQ[0] * v010_010_1;
-    const double v010_200_0 = p.QC[0] * v010_100_0 + p.WQ[0] * v010_100_1 + double(1) * p.oo2n * (v010_000_0 - p.rn * v010_000_1);
-    const double v100_002_0 = p.QC[2] * v100_001_0 + p.WQ[2] * v100_001_1 + double(1) * p.oo2n * (v100_000_0 - p.rn * v100_000_1);
-    const double v100_011_0 = p.QC[1] * v100_001_0 + p.WQ[1] * v100_001_1;
-    const double v100_020_0 = p.QC[1] * v100_010_0 + p.WQ[1] * v100_010_1 + double(1) * p.oo2n * (v100_000_0 - p.rn * v100_000_1);
-    const double v100_101_0 = p.QC[2] * v100_100_0 + p.WQ[2] * v100_100_1;
-    const double v100_110_0 = p.QC[1] * v100_100_0 + p.WQ[1] * v100_100_1;
-    const double v100_200_0 = p.QC[0] * v100_100_0 + p.WQ[0] * v100_100_1 + double(1) * p.oo2n * (v100_000_0 - p.rn * v100_000_1) + double(1) * p.oo2zn * v000_100_1;
-    acc[0] += w[0] * v000_100_0;
-    acc[1] += w[0] * v000_010_0;
-    acc[2] += w[0] * v000_001_0;
-    acc[3] += w[0] * v100_000_0;
-    acc[4] += w[0] * v010_000_0;
-    acc[5] += w[0] * v001_000_0;
-    acc[6] += w[1] * v200_100_0;
-    acc[7] += w[1] * v200_010_0;
-    acc[8] += w[1] * v200_001_0;
-    acc[9] += w[1] * v110_100_0;
-    acc[10] += w[1] * v110_010_0;
-    acc[11] += w[1] * v110_001_0;
-    acc[12] += w[1] * v020_100_0;
-    acc[13] += w[1] * v020_010_0;
-    acc[14] += w[1] * v020_001_0;
-    acc[15] += w[1] * v101_100_0;
-    acc[16] += w[1] * v101_010_0;
-    acc[17] += w[1] * v101_001_0;
-    acc[18] += w[1] * v011_100_0;
-    acc[19] += w[1] * v011_010_0;
-    acc[20] += w[1] * v011_001_0;
-    acc[21] += w[1] * v002_100_0;
-    acc[22] += w[1] * v002_010_0;
-    acc[23] += w[1] * v002_001_0;
-    acc[24] += w[2] * v100_100_0;
-    acc[25] += w[2] * v100_010_0;
-    acc[26] += w[2] * v100_001_0;
-    acc[27] += w[2] * v010_100_0;
-    acc[28] += w[2] * v010_010_0;
-    acc[29] += w[2] * v010_001_0;
-    acc[30] += w[2] * v001_100_0;
-    acc[31] += w[2] * v001_010_0;
-    acc[32] += w[2] * v001_001_0;
-    acc[33] += w[2] * v200_100_0;
-    acc[34] += w[2] * v200_010_0;
-    acc[35] += w[2] * v200_001_0;
-    acc[36] += w[2] * v110_100_0;
-    acc[37] += w[2] * v110_010_0;
-    acc[38] += w[2] * v110_001_0;
-    acc[39] += w[2] * v020_100_0;
-    acc[40] += w[2] * v020_010_0;
-    acc[41] += w[2] * v020_001_0;
-    acc[42] += w[2] * v101_100_0;
-    acc[43] += w[2] * v101_010_0;
-    acc[44] += w[2] * v101_001_0;
-    acc[45] += w[2] * v011_100_0;
-    acc[46] += w[2] * v011_010_0;
-    acc[47] += w[2] * v011_001_0;
-    acc[48] += w[2] * v002_100_0;
-    acc[49] += w[2] * v002_010_0;
-    acc[50] += w[2] * v002_001_0;
-    acc[51] += w[3] * v100_200_0;
-    acc[52] += w[3] * v100_110_0;
-    acc[53] += w[3] * v100_020_0;
-    acc[54] += w[3] * v100_101_0;
-    acc[55] += w[3] * v100_011_0;
-    acc[56] += w[3] * v100_002_0;
-    acc[57] += w[3] * v010_200_0;
-    acc[58] += w[3] * v010_110_0;
-    acc[59] += w[3] * v010_020_0;
-    acc[60] += w[3] * v010_101_0;
-    acc[61] += w[3] * v010_011_0;
-    acc[62] += w[3] * v010_002_0;
-    acc[63] += w[3] * v001_200_0;
-    acc[64] += w[3] * v001_110_0;
-    acc[65] += w[3] * v001_020_0;
-    acc[66] += w[3] * v001_101_0;
-    acc[67] += w[3] * v001_011_0;
-    acc[68] += w[3] * v001_002_0;
+  static constexpr int N1 = 4, NE = 9;   // 1D entries per direction, product table
+  static constexpr int MIN_WAVES = 2;      // waves per SIMD the register budget targets
+  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16
+  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p, rx = -beta/p, ry = alpha/p
+  template <class T>
+  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, double rx, double ry, T out) {
+    const double be100 = X;
+    const double be101 = h;
+    const double bd100 = rx;
+    out[0] = 1.0;
+    out[1] = be100;
+    out[2] = be101;
+    out[3] = bd100;
   }
-  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3], const double (&CD)[3], const double (&Dab)[3], const double (&Dcd)[3], const double (&Dac)[9], const double (&Dad)[3], const double (&Dbc)[3], const double (&Dbd)[1], double hh, double (&g)[9]) {
-    const double bp_b100_100_100_000 = acc[33] + AB[0] * acc[24];
-    const double bp_b100_100_010_000 = acc[34] + AB[0] * acc[25];
-    const double bp_b100_100_001_000 = acc[35] + AB[0] * acc[26];
-    const double bp_b100_010_100_000 = acc[36] + AB[1] * acc[24];
-    const double bp_b100_010_010_000 = acc[37] + AB[1] * acc[25];
-    const double bp_b100_010_001_000 = acc[38] + AB[1] * acc[26];
-    const double bp_b100_001_100_000 = acc[42] + AB[2] * acc[24];
-    const double bp_b100_001_010_000 = acc[43] + AB[2] * acc[25];
-    const double bp_b100_001_001_000 = acc[44] + AB[2] * acc[26];
-    const double bp_b010_100_100_000 = acc[36] + AB[0] * acc[27];
-    const double bp_b010_100_010_000 = acc[37] + AB[0] * acc[28];
-    const double bp_b010_100_001_000 = acc[38] + AB[0] * acc[29];
-    const double bp_b010_010_100_000 = acc[39] + AB[1] * acc[27];
-    const double bp_b010_010_010_000 = acc[40] + AB[1] * acc[28];
-    const double bp_b010_010_001_000 = acc[41] + AB[1] * acc[29];
-    const double bp_b010_001_100_000 = acc[45] + AB[2] * acc[27];
-    const double bp_b010_001_010_000 = acc[46] + AB[2] * acc[28];
-    const double bp_b010_001_001_000 = acc[47] + AB[2] * acc[29];
-    const double bp_b001_100_100_000 = acc[42] + AB[0] * acc[30];
-    const double bp_b001_100_010_000 = acc[43] + AB[0] * acc[31];
-    const double bp_b001_100_001_000 = acc[44] + AB[0] * acc[32];
-    const double bp_b001_010_100_000 = acc[45] + AB[1] * acc[30];
-    const double bp_b001_010_010_000 = acc[46] + AB[1] * acc[31];
-    const double bp_b001_010_001_000 = acc[47] + AB[1] * acc[32];
-    const double bp_b001_001_100_000 = acc[48] + AB[2] * acc[30];
-    const double bp_b001_001_010_000 = acc[49] + AB[2] * acc[31];
-    const double bp_b001_001_001_000 = acc[50] + AB[2] * acc[32];
+  // Dcd with 2 cons, Dbc and Dbd with hyb/2 cons; oc, od: first elements of the a-c and a-d blocks of P
+  template <class ET, class PT, class PU>
+  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a, const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, double rc, double rd, const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[3], const double (&Dbc)[3], const double (&Dbd)[1], double& W, double (&gP)[3], double (&gR)[3], double (&gS)[3]) {
+    double am = pref;
+    const double r000_0 = F[0] * am;
+    am *= m2a;
+    const double r000_1 = F[1] * am;
+    am *= m2a;
+    const double r000_2 = F[2] * am;
+    am *= m2a;
+    const double r000_3 = F[3] * am;
+    const double r100_2 = PQ[0] * r000_3;
+    const double r010_2 = PQ[1] * r000_3;
+    const double r001_2 = PQ[2] * r000_3;
+    const double r100_1 = PQ[0] * r000_2;
+    const double r010_1 = PQ[1] * r000_2;
+    const double r001_1 = PQ[2] * r000_2;
+    const double r200_1 = fma(1.0, r000_2, PQ[0] * r100_2);
+    const double r110_1 = PQ[0] * r010_2;
+    const double r101_1 = PQ[0] * r001_2;
+    const double r020_1 = fma(1.0, r000_2, PQ[1] * r010_2);
+    const double r011_1 = PQ[1] * r001_2;
+    const double r002_1 = fma(1.0, r000_2, PQ[2] * r001_2);
+    const double r100_0 = PQ[0] * r000_1;
+    const double r010_0 = PQ[1] * r000_1;
+    const double r001_0 = PQ[2] * r000_1;
+    const double r200_0 = fma(1.0, r000_1, PQ[0] * r100_1);
+    const double r110_0 = PQ[0] * r010_1;
+    const double r101_0 = PQ[0] * r001_1;
+    const double r020_0 = fma(1.0, r000_1, PQ[1] * r010_1);
+    const double r011_0 = PQ[1] * r001_1;
+    const double r002_0 = fma(1.0, r000_1, PQ[2] * r001_1);
+    const double r300_0 = fma(2.0, r100_1, PQ[0] * r200_1);
+    const double r210_0 = PQ[1] * r200_1;
+    const double r201_0 = PQ[2] * r200_1;
+    const double r120_0 = PQ[0] * r020_1;
+    const double r111_0 = PQ[0] * r011_1;
+    const double r102_0 = PQ[0] * r002_1;
+    const double r030_0 = fma(2.0, r010_1, PQ[1] * r020_1);
+    const double r021_0 = PQ[2] * r020_1;
+    const double r012_0 = PQ[1] * r002_1;
+    const double r003_0 = fma(2.0, r001_1, PQ[2] * r002_1);
+    const double kxe100 = QC[0];
+    const double kxe101 = (-hk);
+    const double kxd100 = rc;
+    const double kye100 = QC[1];
+    const double kye101 = (-hk);
+    const double kyd100 = rc;
+    const double kze100 = QC[2];
+    const double kze101 = (-hk);
+    const double kzd100 = rc;
+    const double k0_0_000 = kxe100;
+    const double k0_0_100 = kxe101;
+    const double k1_0_000 = kye100;
+    const double k1_0_010 = kye101;
+    const double k2_0_000 = kze100;
+    const double k2_0_001 = kze101;
+    double K0_0_000 = 0.0;
+    double K1_0_000 = 0.0;
+    double K2_0_000 = 0.0;
+    double w = 0.0, px = 0.0, py = 0.0, pz = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
     {
-      const double gm = kCons[1][0] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[0] * Dcd[0] - hh * (Dac[0] * Dbd[0] + Dad[0] * Dbc[0]));
-      g[0] += gm * (acc[6] - 1.0 * acc[0]);
-      g[3] += gm * bp_b100_100_100_000;
-      g[6] += gm * (acc[51] - 1.0 * acc[3]);
-      g[1] += gm * acc[9];
-      g[4] += gm * bp_b100_010_100_000;
-      g[7] += gm * acc[52];
-      g[2] += gm * acc[15];
-      g[5] += gm * bp_b100_001_100_000;
-      g[8] += gm * acc[54];
+      const double ac0 = P[oc + 0 * n + 0] * (kCons[1][0] * kCons[1][0]);
+      const double ac1 = P[oc + 0 * n + 1] * (kCons[1][0] * kCons[1][1]);
+      const double ac2 = P[oc + 0 * n + 2] * (kCons[1][0] * kCons[1][2]);
+      const double ad0 = P[od + 0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+      {
+        const double ab = Pab[0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double t200 = fma(y100, r300_0, fma(y010, r210_0, fma(y001, r201_0, y000 * r200_0)));
+        const double e0 = E[0];
+        const double e1 = E[1];
+        w = fma(e1, t100, fma(e0, t000, w));
+        px = fma(e1, t200, fma(e0, t100, px));
+        py = fma(e1, t110, fma(e0, t010, py));
+        pz = fma(e1, t101, fma(e0, t001, pz));
+        sx = fma(E[2], t000, sx);
+        const double z000 = fma(e1, r100_0, e0 * r000_0);
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[1][0] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[0] * Dcd[1] - hh * (Dac[1] * Dbd[0] + Dad[0] * Dbc[1]));
-      g[0] += gm * (acc[7] - 1.0 * acc[1]);
-      g[3] += gm * bp_b100_100_010_000;
-      g[6] += gm * acc[52];
-      g[1] += gm * acc[10];
-      g[4] += gm * bp_b100_010_010_000;
-      g[7] += gm * (acc[53] - 1.0 * acc[3]);
-      g[2] += gm * acc[16];
-      g[5] += gm * bp_b100_001_010_000;
-      g[8] += gm * acc[55];
+      const double ac0 = P[oc + 1 * n + 0] * (kCons[1][1] * kCons[1][0]);
+      const double ac1 = P[oc + 1 * n + 1] * (kCons[1][1] * kCons[1][1]);
+      const double ac2 = P[oc + 1 * n + 2] * (kCons[1][1] * kCons[1][2]);
+      const double ad0 = P[od + 1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+      {
+        const double ab = Pab[1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t020 = fma(y100, r120_0, fma(y010, r030_0, fma(y001, r021_0, y000 * r020_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double e0 = E[3];
+        const double e1 = E[4];
+        w = fma(e1, t010, fma(e0, t000, w));
+        px = fma(e1, t110, fma(e0, t100, px));
+        py = fma(e1, t020, fma(e0, t010, py));
+        pz = fma(e1, t011, fma(e0, t001, pz));
+        sy = fma(E[5], t000, sy);
+        const double z000 = fma(e1, r010_0, e0 * r000_0);
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[1][0] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[0] * Dcd[2] - hh * (Dac[2] * Dbd[0] + Dad[0] * Dbc[2]));
-      g[0] += gm * (acc[8] - 1.0 * acc[2]);
-      g[3] += gm * bp_b100_100_001_000;
-      g[6] += gm * acc[54];
-      g[1] += gm * acc[11];
-      g[4] += gm * bp_b100_010_001_000;
-      g[7] += gm * acc[55];
-      g[2] += gm * acc[17];
-      g[5] += gm * bp_b100_001_001_000;
-      g[8] += gm * (acc[56] - 1.0 * acc[3]);
+      const double ac0 = P[oc + 2 * n + 0] * (kCons[1][2] * kCons[1][0]);
+      const double ac1 = P[oc + 2 * n + 1] * (kCons[1][2] * kCons[1][1]);
+      const double ac2 = P[oc + 2 * n + 2] * (kCons[1][2] * kCons[1][2]);
+      const double ad0 = P[od + 2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+      {
+        const double ab = Pab[2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t002 = fma(y100, r102_0, fma(y010, r012_0, fma(y001, r003_0, y000 * r002_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double e0 = E[6];
+        const double e1 = E[7];
+        w = fma(e1, t001, fma(e0, t000, w));
+        px = fma(e1, t101, fma(e0, t100, px));
+        py = fma(e1, t011, fma(e0, t010, py));
+        pz = fma(e1, t002, fma(e0, t001, pz));
+        sz = fma(E[8], t000, sz);
+        const double z000 = fma(e1, r001_0, e0 * r000_0);
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
-    {
-      const double gm = kCons[1][1] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[1] * Dcd[0] - hh * (Dac[3] * Dbd[0] + Dad[1] * Dbc[0]));
-      g[0] += gm * acc[9];
-      g[3] += gm * bp_b010_100_100_000;
-      g[6] += gm * (acc[57] - 1.0 * acc[4]);
-      g[1] += gm * (acc[12] - 1.0 * acc[0]);
-      g[4] += gm * bp_b010_010_100_000;
-      g[7] += gm * acc[58];
-      g[2] += gm * acc[18];
-      g[5] += gm * bp_b010_001_100_000;
-      g[8] += gm * acc[60];
-    }
-    {
-      const double gm = kCons[1][1] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[1] * Dcd[1] - hh * (Dac[4] * Dbd[0] + Dad[1] * Dbc[1]));
-      g[0] += gm * acc[10];
-      g[3] += gm * bp_b010_100_010_000;
-      g[6] += gm * acc[58];
-      g[1] += gm * (acc[13] - 1.0 * acc[1]);
-      g[4] += gm * bp_b010_010_010_000;
-      g[7] += gm * (acc[59] - 1.0 * acc[4]);
-      g[2] += gm * acc[19];
-      g[5] += gm * bp_b010_001_010_000;
-      g[8] += gm * acc[61];
-    }
-    {
-      const double gm = kCons[1][1] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[1] * Dcd[2] - hh * (Dac[5] * Dbd[0] + Dad[1] * Dbc[2]));
-      g[0] += gm * acc[11];
-      g[3] += gm * bp_b010_100_001_000;
-      g[6] += gm * acc[60];
-      g[1] += gm * (acc[14] - 1.0 * acc[2]);
-      g[4] += gm * bp_b010_010_001_000;
-      g[7] += gm * acc[61];
-      g[2] += gm * acc[20];
-      g[5] += gm * bp_b010_001_001_000;
-      g[8] += gm * (acc[62] - 1.0 * acc[4]);
-    }
-    {
-      const double gm = kCons[1][2] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[2] * Dcd[0] - hh * (Dac[6] * Dbd[0] + Dad[2] * Dbc[0]));
-      g[0] += gm * acc[15];
-      g[3] += gm * bp_b001_100_100_000;
-      g[6] += gm * (acc[63] - 1.0 * acc[5]);
-      g[1] += gm * acc[18];
-      g[4] += gm * bp_b001_010_100_000;
-      g[7] += gm * acc[64];
-      g[2] += gm * (acc[21] - 1.0 * acc[0]);
-      g[5] += gm * bp_b001_001_100_000;
-      g[8] += gm * acc[66];
-    }
-    {
-      const double gm = kCons[1][2] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[2] * Dcd[1] - hh * (Dac[7] * Dbd[0] + Dad[2] * Dbc[1]));
-      g[0] += gm * acc[16];
-      g[3] += gm * bp_b001_100_010_000;
-      g[6] += gm * acc[64];
-      g[1] += gm * acc[19];
-      g[4] += gm * bp_b001_010_010_000;
-      g[7] += gm * (acc[65] - 1.0 * acc[5]);
-      g[2] += gm * (acc[22] - 1.0 * acc[1]);
-      g[5] += gm * bp_b001_001_010_000;
-      g[8] += gm * acc[67];
-    }
-    {
-      const double gm = kCons[1][2] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[2] * Dcd[2] - hh * (Dac[8] * Dbd[0] + Dad[2] * Dbc[2]));
-      g[0] += gm * acc[17];
-      g[3] += gm * bp_b001_100_001_000;
-      g[6] += gm * acc[66];
-      g[1] += gm * acc[20];
-      g[4] += gm * bp_b001_010_001_000;
-      g[7] += gm * acc[67];
-      g[2] += gm * (acc[23] - 1.0 * acc[2]);
-      g[5] += gm * bp_b001_001_001_000;
-      g[8] += gm * (acc[68] - 1.0 * acc[5]);
-    }
+    W = w;
+    gP[0] = px; gP[1] = py; gP[2] = pz;
+    gR[0] = sx; gR[1] = sy; gR[2] = sz;
+    gS[0] = kxd100 * K0_0_000;
+    gS[1] = kyd100 * K1_0_000;
+    gS[2] = kzd100 * K2_0_000;
   }
 };
+__device__ const unsigned kC1010GradMd_index[9] = {1,2,3,256,512,768,65536,131072,196608};
+__device__ inline const unsigned* C1010GradMd::index() { return kC1010GradMd_index; }
 }  // namespace qf

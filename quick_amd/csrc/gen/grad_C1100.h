@@ -28,338 +28,333 @@ __device__ inline const int* C1100Grad::vlev() { return kC1100Grad_vlev; }
 __device__ inline const GradAcc* C1100Grad::acc() { return kC1100Grad_acc; }
 __device__ inline const CoopHNode* C1100Grad::hrr() { return kC1100Grad_hrr; }
 __device__ inline const int* C1100Grad::hlev() { return kC1100Grad_hlev; }
-struct C1100GradLane {
+// (pp|ss): 20 Hermite Coulomb integrals, 63 bra products
+struct C1100GradMd {
   static constexpr int La = 1, Lb = 1, Lc = 0, Ld = 0, L = 3;
-  static constexpr int NACC = 66;
-  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC
-  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p, const double (&w)[4], double (&acc)[NACC]) {
-    const double v000_000_3 = F[3];
-    const double v000_000_2 = F[2];
-    const double v000_000_1 = F[1];
-    const double v000_000_0 = F[0];
-    const double v001_000_2 = p.PA[2] * v000_000_2 + p.WP[2] * v000_000_3;
-    const double v010_000_2 = p.PA[1] * v000_000_2 + p.WP[1] * v000_000_3;
-    const double v100_000_2 = p.PA[0] * v000_000_2 + p.WP[0] * v000_000_3;
-    const double v001_000_1 = p.PA[2] * v000_000_1 + p.WP[2] * v000_000_2;
-    const double v010_000_1 = p.PA[1] * v000_000_1 + p.WP[1] * v000_000_2;
-    const double v100_000_1 = p.PA[0] * v000_000_1 + p.WP[0] * v000_000_2;
-    const double v001_000_0 = p.PA[2] * v000_000_0 + p.WP[2] * v000_000_1;
-    const double v010_000_0 = p.PA[1] * v000_000_0 + p.WP[1] * v000_000_1;
-    const double v100_000_0 = p.PA[0] * v000_000_0 + p.WP[0] * v000_000_1;
-    const double v002_000_1 = p.PA[2] * v001_000_1 + p.WP[2] * v001_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v011_000_1 = p.PA[1] * v001_000_1 + p.WP[1] * v001_000_2;
-    const double v020_000_1 = p.PA[1] * v010_000_1 + p.WP[1] * v010_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v101_000_1 = p.PA[0] * v001_000_1 + p.WP[0] * v001_000_2;
-    const double v110_000_1 = p.PA[0] * v010_000_1 + p.WP[0] * v010_000_2;
-    const double v200_000_1 = p.PA[0] * v100_000_1 + p.WP[0] * v100_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v002_000_0 = p.PA[2] * v001_000_0 + p.WP[2] * v001_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v011_000_0 = p.PA[1] * v001_000_0 + p.WP[1] * v001_000_1;
-    const double v020_000_0 = p.PA[1] * v010_000_0 + p.WP[1] * v010_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v101_000_0 = p.PA[0] * v001_000_0 + p.WP[0] * v001_000_1;
-    const double v110_000_0 = p.PA[0] * v010_000_0 + p.WP[0] * v010_000_1;
-    const double v200_000_0 = p.PA[0] * v100_000_0 + p.WP[0] * v100_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v001_001_0 = p.QC[2] * v001_000_0 + p.WQ[2] * v001_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v001_010_0 = p.QC[1] * v001_000_0 + p.WQ[1] * v001_000_1;
-    const double v001_100_0 = p.QC[0] * v001_000_0 + p.WQ[0] * v001_000_1;
-    const double v010_001_0 = p.QC[2] * v010_000_0 + p.WQ[2] * v010_000_1;
-    const double v010_010_0 = p.QC[1] * v010_000_0 + p.WQ[1] * v010_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v010_100_0 = p.QC[0] * v010_000_0 + p.WQ[0] * v010_000_1;
-    const double v100_001_0 = p.QC[2] * v100_000_0 + p.WQ[2] * v100_000_1;
-    const double v100_010_0 = p.QC[1] * v100_000_0 + p.WQ[1] * v100_000_1;
-    const double v100_100_0 = p.QC[0] * v100_000_0 + p.WQ[0] * v100_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v003_000_0 = p.PA[2] * v002_000_0 + p.WP[2] * v002_000_1 + double(2) * p.oo2z * (v001_000_0 - p.rz * v001_000_1);
-    const double v012_000_0 = p.PA[1] * v002_000_0 + p.WP[1] * v002_000_1;
-    const double v021_000_0 = p.PA[2] * v020_000_0 + p.WP[2] * v020_000_1;
-    const double v030_000_0 = p.PA[1] * v020_000_0 + p.WP[1] * v020_000_1 + double(2) * p.oo2z * (v010_000_0 - p.rz * v010_000_1);
-    const double v102_000_0 = p.PA[0] * v002_000_0 + p.WP[0] * v002_000_1;
-    const double v111_000_0 = p.PA[0] * v011_000_0 + p.WP[0] * v011_000_1;
-    const double v120_000_0 = p.PA[0] * v020_000_0 + p.WP[0] * v020_000_1;
-    const double v201_000_0 = p.PA[2] * v200_000_0 + p.WP[2] * v200_000_1;
-    const double v210_000_0 = p.PA[1] * v200_000_0 + p.WP[1] * v200_000_1;
-    const double v300_000_0 = p.PA[0] * v200_000_0 + p.WP[0] * v200_000_1 + double(2) * p.oo2z * (v100_000_0 - p.rz * v100_000_1);
-    const double v002_001_0 = p.QC[2] * v002_000_0 + p.WQ[2] * v002_000_1 + double(2) * p.oo2zn * v001_000_1;
-    const double v002_010_0 = p.QC[1] * v002_000_0 + p.WQ[1] * v002_000_1;
-    const double v002_100_0 = p.QC[0] * v002_000_0 + p.WQ[0] * v002_000_1;
-    const double v011_001_0 = p.QC[2] * v011_000_0 + p.WQ[2] * v011_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v011_010_0 = p.QC[1] * v011_000_0 + p.WQ[1] * v011_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v011_100_0 = p.QC[0] * v011_000_0 + p.WQ[0] * v011_000_1;
-    const double v020_001_0 = p.QC[2] * v020_000_0 + p.WQ[2] * v020_000_1;
-    const double v020_010_0 = p.QC[1] * v020_000_0 + p.WQ[1] * v020_000_1 + double(2) * p.oo2zn * v010_000_1;
-    const double v020_100_0 = p.QC[0] * v020_000_0 + p.WQ[0] * v020_000_1;
-    const double v101_001_0 = p.QC[2] * v101_000_0 + p.WQ[2] * v101_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v101_010_0 = p.QC[1] * v101_000_0 + p.WQ[1] * v101_000_1;
-    const double v101_100_0 = p.QC[0] * v101_000_0 + p.WQ[0] * v101_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v110_001_0 = p.QC[2] * v110_000_0 + p.WQ[2] * v110_000_1;
-    const double v110_010_0 = p.QC[1] * v110_000_0 + p.WQ[1] * v110_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v110_100_0 = p.QC[0] * v110_000_0 + p.WQ[0] * v110_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v200_001_0 = p.QC[2] * v200_000_0 + p.WQ[2] * v200_000_1;
-    const double v200_010_0 = p.QC[1] * v200_000_0 + p.WQ[1] * v200_000_1;
-    const double v200_100_0 = p.QC[0] * v200_000_0 + p.WQ[0] * v200_000_1 + double(2) * p.oo2zn * v100_000_1;
-    acc[0] += w[0] * v000_000_0;
-    acc[1] += w[0] * v100_000_0;
-    acc[2] += w[0] * v010_000_0;
-    acc[3] += w[0] * v001_000_0;
-    acc[4] += w[1] * v200_000_0;
-    acc[5] += w[1] * v110_000_0;
-    acc[6] += w[1] * v020_000_0;
-    acc[7] += w[1] * v101_000_0;
-    acc[8] += w[1] * v011_000_0;
-    acc[9] += w[1] * v002_000_0;
-    acc[10] += w[1] * v300_000_0;
-    acc[11] += w[1] * v210_000_0;
-    acc[12] += w[1] * v120_000_0;
-    acc[13] += w[1] * v030_000_0;
-    acc[14] += w[1] * v201_000_0;
-    acc[15] += w[1] * v111_000_0;
-    acc[16] += w[1] * v021_000_0;
-    acc[17] += w[1] * v102_000_0;
-    acc[18] += w[1] * v012_000_0;
-    acc[19] += w[1] * v003_000_0;
-    acc[20] += w[2] * v100_000_0;
-    acc[21] += w[2] * v010_000_0;
-    acc[22] += w[2] * v001_000_0;
-    acc[23] += w[2] * v200_000_0;
-    acc[24] += w[2] * v110_000_0;
-    acc[25] += w[2] * v020_000_0;
-    acc[26] += w[2] * v101_000_0;
-    acc[27] += w[2] * v011_000_0;
-    acc[28] += w[2] * v002_000_0;
-    acc[29] += w[2] * v300_000_0;
-    acc[30] += w[2] * v210_000_0;
-    acc[31] += w[2] * v120_000_0;
-    acc[32] += w[2] * v030_000_0;
-    acc[33] += w[2] * v201_000_0;
-    acc[34] += w[2] * v111_000_0;
-    acc[35] += w[2] * v021_000_0;
-    acc[36] += w[2] * v102_000_0;
-    acc[37] += w[2] * v012_000_0;
-    acc[38] += w[2] * v003_000_0;
-    acc[39] += w[3] * v100_100_0;
-    acc[40] += w[3] * v100_010_0;
-    acc[41] += w[3] * v100_001_0;
-    acc[42] += w[3] * v010_100_0;
-    acc[43] += w[3] * v010_010_0;
-    acc[44] += w[3] * v010_001_0;
-    acc[45] += w[3] * v001_100_0;
-    acc[46] += w[3] * v001_010_0;
-    acc[47] += w[3] * v001_001_0;
-    acc[48] += w[3] * v200_100_0;
-    acc[49] += w[3] * v200_010_0;
-    acc[50] += w[3] * v200_001_0;
-    acc[51] += w[3] * v110_100_0;
-    acc[52] += w[3] * v110_010_0;
-    acc[53] += w[3] * v110_001_0;
-    acc[54] += w[3] * v020_100_0;
-    acc[55] += w[3] * v020_010_0;
-    acc[56] += w[3] * v020_001_0;
-    acc[57] += w[3] * v101_100_0;
-    acc[58] += w[3] * v101_010_0;
-    acc[59] += w[3] * v101_001_0;
-    acc[60] += w[3] * v011_100_0;
-    acc[61] += w[3] * v011_010_0;
-    acc[62] += w[3] * v011_001_0;
-    acc[63] += w[3] * v002_100_0;
-    acc[64] += w[3] * v002_010_0;
-    acc[65] += w[3] * v002_001_0;
+  static constexpr int N1 = 12, NE = 63;   // 1D entries per direction, product table
+  static constexpr int MIN_WAVES = 2;      // waves per SIMD the register budget targets
+  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16
+  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p, rx = -beta/p, ry = alpha/p
+  template <class T>
+  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, double rx, double ry, T out) {
+    const double be010 = Y;
+    const double be011 = h;
+    const double bd010 = ry;
+    const double be100 = X;
+    const double be101 = h;
+    const double bd100 = rx;
+    const double be110 = fma(1.0, be101, be100 * Y);
+    const double be111 = fma(be100, h, be101 * Y);
+    const double be112 = be101 * h;
+    const double bd110 = fma(be100, ry, bd100 * Y);
+    const double bd111 = fma(be101, ry, bd100 * h);
+    out[0] = 1.0;
+    out[1] = be010;
+    out[2] = be011;
+    out[3] = bd010;
+    out[4] = be100;
+    out[5] = be101;
+    out[6] = bd100;
+    out[7] = be110;
+    out[8] = be111;
+    out[9] = be112;
+    out[10] = bd110;
+    out[11] = bd111;
   }
-  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3], const double (&CD)[3], const double (&Dab)[9], const double (&Dcd)[1], const double (&Dac)[3], const double (&Dad)[3], const double (&Dbc)[3], const double (&Dbd)[3], double hh, double (&g)[9]) {
-    const double ap_b200_100_000_000 = acc[10] + AB[0] * acc[4];
-    const double ap_b200_010_000_000 = acc[11] + AB[1] * acc[4];
-    const double ap_b200_001_000_000 = acc[14] + AB[2] * acc[4];
-    const double ap_b110_100_000_000 = acc[11] + AB[0] * acc[5];
-    const double ap_b110_010_000_000 = acc[12] + AB[1] * acc[5];
-    const double ap_b110_001_000_000 = acc[15] + AB[2] * acc[5];
-    const double ap_b020_100_000_000 = acc[12] + AB[0] * acc[6];
-    const double ap_b020_010_000_000 = acc[13] + AB[1] * acc[6];
-    const double ap_b020_001_000_000 = acc[16] + AB[2] * acc[6];
-    const double ap_b101_100_000_000 = acc[14] + AB[0] * acc[7];
-    const double ap_b101_010_000_000 = acc[15] + AB[1] * acc[7];
-    const double ap_b101_001_000_000 = acc[17] + AB[2] * acc[7];
-    const double ap_b011_100_000_000 = acc[15] + AB[0] * acc[8];
-    const double ap_b011_010_000_000 = acc[16] + AB[1] * acc[8];
-    const double ap_b011_001_000_000 = acc[18] + AB[2] * acc[8];
-    const double ap_b002_100_000_000 = acc[17] + AB[0] * acc[9];
-    const double ap_b002_010_000_000 = acc[18] + AB[1] * acc[9];
-    const double ap_b002_001_000_000 = acc[19] + AB[2] * acc[9];
-    const double am_b000_100_000_000 = acc[1] + AB[0] * acc[0];
-    const double am_b000_010_000_000 = acc[2] + AB[1] * acc[0];
-    const double am_b000_001_000_000 = acc[3] + AB[2] * acc[0];
-    const double bp_b200_100_000_000 = acc[29] + AB[0] * acc[23];
-    const double bp_b100_100_000_000 = acc[23] + AB[0] * acc[20];
-    const double bp_b100_200_000_000 = bp_b200_100_000_000 + AB[0] * bp_b100_100_000_000;
-    const double bp_b200_010_000_000 = acc[30] + AB[1] * acc[23];
-    const double bp_b100_010_000_000 = acc[24] + AB[1] * acc[20];
-    const double bp_b100_110_000_000 = bp_b200_010_000_000 + AB[0] * bp_b100_010_000_000;
-    const double bp_b110_010_000_000 = acc[31] + AB[1] * acc[24];
-    const double bp_b100_020_000_000 = bp_b110_010_000_000 + AB[1] * bp_b100_010_000_000;
-    const double bp_b200_001_000_000 = acc[33] + AB[2] * acc[23];
-    const double bp_b100_001_000_000 = acc[26] + AB[2] * acc[20];
-    const double bp_b100_101_000_000 = bp_b200_001_000_000 + AB[0] * bp_b100_001_000_000;
-    const double bp_b110_001_000_000 = acc[34] + AB[2] * acc[24];
-    const double bp_b100_011_000_000 = bp_b110_001_000_000 + AB[1] * bp_b100_001_000_000;
-    const double bp_b101_001_000_000 = acc[36] + AB[2] * acc[26];
-    const double bp_b100_002_000_000 = bp_b101_001_000_000 + AB[2] * bp_b100_001_000_000;
-    const double bp_b110_100_000_000 = acc[30] + AB[0] * acc[24];
-    const double bp_b010_100_000_000 = acc[24] + AB[0] * acc[21];
-    const double bp_b010_200_000_000 = bp_b110_100_000_000 + AB[0] * bp_b010_100_000_000;
-    const double bp_b010_010_000_000 = acc[25] + AB[1] * acc[21];
-    const double bp_b010_110_000_000 = bp_b110_010_000_000 + AB[0] * bp_b010_010_000_000;
-    const double bp_b020_010_000_000 = acc[32] + AB[1] * acc[25];
-    const double bp_b010_020_000_000 = bp_b020_010_000_000 + AB[1] * bp_b010_010_000_000;
-    const double bp_b010_001_000_000 = acc[27] + AB[2] * acc[21];
-    const double bp_b010_101_000_000 = bp_b110_001_000_000 + AB[0] * bp_b010_001_000_000;
-    const double bp_b020_001_000_000 = acc[35] + AB[2] * acc[25];
-    const double bp_b010_011_000_000 = bp_b020_001_000_000 + AB[1] * bp_b010_001_000_000;
-    const double bp_b011_001_000_000 = acc[37] + AB[2] * acc[27];
-    const double bp_b010_002_000_000 = bp_b011_001_000_000 + AB[2] * bp_b010_001_000_000;
-    const double bp_b101_100_000_000 = acc[33] + AB[0] * acc[26];
-    const double bp_b001_100_000_000 = acc[26] + AB[0] * acc[22];
-    const double bp_b001_200_000_000 = bp_b101_100_000_000 + AB[0] * bp_b001_100_000_000;
-    const double bp_b101_010_000_000 = acc[34] + AB[1] * acc[26];
-    const double bp_b001_010_000_000 = acc[27] + AB[1] * acc[22];
-    const double bp_b001_110_000_000 = bp_b101_010_000_000 + AB[0] * bp_b001_010_000_000;
-    const double bp_b011_010_000_000 = acc[35] + AB[1] * acc[27];
-    const double bp_b001_020_000_000 = bp_b011_010_000_000 + AB[1] * bp_b001_010_000_000;
-    const double bp_b001_001_000_000 = acc[28] + AB[2] * acc[22];
-    const double bp_b001_101_000_000 = bp_b101_001_000_000 + AB[0] * bp_b001_001_000_000;
-    const double bp_b001_011_000_000 = bp_b011_001_000_000 + AB[1] * bp_b001_001_000_000;
-    const double bp_b002_001_000_000 = acc[38] + AB[2] * acc[28];
-    const double bp_b001_002_000_000 = bp_b002_001_000_000 + AB[2] * bp_b001_001_000_000;
-    const double cp_b100_100_100_000 = acc[48] + AB[0] * acc[39];
-    const double cp_b100_100_010_000 = acc[49] + AB[0] * acc[40];
-    const double cp_b100_100_001_000 = acc[50] + AB[0] * acc[41];
-    const double cp_b100_010_100_000 = acc[51] + AB[1] * acc[39];
-    const double cp_b100_010_010_000 = acc[52] + AB[1] * acc[40];
-    const double cp_b100_010_001_000 = acc[53] + AB[1] * acc[41];
-    const double cp_b100_001_100_000 = acc[57] + AB[2] * acc[39];
-    const double cp_b100_001_010_000 = acc[58] + AB[2] * acc[40];
-    const double cp_b100_001_001_000 = acc[59] + AB[2] * acc[41];
-    const double cp_b010_100_100_000 = acc[51] + AB[0] * acc[42];
-    const double cp_b010_100_010_000 = acc[52] + AB[0] * acc[43];
-    const double cp_b010_100_001_000 = acc[53] + AB[0] * acc[44];
-    const double cp_b010_010_100_000 = acc[54] + AB[1] * acc[42];
-    const double cp_b010_010_010_000 = acc[55] + AB[1] * acc[43];
-    const double cp_b010_010_001_000 = acc[56] + AB[1] * acc[44];
-    const double cp_b010_001_100_000 = acc[60] + AB[2] * acc[42];
-    const double cp_b010_001_010_000 = acc[61] + AB[2] * acc[43];
-    const double cp_b010_001_001_000 = acc[62] + AB[2] * acc[44];
-    const double cp_b001_100_100_000 = acc[57] + AB[0] * acc[45];
-    const double cp_b001_100_010_000 = acc[58] + AB[0] * acc[46];
-    const double cp_b001_100_001_000 = acc[59] + AB[0] * acc[47];
-    const double cp_b001_010_100_000 = acc[60] + AB[1] * acc[45];
-    const double cp_b001_010_010_000 = acc[61] + AB[1] * acc[46];
-    const double cp_b001_010_001_000 = acc[62] + AB[1] * acc[47];
-    const double cp_b001_001_100_000 = acc[63] + AB[2] * acc[45];
-    const double cp_b001_001_010_000 = acc[64] + AB[2] * acc[46];
-    const double cp_b001_001_001_000 = acc[65] + AB[2] * acc[47];
+  // Dcd with 2 cons, Dbc and Dbd with hyb/2 cons; oc, od: first elements of the a-c and a-d blocks of P
+  template <class ET, class PT, class PU>
+  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a, const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, double rc, double rd, const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[1], const double (&Dbc)[3], const double (&Dbd)[3], double& W, double (&gP)[3], double (&gR)[3], double (&gS)[3]) {
+    double am = pref;
+    const double r000_0 = F[0] * am;
+    am *= m2a;
+    const double r000_1 = F[1] * am;
+    am *= m2a;
+    const double r000_2 = F[2] * am;
+    am *= m2a;
+    const double r000_3 = F[3] * am;
+    const double r100_2 = PQ[0] * r000_3;
+    const double r010_2 = PQ[1] * r000_3;
+    const double r001_2 = PQ[2] * r000_3;
+    const double r100_1 = PQ[0] * r000_2;
+    const double r010_1 = PQ[1] * r000_2;
+    const double r001_1 = PQ[2] * r000_2;
+    const double r200_1 = fma(1.0, r000_2, PQ[0] * r100_2);
+    const double r110_1 = PQ[0] * r010_2;
+    const double r101_1 = PQ[0] * r001_2;
+    const double r020_1 = fma(1.0, r000_2, PQ[1] * r010_2);
+    const double r011_1 = PQ[1] * r001_2;
+    const double r002_1 = fma(1.0, r000_2, PQ[2] * r001_2);
+    const double r100_0 = PQ[0] * r000_1;
+    const double r010_0 = PQ[1] * r000_1;
+    const double r001_0 = PQ[2] * r000_1;
+    const double r200_0 = fma(1.0, r000_1, PQ[0] * r100_1);
+    const double r110_0 = PQ[0] * r010_1;
+    const double r101_0 = PQ[0] * r001_1;
+    const double r020_0 = fma(1.0, r000_1, PQ[1] * r010_1);
+    const double r011_0 = PQ[1] * r001_1;
+    const double r002_0 = fma(1.0, r000_1, PQ[2] * r001_1);
+    const double r300_0 = fma(2.0, r100_1, PQ[0] * r200_1);
+    const double r210_0 = PQ[1] * r200_1;
+    const double r201_0 = PQ[2] * r200_1;
+    const double r120_0 = PQ[0] * r020_1;
+    const double r111_0 = PQ[0] * r011_1;
+    const double r102_0 = PQ[0] * r002_1;
+    const double r030_0 = fma(2.0, r010_1, PQ[1] * r020_1);
+    const double r021_0 = PQ[2] * r020_1;
+    const double r012_0 = PQ[1] * r002_1;
+    const double r003_0 = fma(2.0, r001_1, PQ[2] * r002_1);
+    double w = 0.0, px = 0.0, py = 0.0, pz = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
     {
-      const double gm = kCons[1][0] * kCons[1][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[0] * Dcd[0] - hh * (Dac[0] * Dbd[0] + Dad[0] * Dbc[0]));
-      g[0] += gm * (ap_b200_100_000_000 - 1.0 * am_b000_100_000_000);
-      g[3] += gm * (bp_b100_200_000_000 - 1.0 * acc[1]);
-      g[6] += gm * cp_b100_100_100_000;
-      g[1] += gm * ap_b110_100_000_000;
-      g[4] += gm * bp_b100_110_000_000;
-      g[7] += gm * cp_b100_100_010_000;
-      g[2] += gm * ap_b101_100_000_000;
-      g[5] += gm * bp_b100_101_000_000;
-      g[8] += gm * cp_b100_100_001_000;
+      const double ac0 = P[oc + 0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+      const double ad0 = P[od + 0 * n + 0] * (kCons[1][0] * kCons[0][0]);
+      {
+        const double ab = Pab[0 * n + 0] * (kCons[1][0] * kCons[1][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t201 = y000 * r201_0;
+        const double t210 = y000 * r210_0;
+        const double t300 = y000 * r300_0;
+        const double e0 = E[0];
+        const double e1 = E[1];
+        const double e2 = E[2];
+        w = fma(e2, t200, fma(e1, t100, fma(e0, t000, w)));
+        px = fma(e2, t300, fma(e1, t200, fma(e0, t100, px)));
+        py = fma(e2, t210, fma(e1, t110, fma(e0, t010, py)));
+        pz = fma(e2, t201, fma(e1, t101, fma(e0, t001, pz)));
+        sx = fma(E[4], t100, fma(E[3], t000, sx));
+      }
+      {
+        const double ab = Pab[0 * n + 1] * (kCons[1][0] * kCons[1][1]);
+        const double g0_0 = fma(-ad0, Dbc[1], fma(-ac0, Dbd[1], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t111 = y000 * r111_0;
+        const double t120 = y000 * r120_0;
+        const double t210 = y000 * r210_0;
+        const double e0 = E[5];
+        const double e1 = E[6];
+        const double e2 = E[7];
+        const double e3 = E[8];
+        w = fma(e3, t110, fma(e2, t100, fma(e1, t010, fma(e0, t000, w))));
+        px = fma(e3, t210, fma(e2, t200, fma(e1, t110, fma(e0, t100, px))));
+        py = fma(e3, t120, fma(e2, t110, fma(e1, t020, fma(e0, t010, py))));
+        pz = fma(e3, t111, fma(e2, t101, fma(e1, t011, fma(e0, t001, pz))));
+        sx = fma(E[10], t010, fma(E[9], t000, sx));
+        sy = fma(E[12], t100, fma(E[11], t000, sy));
+      }
+      {
+        const double ab = Pab[0 * n + 2] * (kCons[1][0] * kCons[1][2]);
+        const double g0_0 = fma(-ad0, Dbc[2], fma(-ac0, Dbd[2], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t102 = y000 * r102_0;
+        const double t111 = y000 * r111_0;
+        const double t201 = y000 * r201_0;
+        const double e0 = E[13];
+        const double e1 = E[14];
+        const double e2 = E[15];
+        const double e3 = E[16];
+        w = fma(e3, t101, fma(e2, t100, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t201, fma(e2, t200, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t111, fma(e2, t110, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t102, fma(e2, t101, fma(e1, t002, fma(e0, t001, pz))));
+        sx = fma(E[18], t001, fma(E[17], t000, sx));
+        sz = fma(E[20], t100, fma(E[19], t000, sz));
+      }
     }
     {
-      const double gm = kCons[1][0] * kCons[1][1] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[1] * Dcd[0] - hh * (Dac[0] * Dbd[1] + Dad[0] * Dbc[1]));
-      g[0] += gm * (ap_b200_010_000_000 - 1.0 * am_b000_010_000_000);
-      g[3] += gm * bp_b100_110_000_000;
-      g[6] += gm * cp_b100_010_100_000;
-      g[1] += gm * ap_b110_010_000_000;
-      g[4] += gm * (bp_b100_020_000_000 - 1.0 * acc[1]);
-      g[7] += gm * cp_b100_010_010_000;
-      g[2] += gm * ap_b101_010_000_000;
-      g[5] += gm * bp_b100_011_000_000;
-      g[8] += gm * cp_b100_010_001_000;
+      const double ac0 = P[oc + 1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+      const double ad0 = P[od + 1 * n + 0] * (kCons[1][1] * kCons[0][0]);
+      {
+        const double ab = Pab[1 * n + 0] * (kCons[1][1] * kCons[1][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t111 = y000 * r111_0;
+        const double t120 = y000 * r120_0;
+        const double t210 = y000 * r210_0;
+        const double e0 = E[21];
+        const double e1 = E[22];
+        const double e2 = E[23];
+        const double e3 = E[24];
+        w = fma(e3, t110, fma(e2, t100, fma(e1, t010, fma(e0, t000, w))));
+        px = fma(e3, t210, fma(e2, t200, fma(e1, t110, fma(e0, t100, px))));
+        py = fma(e3, t120, fma(e2, t110, fma(e1, t020, fma(e0, t010, py))));
+        pz = fma(e3, t111, fma(e2, t101, fma(e1, t011, fma(e0, t001, pz))));
+        sx = fma(E[26], t010, fma(E[25], t000, sx));
+        sy = fma(E[28], t100, fma(E[27], t000, sy));
+      }
+      {
+        const double ab = Pab[1 * n + 1] * (kCons[1][1] * kCons[1][1]);
+        const double g0_0 = fma(-ad0, Dbc[1], fma(-ac0, Dbd[1], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t110 = y000 * r110_0;
+        const double t021 = y000 * r021_0;
+        const double t030 = y000 * r030_0;
+        const double t120 = y000 * r120_0;
+        const double e0 = E[29];
+        const double e1 = E[30];
+        const double e2 = E[31];
+        w = fma(e2, t020, fma(e1, t010, fma(e0, t000, w)));
+        px = fma(e2, t120, fma(e1, t110, fma(e0, t100, px)));
+        py = fma(e2, t030, fma(e1, t020, fma(e0, t010, py)));
+        pz = fma(e2, t021, fma(e1, t011, fma(e0, t001, pz)));
+        sy = fma(E[33], t010, fma(E[32], t000, sy));
+      }
+      {
+        const double ab = Pab[1 * n + 2] * (kCons[1][1] * kCons[1][2]);
+        const double g0_0 = fma(-ad0, Dbc[2], fma(-ac0, Dbd[2], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t012 = y000 * r012_0;
+        const double t021 = y000 * r021_0;
+        const double t111 = y000 * r111_0;
+        const double e0 = E[34];
+        const double e1 = E[35];
+        const double e2 = E[36];
+        const double e3 = E[37];
+        w = fma(e3, t011, fma(e2, t010, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t111, fma(e2, t110, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t021, fma(e2, t020, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t012, fma(e2, t011, fma(e1, t002, fma(e0, t001, pz))));
+        sy = fma(E[39], t001, fma(E[38], t000, sy));
+        sz = fma(E[41], t010, fma(E[40], t000, sz));
+      }
     }
     {
-      const double gm = kCons[1][0] * kCons[1][2] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[2] * Dcd[0] - hh * (Dac[0] * Dbd[2] + Dad[0] * Dbc[2]));
-      g[0] += gm * (ap_b200_001_000_000 - 1.0 * am_b000_001_000_000);
-      g[3] += gm * bp_b100_101_000_000;
-      g[6] += gm * cp_b100_001_100_000;
-      g[1] += gm * ap_b110_001_000_000;
-      g[4] += gm * bp_b100_011_000_000;
-      g[7] += gm * cp_b100_001_010_000;
-      g[2] += gm * ap_b101_001_000_000;
-      g[5] += gm * (bp_b100_002_000_000 - 1.0 * acc[1]);
-      g[8] += gm * cp_b100_001_001_000;
+      const double ac0 = P[oc + 2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+      const double ad0 = P[od + 2 * n + 0] * (kCons[1][2] * kCons[0][0]);
+      {
+        const double ab = Pab[2 * n + 0] * (kCons[1][2] * kCons[1][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t102 = y000 * r102_0;
+        const double t111 = y000 * r111_0;
+        const double t201 = y000 * r201_0;
+        const double e0 = E[42];
+        const double e1 = E[43];
+        const double e2 = E[44];
+        const double e3 = E[45];
+        w = fma(e3, t101, fma(e2, t100, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t201, fma(e2, t200, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t111, fma(e2, t110, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t102, fma(e2, t101, fma(e1, t002, fma(e0, t001, pz))));
+        sx = fma(E[47], t001, fma(E[46], t000, sx));
+        sz = fma(E[49], t100, fma(E[48], t000, sz));
+      }
+      {
+        const double ab = Pab[2 * n + 1] * (kCons[1][2] * kCons[1][1]);
+        const double g0_0 = fma(-ad0, Dbc[1], fma(-ac0, Dbd[1], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t012 = y000 * r012_0;
+        const double t021 = y000 * r021_0;
+        const double t111 = y000 * r111_0;
+        const double e0 = E[50];
+        const double e1 = E[51];
+        const double e2 = E[52];
+        const double e3 = E[53];
+        w = fma(e3, t011, fma(e2, t010, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t111, fma(e2, t110, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t021, fma(e2, t020, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t012, fma(e2, t011, fma(e1, t002, fma(e0, t001, pz))));
+        sy = fma(E[55], t001, fma(E[54], t000, sy));
+        sz = fma(E[57], t010, fma(E[56], t000, sz));
+      }
+      {
+        const double ab = Pab[2 * n + 2] * (kCons[1][2] * kCons[1][2]);
+        const double g0_0 = fma(-ad0, Dbc[2], fma(-ac0, Dbd[2], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t101 = y000 * r101_0;
+        const double t003 = y000 * r003_0;
+        const double t012 = y000 * r012_0;
+        const double t102 = y000 * r102_0;
+        const double e0 = E[58];
+        const double e1 = E[59];
+        const double e2 = E[60];
+        w = fma(e2, t002, fma(e1, t001, fma(e0, t000, w)));
+        px = fma(e2, t102, fma(e1, t101, fma(e0, t100, px)));
+        py = fma(e2, t012, fma(e1, t011, fma(e0, t010, py)));
+        pz = fma(e2, t003, fma(e1, t002, fma(e0, t001, pz)));
+        sz = fma(E[62], t001, fma(E[61], t000, sz));
+      }
     }
-    {
-      const double gm = kCons[1][1] * kCons[1][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[3] * Dcd[0] - hh * (Dac[1] * Dbd[0] + Dad[1] * Dbc[0]));
-      g[0] += gm * ap_b110_100_000_000;
-      g[3] += gm * (bp_b010_200_000_000 - 1.0 * acc[2]);
-      g[6] += gm * cp_b010_100_100_000;
-      g[1] += gm * (ap_b020_100_000_000 - 1.0 * am_b000_100_000_000);
-      g[4] += gm * bp_b010_110_000_000;
-      g[7] += gm * cp_b010_100_010_000;
-      g[2] += gm * ap_b011_100_000_000;
-      g[5] += gm * bp_b010_101_000_000;
-      g[8] += gm * cp_b010_100_001_000;
-    }
-    {
-      const double gm = kCons[1][1] * kCons[1][1] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[4] * Dcd[0] - hh * (Dac[1] * Dbd[1] + Dad[1] * Dbc[1]));
-      g[0] += gm * ap_b110_010_000_000;
-      g[3] += gm * bp_b010_110_000_000;
-      g[6] += gm * cp_b010_010_100_000;
-      g[1] += gm * (ap_b020_010_000_000 - 1.0 * am_b000_010_000_000);
-      g[4] += gm * (bp_b010_020_000_000 - 1.0 * acc[2]);
-      g[7] += gm * cp_b010_010_010_000;
-      g[2] += gm * ap_b011_010_000_000;
-      g[5] += gm * bp_b010_011_000_000;
-      g[8] += gm * cp_b010_010_001_000;
-    }
-    {
-      const double gm = kCons[1][1] * kCons[1][2] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[5] * Dcd[0] - hh * (Dac[1] * Dbd[2] + Dad[1] * Dbc[2]));
-      g[0] += gm * ap_b110_001_000_000;
-      g[3] += gm * bp_b010_101_000_000;
-      g[6] += gm * cp_b010_001_100_000;
-      g[1] += gm * (ap_b020_001_000_000 - 1.0 * am_b000_001_000_000);
-      g[4] += gm * bp_b010_011_000_000;
-      g[7] += gm * cp_b010_001_010_000;
-      g[2] += gm * ap_b011_001_000_000;
-      g[5] += gm * (bp_b010_002_000_000 - 1.0 * acc[2]);
-      g[8] += gm * cp_b010_001_001_000;
-    }
-    {
-      const double gm = kCons[1][2] * kCons[1][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[6] * Dcd[0] - hh * (Dac[2] * Dbd[0] + Dad[2] * Dbc[0]));
-      g[0] += gm * ap_b101_100_000_000;
-      g[3] += gm * (bp_b001_200_000_000 - 1.0 * acc[3]);
-      g[6] += gm * cp_b001_100_100_000;
-      g[1] += gm * ap_b011_100_000_000;
-      g[4] += gm * bp_b001_110_000_000;
-      g[7] += gm * cp_b001_100_010_000;
-      g[2] += gm * (ap_b002_100_000_000 - 1.0 * am_b000_100_000_000);
-      g[5] += gm * bp_b001_101_000_000;
-      g[8] += gm * cp_b001_100_001_000;
-    }
-    {
-      const double gm = kCons[1][2] * kCons[1][1] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[7] * Dcd[0] - hh * (Dac[2] * Dbd[1] + Dad[2] * Dbc[1]));
-      g[0] += gm * ap_b101_010_000_000;
-      g[3] += gm * bp_b001_110_000_000;
-      g[6] += gm * cp_b001_010_100_000;
-      g[1] += gm * ap_b011_010_000_000;
-      g[4] += gm * (bp_b001_020_000_000 - 1.0 * acc[3]);
-      g[7] += gm * cp_b001_010_010_000;
-      g[2] += gm * (ap_b002_010_000_000 - 1.0 * am_b000_010_000_000);
-      g[5] += gm * bp_b001_011_000_000;
-      g[8] += gm * cp_b001_010_001_000;
-    }
-    {
-      const double gm = kCons[1][2] * kCons[1][2] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[8] * Dcd[0] - hh * (Dac[2] * Dbd[2] + Dad[2] * Dbc[2]));
-      g[0] += gm * ap_b101_001_000_000;
-      g[3] += gm * bp_b001_101_000_000;
-      g[6] += gm * cp_b001_001_100_000;
-      g[1] += gm * ap_b011_001_000_000;
-      g[4] += gm * bp_b001_011_000_000;
-      g[7] += gm * cp_b001_001_010_000;
-      g[2] += gm * (ap_b002_001_000_000 - 1.0 * am_b000_001_000_000);
-      g[5] += gm * (bp_b001_002_000_000 - 1.0 * acc[3]);
-      g[8] += gm * cp_b001_001_001_000;
-    }
+    W = w;
+    gP[0] = px; gP[1] = py; gP[2] = pz;
+    gR[0] = sx; gR[1] = sy; gR[2] = sz;
+    gS[0] = 0.0;
+    gS[1] = 0.0;
+    gS[2] = 0.0;
   }
 };
+__device__ const unsigned kC1100GradMd_index[63] = {7,8,9,10,11,260,516,261,517,262,518,772,773,65540,131076,65541,131077,65542,131078,196612,196613,1025,1281,1026,1282,1027,1283,1537,1538,1792,2048,2304,2560,2816,66560,132096,66816,132352,67072,132608,197632,197888,262145,327681,262146,327682,262147,327683,393217,393218,262400,327936,262656,328192,262912,328448,393472,393728,458752,524288,589824,655360,720896};
+__device__ inline const unsigned* C1100GradMd::index() { return kC1100GradMd_index; }
 }  // namespace qf

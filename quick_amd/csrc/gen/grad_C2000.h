@@ -28,203 +28,258 @@ __device__ inline const int* C2000Grad::vlev() { return kC2000Grad_vlev; }
 __device__ inline const GradAcc* C2000Grad::acc() { return kC2000Grad_acc; }
 __device__ inline const CoopHNode* C2000Grad::hrr() { return kC2000Grad_hrr; }
 __device__ inline const int* C2000Grad::hlev() { return kC2000Grad_hlev; }
-struct C2000GradLane {
+// (ds|ss): 20 Hermite Coulomb integrals, 39 bra products
+struct C2000GradMd {
   static constexpr int La = 2, Lb = 0, Lc = 0, Ld = 0, L = 3;
-  static constexpr int NACC = 47;
-  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC
-  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p, const double (&w)[4], double (&acc)[NACC]) {
-    const double v000_000_3 = F[3];
-    const double v000_000_2 = F[2];
-    const double v000_000_1 = F[1];
-    const double v000_000_0 = F[0];
-    const double v001_000_2 = p.PA[2] * v000_000_2 + p.WP[2] * v000_000_3;
-    const double v010_000_2 = p.PA[1] * v000_000_2 + p.WP[1] * v000_000_3;
-    const double v100_000_2 = p.PA[0] * v000_000_2 + p.WP[0] * v000_000_3;
-    const double v001_000_1 = p.PA[2] * v000_000_1 + p.WP[2] * v000_000_2;
-    const double v010_000_1 = p.PA[1] * v000_000_1 + p.WP[1] * v000_000_2;
-    const double v100_000_1 = p.PA[0] * v000_000_1 + p.WP[0] * v000_000_2;
-    const double v001_000_0 = p.PA[2] * v000_000_0 + p.WP[2] * v000_000_1;
-    const double v010_000_0 = p.PA[1] * v000_000_0 + p.WP[1] * v000_000_1;
-    const double v100_000_0 = p.PA[0] * v000_000_0 + p.WP[0] * v000_000_1;
-    const double v002_000_1 = p.PA[2] * v001_000_1 + p.WP[2] * v001_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v011_000_1 = p.PA[1] * v001_000_1 + p.WP[1] * v001_000_2;
-    const double v020_000_1 = p.PA[1] * v010_000_1 + p.WP[1] * v010_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v101_000_1 = p.PA[0] * v001_000_1 + p.WP[0] * v001_000_2;
-    const double v110_000_1 = p.PA[0] * v010_000_1 + p.WP[0] * v010_000_2;
-    const double v200_000_1 = p.PA[0] * v100_000_1 + p.WP[0] * v100_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v002_000_0 = p.PA[2] * v001_000_0 + p.WP[2] * v001_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v011_000_0 = p.PA[1] * v001_000_0 + p.WP[1] * v001_000_1;
-    const double v020_000_0 = p.PA[1] * v010_000_0 + p.WP[1] * v010_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v101_000_0 = p.PA[0] * v001_000_0 + p.WP[0] * v001_000_1;
-    const double v110_000_0 = p.PA[0] * v010_000_0 + p.WP[0] * v010_000_1;
-    const double v200_000_0 = p.PA[0] * v100_000_0 + p.WP[0] * v100_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v003_000_0 = p.PA[2] * v002_000_0 + p.WP[2] * v002_000_1 + double(2) * p.oo2z * (v001_000_0 - p.rz * v001_000_1);
-    const double v012_000_0 = p.PA[1] * v002_000_0 + p.WP[1] * v002_000_1;
-    const double v021_000_0 = p.PA[2] * v020_000_0 + p.WP[2] * v020_000_1;
-    const double v030_000_0 = p.PA[1] * v020_000_0 + p.WP[1] * v020_000_1 + double(2) * p.oo2z * (v010_000_0 - p.rz * v010_000_1);
-    const double v102_000_0 = p.PA[0] * v002_000_0 + p.WP[0] * v002_000_1;
-    const double v111_000_0 = p.PA[0] * v011_000_0 + p.WP[0] * v011_000_1;
-    const double v120_000_0 = p.PA[0] * v020_000_0 + p.WP[0] * v020_000_1;
-    const double v201_000_0 = p.PA[2] * v200_000_0 + p.WP[2] * v200_000_1;
-    const double v210_000_0 = p.PA[1] * v200_000_0 + p.WP[1] * v200_000_1;
-    const double v300_000_0 = p.PA[0] * v200_000_0 + p.WP[0] * v200_000_1 + double(2) * p.oo2z * (v100_000_0 - p.rz * v100_000_1);
-    const double v002_001_0 = p.QC[2] * v002_000_0 + p.WQ[2] * v002_000_1 + double(2) * p.oo2zn * v001_000_1;
-    const double v002_010_0 = p.QC[1] * v002_000_0 + p.WQ[1] * v002_000_1;
-    const double v002_100_0 = p.QC[0] * v002_000_0 + p.WQ[0] * v002_000_1;
-    const double v011_001_0 = p.QC[2] * v011_000_0 + p.WQ[2] * v011_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v011_010_0 = p.QC[1] * v011_000_0 + p.WQ[1] * v011_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v011_100_0 = p.QC[0] * v011_000_0 + p.WQ[0] * v011_000_1;
-    const double v020_001_0 = p.QC[2] * v020_000_0 + p.WQ[2] * v020_000_1;
-    const double v020_010_0 = p.QC[1] * v020_000_0 + p.WQ[1] * v020_000_1 + double(2) * p.oo2zn * v010_000_1;
-    const double v020_100_0 = p.QC[0] * v020_000_0 + p.WQ[0] * v020_000_1;
-    const double v101_001_0 = p.QC[2] * v101_000_0 + p.WQ[2] * v101_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v101_010_0 = p.QC[1] * v101_000_0 + p.WQ[1] * v101_000_1;
-    const double v101_100_0 = p.QC[0] * v101_000_0 + p.WQ[0] * v101_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v110_001_0 = p.QC[2] * v110_000_0 + p.WQ[2] * v110_000_1;
-    const double v110_010_0 = p.QC[1] * v110_000_0 + p.WQ[1] * v110_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v110_100_0 = p.QC[0] * v110_000_0 + p.WQ[0] * v110_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v200_001_0 = p.QC[2] * v200_000_0 + p.WQ[2] * v200_000_1;
-    const double v200_010_0 = p.QC[1] * v200_000_0 + p.WQ[1] * v200_000_1;
-    const double v200_100_0 = p.QC[0] * v200_000_0 + p.WQ[0] * v200_000_1 + double(2) * p.oo2zn * v100_000_1;
-    acc[0] += w[0] * v100_000_0;
-    acc[1] += w[0] * v010_000_0;
-    acc[2] += w[0] * v001_000_0;
-    acc[3] += w[1] * v300_000_0;
-    acc[4] += w[1] * v210_000_0;
-    acc[5] += w[1] * v120_000_0;
-    acc[6] += w[1] * v030_000_0;
-    acc[7] += w[1] * v201_000_0;
-    acc[8] += w[1] * v111_000_0;
-    acc[9] += w[1] * v021_000_0;
-    acc[10] += w[1] * v102_000_0;
-    acc[11] += w[1] * v012_000_0;
-    acc[12] += w[1] * v003_000_0;
-    acc[13] += w[2] * v200_000_0;
-    acc[14] += w[2] * v110_000_0;
-    acc[15] += w[2] * v020_000_0;
-    acc[16] += w[2] * v101_000_0;
-    acc[17] += w[2] * v011_000_0;
-    acc[18] += w[2] * v002_000_0;
-    acc[19] += w[2] * v300_000_0;
-    acc[20] += w[2] * v210_000_0;
-    acc[21] += w[2] * v120_000_0;
-    acc[22] += w[2] * v030_000_0;
-    acc[23] += w[2] * v201_000_0;
-    acc[24] += w[2] * v111_000_0;
-    acc[25] += w[2] * v021_000_0;
-    acc[26] += w[2] * v102_000_0;
-    acc[27] += w[2] * v012_000_0;
-    acc[28] += w[2] * v003_000_0;
-    acc[29] += w[3] * v200_100_0;
-    acc[30] += w[3] * v200_010_0;
-    acc[31] += w[3] * v200_001_0;
-    acc[32] += w[3] * v110_100_0;
-    acc[33] += w[3] * v110_010_0;
-    acc[34] += w[3] * v110_001_0;
-    acc[35] += w[3] * v020_100_0;
-    acc[36] += w[3] * v020_010_0;
-    acc[37] += w[3] * v020_001_0;
-    acc[38] += w[3] * v101_100_0;
-    acc[39] += w[3] * v101_010_0;
-    acc[40] += w[3] * v101_001_0;
-    acc[41] += w[3] * v011_100_0;
-    acc[42] += w[3] * v011_010_0;
-    acc[43] += w[3] * v011_001_0;
-    acc[44] += w[3] * v002_100_0;
-    acc[45] += w[3] * v002_010_0;
-    acc[46] += w[3] * v002_001_0;
+  static constexpr int N1 = 9, NE = 39;   // 1D entries per direction, product table
+  static constexpr int MIN_WAVES = 2;      // waves per SIMD the register budget targets
+  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16
+  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p, rx = -beta/p, ry = alpha/p
+  template <class T>
+  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, double rx, double ry, T out) {
+    const double be100 = X;
+    const double be101 = h;
+    const double bd100 = rx;
+    const double be200 = fma(1.0, be101, be100 * X);
+    const double be201 = fma(be100, h, be101 * X);
+    const double be202 = be101 * h;
+    const double bd200 = fma(be100, rx, bd100 * X);
+    const double bd201 = fma(be101, rx, bd100 * h);
+    out[0] = 1.0;
+    out[1] = be100;
+    out[2] = be101;
+    out[3] = bd100;
+    out[4] = be200;
+    out[5] = be201;
+    out[6] = be202;
+    out[7] = bd200;
+    out[8] = bd201;
   }
-  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3], const double (&CD)[3], const double (&Dab)[6], const double (&Dcd)[1], const double (&Dac)[6], const double (&Dad)[6], const double (&Dbc)[1], const double (&Dbd)[1], double hh, double (&g)[9]) {
-    const double bp_b200_100_000_000 = acc[19] + AB[0] * acc[13];
-    const double bp_b200_010_000_000 = acc[20] + AB[1] * acc[13];
-    const double bp_b200_001_000_000 = acc[23] + AB[2] * acc[13];
-    const double bp_b110_100_000_000 = acc[20] + AB[0] * acc[14];
-    const double bp_b110_010_000_000 = acc[21] + AB[1] * acc[14];
-    const double bp_b110_001_000_000 = acc[24] + AB[2] * acc[14];
-    const double bp_b020_100_000_000 = acc[21] + AB[0] * acc[15];
-    const double bp_b020_010_000_000 = acc[22] + AB[1] * acc[15];
-    const double bp_b020_001_000_000 = acc[25] + AB[2] * acc[15];
-    const double bp_b101_100_000_000 = acc[23] + AB[0] * acc[16];
-    const double bp_b101_010_000_000 = acc[24] + AB[1] * acc[16];
-    const double bp_b101_001_000_000 = acc[26] + AB[2] * acc[16];
-    const double bp_b011_100_000_000 = acc[24] + AB[0] * acc[17];
-    const double bp_b011_010_000_000 = acc[25] + AB[1] * acc[17];
-    const double bp_b011_001_000_000 = acc[27] + AB[2] * acc[17];
-    const double bp_b002_100_000_000 = acc[26] + AB[0] * acc[18];
-    const double bp_b002_010_000_000 = acc[27] + AB[1] * acc[18];
-    const double bp_b002_001_000_000 = acc[28] + AB[2] * acc[18];
+  // Dcd with 2 cons, Dbc and Dbd with hyb/2 cons; oc, od: first elements of the a-c and a-d blocks of P
+  template <class ET, class PT, class PU>
+  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a, const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, double rc, double rd, const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[1], const double (&Dbc)[1], const double (&Dbd)[1], double& W, double (&gP)[3], double (&gR)[3], double (&gS)[3]) {
+    double am = pref;
+    const double r000_0 = F[0] * am;
+    am *= m2a;
+    const double r000_1 = F[1] * am;
+    am *= m2a;
+    const double r000_2 = F[2] * am;
+    am *= m2a;
+    const double r000_3 = F[3] * am;
+    const double r100_2 = PQ[0] * r000_3;
+    const double r010_2 = PQ[1] * r000_3;
+    const double r001_2 = PQ[2] * r000_3;
+    const double r100_1 = PQ[0] * r000_2;
+    const double r010_1 = PQ[1] * r000_2;
+    const double r001_1 = PQ[2] * r000_2;
+    const double r200_1 = fma(1.0, r000_2, PQ[0] * r100_2);
+    const double r110_1 = PQ[0] * r010_2;
+    const double r101_1 = PQ[0] * r001_2;
+    const double r020_1 = fma(1.0, r000_2, PQ[1] * r010_2);
+    const double r011_1 = PQ[1] * r001_2;
+    const double r002_1 = fma(1.0, r000_2, PQ[2] * r001_2);
+    const double r100_0 = PQ[0] * r000_1;
+    const double r010_0 = PQ[1] * r000_1;
+    const double r001_0 = PQ[2] * r000_1;
+    const double r200_0 = fma(1.0, r000_1, PQ[0] * r100_1);
+    const double r110_0 = PQ[0] * r010_1;
+    const double r101_0 = PQ[0] * r001_1;
+    const double r020_0 = fma(1.0, r000_1, PQ[1] * r010_1);
+    const double r011_0 = PQ[1] * r001_1;
+    const double r002_0 = fma(1.0, r000_1, PQ[2] * r001_1);
+    const double r300_0 = fma(2.0, r100_1, PQ[0] * r200_1);
+    const double r210_0 = PQ[1] * r200_1;
+    const double r201_0 = PQ[2] * r200_1;
+    const double r120_0 = PQ[0] * r020_1;
+    const double r111_0 = PQ[0] * r011_1;
+    const double r102_0 = PQ[0] * r002_1;
+    const double r030_0 = fma(2.0, r010_1, PQ[1] * r020_1);
+    const double r021_0 = PQ[2] * r020_1;
+    const double r012_0 = PQ[1] * r002_1;
+    const double r003_0 = fma(2.0, r001_1, PQ[2] * r002_1);
+    double w = 0.0, px = 0.0, py = 0.0, pz = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
     {
-      const double gm = kCons[2][0] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[0] * Dcd[0] - hh * (Dac[0] * Dbd[0] + Dad[0] * Dbc[0]));
-      g[0] += gm * (acc[3] - 2.0 * acc[0]);
-      g[3] += gm * bp_b200_100_000_000;
-      g[6] += gm * acc[29];
-      g[1] += gm * acc[4];
-      g[4] += gm * bp_b200_010_000_000;
-      g[7] += gm * acc[30];
-      g[2] += gm * acc[7];
-      g[5] += gm * bp_b200_001_000_000;
-      g[8] += gm * acc[31];
+      const double ac0 = P[oc + 0 * n + 0] * (kCons[2][0] * kCons[0][0]);
+      const double ad0 = P[od + 0 * n + 0] * (kCons[2][0] * kCons[0][0]);
+      {
+        const double ab = Pab[0 * n + 0] * (kCons[2][0] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t201 = y000 * r201_0;
+        const double t210 = y000 * r210_0;
+        const double t300 = y000 * r300_0;
+        const double e0 = E[0];
+        const double e1 = E[1];
+        const double e2 = E[2];
+        w = fma(e2, t200, fma(e1, t100, fma(e0, t000, w)));
+        px = fma(e2, t300, fma(e1, t200, fma(e0, t100, px)));
+        py = fma(e2, t210, fma(e1, t110, fma(e0, t010, py)));
+        pz = fma(e2, t201, fma(e1, t101, fma(e0, t001, pz)));
+        sx = fma(E[4], t100, fma(E[3], t000, sx));
+      }
     }
     {
-      const double gm = kCons[2][1] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[1] * Dcd[0] - hh * (Dac[1] * Dbd[0] + Dad[1] * Dbc[0]));
-      g[0] += gm * (acc[4] - 1.0 * acc[1]);
-      g[3] += gm * bp_b110_100_000_000;
-      g[6] += gm * acc[32];
-      g[1] += gm * (acc[5] - 1.0 * acc[0]);
-      g[4] += gm * bp_b110_010_000_000;
-      g[7] += gm * acc[33];
-      g[2] += gm * acc[8];
-      g[5] += gm * bp_b110_001_000_000;
-      g[8] += gm * acc[34];
+      const double ac0 = P[oc + 1 * n + 0] * (kCons[2][1] * kCons[0][0]);
+      const double ad0 = P[od + 1 * n + 0] * (kCons[2][1] * kCons[0][0]);
+      {
+        const double ab = Pab[1 * n + 0] * (kCons[2][1] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t111 = y000 * r111_0;
+        const double t120 = y000 * r120_0;
+        const double t210 = y000 * r210_0;
+        const double e0 = E[5];
+        const double e1 = E[6];
+        const double e2 = E[7];
+        const double e3 = E[8];
+        w = fma(e3, t110, fma(e2, t100, fma(e1, t010, fma(e0, t000, w))));
+        px = fma(e3, t210, fma(e2, t200, fma(e1, t110, fma(e0, t100, px))));
+        py = fma(e3, t120, fma(e2, t110, fma(e1, t020, fma(e0, t010, py))));
+        pz = fma(e3, t111, fma(e2, t101, fma(e1, t011, fma(e0, t001, pz))));
+        sx = fma(E[10], t010, fma(E[9], t000, sx));
+        sy = fma(E[12], t100, fma(E[11], t000, sy));
+      }
     }
     {
-      const double gm = kCons[2][2] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[2] * Dcd[0] - hh * (Dac[2] * Dbd[0] + Dad[2] * Dbc[0]));
-      g[0] += gm * acc[5];
-      g[3] += gm * bp_b020_100_000_000;
-      g[6] += gm * acc[35];
-      g[1] += gm * (acc[6] - 2.0 * acc[1]);
-      g[4] += gm * bp_b020_010_000_000;
-      g[7] += gm * acc[36];
-      g[2] += gm * acc[9];
-      g[5] += gm * bp_b020_001_000_000;
-      g[8] += gm * acc[37];
+      const double ac0 = P[oc + 2 * n + 0] * (kCons[2][2] * kCons[0][0]);
+      const double ad0 = P[od + 2 * n + 0] * (kCons[2][2] * kCons[0][0]);
+      {
+        const double ab = Pab[2 * n + 0] * (kCons[2][2] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t110 = y000 * r110_0;
+        const double t021 = y000 * r021_0;
+        const double t030 = y000 * r030_0;
+        const double t120 = y000 * r120_0;
+        const double e0 = E[13];
+        const double e1 = E[14];
+        const double e2 = E[15];
+        w = fma(e2, t020, fma(e1, t010, fma(e0, t000, w)));
+        px = fma(e2, t120, fma(e1, t110, fma(e0, t100, px)));
+        py = fma(e2, t030, fma(e1, t020, fma(e0, t010, py)));
+        pz = fma(e2, t021, fma(e1, t011, fma(e0, t001, pz)));
+        sy = fma(E[17], t010, fma(E[16], t000, sy));
+      }
     }
     {
-      const double gm = kCons[2][3] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[3] * Dcd[0] - hh * (Dac[3] * Dbd[0] + Dad[3] * Dbc[0]));
-      g[0] += gm * (acc[7] - 1.0 * acc[2]);
-      g[3] += gm * bp_b101_100_000_000;
-      g[6] += gm * acc[38];
-      g[1] += gm * acc[8];
-      g[4] += gm * bp_b101_010_000_000;
-      g[7] += gm * acc[39];
-      g[2] += gm * (acc[10] - 1.0 * acc[0]);
-      g[5] += gm * bp_b101_001_000_000;
-      g[8] += gm * acc[40];
+      const double ac0 = P[oc + 3 * n + 0] * (kCons[2][3] * kCons[0][0]);
+      const double ad0 = P[od + 3 * n + 0] * (kCons[2][3] * kCons[0][0]);
+      {
+        const double ab = Pab[3 * n + 0] * (kCons[2][3] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t200 = y000 * r200_0;
+        const double t102 = y000 * r102_0;
+        const double t111 = y000 * r111_0;
+        const double t201 = y000 * r201_0;
+        const double e0 = E[18];
+        const double e1 = E[19];
+        const double e2 = E[20];
+        const double e3 = E[21];
+        w = fma(e3, t101, fma(e2, t100, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t201, fma(e2, t200, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t111, fma(e2, t110, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t102, fma(e2, t101, fma(e1, t002, fma(e0, t001, pz))));
+        sx = fma(E[23], t001, fma(E[22], t000, sx));
+        sz = fma(E[25], t100, fma(E[24], t000, sz));
+      }
     }
     {
-      const double gm = kCons[2][4] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[4] * Dcd[0] - hh * (Dac[4] * Dbd[0] + Dad[4] * Dbc[0]));
-      g[0] += gm * acc[8];
-      g[3] += gm * bp_b011_100_000_000;
-      g[6] += gm * acc[41];
-      g[1] += gm * (acc[9] - 1.0 * acc[2]);
-      g[4] += gm * bp_b011_010_000_000;
-      g[7] += gm * acc[42];
-      g[2] += gm * (acc[11] - 1.0 * acc[1]);
-      g[5] += gm * bp_b011_001_000_000;
-      g[8] += gm * acc[43];
+      const double ac0 = P[oc + 4 * n + 0] * (kCons[2][4] * kCons[0][0]);
+      const double ad0 = P[od + 4 * n + 0] * (kCons[2][4] * kCons[0][0]);
+      {
+        const double ab = Pab[4 * n + 0] * (kCons[2][4] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t020 = y000 * r020_0;
+        const double t101 = y000 * r101_0;
+        const double t110 = y000 * r110_0;
+        const double t012 = y000 * r012_0;
+        const double t021 = y000 * r021_0;
+        const double t111 = y000 * r111_0;
+        const double e0 = E[26];
+        const double e1 = E[27];
+        const double e2 = E[28];
+        const double e3 = E[29];
+        w = fma(e3, t011, fma(e2, t010, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t111, fma(e2, t110, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t021, fma(e2, t020, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t012, fma(e2, t011, fma(e1, t002, fma(e0, t001, pz))));
+        sy = fma(E[31], t001, fma(E[30], t000, sy));
+        sz = fma(E[33], t010, fma(E[32], t000, sz));
+      }
     }
     {
-      const double gm = kCons[2][5] * kCons[0][0] * kCons[0][0] * kCons[0][0] * (2.0 * Dab[5] * Dcd[0] - hh * (Dac[5] * Dbd[0] + Dad[5] * Dbc[0]));
-      g[0] += gm * acc[10];
-      g[3] += gm * bp_b002_100_000_000;
-      g[6] += gm * acc[44];
-      g[1] += gm * acc[11];
-      g[4] += gm * bp_b002_010_000_000;
-      g[7] += gm * acc[45];
-      g[2] += gm * (acc[12] - 2.0 * acc[2]);
-      g[5] += gm * bp_b002_001_000_000;
-      g[8] += gm * acc[46];
+      const double ac0 = P[oc + 5 * n + 0] * (kCons[2][5] * kCons[0][0]);
+      const double ad0 = P[od + 5 * n + 0] * (kCons[2][5] * kCons[0][0]);
+      {
+        const double ab = Pab[5 * n + 0] * (kCons[2][5] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double y000 = g0_0;
+        const double t000 = y000 * r000_0;
+        const double t001 = y000 * r001_0;
+        const double t010 = y000 * r010_0;
+        const double t100 = y000 * r100_0;
+        const double t002 = y000 * r002_0;
+        const double t011 = y000 * r011_0;
+        const double t101 = y000 * r101_0;
+        const double t003 = y000 * r003_0;
+        const double t012 = y000 * r012_0;
+        const double t102 = y000 * r102_0;
+        const double e0 = E[34];
+        const double e1 = E[35];
+        const double e2 = E[36];
+        w = fma(e2, t002, fma(e1, t001, fma(e0, t000, w)));
+        px = fma(e2, t102, fma(e1, t101, fma(e0, t100, px)));
+        py = fma(e2, t012, fma(e1, t011, fma(e0, t010, py)));
+        pz = fma(e2, t003, fma(e1, t002, fma(e0, t001, pz)));
+        sz = fma(E[38], t001, fma(E[37], t000, sz));
+      }
     }
+    W = w;
+    gP[0] = px; gP[1] = py; gP[2] = pz;
+    gR[0] = sx; gR[1] = sy; gR[2] = sz;
+    gS[0] = 0.0;
+    gS[1] = 0.0;
+    gS[2] = 0.0;
   }
 };
+__device__ const unsigned kC2000GradMd_index[39] = {4,5,6,7,8,257,513,258,514,259,515,769,770,1024,1280,1536,1792,2048,65537,131073,65538,131074,65539,131075,196609,196610,65792,131328,66048,131584,66304,131840,196864,197120,262144,327680,393216,458752,524288};
+__device__ inline const unsigned* C2000GradMd::index() { return kC2000GradMd_index; }
 }  // namespace qf

@@ -28,587 +28,380 @@ __device__ inline const int* C2010Grad::vlev() { return kC2010Grad_vlev; }
 __device__ inline const GradAcc* C2010Grad::acc() { return kC2010Grad_acc; }
 __device__ inline const CoopHNode* C2010Grad::hrr() { return kC2010Grad_hrr; }
 __device__ inline const int* C2010Grad::hlev() { return kC2010Grad_hlev; }
-struct C2010GradLane {
+// (ds|ps): 35 Hermite Coulomb integrals, 39 bra products
+struct C2010GradMd {
   static constexpr int La = 2, Lb = 0, Lc = 1, Ld = 0, L = 4;
-  static constexpr int NACC = 129;
-  // w = 1, 2 alpha, 2 beta, 2 gamma: QUICK's store, storeAA, storeBB, storeCC
-  __device__ static __forceinline__ void vrr(const double (&F)[L + 1], const VrrPar<double>& p, const double (&w)[4], double (&acc)[NACC]) {
-    const double v000_000_4 = F[4];
-    const double v000_000_3 = F[3];
-    const double v000_000_2 = F[2];
-    const double v000_000_1 = F[1];
-    const double v000_000_0 = F[0];
-    const double v001_000_3 = p.PA[2] * v000_000_3 + p.WP[2] * v000_000_4;
-    const double v010_000_3 = p.PA[1] * v000_000_3 + p.WP[1] * v000_000_4;
-    const double v100_000_3 = p.PA[0] * v000_000_3 + p.WP[0] * v000_000_4;
-    const double v001_000_2 = p.PA[2] * v000_000_2 + p.WP[2] * v000_000_3;
-    const double v010_000_2 = p.PA[1] * v000_000_2 + p.WP[1] * v000_000_3;
-    const double v100_000_2 = p.PA[0] * v000_000_2 + p.WP[0] * v000_000_3;
-    const double v001_000_1 = p.PA[2] * v000_000_1 + p.WP[2] * v000_000_2;
-    const double v010_000_1 = p.PA[1] * v000_000_1 + p.WP[1] * v000_000_2;
-    const double v100_000_1 = p.PA[0] * v000_000_1 + p.WP[0] * v000_000_2;
-    const double v001_000_0 = p.PA[2] * v000_000_0 + p.WP[2] * v000_000_1;
-    const double v010_000_0 = p.PA[1] * v000_000_0 + p.WP[1] * v000_000_1;
-    const double v100_000_0 = p.PA[0] * v000_000_0 + p.WP[0] * v000_000_1;
-    const double v002_000_2 = p.PA[2] * v001_000_2 + p.WP[2] * v001_000_3 + double(1) * p.oo2z * (v000_000_2 - p.rz * v000_000_3);
-    const double v011_000_2 = p.PA[1] * v001_000_2 + p.WP[1] * v001_000_3;
-    const double v020_000_2 = p.PA[1] * v010_000_2 + p.WP[1] * v010_000_3 + double(1) * p.oo2z * (v000_000_2 - p.rz * v000_000_3);
-    const double v101_000_2 = p.PA[0] * v001_000_2 + p.WP[0] * v001_000_3;
-    const double v110_000_2 = p.PA[0] * v010_000_2 + p.WP[0] * v010_000_3;
-    const double v200_000_2 = p.PA[0] * v100_000_2 + p.WP[0] * v100_000_3 + double(1) * p.oo2z * (v000_000_2 - p.rz * v000_000_3);
-    const double v002_000_1 = p.PA[2] * v001_000_1 + p.WP[2] * v001_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v011_000_1 = p.PA[1] * v001_000_1 + p.WP[1] * v001_000_2;
-    const double v020_000_1 = p.PA[1] * v010_000_1 + p.WP[1] * v010_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v101_000_1 = p.PA[0] * v001_000_1 + p.WP[0] * v001_000_2;
-    const double v110_000_1 = p.PA[0] * v010_000_1 + p.WP[0] * v010_000_2;
-    const double v200_000_1 = p.PA[0] * v100_000_1 + p.WP[0] * v100_000_2 + double(1) * p.oo2z * (v000_000_1 - p.rz * v000_000_2);
-    const double v002_000_0 = p.PA[2] * v001_000_0 + p.WP[2] * v001_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v011_000_0 = p.PA[1] * v001_000_0 + p.WP[1] * v001_000_1;
-    const double v020_000_0 = p.PA[1] * v010_000_0 + p.WP[1] * v010_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v101_000_0 = p.PA[0] * v001_000_0 + p.WP[0] * v001_000_1;
-    const double v110_000_0 = p.PA[0] * v010_000_0 + p.WP[0] * v010_000_1;
-    const double v200_000_0 = p.PA[0] * v100_000_0 + p.WP[0] * v100_000_1 + double(1) * p.oo2z * (v000_000_0 - p.rz * v000_000_1);
-    const double v001_001_1 = p.QC[2] * v001_000_1 + p.WQ[2] * v001_000_2 + double(1) * p.oo2zn * v000_000_2;
-    const double v001_010_1 = p.QC[1] * v001_000_1 + p.WQ[1] * v001_000_2;
-    const double v001_100_1 = p.QC[0] * v001_000_1 + p.WQ[0] * v001_000_2;
-    const double v010_001_1 = p.QC[2] * v010_000_1 + p.WQ[2] * v010_000_2;
-    const double v010_010_1 = p.QC[1] * v010_000_1 + p.WQ[1] * v010_000_2 + double(1) * p.oo2zn * v000_000_2;
-    const double v010_100_1 = p.QC[0] * v010_000_1 + p.WQ[0] * v010_000_2;
-    const double v100_001_1 = p.QC[2] * v100_000_1 + p.WQ[2] * v100_000_2;
-    const double v100_010_1 = p.QC[1] * v100_000_1 + p.WQ[1] * v100_000_2;
-    const double v100_100_1 = p.QC[0] * v100_000_1 + p.WQ[0] * v100_000_2 + double(1) * p.oo2zn * v000_000_2;
-    const double v001_001_0 = p.QC[2] * v001_000_0 + p.WQ[2] * v001_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v001_010_0 = p.QC[1] * v001_000_0 + p.WQ[1] * v001_000_1;
-    const double v001_100_0 = p.QC[0] * v001_000_0 + p.WQ[0] * v001_000_1;
-    const double v010_001_0 = p.QC[2] * v010_000_0 + p.WQ[2] * v010_000_1;
-    const double v010_010_0 = p.QC[1] * v010_000_0 + p.WQ[1] * v010_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v010_100_0 = p.QC[0] * v010_000_0 + p.WQ[0] * v010_000_1;
-    const double v100_001_0 = p.QC[2] * v100_000_0 + p.WQ[2] * v100_000_1;
-    const double v100_010_0 = p.QC[1] * v100_000_0 + p.WQ[1] * v100_000_1;
-    const double v100_100_0 = p.QC[0] * v100_000_0 + p.WQ[0] * v100_000_1 + double(1) * p.oo2zn * v000_000_1;
-    const double v003_000_1 = p.PA[2] * v002_000_1 + p.WP[2] * v002_000_2 + double(2) * p.oo2z * (v001_000_1 - p.rz * v001_000_2);
-    const double v012_000_1 = p.PA[1] * v002_000_1 + p.WP[1] * v002_000_2;
-    const double v021_000_1 = p.PA[2] * v020_000_1 + p.WP[2] * v020_000_2;
-    const double v030_000_1 = p.PA[1] * v020_000_1 + p.WP[1] * v020_000_2 + double(2) * p.oo2z * (v010_000_1 - p.rz * v010_000_2);
-    const double v102_000_1 = p.PA[0] * v002_000_1 + p.WP[0] * v002_000_2;
-    const double v111_000_1 = p.PA[0] * v011_000_1 + p.WP[0] * v011_000_2;
-    const double v120_000_1 = p.PA[0] * v020_000_1 + p.WP[0] * v020_000_2;
-    const double v201_000_1 = p.PA[2] * v200_000_1 + p.WP[2] * v200_000_2;
-    const double v210_000_1 = p.PA[1] * v200_000_1 + p.WP[1] * v200_000_2;
-    const double v300_000_1 = p.PA[0] * v200_000_1 + p.WP[0] * v200_000_2 + double(2) * p.oo2z * (v100_000_1 - p.rz * v100_000_2);
-    const double v003_000_0 = p.PA[2] * v002_000_0 + p.WP[2] * v002_000_1 + double(2) * p.oo2z * (v001_000_0 - p.rz * v001_000_1);
-    const double v012_000_0 = p.PA[1] * v002_000_0 + p.WP[1] * v002_000_1;
-    const double v021_000_0 = p.PA[2] * v020_000_0 + p.WP[2] * v020_000_1;
-    const double v030_000_0 = p.PA[1] * v020_000_0 + p.WP[1] * v020_000_1 + double(2) * p.oo2z * (v010_000_0 - p.rz * v010_000_1);
-    const double v102_000_0 = p.PA[0] * v002_000_0 + p.WP[0] * v002_000_1;
-    const double v111_000_0 = p.PA[0] * v011_000_0 + p.WP[0] * v011_000_1;
-    const double v120_000_0 = p.PA[0] * v020_000_0 + p.WP[0] * v020_000_1;
-    const double v201_000_0 = p.PA[2] * v200_000_0 + p.WP[2] * v200_000_1;
-    const double v210_000_0 = p.PA[1] * v200_000_0 + p.WP[1] * v200_000_1;
-    const double v300_000_0 = p.PA[0] * v200_000_0 + p.WP[0] * v200_000_1 + double(2) * p.oo2z * (v100_000_0 - p.rz * v100_000_1);
-    const double v002_001_1 = p.QC[2] * v002_000_1 + p.WQ[2] * v002_000_2 + double(2) * p.oo2zn * v001_000_2;
-    const double v002_010_1 = p.QC[1] * v002_000_1 + p.WQ[1] * v002_000_2;
-    const double v002_100_1 = p.QC[0] * v002_000_1 + p.WQ[0] * v002_000_2;
-    const double v011_001_1 = p.QC[2] * v011_000_1 + p.WQ[2] * v011_000_2 + double(1) * p.oo2zn * v010_000_2;
-    const double v011_010_1 = p.QC[1] * v011_000_1 + p.WQ[1] * v011_000_2 + double(1) * p.oo2zn * v001_000_2;
-    const double v011_100_1 = p.QC[0] * v011_000_1 + p.WQ[0] * v011_000_2;
-    const double v020_001_1 = p.QC[2] * v020_000_1 + p.WQ[2] * v020_000_2;
-    const double v020_010_1 = p.QC[1] * v020_000_1 + p.WQ[1] * v020_000_2 + double(2) * p.oo2zn * v010_000_2;
-    const double v020_100_1 = p.QC[0] * v020_000_1 + p.WQ[0] * v020_000_2;
-    const double v101_001_1 = p.QC[2] * v101_000_1 + p.WQ[2] * v101_000_2 + double(1) * p.oo2zn * v100_000_2;
-    const double v101_010_1 = p.QC[1] * v101_000_1 + p.WQ[1] * v101_000_2;
-    const double v101_100_1 = p.QC[0] * v101_000_1 + p.WQ[0] * v101_000_2 + double(1) * p.oo2zn * v001_000_2;
-    const double v110_001_1 = p.QC[2] * v110_000_1 + p.WQ[2] * v110_000_2;
-    const double v110_010_1 = p.QC[1] * v110_000_1 + p.WQ[1] * v110_000_2 + double(1) * p.oo2zn * v100_000_2;
-    const double v110_100_1 = p.QC[0] * v110_000_1 + p.WQ[0] * v110_000_2 + double(1) * p.oo2zn * v010_000_2;
-    const double v200_001_1 = p.QC[2] * v200_000_1 + p.WQ[2] * v200_000_2;
-    const double v200_010_1 = p.QC[1] * v200_000_1 + p.WQ[1] * v200_000_2;
-    const double v200_100_1 = p.QC[0] * v200_000_1 + p.WQ[0] * v200_000_2 + double(2) * p.oo2zn * v100_000_2;
-    const double v002_001_0 = p.QC[2] * v002_000_0 + p.WQ[2] * v002_000_1 + double(2) * p.oo2zn * v001_000_1;
-    const double v002_010_0 = p.QC[1] * v002_000_0 + p.WQ[1] * v002_000_1;
-    const double v002_100_0 = p.QC[0] * v002_000_0 + p.WQ[0] * v002_000_1;
-    const double v011_001_0 = p.QC[2] * v011_000_0 + p.WQ[2] * v011_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v011_010_0 = p.QC[1] * v011_000_0 + p.WQ[1] * v011_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v011_100_0 = p.QC[0] * v011_000_0 + p.WQ[0] * v011_000_1;
-    const double v020_001_0 = p.QC[2] * v020_000_0 + p.WQ[2] * v020_000_1;
-    const double v020_010_0 = p.QC[1] * v020_000_0 + p.WQ[1] * v020_000_1 + double(2) * p.oo2zn * v010_000_1;
-    const double v020_100_0 = p.QC[0] * v020_000_0 + p.WQ[0] * v020_000_1;
-    const double v101_001_0 = p.QC[2] * v101_000_0 + p.WQ[2] * v101_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v101_010_0 = p.QC[1] * v101_000_0 + p.WQ[1] * v101_000_1;
-    const double v101_100_0 = p.QC[0] * v101_000_0 + p.WQ[0] * v101_000_1 + double(1) * p.oo2zn * v001_000_1;
-    const double v110_001_0 = p.QC[2] * v110_000_0 + p.WQ[2] * v110_000_1;
-    const double v110_010_0 = p.QC[1] * v110_000_0 + p.WQ[1] * v110_000_1 + double(1) * p.oo2zn * v100_000_1;
-    const double v110_100_0 = p.QC[0] * v110_000_0 + p.WQ[0] * v110_000_1 + double(1) * p.oo2zn * v010_000_1;
-    const double v200_001_0 = p.QC[2] * v200_000_0 + p.WQ[2] * v200_000_1;
-    const double v200_010_0 = p.QC[1] * v200_000_0 + p.WQ[1] * v200_000_1;
-    const double v200_100_0 = p.QC[0] * v200_000_0 + p.WQ[0] * v200_000_1 + double(2) * p.oo2zn * v100_000_1;
-    const double v003_001_0 = p.QC[2] * v003_000_0 + p.WQ[2] * v003_000_1 + double(3) * p.oo2zn * v002_000_1;
-    const double v003_010_0 = p.QC[1] * v003_000_0 + p.WQ[1] * v003_000_1;
-    const double v003_100_0 = p.QC[0] * v003_000_0 + p.WQ[0] * v003_000_1;
-    const double v012_001_0 = p.QC[2] * v012_000_0 + p.WQ[2] * v012_000_1 + double(2) * p.oo2zn * v011_000_1;
-    const double v012_010_0 = p.QC[1] * v012_000_0 + p.WQ[1] * v012_000_1 + double(1) * p.oo2zn * v002_000_1;
-    const double v012_100_0 = p.QC[0] * v012_000_0 + p.WQ[0] * v012_000_1;
-    const double v021_001_0 = p.QC[2] * v021_000_0 + p.WQ[2] * v021_000_1 + double(1) * p.oo2zn * v020_000_1;
-    const double v021_010_0 = p.QC[1] * v021_000_0 + p.WQ[1] * v021_000_1 + double(2) * p.oo2zn * v011_000_1;
-    const double v021_100_0 = p.QC[0] * v021_000_0 + p.WQ[0] * v021_000_1;
-    const double v030_001_0 = p.QC[2] * v030_000_0 + p.WQ[2] * v030_000_1;
-    const double v030_010_0 = p.QC[1] * v030_000_0 + p.WQ[1] * v030_000_1 + double(3) * p.oo2zn * v020_000_1;
-    const double v030_100_0 = p.QC[0] * v030_000_0 + p.WQ[0] * v030_000_1;
-    const double v102_001_0 = p.QC[2] * v102_000_0 + p.WQ[2] * v102_000_1 + double(2) * p.oo2zn * v101_000_1;
-    const double v102_010_0 = p.QC[1] * v102_000_0 + p.WQ[1] * v102_000_1;
-    const double v102_100_0 = p.QC[0] * v102_000_0 + p.WQ[0] * v102_000_1 + double(1) * p.oo2zn * v002_000_1;
-    const double v111_001_0 = p.QC[2] * v111_000_0 + p.WQ[2] * v111_000_1 + double(1) * p.oo2zn * v110_000_1;
-    const double v111_010_0 = p.QC[1] * v111_000_0 + p.WQ[1] * v111_000_1 + double(1) * p.oo2zn * v101_000_1;
-    const double v111_100_0 = p.QC[0] * v111_000_0 + p.WQ[0] * v111_000_1 + double(1) * p.oo2zn * v011_000_1;
-    const double v120_001_0 = p.QC[2] * v120_000_0 + p.WQ[2] * v120_000_1;
-    const double v120_010_0 = p.QC[1] * v120_000_0 + p.WQ[1] * v120_000_1 + double(2) * p.oo2zn * v110_000_1;
-    const double v120_100_0 = p.QC[0] * v120_000_0 + p.WQ[0] * v120_000_1 + double(1) * p.oo2zn * v020_000_1;
-    const double v201_001_0 = p.QC[2] * v201_000_0 + p.WQ[2] * v201_000_1 + double(1) * p.oo2zn * v200_000_1;
-    const double v201_010_0 = p.QC[1] * v201_000_0 + p.WQ[1] * v201_000_1;
-    const double v201_100_0 = p.QC[0] * v201_000_0 + p.WQ[0] * v201_000_1 + double(2) * p.oo2zn * v101_000_1;
-    const double v210_001_0 = p.QC[2] * v210_000_0 + p.WQ[2] * v210_000_1;
-    const double v210_010_0 = p.QC[1] * v210_000_0 + p.WQ[1] * v210_000_1 + double(1) * p.oo2zn * v200_000_1;
-    const double v210_100_0 = p.QC[0] * v210_000_0 + p.WQ[0] * v210_000_1 + double(2) * p.oo2zn * v110_000_1;
-    const double v300_001_0 = p.QC[2] * v300_000_0 + p.WQ[2] * v300_000_1;
-    const double v300_010_0 = p.QC[1] * v300_000_0 + p.WQ[1] * v300_000_1;
-    const double v300_100_0 = p.QC[0] * v300_000_0 + p.WQ[0] * v300_000_1 + double(3) * p.oo2zn * v200_000_1;
-    const double v002_002_0 = p.QC[2] * v002_001_0 + p.WQ[2] * v002_001_1 + double(1) * p.oo2n * (v002_000_0 - p.rn * v002_000_1) + double(2) * p.oo2zn * v001_001_1;
-    const double v002_011_0 = p.QC[1] * v002_001_0 + p.WQ[1] * v002_001_1;
-    const double v002_020_0 = p.QC[1] * v002_010_0 + p.WQ[1] * v002_010_1 + double(1) * p.oo2n * (v002_000_0 - p.rn * v002_000_1);
-    const double v002_101_0 = p.QC[0] * v002_001_0 + p.WQ[0] * v002_001_1;
-    const double v002_110_0 = p.QC[0] * v002_010_0 + p.WQ[0] * v002_010_1;
-    const double v002_200_0 = p.QC[0] * v002_100_0 + p.WQ[0] * v002_100_1 + double(1) * p.oo2n * (v002_000_0 - p.rn * v002_000_1);
-    const double v011_002_0 = p.QC[2] * v011_001_0 + p.WQ[2] * v011_001_1 + double(1) * p.oo2n * (v011_000_0 - p.rn * v011_000_1) + double(1) * p.oo2zn * v010_001_1;
-    const double v011_011_0 = p.QC[1] * v011_001_0 + p.WQ[1] * v011_001_1 + double(1) * p.oo2zn * v001_001_1;
-    const double v011_020_0 = p.QC[1] * v011_010_0 + p.WQ[1] * v011_010_1 + double(1) * p.oo2n * (v011_000_0 - p.rn * v011_000_1) + double(1) * p.oo2zn * v001_010_1;
-    const double v011_101_0 = p.QC[0] * v011_001_0 + p.WQ[0] * v011_001_1;
-    const double v011_110_0 = p.QC[0] * v011_010_0 + p.WQ[0] * v011_010_1;
-    const double v011_200_0 = p.QC[0] * v011_100_0 + p.WQ[0] * v011_100_1 + double(1) * p.oo2n * (v011_000_0 - p.rn * v011_000_1);
-    const double v020_002_0 = p.QC[2] * v020_001_0 + p.WQ[2] * v020_001_1 + double(1) * p.oo2n * (v020_000_0 - p.rn * v020_000_1);
-    const double v020_011_0 = p.QC[2] * v020_010_0 + p.WQ[2] * v020_010_1;
-    const double v020_020_0 = p.QC[1] * v020_010_0 + p.WQ[1] * v020_010_1 + double(1) * p.oo2n * (v020_000_0 - p.rn * v020_000_1) + double(2) * p.oo2zn * v010_010_1;
-    const double v020_101_0 = p.QC[0] * v020_001_0 + p.WQ[0] * v020_001_1;
-    const double v020_110_0 = p.QC[0] * v020_010_0 + p.WQ[0] * v020_010_1;
-    const double v020_200_0 = p.QC[0] * v020_100_0 + p.WQ[0] * v020_100_1 + double(1) * p.oo2n * (v020_000_0 - p.rn * v020_000_1);
-    const double v101_002_0 = p.QC[2] * v101_001_0 + p.WQ[2] * v101_001_1 + double(1) * p.oo2n * (v101_000_0 - p.rn * v101_000_1) + double(1) * p.oo2zn * v100_001_1;
-    const double v101_011_0 = p.QC[1] * v101_001_0 + p.WQ[1] * v101_001_1;
-    const double v101_020_0 = p.QC[1] * v101_010_0 + p.WQ[1] * v101_010_1 + double(1) * p.oo2n * (v101_000_0 - p.rn * v101_000_1);
-    const double v101_101_0 = p.QC[0] * v101_001_0 + p.WQ[0] * v101_001_1 + double(1) * p.oo2zn * v001_001_1;
-    const double v101_110_0 = p.QC[1] * v101_100_0 + p.WQ[1] * v101_100_1;
-    const double v101_200_0 = p.QC[0] * v101_100_0 + p.WQ[0] * v101_100_1 + double(1) * p.oo2n * (v101_000_0 - p.rn * v101_000_1) + double(1) * p.oo2zn * v001_100_1;
-    const double v110_002_0 = p.QC[2] * v110_001_0 + p.WQ[2] * v110_001_1 + double(1) * p.oo2n * (v110_000_0 - p.rn * v110_000_1);
-    const double v110_011_0 = p.QC[2] * v110_010_0 + p.WQ[2] * v110_010_1;
-    const double v110_020_0 = p.QC[1] * v110_010_0 + p.WQ[1] * v110_010_1 + double(1) * p.oo2n * (v110_000_0 - p.rn * v110_000_1) + double(1) * p.oo2zn * v100_010_1;
-    const double v110_101_0 = p.QC[2] * v110_100_0 + p.WQ[2] * v110_100_1;
-    const double v110_110_0 = p.QC[0] * v110_010_0 + p.WQ[0] * v110_010_1 + double(1) * p.oo2zn * v010_010_1;
-    const double v110_200_0 = p.QC[0] * v110_100_0 + p.WQ[0] * v110_100_1 + double(1) * p.oo2n * (v110_000_0 - p.rn * v110_000_1) + double(1) * p.oo2zn * v010_100_1;
-    const double v200_002_0 = p.QC[2] * v200_001_0 + p.WQ[2] * v200_001_1 + double(1) * p.oo2n * (v200_000_0 - p.rn * v200_000_1);
-    const double v200_011_0 = p.QC[1] * v200_001_0 + p.WQ[1] * v200_001_1;
-    const double v200_020_0 = p.QC[1] * v200_010_0 + p.WQ[1] * v200_010_1 + double(1) * p.oo2n * (v200_000_0 - p.rn * v200_000_1);
-    const double v200_101_0 = p.QC[2] * v200_100_0 + p.WQ[2] * v200_100_1;
-    const double v200_110_0 = p.QC[1] * v200_100_0 + p.WQ[1] * v200_100_1;
-    const double v200_200_0 = p.QC[0] * v200_100_0 + p.WQ[0] * v200_100_1 + double(1) * p.oo2n * (v200_000_0 - p.rn * v200_000_1) + double(2) * p.oo2zn * v100_100_1;
-    acc[0] += w[0] * v100_100_0;
-    acc[1] += w[0] * v100_010_0;
-    acc[2] += w[0] * v100_001_0;
-    acc[3] += w[0] * v010_100_0;
-    acc[4] += w[0] * v010_010_0;
-    acc[5] += w[0] * v010_001_0;
-    acc[6] += w[0] * v001_100_0;
-    acc[7] += w[0] * v001_010_0;
-    acc[8] += w[0] * v001_001_0;
-    acc[9] += w[0] * v200_000_0;
-    acc[10] += w[0] * v110_000_0;
-    acc[11] += w[0] * v020_000_0;
-    acc[12] += w[0] * v101_000_0;
-    acc[13] += w[0] * v011_000_0;
-    acc[14] += w[0] * v002_000_0;
-    acc[15] += w[1] * v300_100_0;
-    acc[16] += w[1] * v300_010_0;
-    acc[17] += w[1] * v300_001_0;
-    acc[18] += w[1] * v210_100_0;
-    acc[19] += w[1] * v210_010_0;
-    acc[20] += w[1] * v210_001_0;
-    acc[21] += w[1] * v120_100_0;
-    acc[22] += w[1] * v120_010_0;
-    acc[23] += w[1] * v120_001_0;
-    acc[24] += w[1] * v030_100_0;
-    acc[25] += w[1] * v030_010_0;
-    acc[26] += w[1] * v030_001_0;
-    acc[27] += w[1] * v201_100_0;
-    acc[28] += w[1] * v201_010_0;
-    acc[29] += w[1] * v201_001_0;
-    acc[30] += w[1] * v111_100_0;
-    acc[31] += w[1] * v111_010_0;
-    acc[32] += w[1] * v111_001_0;
-    acc[33] += w[1] * v021_100_0;
-    acc[34] += w[1] * v021_010_0;
-    acc[35] += w[1] * v021_001_0;
-    acc[36] += w[1] * v102_100_0;
-    acc[37] += w[1] * v102_010_0;
-    acc[38] += w[1] * v102_001_0;
-    acc[39] += w[1] * v012_100_0;
-    acc[40] += w[1] * v012_010_0;
-    acc[41] += w[1] * v012_001_0;
-    acc[42] += w[1] * v003_100_0;
-    acc[43] += w[1] * v003_010_0;
-    acc[44] += w[1] * v003_001_0;
-    acc[45] += w[2] * v200_100_0;
-    acc[46] += w[2] * v200_010_0;
-    acc[47] += w[2] * v200_001_0;
-    acc[48] += w[2] * v110_100_0;
-    acc[49] += w[2] * v110_010_0;
-    acc[50] += w[2] * v110_001_0;
-    acc[51] += w[2] * v020_100_0;
-    acc[52] += w[2] * v020_010_0;
-    acc[53] += w[2] * v020_001_0;
-    acc[54] += w[2] * v101_100_0;
-    acc[55] += w[2] * v101_010_0;
-    acc[56] += w[2] * v101_001_0;
-    acc[57] += w[2] * v011_100_0;
-    acc[58] += w[2] * v011_010_0;
-    acc[59] += w[2] * v011_001_0;
-    acc[60] += w[2] * v002_100_0;
-    acc[61] += w[2] * v002_010_0;
-    acc[62] += w[2] * v002_001_0;
-    acc[63] += w[2] * v300_100_0;
-    acc[64] += w[2] * v300_010_0;
-    acc[65] += w[2] * v300_001_0;
-    acc[66] += w[2] * v210_100_0;
-    acc[67] += w[2] * v210_010_0;
-    acc[68] += w[2] * v210_001_0;
-    acc[69] += w[2] * v120_100_0;
-    acc[70] += w[2] * v120_010_0;
-    acc[71] += w[2] * v120_001_0;
-    acc[72] += w[2] * v030_100_0;
-    acc[73] += w[2] * v030_010_0;
-    acc[74] += w[2] * v030_001_0;
-    acc[75] += w[2] * v201_100_0;
-    acc[76] += w[2] * v201_010_0;
-    acc[77] += w[2] * v201_001_0;
-    acc[78] += w[2] * v111_100_0;
-    acc[79] += w[2] * v111_010_0;
-    acc[80] += w[2] * v111_001_0;
-    acc[81] += w[2] * v021_100_0;
-    acc[82] += w[2] * v021_010_0;
-    acc[83] += w[2] * v021_001_0;
-    acc[84] += w[2] * v102_100_0;
-    acc[85] += w[2] * v102_010_0;
-    acc[86] += w[2] * v102_001_0;
-    acc[87] += w[2] * v012_100_0;
-    acc[88] += w[2] * v012_010_0;
-    acc[89] += w[2] * v012_001_0;
-    acc[90] += w[2] * v003_100_0;
-    acc[91] += w[2] * v003_010_0;
-    acc[92] += w[2] * v003_001_0;
-    acc[93] += w[3] * v200_200_0;
-    acc[94] += w[3] * v200_110_0;
-    acc[95] += w[3] * v200_020_0;
-    acc[96] += w[3] * v200_101_0;
-    acc[97] += w[3] * v200_011_0;
-    acc[98] += w[3] * v200_002_0;
-    acc[99] += w[3] * v110_200_0;
-    acc[100] += w[3] * v110_110_0;
-    acc[101] += w[3] * v110_020_0;
-    acc[102] += w[3] * v110_101_0;
-    acc[103] += w[3] * v110_011_0;
-    acc[104] += w[3] * v110_002_0;
-    acc[105] += w[3] * v020_200_0;
-    acc[106] += w[3] * v020_110_0;
-    acc[107] += w[3] * v020_020_0;
-    acc[108] += w[3] * v020_101_0;
-    acc[109] += w[3] * v020_011_0;
-    acc[110] += w[3] * v020_002_0;
-    acc[111] += w[3] * v101_200_0;
-    acc[112] += w[3] * v101_110_0;
-    acc[113] += w[3] * v101_020_0;
-    acc[114] += w[3] * v101_101_0;
-    acc[115] += w[3] * v101_011_0;
-    acc[116] += w[3] * v101_002_0;
-    acc[117] += w[3] * v011_200_0;
-    acc[118] += w[3] * v011_110_0;
-    acc[119] += w[3] * v011_020_0;
-    acc[120] += w[3] * v011_101_0;
-    acc[121] += w[3] * v011_011_0;
-    acc[122] += w[3] * v011_002_0;
-    acc[123] += w[3] * v002_200_0;
-    acc[124] += w[3] * v002_110_0;
-    acc[125] += w[3] * v002_020_0;
-    acc[126] += w[3] * v002_101_0;
-    acc[127] += w[3] * v002_011_0;
-    acc[128] += w[3] * v002_002_0;
+  static constexpr int N1 = 9, NE = 39;   // 1D entries per direction, product table
+  static constexpr int MIN_WAVES = 1;      // waves per SIMD the register budget targets
+  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16
+  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p, rx = -beta/p, ry = alpha/p
+  template <class T>
+  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, double rx, double ry, T out) {
+    const double be100 = X;
+    const double be101 = h;
+    const double bd100 = rx;
+    const double be200 = fma(1.0, be101, be100 * X);
+    const double be201 = fma(be100, h, be101 * X);
+    const double be202 = be101 * h;
+    const double bd200 = fma(be100, rx, bd100 * X);
+    const double bd201 = fma(be101, rx, bd100 * h);
+    out[0] = 1.0;
+    out[1] = be100;
+    out[2] = be101;
+    out[3] = bd100;
+    out[4] = be200;
+    out[5] = be201;
+    out[6] = be202;
+    out[7] = bd200;
+    out[8] = bd201;
   }
-  __device__ static __forceinline__ void digest(const double (&acc)[NACC], const double (&AB)[3], const double (&CD)[3], const double (&Dab)[6], const double (&Dcd)[3], const double (&Dac)[18], const double (&Dad)[6], const double (&Dbc)[3], const double (&Dbd)[1], double hh, double (&g)[9]) {
-    const double bp_b200_100_100_000 = acc[63] + AB[0] * acc[45];
-    const double bp_b200_100_010_000 = acc[64] + AB[0] * acc[46];
-    const double bp_b200_100_001_000 = acc[65] + AB[0] * acc[47];
-    const double bp_b200_010_100_000 = acc[66] + AB[1] * acc[45];
-    const double bp_b200_010_010_000 = acc[67] + AB[1] * acc[46];
-    const double bp_b200_010_001_000 = acc[68] + AB[1] * acc[47];
-    const double bp_b200_001_100_000 = acc[75] + AB[2] * acc[45];
-    const double bp_b200_001_010_000 = acc[76] + AB[2] * acc[46];
-    const double bp_b200_001_001_000 = acc[77] + AB[2] * acc[47];
-    const double bp_b110_100_100_000 = acc[66] + AB[0] * acc[48];
-    const double bp_b110_100_010_000 = acc[67] + AB[0] * acc[49];
-    const double bp_b110_100_001_000 = acc[68] + AB[0] * acc[50];
-    const double bp_b110_010_100_000 = acc[69] + AB[1] * acc[48];
-    const double bp_b110_010_010_000 = acc[70] + AB[1] * acc[49];
-    const double bp_b110_010_001_000 = acc[71] + AB[1] * acc[50];
-    const double bp_b110_001_100_000 = acc[78] + AB[2] * acc[48];
-    const double bp_b110_001_010_000 = acc[79] + AB[2] * acc[49];
-    const double bp_b110_001_001_000 = acc[80] + AB[2] * acc[50];
-    const double bp_b020_100_100_000 = acc[69] + AB[0] * acc[51];
-    const double bp_b020_100_010_000 = acc[70] + AB[0] * acc[52];
-    const double bp_b020_100_001_000 = acc[71] + AB[0] * acc[53];
-    const double bp_b020_010_100_000 = acc[72] + AB[1] * acc[51];
-    const double bp_b020_010_010_000 = acc[73] + AB[1] * acc[52];
-    const double bp_b020_010_001_000 = acc[74] + AB[1] * acc[53];
-    const double bp_b020_001_100_000 = acc[81] + AB[2] * acc[51];
-    const double bp_b020_001_010_000 = acc[82] + AB[2] * acc[52];
-    const double bp_b020_001_001_000 = acc[83] + AB[2] * acc[53];
-    const double bp_b101_100_100_000 = acc[75] + AB[0] * acc[54];
-    const double bp_b101_100_010_000 = acc[76] + AB[0] * acc[55];
-    const double bp_b101_100_001_000 = acc[77] + AB[0] * acc[56];
-    const double bp_b101_010_100_000 = acc[78] + AB[1] * acc[54];
-    const double bp_b101_010_010_000 = acc[79] + AB[1] * acc[55];
-    const double bp_b101_010_001_000 = acc[80] + AB[1] * acc[56];
-    const double bp_b101_001_100_000 = acc[84] + AB[2] * acc[54];
-    const double bp_b101_001_010_000 = acc[85] + AB[2] * acc[55];
-    const double bp_b101_001_001_000 = acc[86] + AB[2] * acc[56];
-    const double bp_b011_100_100_000 = acc[78] + AB[0] * acc[57];
-    const double bp_b011_100_010_000 = acc[79] + AB[0] * acc[58];
-    const double bp_b011_100_001_000 = acc[80] + AB[0] * acc[59];
-    const double bp_b011_010_100_000 = acc[81] + AB[1] * acc[57];
-    const double bp_b011_010_010_000 = acc[82] + AB[1] * acc[58];
-    const double bp_b011_010_001_000 = acc[83] + AB[1] * acc[59];
-    const double bp_b011_001_100_000 = acc[87] + AB[2] * acc[57];
-    const double bp_b011_001_010_000 = acc[88] + AB[2] * acc[58];
-    const double bp_b011_001_001_000 = acc[89] + AB[2] * acc[59];
-    const double bp_b002_100_100_000 = acc[84] + AB[0] * acc[60];
-    const double bp_b002_100_010_000 = acc[85] + AB[0] * acc[61];
-    const double bp_b002_100_001_000 = acc[86] + AB[0] * acc[62];
-    const double bp_b002_010_100_000 = acc[87] + AB[1] * acc[60];
-    const double bp_b002_010_010_000 = acc[88] + AB[1] * acc[61];
-    const double bp_b002_010_001_000 = acc[89] + AB[1] * acc[62];
-    const double bp_b002_001_100_000 = acc[90] + AB[2] * acc[60];
-    const double bp_b002_001_010_000 = acc[91] + AB[2] * acc[61];
-    const double bp_b002_001_001_000 = acc[92] + AB[2] * acc[62];
+  // Dcd with 2 cons, Dbc and Dbd with hyb/2 cons; oc, od: first elements of the a-c and a-d blocks of P
+  template <class ET, class PT, class PU>
+  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a, const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, double rc, double rd, const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[3], const double (&Dbc)[3], const double (&Dbd)[1], double& W, double (&gP)[3], double (&gR)[3], double (&gS)[3]) {
+    double am = pref;
+    const double r000_0 = F[0] * am;
+    am *= m2a;
+    const double r000_1 = F[1] * am;
+    am *= m2a;
+    const double r000_2 = F[2] * am;
+    am *= m2a;
+    const double r000_3 = F[3] * am;
+    am *= m2a;
+    const double r000_4 = F[4] * am;
+    const double r100_3 = PQ[0] * r000_4;
+    const double r010_3 = PQ[1] * r000_4;
+    const double r001_3 = PQ[2] * r000_4;
+    const double r100_2 = PQ[0] * r000_3;
+    const double r010_2 = PQ[1] * r000_3;
+    const double r001_2 = PQ[2] * r000_3;
+    const double r200_2 = fma(1.0, r000_3, PQ[0] * r100_3);
+    const double r110_2 = PQ[0] * r010_3;
+    const double r101_2 = PQ[0] * r001_3;
+    const double r020_2 = fma(1.0, r000_3, PQ[1] * r010_3);
+    const double r011_2 = PQ[1] * r001_3;
+    const double r002_2 = fma(1.0, r000_3, PQ[2] * r001_3);
+    const double r100_1 = PQ[0] * r000_2;
+    const double r010_1 = PQ[1] * r000_2;
+    const double r001_1 = PQ[2] * r000_2;
+    const double r200_1 = fma(1.0, r000_2, PQ[0] * r100_2);
+    const double r110_1 = PQ[0] * r010_2;
+    const double r101_1 = PQ[0] * r001_2;
+    const double r020_1 = fma(1.0, r000_2, PQ[1] * r010_2);
+    const double r011_1 = PQ[1] * r001_2;
+    const double r002_1 = fma(1.0, r000_2, PQ[2] * r001_2);
+    const double r300_1 = fma(2.0, r100_2, PQ[0] * r200_2);
+    const double r210_1 = PQ[1] * r200_2;
+    const double r201_1 = PQ[2] * r200_2;
+    const double r120_1 = PQ[0] * r020_2;
+    const double r111_1 = PQ[0] * r011_2;
+    const double r102_1 = PQ[0] * r002_2;
+    const double r030_1 = fma(2.0, r010_2, PQ[1] * r020_2);
+    const double r021_1 = PQ[2] * r020_2;
+    const double r012_1 = PQ[1] * r002_2;
+    const double r003_1 = fma(2.0, r001_2, PQ[2] * r002_2);
+    const double r100_0 = PQ[0] * r000_1;
+    const double r010_0 = PQ[1] * r000_1;
+    const double r001_0 = PQ[2] * r000_1;
+    const double r200_0 = fma(1.0, r000_1, PQ[0] * r100_1);
+    const double r110_0 = PQ[0] * r010_1;
+    const double r101_0 = PQ[0] * r001_1;
+    const double r020_0 = fma(1.0, r000_1, PQ[1] * r010_1);
+    const double r011_0 = PQ[1] * r001_1;
+    const double r002_0 = fma(1.0, r000_1, PQ[2] * r001_1);
+    const double r300_0 = fma(2.0, r100_1, PQ[0] * r200_1);
+    const double r210_0 = PQ[1] * r200_1;
+    const double r201_0 = PQ[2] * r200_1;
+    const double r120_0 = PQ[0] * r020_1;
+    const double r111_0 = PQ[0] * r011_1;
+    const double r102_0 = PQ[0] * r002_1;
+    const double r030_0 = fma(2.0, r010_1, PQ[1] * r020_1);
+    const double r021_0 = PQ[2] * r020_1;
+    const double r012_0 = PQ[1] * r002_1;
+    const double r003_0 = fma(2.0, r001_1, PQ[2] * r002_1);
+    const double r400_0 = fma(3.0, r200_1, PQ[0] * r300_1);
+    const double r310_0 = PQ[1] * r300_1;
+    const double r301_0 = PQ[2] * r300_1;
+    const double r220_0 = fma(1.0, r020_1, PQ[0] * r120_1);
+    const double r211_0 = PQ[1] * r201_1;
+    const double r202_0 = fma(1.0, r002_1, PQ[0] * r102_1);
+    const double r130_0 = PQ[0] * r030_1;
+    const double r121_0 = PQ[0] * r021_1;
+    const double r112_0 = PQ[0] * r012_1;
+    const double r103_0 = PQ[0] * r003_1;
+    const double r040_0 = fma(3.0, r020_1, PQ[1] * r030_1);
+    const double r031_0 = PQ[2] * r030_1;
+    const double r022_0 = fma(1.0, r002_1, PQ[1] * r012_1);
+    const double r013_0 = PQ[1] * r003_1;
+    const double r004_0 = fma(3.0, r002_1, PQ[2] * r003_1);
+    const double kxe100 = QC[0];
+    const double kxe101 = (-hk);
+    const double kxd100 = rc;
+    const double kye100 = QC[1];
+    const double kye101 = (-hk);
+    const double kyd100 = rc;
+    const double kze100 = QC[2];
+    const double kze101 = (-hk);
+    const double kzd100 = rc;
+    const double k0_0_000 = kxe100;
+    const double k0_0_100 = kxe101;
+    const double k1_0_000 = kye100;
+    const double k1_0_010 = kye101;
+    const double k2_0_000 = kze100;
+    const double k2_0_001 = kze101;
+    double K0_0_000 = 0.0;
+    double K1_0_000 = 0.0;
+    double K2_0_000 = 0.0;
+    double w = 0.0, px = 0.0, py = 0.0, pz = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
+    QF_OPAQUE(oc);
+    QF_OPAQUE(od);
     {
-      const double gm = kCons[2][0] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[0] * Dcd[0] - hh * (Dac[0] * Dbd[0] + Dad[0] * Dbc[0]));
-      g[0] += gm * (acc[15] - 2.0 * acc[0]);
-      g[3] += gm * bp_b200_100_100_000;
-      g[6] += gm * (acc[93] - 1.0 * acc[9]);
-      g[1] += gm * acc[18];
-      g[4] += gm * bp_b200_010_100_000;
-      g[7] += gm * acc[94];
-      g[2] += gm * acc[27];
-      g[5] += gm * bp_b200_001_100_000;
-      g[8] += gm * acc[96];
+      const double ac0 = P[oc + 0 * n + 0] * (kCons[2][0] * kCons[1][0]);
+      const double ac1 = P[oc + 0 * n + 1] * (kCons[2][0] * kCons[1][1]);
+      const double ac2 = P[oc + 0 * n + 2] * (kCons[2][0] * kCons[1][2]);
+      const double ad0 = P[od + 0 * n + 0] * (kCons[2][0] * kCons[0][0]);
+      {
+        const double ab = Pab[0 * n + 0] * (kCons[2][0] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double t200 = fma(y100, r300_0, fma(y010, r210_0, fma(y001, r201_0, y000 * r200_0)));
+        const double t201 = fma(y100, r301_0, fma(y010, r211_0, fma(y001, r202_0, y000 * r201_0)));
+        const double t210 = fma(y100, r310_0, fma(y010, r220_0, fma(y001, r211_0, y000 * r210_0)));
+        const double t300 = fma(y100, r400_0, fma(y010, r310_0, fma(y001, r301_0, y000 * r300_0)));
+        const double e0 = E[0];
+        const double e1 = E[1];
+        const double e2 = E[2];
+        w = fma(e2, t200, fma(e1, t100, fma(e0, t000, w)));
+        px = fma(e2, t300, fma(e1, t200, fma(e0, t100, px)));
+        py = fma(e2, t210, fma(e1, t110, fma(e0, t010, py)));
+        pz = fma(e2, t201, fma(e1, t101, fma(e0, t001, pz)));
+        sx = fma(E[4], t100, fma(E[3], t000, sx));
+        const double z000 = fma(e2, r200_0, fma(e1, r100_0, e0 * r000_0));
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[2][0] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[0] * Dcd[1] - hh * (Dac[1] * Dbd[0] + Dad[0] * Dbc[1]));
-      g[0] += gm * (acc[16] - 2.0 * acc[1]);
-      g[3] += gm * bp_b200_100_010_000;
-      g[6] += gm * acc[94];
-      g[1] += gm * acc[19];
-      g[4] += gm * bp_b200_010_010_000;
-      g[7] += gm * (acc[95] - 1.0 * acc[9]);
-      g[2] += gm * acc[28];
-      g[5] += gm * bp_b200_001_010_000;
-      g[8] += gm * acc[97];
+      const double ac0 = P[oc + 1 * n + 0] * (kCons[2][1] * kCons[1][0]);
+      const double ac1 = P[oc + 1 * n + 1] * (kCons[2][1] * kCons[1][1]);
+      const double ac2 = P[oc + 1 * n + 2] * (kCons[2][1] * kCons[1][2]);
+      const double ad0 = P[od + 1 * n + 0] * (kCons[2][1] * kCons[0][0]);
+      {
+        const double ab = Pab[1 * n + 0] * (kCons[2][1] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t020 = fma(y100, r120_0, fma(y010, r030_0, fma(y001, r021_0, y000 * r020_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double t200 = fma(y100, r300_0, fma(y010, r210_0, fma(y001, r201_0, y000 * r200_0)));
+        const double t111 = fma(y100, r211_0, fma(y010, r121_0, fma(y001, r112_0, y000 * r111_0)));
+        const double t120 = fma(y100, r220_0, fma(y010, r130_0, fma(y001, r121_0, y000 * r120_0)));
+        const double t210 = fma(y100, r310_0, fma(y010, r220_0, fma(y001, r211_0, y000 * r210_0)));
+        const double e0 = E[5];
+        const double e1 = E[6];
+        const double e2 = E[7];
+        const double e3 = E[8];
+        w = fma(e3, t110, fma(e2, t100, fma(e1, t010, fma(e0, t000, w))));
+        px = fma(e3, t210, fma(e2, t200, fma(e1, t110, fma(e0, t100, px))));
+        py = fma(e3, t120, fma(e2, t110, fma(e1, t020, fma(e0, t010, py))));
+        pz = fma(e3, t111, fma(e2, t101, fma(e1, t011, fma(e0, t001, pz))));
+        sx = fma(E[10], t010, fma(E[9], t000, sx));
+        sy = fma(E[12], t100, fma(E[11], t000, sy));
+        const double z000 = fma(e3, r110_0, fma(e2, r100_0, fma(e1, r010_0, e0 * r000_0)));
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[2][0] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[0] * Dcd[2] - hh * (Dac[2] * Dbd[0] + Dad[0] * Dbc[2]));
-      g[0] += gm * (acc[17] - 2.0 * acc[2]);
-      g[3] += gm * bp_b200_100_001_000;
-      g[6] += gm * acc[96];
-      g[1] += gm * acc[20];
-      g[4] += gm * bp_b200_010_001_000;
-      g[7] += gm * acc[97];
-      g[2] += gm * acc[29];
-      g[5] += gm * bp_b200_001_001_000;
-      g[8] += gm * (acc[98] - 1.0 * acc[9]);
+      const double ac0 = P[oc + 2 * n + 0] * (kCons[2][2] * kCons[1][0]);
+      const double ac1 = P[oc + 2 * n + 1] * (kCons[2][2] * kCons[1][1]);
+      const double ac2 = P[oc + 2 * n + 2] * (kCons[2][2] * kCons[1][2]);
+      const double ad0 = P[od + 2 * n + 0] * (kCons[2][2] * kCons[0][0]);
+      {
+        const double ab = Pab[2 * n + 0] * (kCons[2][2] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t020 = fma(y100, r120_0, fma(y010, r030_0, fma(y001, r021_0, y000 * r020_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double t021 = fma(y100, r121_0, fma(y010, r031_0, fma(y001, r022_0, y000 * r021_0)));
+        const double t030 = fma(y100, r130_0, fma(y010, r040_0, fma(y001, r031_0, y000 * r030_0)));
+        const double t120 = fma(y100, r220_0, fma(y010, r130_0, fma(y001, r121_0, y000 * r120_0)));
+        const double e0 = E[13];
+        const double e1 = E[14];
+        const double e2 = E[15];
+        w = fma(e2, t020, fma(e1, t010, fma(e0, t000, w)));
+        px = fma(e2, t120, fma(e1, t110, fma(e0, t100, px)));
+        py = fma(e2, t030, fma(e1, t020, fma(e0, t010, py)));
+        pz = fma(e2, t021, fma(e1, t011, fma(e0, t001, pz)));
+        sy = fma(E[17], t010, fma(E[16], t000, sy));
+        const double z000 = fma(e2, r020_0, fma(e1, r010_0, e0 * r000_0));
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[2][1] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[1] * Dcd[0] - hh * (Dac[3] * Dbd[0] + Dad[1] * Dbc[0]));
-      g[0] += gm * (acc[18] - 1.0 * acc[3]);
-      g[3] += gm * bp_b110_100_100_000;
-      g[6] += gm * (acc[99] - 1.0 * acc[10]);
-      g[1] += gm * (acc[21] - 1.0 * acc[0]);
-      g[4] += gm * bp_b110_010_100_000;
-      g[7] += gm * acc[100];
-      g[2] += gm * acc[30];
-      g[5] += gm * bp_b110_001_100_000;
-      g[8] += gm * acc[102];
+      const double ac0 = P[oc + 3 * n + 0] * (kCons[2][3] * kCons[1][0]);
+      const double ac1 = P[oc + 3 * n + 1] * (kCons[2][3] * kCons[1][1]);
+      const double ac2 = P[oc + 3 * n + 2] * (kCons[2][3] * kCons[1][2]);
+      const double ad0 = P[od + 3 * n + 0] * (kCons[2][3] * kCons[0][0]);
+      {
+        const double ab = Pab[3 * n + 0] * (kCons[2][3] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t002 = fma(y100, r102_0, fma(y010, r012_0, fma(y001, r003_0, y000 * r002_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double t200 = fma(y100, r300_0, fma(y010, r210_0, fma(y001, r201_0, y000 * r200_0)));
+        const double t102 = fma(y100, r202_0, fma(y010, r112_0, fma(y001, r103_0, y000 * r102_0)));
+        const double t111 = fma(y100, r211_0, fma(y010, r121_0, fma(y001, r112_0, y000 * r111_0)));
+        const double t201 = fma(y100, r301_0, fma(y010, r211_0, fma(y001, r202_0, y000 * r201_0)));
+        const double e0 = E[18];
+        const double e1 = E[19];
+        const double e2 = E[20];
+        const double e3 = E[21];
+        w = fma(e3, t101, fma(e2, t100, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t201, fma(e2, t200, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t111, fma(e2, t110, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t102, fma(e2, t101, fma(e1, t002, fma(e0, t001, pz))));
+        sx = fma(E[23], t001, fma(E[22], t000, sx));
+        sz = fma(E[25], t100, fma(E[24], t000, sz));
+        const double z000 = fma(e3, r101_0, fma(e2, r100_0, fma(e1, r001_0, e0 * r000_0)));
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[2][1] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[1] * Dcd[1] - hh * (Dac[4] * Dbd[0] + Dad[1] * Dbc[1]));
-      g[0] += gm * (acc[19] - 1.0 * acc[4]);
-      g[3] += gm * bp_b110_100_010_000;
-      g[6] += gm * acc[100];
-      g[1] += gm * (acc[22] - 1.0 * acc[1]);
-      g[4] += gm * bp_b110_010_010_000;
-      g[7] += gm * (acc[101] - 1.0 * acc[10]);
-      g[2] += gm * acc[31];
-      g[5] += gm * bp_b110_001_010_000;
-      g[8] += gm * acc[103];
+      const double ac0 = P[oc + 4 * n + 0] * (kCons[2][4] * kCons[1][0]);
+      const double ac1 = P[oc + 4 * n + 1] * (kCons[2][4] * kCons[1][1]);
+      const double ac2 = P[oc + 4 * n + 2] * (kCons[2][4] * kCons[1][2]);
+      const double ad0 = P[od + 4 * n + 0] * (kCons[2][4] * kCons[0][0]);
+      {
+        const double ab = Pab[4 * n + 0] * (kCons[2][4] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t002 = fma(y100, r102_0, fma(y010, r012_0, fma(y001, r003_0, y000 * r002_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t020 = fma(y100, r120_0, fma(y010, r030_0, fma(y001, r021_0, y000 * r020_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double t110 = fma(y100, r210_0, fma(y010, r120_0, fma(y001, r111_0, y000 * r110_0)));
+        const double t012 = fma(y100, r112_0, fma(y010, r022_0, fma(y001, r013_0, y000 * r012_0)));
+        const double t021 = fma(y100, r121_0, fma(y010, r031_0, fma(y001, r022_0, y000 * r021_0)));
+        const double t111 = fma(y100, r211_0, fma(y010, r121_0, fma(y001, r112_0, y000 * r111_0)));
+        const double e0 = E[26];
+        const double e1 = E[27];
+        const double e2 = E[28];
+        const double e3 = E[29];
+        w = fma(e3, t011, fma(e2, t010, fma(e1, t001, fma(e0, t000, w))));
+        px = fma(e3, t111, fma(e2, t110, fma(e1, t101, fma(e0, t100, px))));
+        py = fma(e3, t021, fma(e2, t020, fma(e1, t011, fma(e0, t010, py))));
+        pz = fma(e3, t012, fma(e2, t011, fma(e1, t002, fma(e0, t001, pz))));
+        sy = fma(E[31], t001, fma(E[30], t000, sy));
+        sz = fma(E[33], t010, fma(E[32], t000, sz));
+        const double z000 = fma(e3, r011_0, fma(e2, r010_0, fma(e1, r001_0, e0 * r000_0)));
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
     {
-      const double gm = kCons[2][1] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[1] * Dcd[2] - hh * (Dac[5] * Dbd[0] + Dad[1] * Dbc[2]));
-      g[0] += gm * (acc[20] - 1.0 * acc[5]);
-      g[3] += gm * bp_b110_100_001_000;
-      g[6] += gm * acc[102];
-      g[1] += gm * (acc[23] - 1.0 * acc[2]);
-      g[4] += gm * bp_b110_010_001_000;
-      g[7] += gm * acc[103];
-      g[2] += gm * acc[32];
-      g[5] += gm * bp_b110_001_001_000;
-      g[8] += gm * (acc[104] - 1.0 * acc[10]);
+      const double ac0 = P[oc + 5 * n + 0] * (kCons[2][5] * kCons[1][0]);
+      const double ac1 = P[oc + 5 * n + 1] * (kCons[2][5] * kCons[1][1]);
+      const double ac2 = P[oc + 5 * n + 2] * (kCons[2][5] * kCons[1][2]);
+      const double ad0 = P[od + 5 * n + 0] * (kCons[2][5] * kCons[0][0]);
+      {
+        const double ab = Pab[5 * n + 0] * (kCons[2][5] * kCons[0][0]);
+        const double g0_0 = fma(-ad0, Dbc[0], fma(-ac0, Dbd[0], ab * Dcd[0]));
+        const double g1_0 = fma(-ad0, Dbc[1], fma(-ac1, Dbd[0], ab * Dcd[1]));
+        const double g2_0 = fma(-ad0, Dbc[2], fma(-ac2, Dbd[0], ab * Dcd[2]));
+        const double y000 = fma(k2_0_000, g2_0, fma(k1_0_000, g1_0, k0_0_000 * g0_0));
+        const double y001 = k2_0_001 * g2_0;
+        const double y010 = k1_0_010 * g1_0;
+        const double y100 = k0_0_100 * g0_0;
+        const double t000 = fma(y100, r100_0, fma(y010, r010_0, fma(y001, r001_0, y000 * r000_0)));
+        const double t001 = fma(y100, r101_0, fma(y010, r011_0, fma(y001, r002_0, y000 * r001_0)));
+        const double t010 = fma(y100, r110_0, fma(y010, r020_0, fma(y001, r011_0, y000 * r010_0)));
+        const double t100 = fma(y100, r200_0, fma(y010, r110_0, fma(y001, r101_0, y000 * r100_0)));
+        const double t002 = fma(y100, r102_0, fma(y010, r012_0, fma(y001, r003_0, y000 * r002_0)));
+        const double t011 = fma(y100, r111_0, fma(y010, r021_0, fma(y001, r012_0, y000 * r011_0)));
+        const double t101 = fma(y100, r201_0, fma(y010, r111_0, fma(y001, r102_0, y000 * r101_0)));
+        const double t003 = fma(y100, r103_0, fma(y010, r013_0, fma(y001, r004_0, y000 * r003_0)));
+        const double t012 = fma(y100, r112_0, fma(y010, r022_0, fma(y001, r013_0, y000 * r012_0)));
+        const double t102 = fma(y100, r202_0, fma(y010, r112_0, fma(y001, r103_0, y000 * r102_0)));
+        const double e0 = E[34];
+        const double e1 = E[35];
+        const double e2 = E[36];
+        w = fma(e2, t002, fma(e1, t001, fma(e0, t000, w)));
+        px = fma(e2, t102, fma(e1, t101, fma(e0, t100, px)));
+        py = fma(e2, t012, fma(e1, t011, fma(e0, t010, py)));
+        pz = fma(e2, t003, fma(e1, t002, fma(e0, t001, pz)));
+        sz = fma(E[38], t001, fma(E[37], t000, sz));
+        const double z000 = fma(e2, r002_0, fma(e1, r001_0, e0 * r000_0));
+        K0_0_000 = fma(g0_0, z000, K0_0_000);
+        K1_0_000 = fma(g1_0, z000, K1_0_000);
+        K2_0_000 = fma(g2_0, z000, K2_0_000);
+      }
     }
-    {
-      const double gm = kCons[2][2] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[2] * Dcd[0] - hh * (Dac[6] * Dbd[0] + Dad[2] * Dbc[0]));
-      g[0] += gm * acc[21];
-      g[3] += gm * bp_b020_100_100_000;
-      g[6] += gm * (acc[105] - 1.0 * acc[11]);
-      g[1] += gm * (acc[24] - 2.0 * acc[3]);
-      g[4] += gm * bp_b020_010_100_000;
-      g[7] += gm * acc[106];
-      g[2] += gm * acc[33];
-      g[5] += gm * bp_b020_001_100_000;
-      g[8] += gm * acc[108];
-    }
-    {
-      const double gm = kCons[2][2] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[2] * Dcd[1] - hh * (Dac[7] * Dbd[0] + Dad[2] * Dbc[1]));
-      g[0] += gm * acc[22];
-      g[3] += gm * bp_b020_100_010_000;
-      g[6] += gm * acc[106];
-      g[1] += gm * (acc[25] - 2.0 * acc[4]);
-      g[4] += gm * bp_b020_010_010_000;
-      g[7] += gm * (acc[107] - 1.0 * acc[11]);
-      g[2] += gm * acc[34];
-      g[5] += gm * bp_b020_001_010_000;
-      g[8] += gm * acc[109];
-    }
-    {
-      const double gm = kCons[2][2] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[2] * Dcd[2] - hh * (Dac[8] * Dbd[0] + Dad[2] * Dbc[2]));
-      g[0] += gm * acc[23];
-      g[3] += gm * bp_b020_100_001_000;
-      g[6] += gm * acc[108];
-      g[1] += gm * (acc[26] - 2.0 * acc[5]);
-      g[4] += gm * bp_b020_010_001_000;
-      g[7] += gm * acc[109];
-      g[2] += gm * acc[35];
-      g[5] += gm * bp_b020_001_001_000;
-      g[8] += gm * (acc[110] - 1.0 * acc[11]);
-    }
-    {
-      const double gm = kCons[2][3] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[3] * Dcd[0] - hh * (Dac[9] * Dbd[0] + Dad[3] * Dbc[0]));
-      g[0] += gm * (acc[27] - 1.0 * acc[6]);
-      g[3] += gm * bp_b101_100_100_000;
-      g[6] += gm * (acc[111] - 1.0 * acc[12]);
-      g[1] += gm * acc[30];
-      g[4] += gm * bp_b101_010_100_000;
-      g[7] += gm * acc[112];
-      g[2] += gm * (acc[36] - 1.0 * acc[0]);
-      g[5] += gm * bp_b101_001_100_000;
-      g[8] += gm * acc[114];
-    }
-    {
-      const double gm = kCons[2][3] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[3] * Dcd[1] - hh * (Dac[10] * Dbd[0] + Dad[3] * Dbc[1]));
-      g[0] += gm * (acc[28] - 1.0 * acc[7]);
-      g[3] += gm * bp_b101_100_010_000;
-      g[6] += gm * acc[112];
-      g[1] += gm * acc[31];
-      g[4] += gm * bp_b101_010_010_000;
-      g[7] += gm * (acc[113] - 1.0 * acc[12]);
-      g[2] += gm * (acc[37] - 1.0 * acc[1]);
-      g[5] += gm * bp_b101_001_010_000;
-      g[8] += gm * acc[115];
-    }
-    {
-      const double gm = kCons[2][3] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[3] * Dcd[2] - hh * (Dac[11] * Dbd[0] + Dad[3] * Dbc[2]));
-      g[0] += gm * (acc[29] - 1.0 * acc[8]);
-      g[3] += gm * bp_b101_100_001_000;
-      g[6] += gm * acc[114];
-      g[1] += gm * acc[32];
-      g[4] += gm * bp_b101_010_001_000;
-      g[7] += gm * acc[115];
-      g[2] += gm * (acc[38] - 1.0 * acc[2]);
-      g[5] += gm * bp_b101_001_001_000;
-      g[8] += gm * (acc[116] - 1.0 * acc[12]);
-    }
-    {
-      const double gm = kCons[2][4] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[4] * Dcd[0] - hh * (Dac[12] * Dbd[0] + Dad[4] * Dbc[0]));
-      g[0] += gm * acc[30];
-      g[3] += gm * bp_b011_100_100_000;
-      g[6] += gm * (acc[117] - 1.0 * acc[13]);
-      g[1] += gm * (acc[33] - 1.0 * acc[6]);
-      g[4] += gm * bp_b011_010_100_000;
-      g[7] += gm * acc[118];
-      g[2] += gm * (acc[39] - 1.0 * acc[3]);
-      g[5] += gm * bp_b011_001_100_000;
-      g[8] += gm * acc[120];
-    }
-    {
-      const double gm = kCons[2][4] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[4] * Dcd[1] - hh * (Dac[13] * Dbd[0] + Dad[4] * Dbc[1]));
-      g[0] += gm * acc[31];
-      g[3] += gm * bp_b011_100_010_000;
-      g[6] += gm * acc[118];
-      g[1] += gm * (acc[34] - 1.0 * acc[7]);
-      g[4] += gm * bp_b011_010_010_000;
-      g[7] += gm * (acc[119] - 1.0 * acc[13]);
-      g[2] += gm * (acc[40] - 1.0 * acc[4]);
-      g[5] += gm * bp_b011_001_010_000;
-      g[8] += gm * acc[121];
-    }
-    {
-      const double gm = kCons[2][4] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[4] * Dcd[2] - hh * (Dac[14] * Dbd[0] + Dad[4] * Dbc[2]));
-      g[0] += gm * acc[32];
-      g[3] += gm * bp_b011_100_001_000;
-      g[6] += gm * acc[120];
-      g[1] += gm * (acc[35] - 1.0 * acc[8]);
-      g[4] += gm * bp_b011_010_001_000;
-      g[7] += gm * acc[121];
-      g[2] += gm * (acc[41] - 1.0 * acc[5]);
-      g[5] += gm * bp_b011_001_001_000;
-      g[8] += gm * (acc[122] - 1.0 * acc[13]);
-    }
-    {
-      const double gm = kCons[2][5] * kCons[0][0] * kCons[1][0] * kCons[0][0] * (2.0 * Dab[5] * Dcd[0] - hh * (Dac[15] * Dbd[0] + Dad[5] * Dbc[0]));
-      g[0] += gm * acc[36];
-      g[3] += gm * bp_b002_100_100_000;
-      g[6] += gm * (acc[123] - 1.0 * acc[14]);
-      g[1] += gm * acc[39];
-      g[4] += gm * bp_b002_010_100_000;
-      g[7] += gm * acc[124];
-      g[2] += gm * (acc[42] - 2.0 * acc[6]);
-      g[5] += gm * bp_b002_001_100_000;
-      g[8] += gm * acc[126];
-    }
-    {
-      const double gm = kCons[2][5] * kCons[0][0] * kCons[1][1] * kCons[0][0] * (2.0 * Dab[5] * Dcd[1] - hh * (Dac[16] * Dbd[0] + Dad[5] * Dbc[1]));
-      g[0] += gm * acc[37];
-      g[3] += gm * bp_b002_100_010_000;
-      g[6] += gm * acc[124];
-      g[1] += gm * acc[40];
-      g[4] += gm * bp_b002_010_010_000;
-      g[7] += gm * (acc[125] - 1.0 * acc[14]);
-      g[2] += gm * (acc[43] - 2.0 * acc[7]);
-      g[5] += gm * bp_b002_001_010_000;
-      g[8] += gm * acc[127];
-    }
-    {
-      const double gm = kCons[2][5] * kCons[0][0] * kCons[1][2] * kCons[0][0] * (2.0 * Dab[5] * Dcd[2] - hh * (Dac[17] * Dbd[0] + Dad[5] * Dbc[2]));
-      g[0] += gm * acc[38];
-      g[3] += gm * bp_b002_100_001_000;
-      g[6] += gm * acc[126];
-      g[1] += gm * acc[41];
-      g[4] += gm * bp_b002_010_001_000;
-      g[7] += gm * acc[127];
-      g[2] += gm * (acc[44] - 2.0 * acc[8]);
-      g[5] += gm * bp_b002_001_001_000;
-      g[8] += gm * (acc[128] - 1.0 * acc[14]);
-    }
+    W = w;
+    gP[0] = px; gP[1] = py; gP[2] = pz;
+    gR[0] = sx; gR[1] = sy; gR[2] = sz;
+    gS[0] = kxd100 * K0_0_000;
+    gS[1] = kyd100 * K1_0_000;
+    gS[2] = kzd100 * K2_0_000;
   }
 };
+__device__ const unsigned kC2010GradMd_index[39] = {4,5,6,7,8,257,513,258,514,259,515,769,770,1024,1280,1536,1792,2048,65537,131073,65538,131074,65539,131075,196609,196610,65792,131328,66048,131584,66304,131840,196864,197120,262144,327680,393216,458752,524288};
+__device__ inline const unsigned* C2010GradMd::index() { return kC2010GradMd_index; }
 }  // namespace qf

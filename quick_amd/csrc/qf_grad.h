@@ -278,91 +278,54 @@ __global__ __launch_bounds__(D::NT) void grad_coop_kernel(const Task* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// Per-lane gradient kernel for the light classes: the layout of the per-lane
-// Fock kernels (one ket pair per lane, the wave's bras sharing the first
-// Q-shell a), with the raised VRR, the four weighted sets, the six HRR
-// blocks and the contraction with the density in registers (generated
-// C::vrr and C::digest).  Atom A is the same for the whole task and atoms
-// C, D for a lane, so dE/dA, dE/dC and dE/dD are summed in registers over
-// the bra loop; dE/dB is summed over the wave per bra.  Sums go to the
-// workgroup's LDS gradient (or straight to md.grad when it does not fit).
+// Per-lane gradient kernel for the classes with La+Lb+Lc+Ld <= 5: the layout
+// of the per-lane Fock kernels (one ket pair per lane, the wave's bras sharing
+// the first Q-shell a), every primitive quartet contracted with the
+// two-particle density on the spot in Hermite Gaussians (gen_md.py, C::prim),
+// so a lane keeps nine sums and no derivative integrals.  Atom A is the same
+// for the whole task and atoms C, D for a lane, so dE/dA, dE/dC and dE/dD are
+// summed in registers over the bra loop; dE/dB is summed over the wave per
+// bra.  Sums go to the workgroup's LDS gradient (or straight to md.grad when
+// it does not fit).
+//
+// Bound: FP64 VALU and its latency at one or two waves per SIMD.  The form it
+// replaces kept the four weighted sets of contracted [e0|f0] and the HRR
+// blocks of a quartet, 2 to 10 KB per lane of them in scratch, and waited for
+// that memory: (H2O)16 6-31G*, ms per gradient before -> now, (dp|pp) 10.6 ->
+// 0.78, (pp|pp) 9.8 -> 0.61, (ds|pp) 8.2 -> 0.68, (dp|ds) 6.8 -> 1.07, (dp|ps)
+// 5.1 -> 0.63, (dd|ps) 4.4 -> 0.60, (ds|ds) 2.5 -> 0.39, (pp|ps) 2.4 -> 0.54,
+// (ps|ss) 1.29 -> 1.06.  The bra primitive is the outer loop (the ket
+// primitive was), so its product table is filled once per bra primitive; both
+// orders keep the same set of primitive quartets, as both pairs are sorted by
+// cutprim.
 // ---------------------------------------------------------------------------
-template <class C, typename Tab>
-__device__ __forceinline__ void grad_lane_contract(const PairBlock& bb, int i, const PairInfo& bi, const PairBlock& kb,
-                                                   int j, const PairInfo& ki, double dn, double primlim, int maxm,
-                                                   double (&acc)[C::NACC], Tab boys_tab, int pb, int pe, int qb,
-                                                   int qe)
-{
-    const auto bpc = cptr(bb.prim);
-    const auto kp = gptr(kb.prim);
-    const int bn = bb.n, bK = bb.K, kn = kb.n, kK = kb.K;
-    const size_t bfs = (size_t)bK * bn, kfs = (size_t)kK * kn;
-#define BP(f, q) (*(const QF_AS_CONST double*)((const QF_AS_CONST char*)(bpc + (f) * bfs) + (uint32_t)((q) * bn + i) * 8u))
-#define KP(f, off) (*(const QF_AS_GLOBAL double*)((const QF_AS_GLOBAL char*)(kp + (f) * kfs) + (off)))
-    const double c0 = dn * BP(PF_CUT, 0);
-    for (int jp = qb; jp < qe; ++jp) {
-        const uint32_t ko = (uint32_t)(jp * kn + j) * 8u;
-        const double cutk = KP(PF_CUT, ko);
-        if (!(c0 * cutk > primlim)) break;
-        const double zk = KP(PF_ZETA, ko);
-        const double ozk = KP(PF_OOZ2, ko);
-        const double Kk = KP(PF_KC, ko);
-        const double gk = KP(PF_ALPHA, ko);
-        const double Qk[3] = {KP(PF_PX, ko), KP(PF_PY, ko), KP(PF_PZ, ko)};
-        const double QC[3] = {Qk[0] - ki.A[0], Qk[1] - ki.A[1], Qk[2] - ki.A[2]};
-        for (int ip0 = pb; ip0 < pe; ++ip0) {
-            const int ip = wave_uniform(ip0);    // the active lanes agree: scalar loads of the bra data
-            if (!((dn * BP(PF_CUT, ip)) * cutk > primlim)) break;
-            const double zb = BP(PF_ZETA, ip);
-            const double ozb = BP(PF_OOZ2, ip);
-            const double ab = BP(PF_ALPHA, ip);
-            const double Pb[3] = {BP(PF_PX, ip), BP(PF_PY, ip), BP(PF_PZ, ip)};
-            const double Kb = BP(PF_KC, ip);
-            const double rs = qf_rsqrt(zb + zk);
-            const double inv = rs * rs;
-            const double PQ[3] = {Pb[0] - Qk[0], Pb[1] - Qk[1], Pb[2] - Qk[2]};
-            const double rpq = PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2];
-            const double T = rpq * (zb * zk * inv);
-            double F[C::L + 1];
-            boys_quick<C::L, Tab, 4>(T, maxm, F, boys_tab);
-            const double pref = Kb * Kk * rs;
-#pragma unroll
-            for (int m = 0; m <= C::L; ++m) F[m] *= pref;
-            VrrPar<double> p;
-            const double wp = zk * inv, wq = zb * inv;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                p.PA[d] = Pb[d] - bi.A[d];
-                p.WP[d] = -wp * PQ[d];
-                p.QC[d] = QC[d];
-                p.WQ[d] = wq * PQ[d];
-            }
-            p.oo2z = ozb;
-            p.oo2n = ozk;
-            p.oo2zn = 0.5 * inv;
-            p.rz = wp;
-            p.rn = wq;
-            const double w[4] = {1.0, 2.0 * ab, 2.0 * (zb - ab), 2.0 * gk};
-            C::vrr(F, p, w, acc);
-        }
-    }
-#undef BP
-#undef KP
-}
+#if defined(__HIP_DEVICE_COMPILE__)
+// x in a vector (scalar) register of unknown value: what is loaded from it
+// cannot be hoisted out of a loop
+#define QF_OPAQUE(x) asm volatile("" : "+v"(x))
+#define QF_OPAQUE_S(x) asm volatile("" : "+s"(x))
+#else
+#define QF_OPAQUE(x)
+#define QF_OPAQUE_S(x)
+#endif
 
 template <class C>
-__global__ __launch_bounds__(WAVE) void grad_lane_kernel(const Task* __restrict__ tasks, int ntasks,
-                                                        const PairBlock* __restrict__ blocks,
-                                                        const MolDesc* __restrict__ mols, int tile, int fp32)
+__global__ __attribute__((amdgpu_flat_work_group_size(WAVE, WAVE), amdgpu_waves_per_eu(C::MIN_WAVES)))
+void grad_md_kernel(const Task* __restrict__ tasks, int ntasks, const PairBlock* __restrict__ blocks,
+                    const MolDesc* __restrict__ mols, int tile, int fp32)
 {
-    constexpr int na = ncart(C::La), nb = ncart(C::Lb), nc = ncart(C::Lc), nd = ncart(C::Ld);
+    constexpr int nb = ncart(C::Lb), nc = ncart(C::Lc), nd = ncart(C::Ld);
     QF_BOYS_LDS_DECL;
     QF_BOYS_LDS_FILL();
+    // bra primitive: 1D coefficients of x, y, z, then the products C::prim reads
+    __shared__ double qf_bra[3 * C::N1 + (C::NE > 0 ? C::NE : 1)];
+    QF_AS_LDS double* bra = (QF_AS_LDS double*)qf_bra;
     extern __shared__ double qf_lds[];
     QF_AS_LDS double* gt = (QF_AS_LDS double*)qf_lds;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x % WAVE;
     for (int x = lane; x < tile; x += WAVE) gt[x] = 0.0;
     __syncthreads();
+    const auto index = gptr(C::index());
     const MolDesc* md_last = nullptr;
     for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
         const Task t = cptr(tasks)[ti];
@@ -370,12 +333,16 @@ __global__ __launch_bounds__(WAVE) void grad_lane_kernel(const Task* __restrict_
         const PairBlock kb = cptr(blocks)[t.ket_block];
         const MolDesc md = cptr(mols)[bb.mol];
         md_last = mols + bb.mol;
+        const int n = md.nbasis, ns = md.nshell;
         const auto grad = gptr_rw(md.grad);
-        const int ns = md.nshell, n = md.nbasis;
         const auto cm = gptr(md.cutmat);
         const auto sat = gptr(md.shell_atom);
         const auto P = gptr(md.P);
+        const auto Pu = cptr(md.P);
         const auto bperm = cptr(bb.bperm);
+        const auto bp = cptr(bb.prim);     // bra data, the same in every lane: scalar loads
+        const auto kp = gptr(kb.prim);
+        const int bn = bb.n, bK = bb.K, kn = kb.n, kK = kb.K;
         const bool in_range = lane < t.ket_count;
         const int j = t.ket_start + (in_range ? lane : 0);
         const PairInfo ki = gptr(kb.info)[j];
@@ -383,10 +350,11 @@ __global__ __launch_bounds__(WAVE) void grad_lane_kernel(const Task* __restrict_
         const double hh = 0.5 * md.hyb;
         double gA[3] = {0.0, 0.0, 0.0}, gC[3] = {0.0, 0.0, 0.0}, gD[3] = {0.0, 0.0, 0.0};
         int atA = 0;
-        // density blocks of the ket pair (the same for every bra)
+        // density block of the ket pair (the same for every bra), scaled as C::prim takes it
         double Dcd[nc * nd];
 #pragma unroll
-        for (int x = 0; x < nc * nd; ++x) Dcd[x] = P[(ki.fa + x / nd) * n + ki.fb + x % nd];
+        for (int x = 0; x < nc * nd; ++x)
+            Dcd[x] = P[(ki.fa + x / nd) * n + ki.fb + x % nd] * (2.0 * kCons[C::Lc][x / nd] * kCons[C::Ld][x % nd]);
         for (int kk0 = t.kb; kk0 < t.ke; ++kk0) {
             const int kk = wave_uniform(kk0);
             const int i = bperm[kk];
@@ -400,41 +368,98 @@ __global__ __launch_bounds__(WAVE) void grad_lane_kernel(const Task* __restrict_
             dn = fmax(dn, cm[bi.sb * ns + ki.sa]);
             dn = fmax(dn, cm[bi.sb * ns + ki.sb]);
             const bool one_atom = atA == atB && atA == atC && atA == atD;
+            // the two precision halves of a split class share boundary windows: each
+            // launch keeps its own side of md.split, as the Fock kernels do
             const bool half = fp32 ? (ytest < md.split) : (t.all_fp64 || ytest >= md.split);
             const bool valid = in_range && !one_atom && half && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
                                (!t.same_block || j <= i);
+            if (!__any(valid)) continue;
+            double Dbc[nb * nc], Dbd[nb * nd];
+#pragma unroll
+            for (int x = 0; x < nb * nc; ++x)
+                Dbc[x] = P[(bi.fb + x / nc) * n + ki.fa + x % nc] * (hh * (kCons[C::Lb][x / nc] * kCons[C::Lc][x % nc]));
+#pragma unroll
+            for (int x = 0; x < nb * nd; ++x)
+                Dbd[x] = P[(bi.fb + x / nd) * n + ki.fb + x % nd] * (hh * (kCons[C::Lb][x / nd] * kCons[C::Ld][x % nd]));
+            // QUICK's CPU gradient evaluates FmT with NABCD + 2 (eri_grad.fh:104-106)
+            const int maxm = bi.qfs + ki.qfs + 2;
             double g[9];
 #pragma unroll
             for (int k = 0; k < 9; ++k) g[k] = 0.0;
-            if (valid) {
-                double acc[C::NACC];
+            for (int ip0 = t.pb; ip0 < t.pe; ++ip0) {
+                const int ip = wave_uniform(ip0);
+                const double cb = dn * bp[(PF_CUT * bK + ip) * bn + i];
+                if (!__any(valid && cb * kp[(PF_CUT * kK + t.qb) * kn + j] > md.primlim)) break;
+                const double zb = bp[(PF_ZETA * bK + ip) * bn + i];
+                const double hb = bp[(PF_OOZ2 * bK + ip) * bn + i];
+                const double ab = bp[(PF_ALPHA * bK + ip) * bn + i];
+                const double Pb[3] = {bp[(PF_PX * bK + ip) * bn + i], bp[(PF_PY * bK + ip) * bn + i],
+                                      bp[(PF_PZ * bK + ip) * bn + i]};
+                const double Kb = bp[(PF_KC * bK + ip) * bn + i];
+                const double wa = 2.0 * hb * ab, wb = 2.0 * hb * (zb - ab);   // alpha/p, beta/p
+                if constexpr (C::NE > 0) {
+                    __syncthreads();   // the previous primitive's table has been read
+                    const int dir = lane % 3;
+                    const double PA = dir == 0 ? Pb[0] - bi.A[0] : dir == 1 ? Pb[1] - bi.A[1] : Pb[2] - bi.A[2];
+                    const double AB = dir == 0 ? bi.AB[0] : dir == 1 ? bi.AB[1] : bi.AB[2];
+                    if (lane < 3) C::bra1d(PA, PA + AB, hb, -wb, wa, bra + lane * C::N1);
+                    __syncthreads();
 #pragma unroll
-                for (int x = 0; x < C::NACC; ++x) acc[x] = 0.0;
-                grad_lane_contract<C>(bb, i, bi, kb, j, ki, dn, md.primlim, bi.qfs + ki.qfs + 2, acc,
-                                      QF_BOYS_LDS_PTR, t.pb, t.pe, t.qb, t.qe);
-                double Dab[na * nb], Dac[na * nc], Dad[na * nd], Dbc[nb * nc], Dbd[nb * nd];
+                    for (int x0 = 0; x0 < C::NE; x0 += WAVE) {
+                        const int x = x0 + lane;
+                        const unsigned id = index[x < C::NE ? x : 0];
+                        const double v = bra[id & 255] * bra[C::N1 + ((id >> 8) & 255)] * bra[2 * C::N1 + (id >> 16)];
+                        if (x < C::NE) bra[3 * C::N1 + x] = v;
+                    }
+                    __syncthreads();
+                }
+                const double mu2 = -2.0 * wa * (zb - ab);    // -2 alpha beta / p
+                for (int jp0 = t.qb; jp0 < t.qe; ++jp0) {
+                    const int jp = wave_uniform(jp0);
+                    const size_t ko = (size_t)jp * kn + j, kf = (size_t)kK * kn;
+                    const bool act = valid && cb * kp[PF_CUT * kf + ko] > md.primlim;
+                    if (!__any(act)) break;
+                    if (act) {
+                        const double zk = kp[PF_ZETA * kf + ko], hk = kp[PF_OOZ2 * kf + ko];
+                        const double gk = kp[PF_ALPHA * kf + ko], Kk = kp[PF_KC * kf + ko];
+                        const double Qk[3] = {kp[PF_PX * kf + ko], kp[PF_PY * kf + ko], kp[PF_PZ * kf + ko]};
+                        const double QC[3] = {Qk[0] - ki.A[0], Qk[1] - ki.A[1], Qk[2] - ki.A[2]};
+                        const double QD[3] = {QC[0] + ki.AB[0], QC[1] + ki.AB[1], QC[2] + ki.AB[2]};
+                        const double PQ[3] = {Pb[0] - Qk[0], Pb[1] - Qk[1], Pb[2] - Qk[2]};
+                        const double rs = qf_rsqrt(zb + zk);
+                        const double al = zb * zk * (rs * rs);
+                        const double rpq = PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2];
+                        double F[C::L + 1];
+                        boys_quick<C::L, const QF_AS_LDS double*, 4>(rpq * al, maxm, F, QF_BOYS_LDS_PTR);
+                        const double wc = 2.0 * hk * gk, wd = 2.0 * hk * (zk - gk);   // gamma/q, delta/q
+                        double W, gP[3], gR[3], gS[3];
+                        // the product table and the a-b block are the same for every ket
+                        // primitive: hoisted, they would be hundreds of registers
+                        int eo = 3 * C::N1, po = bi.fa * n + bi.fb;
+                        QF_OPAQUE(eo);
+                        QF_OPAQUE_S(po);
+                        C::prim(F, Kb * Kk * rs, -2.0 * al, PQ, QC, QD, hk, -wd, wc, bra + eo, Pu + po, P, n, bi.fa * n + ki.fa, bi.fa * n + ki.fb, Dcd, Dbc, Dbd, W,
+                                gP, gR, gS);
+                        const double nu2 = -2.0 * wc * (zk - gk);
 #pragma unroll
-                for (int x = 0; x < na * nb; ++x) Dab[x] = P[(bi.fa + x / nb) * n + bi.fb + x % nb];
-#pragma unroll
-                for (int x = 0; x < na * nc; ++x) Dac[x] = P[(bi.fa + x / nc) * n + ki.fa + x % nc];
-#pragma unroll
-                for (int x = 0; x < na * nd; ++x) Dad[x] = P[(bi.fa + x / nd) * n + ki.fb + x % nd];
-#pragma unroll
-                for (int x = 0; x < nb * nc; ++x) Dbc[x] = P[(bi.fb + x / nc) * n + ki.fa + x % nc];
-#pragma unroll
-                for (int x = 0; x < nb * nd; ++x) Dbd[x] = P[(bi.fb + x / nd) * n + ki.fb + x % nd];
-                C::digest(acc, bi.AB, ki.AB, Dab, Dcd, Dac, Dad, Dbc, Dbd, hh, g);
-                const double sdeg = 0.25 * (bi.qa != bi.qb ? 2.0 : 1.0) * (ki.qa != ki.qb ? 2.0 : 1.0) *
-                                    (bi.id != ki.id ? 2.0 : 1.0);
-#pragma unroll
-                for (int k = 0; k < 9; ++k) g[k] *= sdeg;
+                        for (int x = 0; x < 3; ++x) {
+                            const double r = fma(mu2 * bi.AB[x], W, gR[x]), s = fma(nu2 * ki.AB[x], W, gS[x]);
+                            g[x] += fma(wa, gP[x], r);
+                            g[3 + x] += fma(wb, gP[x], -r);
+                            g[6 + x] += fma(-wc, gP[x], s);
+                        }
+                    }
+                }
             }
+            const double sdeg = 0.25 * (bi.qa != bi.qb ? 2.0 : 1.0) * (ki.qa != ki.qb ? 2.0 : 1.0) *
+                                (bi.id != ki.id ? 2.0 : 1.0);
 #pragma unroll
             for (int x = 0; x < 3; ++x) {
-                gA[x] += g[x];
-                gC[x] += g[6 + x];
-                gD[x] -= g[x] + g[3 + x] + g[6 + x];
-                const double b = wave_sum_all_active(g[3 + x]);
+                const double a = sdeg * g[x], bs = sdeg * g[3 + x], c = sdeg * g[6 + x];
+                gA[x] += a;
+                gC[x] += c;
+                gD[x] -= a + bs + c;
+                const double b = wave_sum_all_active(bs);
                 if (lane == 0) {
                     if (tile)
                         lds_add(gt + 3 * atB + x, b);
