@@ -47,6 +47,7 @@ def _deps(src):
     if base.startswith("eri_"):
         deps.append(os.path.join(CSRC, "gen", base[4:-4] + ".h"))
         deps.append(os.path.join(CSRC, "gen", "coop_" + base[4:-4] + ".h"))
+        deps += [os.path.join(CSRC, "qf_md.h"), os.path.join(CSRC, "gen", "md_" + base[4:-4] + ".h")]
     if base.startswith("egrad_"):
         deps += [os.path.join(CSRC, "qf_grad.h"), os.path.join(CSRC, "gen", "grad_maps.h"),
                  os.path.join(CSRC, "gen", "grad_" + base[6:-4] + ".h")]

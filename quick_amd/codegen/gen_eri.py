@@ -621,13 +621,31 @@ def gen_class(La, Lb, Lc, Ld):
                                              vrr_flop=vflops, hrr_flop=hflops, nodes=len(vrr.nodes))
 
 
-def launcher_source(name, diag, coop=False, lane=True, fp32=True):
+# Classes whose closed-shell FP64 LDS-tile launches run in Hermite Gaussians
+# (fock_md_kernel, gen_md.py) instead of the contracted recursions.  One launch
+# alone, ms, (H2O)32 6-31G* / (Gly)4 6-31G**, best shape of each form: (dp|pp)
+# 0.72 / 0.80 -> 0.38 / 0.39, (dd|ds) 0.76 / 0.35 (wave per quartet) -> 0.51 /
+# 0.38, (dd|pp) 0.43 / 0.39 -> 0.55 / 0.43, (dp|dp) 0.52 / 0.62 -> 0.86 / 1.16:
+# the last two gain beside other launches, as they issue fewer instructions
+# (engine.hip, make_tasks).  Not kept: (pp|pp) 0.29 -> 0.44, (ds|pp) 0.32 ->
+# 0.67, (ds|ds) 0.26 -> 0.46, (dp|ps) 0.44 -> 0.74, (dd|ps) 0.22 -> 0.38, (dp|ds)
+# 0.66 / 0.35 -> 0.62 / 0.40: contracted quartets repeat the digestion for every
+# primitive quartet.
+MD_CLASSES = [(2, 1, 1, 1), (2, 2, 2, 0), (2, 1, 2, 1), (2, 2, 1, 1)]
+
+
+def has_tile_kernels(La, Lb, Lc, Ld):
+    return has_lane_kernels(La, Lb, Lc, Ld) or (La, Lb, Lc, Ld) in MD_CLASSES
+
+
+def launcher_source(name, diag, coop=False, lane=True, fp32=True, md=False):
     """Launchers of one class.  ``lane``: the class has per-lane kernels
     (direct FP64 and LDS-tile FP64/FP32); without them every launch of the
     class goes to the wave-per-quartet kernel and its Schwarz diagonal to the
     wave-per-quartet Schwarz kernel."""
     out = ["// Generated by quick_amd/codegen/gen_eri.py - do not edit."]
     out += (['#include "%s.h"' % name] if lane else []) + (['#include "coop_%s.h"' % name] if coop else [])
+    out += ['#include "md_%s.h"' % name] if md else []
     out += ["", "namespace qf {", ""]
     if lane:
         out += ["// Direct-atomic launch; FP64 only.  The FP32 instantiation of the direct",
@@ -671,9 +689,22 @@ def launcher_source(name, diag, coop=False, lane=True, fp32=True):
                 "    else if (os)",
                 "        hipLaunchKernelGGL((fock_tile_kernel<%s, double, true>), dim3(grid), dim3(waves * WAVE), lds, s,"
                 " g, ng, t, b, m, k2);" % name,
-                "    else",
-                "        hipLaunchKernelGGL((fock_tile_kernel<%s, double>), dim3(grid), dim3(waves * WAVE), lds, s,"
-                " g, ng, t, b, m, 0);" % name,
+                "    else"]
+        out += (["        hipLaunchKernelGGL((fock_md_kernel<%sMd>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                 " g, ng, t, b, m);" % name] if md else
+                ["        hipLaunchKernelGGL((fock_tile_kernel<%s, double>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                 " g, ng, t, b, m, 0);" % name])
+        out += ["}", ""]
+    elif md:
+        out += ["// closed shell, FP64 only (an open-shell build runs the class in two passes)",
+                "void launch_fock_tile_%s(const TileGroup* g, int ng, const Task* t, const PairBlock* b,"
+                " const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)" % name, "{",
+                "    if (ng <= 0) return;",
+                "    if (grid <= 0 || grid > ng) grid = ng;",
+                "    (void)fp32;",
+                "    (void)os;",
+                "    hipLaunchKernelGGL((fock_md_kernel<%sMd>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m);"
+                % name,
                 "}", ""]
     if coop:
         out += ["// gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its",
@@ -719,6 +750,7 @@ def _write(path, text):
 
 
 def main():
+    from . import gen_md
     os.makedirs(OUT, exist_ok=True)
     table = {}
     names = []
@@ -738,7 +770,13 @@ def main():
         lane = has_lane_kernels(La, Lb, Lc, Ld)
         assert lane or coop, "a class needs per-lane or wave-per-quartet kernels"
         _write(os.path.join(OUT, "eri_" + name + ".hip"), launcher_source(name, diag, coop, lane,
-                                                                           has_fp32_kernels(La, Lb, Lc, Ld)))
+                                                                           has_fp32_kernels(La, Lb, Lc, Ld),
+                                                                           (La, Lb, Lc, Ld) in MD_CLASSES))
+        if (La, Lb, Lc, Ld) in MD_CLASSES:
+            _write(os.path.join(OUT, "md_" + name + ".h"),
+                   "// Generated by quick_amd/codegen/gen_md.py - do not edit.\n#pragma once\n"
+                   "#include \"../qf_md.h\"\nnamespace qf {\n" + gen_md.md_fock_source(name, La, Lb, Lc, Ld)[1] +
+                   "}  // namespace qf\n")
         names.append((name, La, Lb, Lc, Ld, diag))
         info["boys_setup_flop"] = boys_setup_flop(La + Lb + Lc + Ld)
         info["prim_flop"] = info["vrr_flop"] + info["boys_setup_flop"]
@@ -762,6 +800,7 @@ def main():
         if has_lane_kernels(La, Lb, Lc, Ld):
             lines.append("int launch_fock_%s(const Task*, int, const PairBlock*, const MolDesc*, int, int, int,"
                          " hipStream_t);" % name)
+        if has_tile_kernels(La, Lb, Lc, Ld):
             lines.append("void launch_fock_tile_%s(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*,"
                          " int, int, int, size_t, int, hipStream_t);" % name)
         if (La, Lb, Lc, Ld) in COOP_CLASSES:
@@ -790,9 +829,13 @@ def main():
             lines.append("    if (cb == %d && ck == %d) return launch_fock_%s;" % (pc[(La, Lb)], pc[(Lc, Ld)], name))
     lines += ["    return nullptr;", "}", "", "inline FockTileLaunch fock_tile_launcher(int cb, int ck)", "{"]
     for (name, La, Lb, Lc, Ld, diag) in names:
-        if has_lane_kernels(La, Lb, Lc, Ld):
+        if has_tile_kernels(La, Lb, Lc, Ld):
             lines.append("    if (cb == %d && ck == %d) return launch_fock_tile_%s;" % (pc[(La, Lb)], pc[(Lc, Ld)], name))
-    lines += ["    return nullptr;", "}", "", "// wave-per-quartet kernels (nullptr: the class has none)",
+    lines += ["    return nullptr;", "}", "",
+              "// the class's closed-shell FP64 tile kernel runs in Hermite Gaussians (fock_md_kernel)",
+              "inline bool fock_tile_is_md(int cb, int ck)", "{",
+              "    return %s;" % " || ".join("(cb == %d && ck == %d)" % (pc[c[:2]], pc[c[2:]]) for c in MD_CLASSES), "}"]
+    lines += ["", "// wave-per-quartet kernels (nullptr: the class has none)",
               "inline FockCoopLaunch fock_coop_launcher(int cb, int ck)", "{"]
     for (name, La, Lb, Lc, Ld, diag) in names:
         if (La, Lb, Lc, Ld) in COOP_CLASSES:

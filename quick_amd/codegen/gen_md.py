@@ -1,5 +1,6 @@
-"""Per-lane gradient kernels in Hermite Gaussians (McMurchie and Davidson,
-J. Comput. Phys. 26, 218 (1978)): straight-line code of one primitive quartet.
+"""Per-lane kernels in Hermite Gaussians (McMurchie and Davidson, J. Comput.
+Phys. 26, 218 (1978)): straight-line code of one primitive quartet, for the
+gradient (md_grad_source) and for the Fock build (md_fock_source).
 
 With Hermite expansions of the bra and ket pairs, E^{ab}_P and E^{cd}_Q, and
 the Hermite Coulomb integrals R_N(P - Q), N = (t, u, v),
@@ -25,7 +26,14 @@ expansion coefficients and one component pair (a, b) at a time:
 
 after all (a, b), dW/dS_x = sum_{cd,Q} (dE^{cd}_Q/dS_x) K_{cd,Q}.  E without
 the factor exp(-mu R^2), which the primitive table holds; its derivative is
--2 mu R_x W.  The bra pair is the same in every lane: its products
+-2 mu R_x W.
+
+The Fock build takes one component pair (a, b) at a time too: Z_Q as above,
+(ab|cd) = sum_Q E^{cd}_Q Z_Q, and each integral goes into J and K at once, per
+primitive quartet: no contracted integrals or recursion intermediates are
+kept, which in the classes from (dp|pp) up fill more than the registers.
+
+The bra pair is the same in every lane: its products
 E_x E_y E_z and (dE_x) E_y E_z come from a table in LDS that the wave fills
 once per bra primitive (bra1d and the index list).
 """
@@ -278,6 +286,107 @@ def md_grad_source(name, La, Lb, Lc, Ld):
             " const ET E, const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[%d],"
             " const double (&Dbc)[%d], const double (&Dbd)[%d], double& W, double (&gP)[3], double (&gR)[3],"
             " double (&gS)[3]) {" % (nc * nd, nb * nc, nb * nd)]
+    src += ["    " + l for l in lines]
+    src += ["  }", "};"]
+    idx = sorted(prods, key=prods.get)
+    src += ["__device__ const unsigned k%s_index[%d] = {%s};"
+            % (g, max(1, len(idx)), ",".join(str(x | y << 8 | z << 16) for x, y, z in idx) or "0"),
+            "__device__ inline const unsigned* %s::index() { return k%s_index; }" % (g, g)]
+    return g, "\n".join(src) + "\n"
+
+
+def md_fock_source(name, La, Lb, Lc, Ld):
+    """Fock digestion of one primitive quartet.  ``out`` takes the sums that
+    leave the lane: jab_add(k, v) for element k of J_ab, rows(ia, c, d) for row ia
+    of the a-c and a-d exchange blocks."""
+    ca, cb, cc, cd = comps(La), comps(Lb), comps(Lc), comps(Ld)
+    nb, nc, nd = len(cb), len(cc), len(cd)
+    L = La + Lb + Lc + Ld
+    bra = Table1D(La, Lb, "b", "h", "X", "Y", "0.0", "0.0")
+    order = [k for k in bra.order if k[0] == "e"]
+    index1 = {("e", 0, 0, 0): 0}
+    for k in order:
+        index1[k] = len(index1)
+    n1 = len(index1)
+    prods = {}
+
+    def bra_entry(a, b, P):
+        ids = tuple(index1[("e", a[x], b[x], P[x])] for x in range(3))
+        if ids == (0, 0, 0):
+            return "1"
+        if ids not in prods:
+            prods[ids] = len(prods)
+        return "E[%d]" % prods[ids]
+
+    lines = list(r_lines(L))
+    ket = []
+    for x in range(3):
+        t = Table1D(Lc, Ld, "k%s" % "xyz"[x], "hk", "QC[%d]" % x, "QD[%d]" % x, "0.0", "0.0", sign=-1)
+        lines += [l for l in t.lines if l.startswith("const double k%se" % "xyz"[x])]
+        ket.append(t)
+    kets = [(ic, id_, c, d) for ic, c in enumerate(cc) for id_, d in enumerate(cd)]
+    for ic, id_, c, d in kets:
+        for Q in box(c, d):
+            p = product([ket[x].get("e", c[x], d[x], Q[x]) for x in range(3)])
+            lines.append("const double k%d_%d_%d%d%d = %s(kCons[%d][%d] * kCons[%d][%d]);"
+                         % ((ic, id_) + Q + ("" if p == "1" else p + " * ", Lc, ic, Ld, id_)))
+    Qall = sorted({Q for _, _, c, d in kets for Q in box(c, d)}, key=lambda q: (sum(q), q))
+    lines += ["QF_OPAQUE(oc);", "QF_OPAQUE(od);"]
+    for ia, a in enumerate(ca):
+        lines.append("{")
+        for ic in range(nc):
+            lines.append("  const double ac%d = P[oc + %d * n + %d] * kCons[%d][%d];" % (ic, ia, ic, La, ia))
+        for id_ in range(nd):
+            lines.append("  const double ad%d = P[od + %d * n + %d] * kCons[%d][%d];" % (id_, ia, id_, La, ia))
+        for ib, b in enumerate(cb):
+            lines.append("  {")
+            o = "    "
+            lines.append(o + "const double ab = Pab[%d * n + %d] * (kCons[%d][%d] * kCons[%d][%d]);"
+                         % (ia, ib, La, ia, Lb, ib))
+            B = box(a, b)
+            for k, P in enumerate(B):
+                e = bra_entry(a, b, P)
+                if e != "1":
+                    lines.append(o + "const double e%d = %s;" % (k, e))
+            for Q in Qall:
+                lines.append(o + "const double z%d%d%d = %s;" % (Q + (sum_of(
+                    [("1" if bra_entry(a, b, P) == "1" else "e%d" % k, rn(plus(P, Q))) for k, P in enumerate(B)]),)))
+            lines.append(o + "double j = 0.0;")
+            for ic, id_, c, d in kets:
+                v = sum_of([("k%d_%d_%d%d%d" % ((ic, id_) + Q), "z%d%d%d" % Q) for Q in box(c, d)])
+                lines.append(o + "{")
+                lines.append(o + "  const double v = %s;" % v)
+                lines.append(o + "  j = fma(Dcd[%d], v, j);" % (ic * nd + id_))
+                lines.append(o + "  Jcd[%d] = fma(ab, v, Jcd[%d]);" % (ic * nd + id_, ic * nd + id_))
+                lines.append(o + "  Kac[%d] = fma(Dbd[%d], v, Kac[%d]);" % (ia * nc + ic, ib * nd + id_, ia * nc + ic))
+                lines.append(o + "  Kad[%d] = fma(Dbc[%d], v, Kad[%d]);" % (ia * nd + id_, ib * nc + ic, ia * nd + id_))
+                lines.append(o + "  Kbc[%d] = fma(ad%d, v, Kbc[%d]);" % (ib * nc + ic, id_, ib * nc + ic))
+                lines.append(o + "  Kbd[%d] = fma(ac%d, v, Kbd[%d]);" % (ib * nd + id_, ic, ib * nd + id_))
+                lines.append(o + "}")
+            lines.append(o + "Jab[%d] += j;" % (ia * nb + ib))
+            lines.append("  }")
+        lines.append("}")
+    g = name + "Md"
+    src = ["// (%s%s|%s%s): %d Hermite Coulomb integrals, %d bra products"
+           % ("spd"[La], "spd"[Lb], "spd"[Lc], "spd"[Ld], len(hermites(L)), len(prods)),
+           "struct %s {" % g,
+           "  static constexpr int La = %d, Lb = %d, Lc = %d, Ld = %d, L = %d;" % (La, Lb, Lc, Ld, L),
+           "  static constexpr int N1 = %d, NE = %d;   // 1D entries per direction, product table" % (n1, len(prods)),
+           "  __device__ static const unsigned* index();   // 1D entries of a product, x | y << 8 | z << 16",
+           "  // 1D coefficients of one direction: X = P - A, Y = P - B, h = 1/2p",
+           "  template <class T>",
+           "  __host__ __device__ static __forceinline__ void bra1d(double X, double Y, double h, T out) {"]
+    src += ["    " + l for l in bra.lines if l.startswith("const double be")]
+    src += ["    out[0] = 1.0;"] + ["    out[%d] = %s;" % (index1[k], bra.names[k]) for k in order]
+    src += ["  }",
+            "  // Dbc and Dbd with the cons of b; oc, od: first elements of the a-c and a-d blocks of P",
+            "  template <class ET, class PT, class PU>",
+            "  __host__ __device__ static __forceinline__ void prim(const double (&F)[L + 1], double pref, double m2a,"
+            " const double (&PQ)[3], const double (&QC)[3], const double (&QD)[3], double hk, const ET E,"
+            " const PU Pab, const PT P, int n, int oc, int od, const double (&Dcd)[%d], const double (&Dbc)[%d],"
+            " const double (&Dbd)[%d], double (&Jcd)[%d], double (&Kbc)[%d], double (&Kbd)[%d], double (&Jab)[%d], double (&Kac)[%d],"
+            " double (&Kad)[%d]) {"
+            % (nc * nd, nb * nc, nb * nd, nc * nd, nb * nc, nb * nd, len(ca) * nb, len(ca) * nc, len(ca) * nd)]
     src += ["    " + l for l in lines]
     src += ["  }", "};"]
     idx = sorted(prods, key=prods.get)

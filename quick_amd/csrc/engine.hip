@@ -402,6 +402,8 @@ struct qf_engine {
         size_t lds_os;   // open-shell pass with a second exchange tile (0: it does not fit)
         int os_split;    // open-shell builds run this class as two closed-shell passes
         int os_lean;     // ... or, on the tile kernel, in the fused lean form
+        int alt_offset, alt_count;   // wave-per-quartet tasks of a class whose tile kernel is closed-shell Fock
+                                     // only: open-shell builds and gradients run these (alt_count 0: none)
         size_t gslot;    // first double of its region of the global slot buffer (classes that need one)
     };
     std::vector<Launch> launches;
@@ -822,12 +824,12 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // 1447, C20H42 3-21G (264) 1825 / 1105 / 912 / 897 / 994, (H2O)16
                 // 3703 / 2940 / 3133 / 3171 / 3142, (H2O)32 25512 / 14599 / 12000 / 11245 /
                 // 10973)
-                const int tile_tasks = ct.tpg > 0        ? ct.tpg
+                int tile_tasks = ct.tpg > 0        ? ct.tpg
                                        : e->tile_tasks > 0 ? e->tile_tasks
                                        : size <= 200       ? 2
                                        : size <= 400       ? 4
                                                            : 16;
-                const int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
+                int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
                 // LDS tile: (na + m*nb) x ncol exchange terms + m*na*nb Coulomb terms
                 int maxcol = 0;
                 for (const auto& Kb : e->blocks)
@@ -873,10 +875,29 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // 15.8x -> 18.0x, PSB5 6-31G 26x -> 34x QUICK's build times;
                 // up to 48 functions and at 5 the wave-per-quartet kernel wins)
                 const int coop_lmin = size <= 48 ? 4 : size <= 128 ? 5 : 6;
-                const bool want_coop = !lane_class || ct.tile == 2 || (ct.tile < 0 && e->tile != 0 && Lsum >= coop_lmin);
+                const bool tile_class = qf::fock_tile_launcher(cb, ck) != nullptr;
+                const bool tile_ok = tile_class && mfit >= 1;
+                // Classes whose FP64 tile kernel runs in Hermite Gaussians: above 256
+                // functions it takes over from the wave-per-quartet kernel ((dd|ds),
+                // (dd|pp) and (dp|dp) together: (H2O)32 10.65 -> 10.2 ms a build, (Gly)10
+                // mixed 29.4 -> 26.0; below, too few quartets fill its waves: glycine
+                // 6-31G** 0.63 -> 0.93, (H2O)8 cc-pVDZ 1.08 -> 1.26, which a batch does
+                // not change: 48 molecules 16.0 -> 16.9), with two waves,
+                // four tasks of one bra a workgroup ((dp|pp), (H2O)32: 10.5 ms against
+                // 10.7 with the other classes' shapes).
+                const bool md = !fp32 && tile_ok && qf::fock_tile_is_md(cb, ck);
+                const bool md_shape = md && e->nbasis > 256 && ct.tile < 0 && e->tile != 0;
+                if (md_shape && ct.mmax == 0) mmax = 1;
+                if (md_shape && ct.tpg == 0 && e->tile_tasks == 0) tile_tasks = 4;
+                if (md_shape && ct.waves == 0) tile_waves = std::min(tile_waves, 2);
+                const bool want_coop = ct.tile == 2   ? true
+                                       : ct.tile == 1 ? !lane_class && !tile_ok
+                                       : ct.tile == 0 || e->tile == 0 ? !lane_class
+                                       : md_shape ? false
+                                                  : Lsum >= coop_lmin || (!lane_class && !tile_ok);
                 const bool coop = !fp32 && want_coop && qf::fock_coop_launcher(cb, ck) != nullptr;
-                if (!coop && !lane_class) return fail(QF_ERR_STATE, "class has neither per-lane nor wave-per-quartet kernels");
-                const bool tile = !coop && (fp32 || (ct.tile >= 0 ? ct.tile != 0 : e->tile != 0)) && mfit >= 1;
+                if (!coop && !lane_class && !tile_ok) return fail(QF_ERR_STATE, "class has no kernel for its launch");
+                const bool tile = !coop && tile_ok && (fp32 || !lane_class || (ct.tile >= 0 ? ct.tile != 0 : e->tile != 0));
                 if (tile) mmax = (int)std::min<long long>(mmax, mfit);
                 // kets per task: a full wave for the per-lane kernels; for the
                 // wave-per-quartet kernel a window (the class tuning's
@@ -889,89 +910,98 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_win) : qf::WAVE;
                 size_t lds = 0, lds_os = 0;
                 long long group_tasks = 0;
-                for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
-                    const HostBlock& B = e->blocks[bbk];
-                    if (B.cls != cb) continue;
-                    for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
-                        const HostBlock& Kb = e->blocks[kbk];
-                        if (Kb.cls != ck) continue;
-                        if (cb == ck && kbk > bbk) continue;
-                        const bool same = (cb == ck && kbk == bbk);
-                        std::vector<std::pair<int, int>> chunks;
-                        for (const auto& g : B.groups)
-                            for (int c0 = g.first; c0 < g.second; c0 += mmax)
-                                chunks.push_back({c0, std::min(g.second, c0 + mmax)});
-                        for (const auto& g : chunks) {
-                            // per bra of the group: ket range [lo, hi) of this precision
-                            const int M = g.second - g.first;
-                            std::vector<int> lo(M), hi(M);
-                            int nmax = 0;
-                            for (int k = 0; k < M; ++k) {
-                                const int i = B.bperm[g.first + k];
-                                const double yi = B.info[i].ycut;
-                                int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
-                                if (same) n = std::min(n, i + 1);
-                                if (!fp32 && stats) stats->n_quartets_bound += n;
-                                int n64 = n;
-                                if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
-                                lo[k] = fp32 ? n64 : 0;
-                                hi[k] = fp32 ? n : n64;
-                                nmax = std::max(nmax, hi[k]);
-                            }
-                            const int chunk_first = (int)tasks.size();
-                            for (int s0 = 0; s0 < nmax; s0 += win) {
-                                int kb = -1, ke = -1;
-                                for (int k = 0; k < M; ++k)
-                                    if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
-                                        if (kb < 0) kb = k;
-                                        ke = k + 1;
-                                    }
-                                if (kb < 0) continue;
-                                qf::Task t{};
-                                t.bra_block = (int)bbk;
-                                t.kb = g.first + kb;
-                                t.ke = g.first + ke;
-                                t.ket_block = (int)kbk;
-                                t.ket_start = s0;
-                                t.ket_count = std::min(win, nmax - s0);
-                                t.same_block = same ? 1 : 0;
-                                t.all_fp64 = split_class ? 0 : 1;
-                                // highly contracted pairs: spread the primitive
-                                // pairs of the window over several tasks
-                                const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
-                                const int nbp = (B.K + cpiece - 1) / cpiece, nkp = (Kb.K + cpiece - 1) / cpiece;
-                                const int sb = (B.K + nbp - 1) / nbp, sk = (Kb.K + nkp - 1) / nkp;
-                                for (int pbi = 0; pbi < B.K; pbi += sb)
-                                    for (int qbi = 0; qbi < Kb.K; qbi += sk) {
-                                        t.pb = pbi;
-                                        t.pe = std::min(B.K, pbi + sb);
-                                        t.qb = qbi;
-                                        t.qe = std::min(Kb.K, qbi + sk);
-                                        tasks.push_back(t);
-                                    }
-                            }
-                            if (!tile) continue;
-                            // workgroups of the chunk: consecutive runs of its tasks
-                            const int chunk_end = (int)tasks.size();
-                            for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
-                                qf::TileGroup tg{};
-                                tg.task_begin = t0;
-                                tg.task_end = std::min(chunk_end, t0 + tile_tasks);
-                                tg.chunk_kb = g.first;
-                                tg.nbra = M;
-                                groups.push_back(tg);
-                                group_tasks += tg.task_end - tg.task_begin;
-                            }
-                            if (chunk_end > chunk_first) {
-                                const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
-                                lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
-                                lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
+                // tasks of this launch (and its tile groups), or with alt the
+                // wave-per-quartet tasks of the same quartets
+                auto emit = [&](int win, int mmax, bool alt) {
+                    for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
+                        const HostBlock& B = e->blocks[bbk];
+                        if (B.cls != cb) continue;
+                        for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
+                            const HostBlock& Kb = e->blocks[kbk];
+                            if (Kb.cls != ck) continue;
+                            if (cb == ck && kbk > bbk) continue;
+                            const bool same = (cb == ck && kbk == bbk);
+                            std::vector<std::pair<int, int>> chunks;
+                            for (const auto& g : B.groups)
+                                for (int c0 = g.first; c0 < g.second; c0 += mmax)
+                                    chunks.push_back({c0, std::min(g.second, c0 + mmax)});
+                            for (const auto& g : chunks) {
+                                // per bra of the group: ket range [lo, hi) of this precision
+                                const int M = g.second - g.first;
+                                std::vector<int> lo(M), hi(M);
+                                int nmax = 0;
+                                for (int k = 0; k < M; ++k) {
+                                    const int i = B.bperm[g.first + k];
+                                    const double yi = B.info[i].ycut;
+                                    int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
+                                    if (same) n = std::min(n, i + 1);
+                                    if (!fp32 && stats && !alt) stats->n_quartets_bound += n;
+                                    int n64 = n;
+                                    if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
+                                    lo[k] = fp32 ? n64 : 0;
+                                    hi[k] = fp32 ? n : n64;
+                                    nmax = std::max(nmax, hi[k]);
+                                }
+                                const int chunk_first = (int)tasks.size();
+                                for (int s0 = 0; s0 < nmax; s0 += win) {
+                                    int kb = -1, ke = -1;
+                                    for (int k = 0; k < M; ++k)
+                                        if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
+                                            if (kb < 0) kb = k;
+                                            ke = k + 1;
+                                        }
+                                    if (kb < 0) continue;
+                                    qf::Task t{};
+                                    t.bra_block = (int)bbk;
+                                    t.kb = g.first + kb;
+                                    t.ke = g.first + ke;
+                                    t.ket_block = (int)kbk;
+                                    t.ket_start = s0;
+                                    t.ket_count = std::min(win, nmax - s0);
+                                    t.same_block = same ? 1 : 0;
+                                    t.all_fp64 = split_class ? 0 : 1;
+                                    // highly contracted pairs: spread the primitive
+                                    // pairs of the window over several tasks
+                                    const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
+                                    const int nbp = (B.K + cpiece - 1) / cpiece, nkp = (Kb.K + cpiece - 1) / cpiece;
+                                    const int sb = (B.K + nbp - 1) / nbp, sk = (Kb.K + nkp - 1) / nkp;
+                                    for (int pbi = 0; pbi < B.K; pbi += sb)
+                                        for (int qbi = 0; qbi < Kb.K; qbi += sk) {
+                                            t.pb = pbi;
+                                            t.pe = std::min(B.K, pbi + sb);
+                                            t.qb = qbi;
+                                            t.qe = std::min(Kb.K, qbi + sk);
+                                            tasks.push_back(t);
+                                        }
+                                }
+                                if (!tile || alt) continue;
+                                // workgroups of the chunk: consecutive runs of its tasks
+                                const int chunk_end = (int)tasks.size();
+                                for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
+                                    qf::TileGroup tg{};
+                                    tg.task_begin = t0;
+                                    tg.task_end = std::min(chunk_end, t0 + tile_tasks);
+                                    tg.chunk_kb = g.first;
+                                    tg.nbra = M;
+                                    groups.push_back(tg);
+                                    group_tasks += tg.task_end - tg.task_begin;
+                                }
+                                if (chunk_end > chunk_first) {
+                                    const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
+                                    lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
+                                    lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
+                                }
                             }
                         }
                     }
-                }
+                };
+                emit(win, mmax, false);
                 const int count = (int)tasks.size() - offset;
                 const int gcount = (int)groups.size() - goffset;
+                // open-shell builds and gradients of a class whose tile kernel has neither
+                const int alt_offset = (int)tasks.size();
+                if (tile && !fp32 && !lane_class && stats) emit(coop_win, 1, true);
+                const int alt_count = (int)tasks.size() - alt_offset;
                 // work of a task: bras x kets x primitive pairs (bra and ket);
                 // without the primitive factor the longest-first order misjudges
                 // the contracted classes (13 % of the (H2O)32 build)
@@ -1005,8 +1035,12 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                     std::stable_sort(tasks.begin() + offset, tasks.end(),
                                      [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
                 }
+                std::stable_sort(tasks.begin() + alt_offset, tasks.end(),
+                                 [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
                 if (count > 0) {
                     qf_engine::Launch L{};
+                    L.alt_offset = alt_offset;
+                    L.alt_count = alt_count;
                     L.cb = cb;
                     L.ck = ck;
                     L.fp32 = fp32;
@@ -1327,10 +1361,11 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     if (orc) return orc;
     // one class launch with descriptor m on stream q; los: its open-shell form
     auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, hipStream_t q) -> int {
-        if (L.tile == 2) {
+        const bool alt = los && L.alt_count > 0;
+        if (L.tile == 2 || alt) {
             qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
             if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
-            fc(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p + L.gslot, q);
+            fc(e->d_tasks.p + (alt ? L.alt_offset : L.offset), alt ? L.alt_count : L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p + L.gslot, q);
         } else if (L.tile) {
             qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
             if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
@@ -1630,7 +1665,8 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
             return fail(QF_ERR_ARG, "ERI gradients cover shells up to d; this basis has f shells");
         gslot.push_back(gdoubles);
         if (!lane_kernel(L))
-            gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) * std::min(L.count, qf::COOP_GLOBAL_SLICES);
+            gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) *
+                        std::min(std::max(L.count, L.alt_count), qf::COOP_GLOBAL_SLICES);
     }
     if (gdoubles && e->d_gscratch.n < gdoubles) QF_HIP(e->d_gscratch.resize(gdoubles));
     qf::MolDesc md{};
@@ -1668,8 +1704,11 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
         const size_t tile = slots + tile_bytes <= kGradLdsMax ? tile_bytes : 0;
         // one workgroup per task unless the engine caps the grid (qf_set_persistent):
         // the hardware then hands out tasks as workgroups finish
-        const int grid = e->persist > 0 ? std::min(L.count, e->persist) : L.count;
-        (lane ? lane : qf::grad_launcher(L.cb, L.ck))(e->d_tasks.p + L.offset, L.count, e->d_blocks.p, dmol, grid,
+        const bool alt = L.alt_count > 0;
+        const int count = alt ? L.alt_count : L.count;
+        const int grid = e->persist > 0 ? std::min(count, e->persist) : count;
+        (lane ? lane : qf::grad_launcher(L.cb, L.ck))(e->d_tasks.p + (alt ? L.alt_offset : L.offset), count,
+                                                      e->d_blocks.p, dmol, grid,
                                                       tile, e->d_gscratch.p + gslot[li], L.fp32, q);
         return QF_OK;
     };

@@ -1,6 +1,7 @@
 // Generated by quick_amd/codegen/gen_eri.py - do not edit.
 #include "C2111.h"
 #include "coop_C2111.h"
+#include "md_C2111.h"
 
 namespace qf {
 
@@ -39,7 +40,7 @@ void launch_fock_tile_C2111(const TileGroup* g, int ng, const Task* t, const Pai
     else if (os)
         hipLaunchKernelGGL((fock_tile_kernel<C2111, double, true>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, k2);
     else
-        hipLaunchKernelGGL((fock_tile_kernel<C2111, double>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, 0);
+        hipLaunchKernelGGL((fock_md_kernel<C2111Md>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m);
 }
 
 // gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its

@@ -1,7 +1,18 @@
 // Generated by quick_amd/codegen/gen_eri.py - do not edit.
 #include "coop_C2220.h"
+#include "md_C2220.h"
 
 namespace qf {
+
+// closed shell, FP64 only (an open-shell build runs the class in two passes)
+void launch_fock_tile_C2220(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)
+{
+    if (ng <= 0) return;
+    if (grid <= 0 || grid > ng) grid = ng;
+    (void)fp32;
+    (void)os;
+    hipLaunchKernelGGL((fock_md_kernel<C2220Md>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m);
+}
 
 // gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its
 // slots in global memory (the grid is then capped to that many workgroups)

@@ -51,6 +51,7 @@ void launch_fock_coop_C2111(const Task*, int, const PairBlock*, const MolDesc*, 
 int launch_fock_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
 void launch_fock_tile_C2120(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+void launch_fock_tile_C2121(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C2121(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_schwarz_C2121(PairBlock, double*, double*, hipStream_t);
 int launch_fock_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
@@ -59,7 +60,9 @@ void launch_fock_coop_C2200(const Task*, int, const PairBlock*, const MolDesc*, 
 int launch_fock_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
 void launch_fock_tile_C2210(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+void launch_fock_tile_C2211(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C2211(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+void launch_fock_tile_C2220(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
 void launch_fock_coop_C2220(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C2221(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
 void launch_fock_coop_C2222(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
@@ -225,8 +228,11 @@ inline FockTileLaunch fock_tile_launcher(int cb, int ck)
     if (cb == 4 && ck == 1) return launch_fock_tile_C2110;
     if (cb == 4 && ck == 2) return launch_fock_tile_C2111;
     if (cb == 4 && ck == 3) return launch_fock_tile_C2120;
+    if (cb == 4 && ck == 4) return launch_fock_tile_C2121;
     if (cb == 5 && ck == 0) return launch_fock_tile_C2200;
     if (cb == 5 && ck == 1) return launch_fock_tile_C2210;
+    if (cb == 5 && ck == 2) return launch_fock_tile_C2211;
+    if (cb == 5 && ck == 3) return launch_fock_tile_C2220;
     if (cb == 6 && ck == 0) return launch_fock_tile_C3000;
     if (cb == 6 && ck == 1) return launch_fock_tile_C3010;
     if (cb == 6 && ck == 2) return launch_fock_tile_C3011;
@@ -235,6 +241,12 @@ inline FockTileLaunch fock_tile_launcher(int cb, int ck)
     if (cb == 7 && ck == 1) return launch_fock_tile_C3110;
     if (cb == 8 && ck == 0) return launch_fock_tile_C3200;
     return nullptr;
+}
+
+// the class's closed-shell FP64 tile kernel runs in Hermite Gaussians (fock_md_kernel)
+inline bool fock_tile_is_md(int cb, int ck)
+{
+    return (cb == 4 && ck == 2) || (cb == 5 && ck == 3) || (cb == 4 && ck == 4) || (cb == 5 && ck == 2);
 }
 
 // wave-per-quartet kernels (nullptr: the class has none)

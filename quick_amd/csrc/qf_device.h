@@ -42,6 +42,16 @@ __device__ __forceinline__ QF_AS_GLOBAL T* gptr_rw(T* p)
     return (QF_AS_GLOBAL T*)(p);
 }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+// x in a vector (scalar) register of unknown value: what is loaded from it
+// cannot be hoisted out of a loop
+#define QF_OPAQUE(x) asm volatile("" : "+v"(x))
+#define QF_OPAQUE_S(x) asm volatile("" : "+s"(x))
+#else
+#define QF_OPAQUE(x)
+#define QF_OPAQUE_S(x)
+#endif
+
 // A value that the caller knows to be the same in every active lane, moved
 // to a scalar register.  Loop counters of loops whose exit differs between
 // lanes are kept in vector registers by the compiler (it cannot tell that
@@ -867,6 +877,42 @@ void fock_kernel(const Task* __restrict__ tasks, int ntasks, const PairBlock* __
     }
 }
 
+// Adds the non-zero elements of a workgroup's LDS tile to G (and, from element
+// ntile on, to G2): row r -> function of a (r < na) or of b_k, column q ->
+// colf[q]; then the Coulomb terms of the bras.
+template <int na, int nb>
+__device__ __forceinline__ void tile_flush(QF_AS_LDS double* lds, int nk, int ntile, int njab, int ncol,
+                                           const TileGroup& g, const PairBlock& bb, const PairBlock& kb,
+                                           const MolDesc& md, QF_AS_GLOBAL double* G, QF_AS_GLOBAL double* G2)
+{
+    const int n = md.nbasis;
+    const double kscale = -0.25 * md.hyb;
+    const auto bperm = cptr(bb.bperm);
+    const auto colf = gptr(kb.colf);
+    const int fa = cptr(bb.info)[bperm[g.chunk_kb]].fa;
+    for (int x = threadIdx.x; x < nk; x += blockDim.x) {
+        const double v = lds[x];
+        if (v == 0.0) continue;
+        const int xt = x < ntile ? x : x - ntile;
+        const int r = xt / ncol, q = xt - r * ncol;
+        int fr;
+        if (r < na) {
+            fr = fa + r;
+        } else {
+            const int k = (r - na) / nb;
+            fr = gptr(bb.info)[bperm[g.chunk_kb + k]].fb + (r - na - k * nb);
+        }
+        atomic_add(&(x < ntile ? G : G2)[fr * n + colf[q]], kscale * v);
+    }
+    for (int x = threadIdx.x; x < njab; x += blockDim.x) {
+        const double v = lds[nk + x];
+        if (v == 0.0) continue;
+        const int k = x / (na * nb), ab = x - k * (na * nb);
+        const PairInfo bi = gptr(bb.info)[bperm[g.chunk_kb + k]];
+        atomic_add(&G[(bi.fa + ab / nb) * n + bi.fb + ab % nb], v);
+    }
+}
+
 // One workgroup per TileGroup (striding over the groups when the grid is
 // smaller): its waves take the group's tasks in turn and accumulate J_ab
 // and the exchange terms in LDS; after a barrier the workgroup adds the
@@ -921,32 +967,7 @@ void fock_tile_kernel(const TileGroup* __restrict__ groups, int ngroups, const T
         }
         __syncthreads();
 
-        // flush: row r -> function of a (r < na) or of b_k; column q -> colf[q]
-        const double kscale = -0.25 * md.hyb;
-        const auto bperm = cptr(bb.bperm);
-        const auto colf = gptr(kb.colf);
-        const int fa = cptr(bb.info)[bperm[g.chunk_kb]].fa;
-        for (int x = threadIdx.x; x < nk; x += blockDim.x) {
-            const double v = lds[x];
-            if (v == 0.0) continue;
-            const int xt = x < ntile ? x : x - ntile;
-            const int r = xt / ncol, q = xt - r * ncol;
-            int fr;
-            if (r < na) {
-                fr = fa + r;
-            } else {
-                const int k = (r - na) / nb;
-                fr = gptr(bb.info)[bperm[g.chunk_kb + k]].fb + (r - na - k * nb);
-            }
-            atomic_add(&(x < ntile ? G : G2)[fr * n + colf[q]], kscale * v);
-        }
-        for (int x = threadIdx.x; x < njab; x += blockDim.x) {
-            const double v = lds[nk + x];
-            if (v == 0.0) continue;
-            const int k = x / (na * nb), ab = x - k * (na * nb);
-            const PairInfo bi = gptr(bb.info)[bperm[g.chunk_kb + k]];
-            atomic_add(&G[(bi.fa + ab / nb) * n + bi.fb + ab % nb], v);
-        }
+        tile_flush<na, nb>(lds, nk, ntile, njab, ncol, g, bb, kb, md, G, G2);
         __syncthreads();   // the next group reuses the tile
     }
 }

@@ -299,16 +299,6 @@ __global__ __launch_bounds__(D::NT) void grad_coop_kernel(const Task* __restrict
 // orders keep the same set of primitive quartets, as both pairs are sorted by
 // cutprim.
 // ---------------------------------------------------------------------------
-#if defined(__HIP_DEVICE_COMPILE__)
-// x in a vector (scalar) register of unknown value: what is loaded from it
-// cannot be hoisted out of a loop
-#define QF_OPAQUE(x) asm volatile("" : "+v"(x))
-#define QF_OPAQUE_S(x) asm volatile("" : "+s"(x))
-#else
-#define QF_OPAQUE(x)
-#define QF_OPAQUE_S(x)
-#endif
-
 template <class C>
 __global__ __attribute__((amdgpu_flat_work_group_size(WAVE, WAVE), amdgpu_waves_per_eu(C::MIN_WAVES)))
 void grad_md_kernel(const Task* __restrict__ tasks, int ntasks, const PairBlock* __restrict__ blocks,
