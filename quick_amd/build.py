@@ -41,7 +41,7 @@ def sources():
 
 
 def _deps(src):
-    deps = [src, os.path.join(CSRC, "qf_types.h"), os.path.join(CSRC, "qf_device.h"), os.path.join(CSRC, "qf_coop.h"),
+    deps = [src, os.path.join(CSRC, "qf_types.h"), os.path.join(CSRC, "qf_launch.h"), os.path.join(CSRC, "qf_device.h"), os.path.join(CSRC, "qf_coop.h"),
             os.path.join(os.path.dirname(PKG), "include", "quickfock.h"), os.path.join(CSRC, "gen", "launchers.h")]
     base = os.path.basename(src)
     if base.startswith("eri_"):

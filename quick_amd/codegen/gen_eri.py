@@ -653,74 +653,74 @@ def launcher_source(name, diag, coop=False, lane=True, fp32=True, md=False):
                 "// found): a request for it is refused with a nonzero return.",
                 "// os: 1 = the fused open-shell pass (second exchange density)",
                 "int launch_fock_%s(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int fp32,"
-                " int os, int grid, hipStream_t s)" % name, "{",
+                " int os, int grid, LaunchTo& q)" % name, "{",
                 "    if (fp32) return 1;",
                 "    if (nt <= 0) return 0;",
                 "    if (grid <= 0 || grid > nt) grid = nt;",
                 "    if (os)",
-                "        hipLaunchKernelGGL((fock_kernel<%s, double, true>), dim3(grid), dim3(WAVE), 0, s, t, nt, b, m);"
+                "        q((fock_kernel<%s, double, true>), dim3(grid), dim3(WAVE), 0, t, nt, b, m);"
                 % name,
                 "    else",
-                "        hipLaunchKernelGGL((fock_kernel<%s, double>), dim3(grid), dim3(WAVE), 0, s, t, nt, b, m);" % name,
+                "        q((fock_kernel<%s, double>), dim3(grid), dim3(WAVE), 0, t, nt, b, m);" % name,
                 "    return 0;",
                 "}", "",
                 "// os & 3: 0 closed shell, 1 open shell with a second LDS tile, 2 open",
                 "// shell with the second exchange terms straight to G2; os & 4: the lean",
                 "// open-shell form (FP64; FP32 launches take the register form)",
                 "void launch_fock_tile_%s(const TileGroup* g, int ng, const Task* t, const PairBlock* b,"
-                " const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)" % name, "{",
+                " const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, LaunchTo& q)" % name, "{",
                 "    if (ng <= 0) return;",
                 "    if (grid <= 0 || grid > ng) grid = ng;",
                 "    const bool lean = (os & 4) != 0;",
                 "    os &= 3;",
                 "    const int k2 = os == 1;"]
         out += (["    if (fp32 && os)",
-                 "        hipLaunchKernelGGL((fock_tile_kernel<%s, float, true>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                 "        q((fock_tile_kernel<%s, float, true>), dim3(grid), dim3(waves * WAVE), lds,"
                  " g, ng, t, b, m, k2);" % name,
                  "    else if (fp32)",
-                 "        hipLaunchKernelGGL((fock_tile_kernel<%s, float>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                 "        q((fock_tile_kernel<%s, float>), dim3(grid), dim3(waves * WAVE), lds,"
                  " g, ng, t, b, m, 0);" % name,
                  "    else if (os && lean)"] if fp32 else
                 ["    (void)fp32;   // f classes are never split",
                  "    if (os && lean)"])
         out += [
-                "        hipLaunchKernelGGL((fock_tile_kernel<%s, double, true, true>), dim3(grid), dim3(waves * WAVE), lds,"
-                " s, g, ng, t, b, m, k2);" % name,
+                "        q((fock_tile_kernel<%s, double, true, true>), dim3(grid), dim3(waves * WAVE), lds,"
+                " g, ng, t, b, m, k2);" % name,
                 "    else if (os)",
-                "        hipLaunchKernelGGL((fock_tile_kernel<%s, double, true>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                "        q((fock_tile_kernel<%s, double, true>), dim3(grid), dim3(waves * WAVE), lds,"
                 " g, ng, t, b, m, k2);" % name,
                 "    else"]
-        out += (["        hipLaunchKernelGGL((fock_md_kernel<%sMd>), dim3(grid), dim3(waves * WAVE), lds, s,"
+        out += (["        q((fock_md_kernel<%sMd>), dim3(grid), dim3(waves * WAVE), lds,"
                  " g, ng, t, b, m);" % name] if md else
-                ["        hipLaunchKernelGGL((fock_tile_kernel<%s, double>), dim3(grid), dim3(waves * WAVE), lds, s,"
+                ["        q((fock_tile_kernel<%s, double>), dim3(grid), dim3(waves * WAVE), lds,"
                  " g, ng, t, b, m, 0);" % name])
         out += ["}", ""]
     elif md:
         out += ["// closed shell, FP64 only (an open-shell build runs the class in two passes)",
                 "void launch_fock_tile_%s(const TileGroup* g, int ng, const Task* t, const PairBlock* b,"
-                " const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)" % name, "{",
+                " const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, LaunchTo& q)" % name, "{",
                 "    if (ng <= 0) return;",
                 "    if (grid <= 0 || grid > ng) grid = ng;",
                 "    (void)fp32;",
                 "    (void)os;",
-                "    hipLaunchKernelGGL((fock_md_kernel<%sMd>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m);"
+                "    q((fock_md_kernel<%sMd>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m);"
                 % name,
                 "}", ""]
     if coop:
         out += ["// gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its",
                 "// slots in global memory (the grid is then capped to that many workgroups)",
                 "void launch_fock_coop_%s(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int os,"
-                " int grid, double* gscratch, hipStream_t s)" % name, "{",
+                " int grid, double* gscratch, LaunchTo& q)" % name, "{",
                 "    using D = %sCoop;" % name,
                 "    if (nt <= 0) return;",
                 "    if (grid <= 0 || grid > nt) grid = nt;",
                 "    if (D::GLOBAL_SLOTS && grid > COOP_GLOBAL_SLICES) grid = COOP_GLOBAL_SLICES;",
                 "    const size_t lds = D::GLOBAL_SLOTS ? 0 : D::LDS * sizeof(double);",
                 "    if (os)",
-                "        hipLaunchKernelGGL((fock_coop_kernel<D, true>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m,"
+                "        q((fock_coop_kernel<D, true>), dim3(grid), dim3(D::NT), lds, t, nt, b, m,"
                 " gscratch);",
                 "    else",
-                "        hipLaunchKernelGGL((fock_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch);",
+                "        q((fock_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch);",
                 "}", ""]
     if diag:
         out += ["void launch_schwarz_%s(PairBlock blk, double* out, double* gscratch, hipStream_t s)" % name, "{",
@@ -785,27 +785,27 @@ def main():
     # launch table
     pc = {pcl: k for k, pcl in enumerate(PAIR_CLASSES)}
     lines = ["// Generated by quick_amd/codegen/gen_eri.py - do not edit.", "#pragma once",
-             "#include <hip/hip_runtime.h>", '#include "../qf_types.h"', "", "namespace qf {", "",
+             "#include <hip/hip_runtime.h>", '#include "../qf_launch.h"', '#include "../qf_types.h"', "", "namespace qf {", "",
              "// returns nonzero when the launch is refused (FP32 on the direct kernel)",
-             "// (tasks, ntasks, blocks, mols, fp32, os, grid, stream)",
-             "using FockLaunch = int (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);",
-             "// (groups, ngroups, tasks, blocks, mols, fp32, os, waves, lds bytes, grid, stream)",
+             "// (tasks, ntasks, blocks, mols, fp32, os, grid, target)",
+             "using FockLaunch = int (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);",
+             "// (groups, ngroups, tasks, blocks, mols, fp32, os, waves, lds bytes, grid, target)",
              "using FockTileLaunch = void (*)(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*,"
-             " int, int, int, size_t, int, hipStream_t);",
-             "// (tasks, ntasks, blocks, mols, os, grid, global slots, stream)",
+             " int, int, int, size_t, int, LaunchTo&);",
+             "// (tasks, ntasks, blocks, mols, os, grid, global slots, target)",
              "using FockCoopLaunch = void (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*,"
-             " hipStream_t);",
+             " LaunchTo&);",
              "using SchwarzLaunch = void (*)(PairBlock, double*, double*, hipStream_t);", ""]
     for (name, La, Lb, Lc, Ld, diag) in names:
         if has_lane_kernels(La, Lb, Lc, Ld):
             lines.append("int launch_fock_%s(const Task*, int, const PairBlock*, const MolDesc*, int, int, int,"
-                         " hipStream_t);" % name)
+                         " LaunchTo&);" % name)
         if has_tile_kernels(La, Lb, Lc, Ld):
             lines.append("void launch_fock_tile_%s(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*,"
-                         " int, int, int, size_t, int, hipStream_t);" % name)
+                         " int, int, int, size_t, int, LaunchTo&);" % name)
         if (La, Lb, Lc, Ld) in COOP_CLASSES:
             lines.append("void launch_fock_coop_%s(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*,"
-                         " hipStream_t);" % name)
+                         " LaunchTo&);" % name)
         if diag:
             lines.append("void launch_schwarz_%s(PairBlock, double*, double*, hipStream_t);" % name)
     # FLOP model (FMA = 2): per surviving primitive quartet the VRR plus

@@ -333,11 +333,11 @@ def launcher_source(name, g, lane):
         extra = [
             "// per-lane kernel: grad_tile as above; no global slots",
             "void launch_grad_lane_%s(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int grid,"
-            " size_t grad_tile, double* gscratch, int fp32, hipStream_t s)" % name, "{",
+            " size_t grad_tile, double* gscratch, int fp32, LaunchTo& q)" % name, "{",
             "    (void)gscratch;",
             "    if (nt <= 0) return;",
             "    if (grid <= 0 || grid > nt) grid = nt;",
-            "    hipLaunchKernelGGL((grad_md_kernel<%sGradMd>), dim3(grid), dim3(WAVE), grad_tile, s, t, nt, b, m,"
+            "    q((grad_md_kernel<%sGradMd>), dim3(grid), dim3(WAVE), grad_tile, t, nt, b, m,"
             " (int)(grad_tile / sizeof(double)), fp32);" % name,
             "}", ""]
     return "\n".join([
@@ -347,13 +347,13 @@ def launcher_source(name, g, lane):
         "// straight to md.grad); gscratch: COOP_GLOBAL_SLICES slices when the class",
         "// keeps its slots in global memory",
         "void launch_grad_%s(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int grid,"
-        " size_t grad_tile, double* gscratch, int fp32, hipStream_t s)" % name, "{",
+        " size_t grad_tile, double* gscratch, int fp32, LaunchTo& q)" % name, "{",
         "    using D = %s;" % g,
         "    if (nt <= 0) return;",
         "    if (grid <= 0 || grid > nt) grid = nt;",
         "    if (D::GLOBAL_SLOTS && grid > COOP_GLOBAL_SLICES) grid = COOP_GLOBAL_SLICES;",
         "    const size_t lds = (D::GLOBAL_SLOTS ? 0 : D::LDS * sizeof(double)) + grad_tile;",
-        "    hipLaunchKernelGGL((grad_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch,"
+        "    q((grad_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch,"
         " (int)(grad_tile / sizeof(double)), fp32);",
         "}", ""] + extra + ["}  // namespace qf", ""])
 
@@ -376,15 +376,15 @@ def main(outdir, write):
     plus, minus, power = grad_index_tables()
     fmt = lambda rows: ",".join("{%s}" % ",".join(map(str, r)) for r in rows)
     lines = ["// Generated by quick_amd/codegen/gen_grad.py - do not edit.", "#pragma once",
-             "#include <hip/hip_runtime.h>", '#include "../qf_types.h"', "", "namespace qf {", "",
+             "#include <hip/hip_runtime.h>", '#include "../qf_launch.h"', '#include "../qf_types.h"', "", "namespace qf {", "",
              "using GradLaunch = void (*)(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*,"
-             " int, hipStream_t);", ""]
+             " int, LaunchTo&);", ""]
     for (name, La, Lb, Lc, Ld, t) in names:
         lines.append("void launch_grad_%s(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*,"
-                     " int, hipStream_t);" % name)
+                     " int, LaunchTo&);" % name)
         if has_lane_grad(La, Lb, Lc, Ld):
             lines.append("void launch_grad_lane_%s(const Task*, int, const PairBlock*, const MolDesc*, int, size_t,"
-                         " double*, int, hipStream_t);" % name)
+                         " double*, int, LaunchTo&);" % name)
     lines += ["", "// nullptr: no gradient kernel for the class (f shells)",
               "inline GradLaunch grad_launcher(int cb, int ck)", "{"]
     for (name, La, Lb, Lc, Ld, t) in names:

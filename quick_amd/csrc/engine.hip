@@ -186,17 +186,22 @@ private:
     std::vector<SideStreams*> free_;
 };
 
+bool is_capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;    // unknown: only plain launches
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // Makes sure `side` has its streams, unless s is being captured (creating
 // streams is no work for a capture; without them everything runs on s).
 bool side_ready(SideStreams*& side, int device, hipStream_t s)
 {
     if (side) return true;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    if (st != hipStreamCaptureStatusNone) return false;
+    if (is_capturing(s)) return false;
     side = SidePool::get().take(device);
     return side != nullptr;
 }
@@ -254,12 +259,11 @@ __global__ __launch_bounds__(256) void k_open(const OpenArgs a)
         for (size_t i = first; i < a.ng; i += step) a.G2[i] = 0.0;
 }
 
-int open_build(const OpenArgs& a, hipStream_t s)
+void open_build(const OpenArgs& a, qf::LaunchTo& q)
 {
     const size_t work = std::max((size_t)a.n * a.n, a.G ? a.ng : (size_t)0);
     const int grid = (int)std::min<size_t>(2048, (work + 255) / 256);
-    hipLaunchKernelGGL(k_open, dim3(grid), dim3(256), 0, s, a);
-    return hipGetLastError() == hipSuccess ? QF_OK : fail(QF_ERR_HIP, "k_open");
+    q(k_open, dim3(grid), dim3(256), 0, a);
 }
 
 __global__ void k_zero(double* __restrict__ p, size_t count)
@@ -268,38 +272,57 @@ __global__ void k_zero(double* __restrict__ p, size_t count)
         p[i] = 0.0;
 }
 
-__global__ void k_finalize(const double* __restrict__ Gt, int replicas, double* __restrict__ Gs,
-                           double* __restrict__ F, int n)
+// Closing kernel of a build.  Closed shell: G = sum over copies of (Gt +
+// Gt^T), F += G.  Open shell (Gt2): A = the sum of Gt (J and exchange of Pt), B
+// = the sum of Gt2 (exchange of Ps); Fa += A + B, Fb += A - B, Gs = A.
+struct CloseArgs {
+    const double *Gt, *Gt2;
+    double *Gs, *F, *F2;
+    int replicas, n;
+};
+
+__global__ __launch_bounds__(256) void k_close(const CloseArgs a)
 {
-    // G = sum over copies of (Gt + Gt^T); F += G
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n * n) return;
-    const int i = idx / n, j = idx % n;
-    const size_t n2 = (size_t)n * n;
-    double g = 0.0;
-    for (int r = 0; r < replicas; ++r) g += Gt[r * n2 + i * n + j] + Gt[r * n2 + j * n + i];
-    Gs[idx] = g;
-    if (F) F[idx] += g;
+    if (idx >= a.n * a.n) return;
+    const int i = idx / a.n, j = idx % a.n;
+    const size_t n2 = (size_t)a.n * a.n, ij = (size_t)i * a.n + j, ji = (size_t)j * a.n + i;
+    double g = 0.0, h = 0.0;
+    for (int r = 0; r < a.replicas; ++r) g += a.Gt[r * n2 + ij] + a.Gt[r * n2 + ji];
+    if (a.Gt2)
+        for (int r = 0; r < a.replicas; ++r) h += a.Gt2[r * n2 + ij] + a.Gt2[r * n2 + ji];
+    a.Gs[idx] = g;
+    if (a.F) a.F[idx] += g + h;
+    if (a.F2) a.F2[idx] += g - h;
 }
 
-// Open-shell pass: A = sum(Gt + Gt^T) (J and exchange of Pt), B = sum(Gt2 +
-// Gt2^T) (exchange of Ps); Fa += A + B, Fb += A - B, Gs = A.
-__global__ void k_finalize_os(const double* __restrict__ Gt, const double* __restrict__ Gt2, int replicas,
-                              double* __restrict__ Gs, double* __restrict__ Fa, double* __restrict__ Fb, int n)
+void close_build(const CloseArgs& a, qf::LaunchTo& q)
 {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= n * n) return;
-    const int i = idx / n, j = idx % n;
-    const size_t n2 = (size_t)n * n;
-    double a = 0.0, b = 0.0;
-    for (int r = 0; r < replicas; ++r) {
-        a += Gt[r * n2 + i * n + j] + Gt[r * n2 + j * n + i];
-        b += Gt2[r * n2 + i * n + j] + Gt2[r * n2 + j * n + i];
-    }
-    Gs[idx] = a;
-    Fa[idx] += a + b;
-    Fb[idx] += a - b;
+    q(k_close, dim3((a.n * a.n + 255) / 256), dim3(256), 0, a);
 }
+
+// The launches of one kind of build as an instantiated graph.
+struct Replay {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    hipGraphNode_t first = nullptr, last = nullptr;   // the opening and the closing kernel
+    OpenArgs open{};        // arguments that `first` and `last` hold
+    CloseArgs close{};
+    int uses = 0;           // builds of this kind since the last prepare
+    bool failed = false;    // could not be built: the launches stay eager
+    void drop()
+    {
+        if (exec) {
+            (void)hipDeviceSynchronize();   // a replay may still run
+            (void)hipGraphExecDestroy(exec);
+        }
+        if (graph) (void)hipGraphDestroy(graph);
+        exec = nullptr;
+        graph = nullptr;
+        uses = 0;
+        failed = false;
+    }
+};
 
 // Counts, per quartet class, the quartets and primitive quartets that pass
 // the screens (same tests as the Fock kernel); used for the FLOP model.
@@ -408,7 +431,13 @@ struct qf_engine {
     };
     std::vector<Launch> launches;
     std::vector<std::pair<int, int>> order;   // issue order: (launch index, stream 0..kSide)
-    SideStreams* side = nullptr;              // taken at the first build
+    double fork_gain = 0.0;                   // seconds the forked order saves (estimate)
+    SideStreams* side = nullptr;              // taken at the first forked build
+    Replay replay[3];                         // closed shell, open shell, gradient
+    void drop_replays()
+    {
+        for (auto& r : replay) r.drop();
+    }
     bool prepared = false;
     unsigned long long generation = 0;   // bumped by every prepare(): batches check it
     bool built = false;                  // a build has run since the last prepare()
@@ -443,6 +472,7 @@ struct qf_engine {
     std::vector<int> ev_launch;        // launch index of each recorded (start, stop) pair
     ~qf_engine()
     {
+        drop_replays();
         for (hipEvent_t ev : ev_pool) (void)hipEventDestroy(ev);
         SidePool::get().give(side);
     }
@@ -733,7 +763,7 @@ size_t place_slots(std::vector<qf_engine::Launch>& launches)
 // of the per-lane kernels, and at the 1.2 and 6 TFLOP/s that whole launches
 // reach.
 std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launch>& launches,
-                                              const std::vector<qf::Task>& tasks)
+                                              const std::vector<qf::Task>& tasks, double* gain = nullptr)
 {
     const int n = (int)launches.size();
     std::vector<double> t(n);
@@ -762,6 +792,7 @@ std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launc
         load[to] += t[l];
         out.push_back({l, to});
     }
+    if (gain) *gain = std::accumulate(t.begin(), t.end(), 0.0) - *std::max_element(load, load + kSide + 1);
     return out;
 }
 
@@ -1175,7 +1206,8 @@ int prepare(qf_engine* e)
     if (rc) return rc;
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
-    e->order = stream_order(e->launches, e->tasks);
+    e->order = stream_order(e->launches, e->tasks, &e->fork_gain);
+    e->drop_replays();
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
     const size_t gdoubles = place_slots(e->launches);
@@ -1261,7 +1293,7 @@ struct GBufs {
     int replicas;
     double* Gs;
     bool timing;   // per-launch HIP events (never in the no-alloc path: it creates events)
-    bool fork;     // spread the class launches over side streams (not in the no-alloc path)
+    bool fork;     // side streams and replay (not in the no-alloc path: they allocate)
     double* Gt2 = nullptr;   // open-shell pass: accumulators of the second exchange density
 };
 
@@ -1299,11 +1331,112 @@ int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<i
     return rc;
 }
 
+// Records the start event of a timed launch; *stop is the event that ends it.
+int timing_begin(qf_engine* e, int li, hipStream_t s, hipEvent_t* stop)
+{
+    while (e->ev_pool.size() < e->ev_used + 2) {
+        hipEvent_t ev;
+        QF_HIP(hipEventCreate(&ev));
+        e->ev_pool.push_back(ev);
+    }
+    QF_HIP(hipEventRecord(e->ev_pool[e->ev_used], s));
+    *stop = e->ev_pool[e->ev_used + 1];
+    e->ev_used += 2;
+    e->ev_launch.push_back(li);
+    return QF_OK;
+}
+
+// Issues one kind of build (0 closed shell, 1 open shell, 2 gradient): the
+// opening kernel, the class launches by issue(launch index, target) and the
+// closing kernel (none where close is null).  The first build since a prepare
+// is issued launch by launch, the classes forked over the side streams where
+// that saves more than its ten event calls cost (about 60 us).  From the second
+// on it is replayed from a graph of the same four chains; of its arguments
+// only those of the opening and closing kernels change (densities and results
+// reach the class kernels through the descriptor that the opening kernel
+// writes).  What bounds a small build is host time and the waits between
+// streams.  Device builds, us, one stream / forked launches / replay: water
+// STO-3G 73 / 94 / 72, water 6-31G* 314 / 217 / 132, glycine 6-31G** 1497 / 1018 /
+// 670, ethane def2-TZVP 4482 / 2498 / 1568.  A build under capture is issued
+// launch by launch.
+template <class F>
+int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, const CloseArgs* close, F&& issue)
+{
+    Replay& r = e->replay[kind];
+    const bool captured = is_capturing(s);
+    if (!captured && !r.exec && !r.failed && !e->order.empty() && ++r.uses > 1) {
+        hipGraphNode_t last[kSide + 1] = {};
+        bool ok = hipGraphCreate(&r.graph, 0) == hipSuccess;
+        if (ok) {
+            qf::LaunchTo to(r.graph, nullptr, 0);
+            open_build(open, to);
+            r.first = to.node;
+            ok = to.err == hipSuccess;
+        }
+        for (const auto& o : e->order) {
+            if (!ok) break;
+            qf::LaunchTo to(r.graph, last[o.second] ? &last[o.second] : &r.first, 1);
+            const int rc = issue(o.first, to);
+            if (rc) {
+                r.drop();
+                return rc;
+            }
+            last[o.second] = to.node;
+            ok = to.err == hipSuccess;
+        }
+        if (ok && close) {
+            hipGraphNode_t ends[kSide + 1];
+            int n = 0;
+            for (auto x : last)
+                if (x) ends[n++] = x;
+            qf::LaunchTo to(r.graph, ends, n);
+            close_build(*close, to);
+            r.last = to.node;
+            ok = to.err == hipSuccess;
+        }
+        ok = ok && hipGraphInstantiate(&r.exec, r.graph, nullptr, nullptr, 0) == hipSuccess;
+        if (ok) {
+            r.open = open;
+            if (close) r.close = *close;
+        } else {
+            (void)hipGetLastError();
+            r.drop();
+            r.failed = true;
+        }
+    }
+    if (!captured && r.exec) {
+        if (std::memcmp(&r.open, &open, sizeof(open))) {
+            qf::LaunchTo to(r.exec, r.first);
+            open_build(open, to);
+            QF_HIP(to.err);
+            r.open = open;
+        }
+        if (close && std::memcmp(&r.close, close, sizeof(*close))) {
+            qf::LaunchTo to(r.exec, r.last);
+            close_build(*close, to);
+            QF_HIP(to.err);
+            r.close = *close;
+        }
+        QF_HIP(hipGraphLaunch(r.exec, s));
+        return QF_OK;
+    }
+    qf::LaunchTo to(s);
+    open_build(open, to);
+    const bool forked = e->order.size() > 1 && (e->side || e->fork_gain > 8e-5) && side_ready(e->side, e->device, s);
+    const int rc = issue_forked(forked ? e->side : nullptr, s, e->order, [&](int li, hipStream_t q) {
+        qf::LaunchTo x(q);
+        return issue(li, x);
+    });
+    if (rc) return rc;
+    if (close) close_build(*close, to);
+    return QF_OK;
+}
+
 // cm_out: where the opening kernel puts the density screen matrix (null: dcm
 // is the caller's).  dPb != nullptr: the open-shell pass.  Every integral is
 // digested with dP (Coulomb and exchange, into Gt) and with the spin density
 // dP2 (exchange only, into gb.Gt2);
-// then dF += A + B and dF2 += A - B (k_finalize_os).  A class with os_split
+// then dF += A + B and dF2 += A - B (k_close).  A class with os_split
 // runs as two closed-shell launches instead of the fused one: dP into Gt,
 // then dP2 with a zero Coulomb density (e->d_zero) into Gt2 (descriptor slot
 // 1).
@@ -1357,10 +1490,16 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     oa.f1 = e->d_f1.p;
     oa.n = n;
     oa.nshell = ns;
-    const int orc = open_build(oa, s);
-    if (orc) return orc;
+    CloseArgs ca{};
+    ca.Gt = gb.Gt;
+    ca.Gt2 = os ? gb.Gt2 : nullptr;
+    ca.Gs = gb.Gs;
+    ca.F = dF;
+    ca.F2 = os ? dF2 : nullptr;
+    ca.replicas = gb.replicas;
+    ca.n = n;
     // one class launch with descriptor m on stream q; los: its open-shell form
-    auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, hipStream_t q) -> int {
+    auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, qf::LaunchTo& q) -> int {
         const bool alt = los && L.alt_count > 0;
         if (L.tile == 2 || alt) {
             qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
@@ -1381,39 +1520,28 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         }
         return QF_OK;
     };
-    auto class_launch = [&](const qf_engine::Launch& L, hipStream_t q) -> int {
+    auto class_launch = [&](const qf_engine::Launch& L, qf::LaunchTo& q) -> int {
         if (!(os && L.os_split)) return launch(L, dmol, os, q);
         const int rc = launch(L, dmol, 0, q);
         return rc ? rc : launch(L, dmol_x, 0, q);
     };
-    if (gb.timing) {
-        // timed launches run one after another on s
-        for (size_t li = 0; li < e->launches.size(); ++li) {
-            while (e->ev_pool.size() < e->ev_used + 2) {
-                hipEvent_t ev;
-                QF_HIP(hipEventCreate(&ev));
-                e->ev_pool.push_back(ev);
-            }
-            hipEvent_t ea = e->ev_pool[e->ev_used], eb = e->ev_pool[e->ev_used + 1];
-            e->ev_used += 2;
-            e->ev_launch.push_back((int)li);
-            QF_HIP(hipEventRecord(ea, s));
-            const int rc = class_launch(e->launches[li], s);
-            if (rc) return rc;
-            QF_HIP(hipEventRecord(eb, s));
-        }
-    } else {
-        const bool forked = gb.fork && e->order.size() > 1 && side_ready(e->side, e->device, s);
-        const int rc = issue_forked(forked ? e->side : nullptr, s, e->order,
-                                    [&](int li, hipStream_t q) { return class_launch(e->launches[li], q); });
+    if (gb.fork && !gb.timing) {
+        const int rc = issue_build(e, os, s, oa, &ca,
+                                   [&](int li, qf::LaunchTo& q) { return class_launch(e->launches[li], q); });
         if (rc) return rc;
+    } else {
+        // one after another on s, timed ones between events
+        qf::LaunchTo to(s);
+        open_build(oa, to);
+        for (size_t li = 0; li < e->launches.size(); ++li) {
+            hipEvent_t eb = nullptr;
+            if (gb.timing && timing_begin(e, (int)li, s, &eb)) return QF_ERR_HIP;
+            const int rc = class_launch(e->launches[li], to);
+            if (rc) return rc;
+            if (eb) QF_HIP(hipEventRecord(eb, s));
+        }
+        close_build(ca, to);
     }
-    if (os)
-        hipLaunchKernelGGL(k_finalize_os, dim3((n * n + 255) / 256), dim3(256), 0, s, gb.Gt, gb.Gt2, gb.replicas,
-                           gb.Gs, dF, dF2, n);
-    else
-        hipLaunchKernelGGL(k_finalize, dim3((n * n + 255) / 256), dim3(256), 0, s, gb.Gt, gb.replicas, gb.Gs,
-                           dF, n);
     QF_HIP(hipGetLastError());
     return QF_OK;
 }
@@ -1668,7 +1796,10 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
             gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) *
                         std::min(std::max(L.count, L.alt_count), qf::COOP_GLOBAL_SLICES);
     }
-    if (gdoubles && e->d_gscratch.n < gdoubles) QF_HIP(e->d_gscratch.resize(gdoubles));
+    if (gdoubles && e->d_gscratch.n < gdoubles) {
+        e->replay[2].drop();   // it holds the old buffer
+        QF_HIP(e->d_gscratch.resize(gdoubles));
+    }
     qf::MolDesc md{};
     md.P = dP;
     md.PJ = dP;
@@ -1694,10 +1825,8 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     oa.f1 = e->d_f1.p;
     oa.n = e->nbasis;
     oa.nshell = e->nshell;
-    const int orc = open_build(oa, s);
-    if (orc) return orc;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
-    auto launch = [&](int li, hipStream_t q) -> int {
+    auto launch = [&](int li, qf::LaunchTo& q) -> int {
         const auto& L = e->launches[li];
         const qf::GradLaunch lane = lane_kernel(L);
         const size_t slots = lane ? 0 : (size_t)qf::grad_lds_doubles(L.cb, L.ck) * sizeof(double);
@@ -1712,24 +1841,18 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
                                                       tile, e->d_gscratch.p + gslot[li], L.fp32, q);
         return QF_OK;
     };
-    if (e->timing) {
+    if (!e->timing) {
+        const int rc = issue_build(e, 2, s, oa, nullptr, launch);
+        if (rc) return rc;
+    } else {
+        qf::LaunchTo to(s);
+        open_build(oa, to);
         for (size_t li = 0; li < e->launches.size(); ++li) {
-            while (e->ev_pool.size() < e->ev_used + 2) {
-                hipEvent_t ev;
-                QF_HIP(hipEventCreate(&ev));
-                e->ev_pool.push_back(ev);
-            }
-            hipEvent_t ea = e->ev_pool[e->ev_used], eb = e->ev_pool[e->ev_used + 1];
-            e->ev_used += 2;
-            e->ev_launch.push_back((int)li);
-            QF_HIP(hipEventRecord(ea, s));
-            launch((int)li, s);
+            hipEvent_t eb = nullptr;
+            if (timing_begin(e, (int)li, s, &eb)) return QF_ERR_HIP;
+            launch((int)li, to);
             QF_HIP(hipEventRecord(eb, s));
         }
-    } else {
-        const bool forked = e->order.size() > 1 && side_ready(e->side, e->device, s);
-        const int rc = issue_forked(forked ? e->side : nullptr, s, e->order, launch);
-        if (rc) return rc;
     }
     QF_HIP(hipGetLastError());
     return QF_OK;
@@ -1749,6 +1872,7 @@ int qf_set_grad_kernel(qf_engine* e, int lane)
 {
     if (!e) return fail(QF_ERR_ARG, "engine is NULL");
     e->grad_lane = lane != 0;
+    e->replay[2].drop();
     return QF_OK;
 }
 
@@ -1758,6 +1882,7 @@ int qf_set_grad_class(qf_engine* e, int cb, int ck, int mode)
     if (cb < 0 || cb >= kNPC || ck < 0 || ck > cb) return fail(QF_ERR_ARG, "class index out of range");
     if (mode < -1 || mode > 1) return fail(QF_ERR_ARG, "mode must be -1, 0 (wave-per-quartet) or 1 (per-lane)");
     e->ctune[cb][ck].grad = mode;
+    e->replay[2].drop();
     return QF_OK;
 }
 
@@ -2057,6 +2182,7 @@ int qf_set_persistent(qf_engine* e, int max_workgroups)
 {
     if (!e || max_workgroups < 0) return fail(QF_ERR_ARG, "max_workgroups must be >= 0");
     e->persist = max_workgroups;
+    e->drop_replays();
     return QF_OK;
 }
 
@@ -2201,7 +2327,8 @@ int batch_issue(qf_batch* b, hipStream_t s)
     const int nm = (int)b->mols.size();
     hipLaunchKernelGGL(k_cutmat_batch, dim3((b->max_ns2 + 255) / 256, nm), dim3(256), 0, s, b->d_bm.p);
     hipLaunchKernelGGL(k_zero, dim3(1024), dim3(256), 0, s, b->d_Gt.p, b->gt_total);
-    auto class_launch = [&](const qf_engine::Launch& L, hipStream_t q) -> int {
+    auto class_launch = [&](const qf_engine::Launch& L, hipStream_t stream) -> int {
+        qf::LaunchTo q(stream);
         if (L.tile == 2) {
             qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
             if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");

@@ -6,23 +6,23 @@ namespace qf {
 // grad_tile: 3 natom doubles of LDS for the workgroup's gradient (0: atomics
 // straight to md.grad); gscratch: COOP_GLOBAL_SLICES slices when the class
 // keeps its slots in global memory
-void launch_grad_C1110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int grid, size_t grad_tile, double* gscratch, int fp32, hipStream_t s)
+void launch_grad_C1110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int grid, size_t grad_tile, double* gscratch, int fp32, LaunchTo& q)
 {
     using D = C1110Grad;
     if (nt <= 0) return;
     if (grid <= 0 || grid > nt) grid = nt;
     if (D::GLOBAL_SLOTS && grid > COOP_GLOBAL_SLICES) grid = COOP_GLOBAL_SLICES;
     const size_t lds = (D::GLOBAL_SLOTS ? 0 : D::LDS * sizeof(double)) + grad_tile;
-    hipLaunchKernelGGL((grad_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch, (int)(grad_tile / sizeof(double)), fp32);
+    q((grad_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch, (int)(grad_tile / sizeof(double)), fp32);
 }
 
 // per-lane kernel: grad_tile as above; no global slots
-void launch_grad_lane_C1110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int grid, size_t grad_tile, double* gscratch, int fp32, hipStream_t s)
+void launch_grad_lane_C1110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int grid, size_t grad_tile, double* gscratch, int fp32, LaunchTo& q)
 {
     (void)gscratch;
     if (nt <= 0) return;
     if (grid <= 0 || grid > nt) grid = nt;
-    hipLaunchKernelGGL((grad_md_kernel<C1110GradMd>), dim3(grid), dim3(WAVE), grad_tile, s, t, nt, b, m, (int)(grad_tile / sizeof(double)), fp32);
+    q((grad_md_kernel<C1110GradMd>), dim3(grid), dim3(WAVE), grad_tile, t, nt, b, m, (int)(grad_tile / sizeof(double)), fp32);
 }
 
 }  // namespace qf

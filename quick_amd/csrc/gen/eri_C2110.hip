@@ -7,22 +7,22 @@ namespace qf {
 // kernel is not built (it gave wrong Fock matrices on gfx950, cause not
 // found): a request for it is refused with a nonzero return.
 // os: 1 = the fused open-shell pass (second exchange density)
-int launch_fock_C2110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int fp32, int os, int grid, hipStream_t s)
+int launch_fock_C2110(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int fp32, int os, int grid, LaunchTo& q)
 {
     if (fp32) return 1;
     if (nt <= 0) return 0;
     if (grid <= 0 || grid > nt) grid = nt;
     if (os)
-        hipLaunchKernelGGL((fock_kernel<C2110, double, true>), dim3(grid), dim3(WAVE), 0, s, t, nt, b, m);
+        q((fock_kernel<C2110, double, true>), dim3(grid), dim3(WAVE), 0, t, nt, b, m);
     else
-        hipLaunchKernelGGL((fock_kernel<C2110, double>), dim3(grid), dim3(WAVE), 0, s, t, nt, b, m);
+        q((fock_kernel<C2110, double>), dim3(grid), dim3(WAVE), 0, t, nt, b, m);
     return 0;
 }
 
 // os & 3: 0 closed shell, 1 open shell with a second LDS tile, 2 open
 // shell with the second exchange terms straight to G2; os & 4: the lean
 // open-shell form (FP64; FP32 launches take the register form)
-void launch_fock_tile_C2110(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)
+void launch_fock_tile_C2110(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, LaunchTo& q)
 {
     if (ng <= 0) return;
     if (grid <= 0 || grid > ng) grid = ng;
@@ -30,15 +30,15 @@ void launch_fock_tile_C2110(const TileGroup* g, int ng, const Task* t, const Pai
     os &= 3;
     const int k2 = os == 1;
     if (fp32 && os)
-        hipLaunchKernelGGL((fock_tile_kernel<C2110, float, true>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, k2);
+        q((fock_tile_kernel<C2110, float, true>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m, k2);
     else if (fp32)
-        hipLaunchKernelGGL((fock_tile_kernel<C2110, float>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, 0);
+        q((fock_tile_kernel<C2110, float>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m, 0);
     else if (os && lean)
-        hipLaunchKernelGGL((fock_tile_kernel<C2110, double, true, true>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, k2);
+        q((fock_tile_kernel<C2110, double, true, true>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m, k2);
     else if (os)
-        hipLaunchKernelGGL((fock_tile_kernel<C2110, double, true>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, k2);
+        q((fock_tile_kernel<C2110, double, true>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m, k2);
     else
-        hipLaunchKernelGGL((fock_tile_kernel<C2110, double>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m, 0);
+        q((fock_tile_kernel<C2110, double>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m, 0);
 }
 
 }  // namespace qf

@@ -5,18 +5,18 @@
 namespace qf {
 
 // closed shell, FP64 only (an open-shell build runs the class in two passes)
-void launch_fock_tile_C2121(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, hipStream_t s)
+void launch_fock_tile_C2121(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, LaunchTo& q)
 {
     if (ng <= 0) return;
     if (grid <= 0 || grid > ng) grid = ng;
     (void)fp32;
     (void)os;
-    hipLaunchKernelGGL((fock_md_kernel<C2121Md>), dim3(grid), dim3(waves * WAVE), lds, s, g, ng, t, b, m);
+    q((fock_md_kernel<C2121Md>), dim3(grid), dim3(waves * WAVE), lds, g, ng, t, b, m);
 }
 
 // gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its
 // slots in global memory (the grid is then capped to that many workgroups)
-void launch_fock_coop_C2121(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int os, int grid, double* gscratch, hipStream_t s)
+void launch_fock_coop_C2121(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int os, int grid, double* gscratch, LaunchTo& q)
 {
     using D = C2121Coop;
     if (nt <= 0) return;
@@ -24,9 +24,9 @@ void launch_fock_coop_C2121(const Task* t, int nt, const PairBlock* b, const Mol
     if (D::GLOBAL_SLOTS && grid > COOP_GLOBAL_SLICES) grid = COOP_GLOBAL_SLICES;
     const size_t lds = D::GLOBAL_SLOTS ? 0 : D::LDS * sizeof(double);
     if (os)
-        hipLaunchKernelGGL((fock_coop_kernel<D, true>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch);
+        q((fock_coop_kernel<D, true>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch);
     else
-        hipLaunchKernelGGL((fock_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch);
+        q((fock_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch);
 }
 
 void launch_schwarz_C2121(PairBlock blk, double* out, double* gscratch, hipStream_t s)

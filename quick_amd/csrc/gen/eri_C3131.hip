@@ -5,7 +5,7 @@ namespace qf {
 
 // gscratch: COOP_GLOBAL_SLICES slices of LDS doubles when the class keeps its
 // slots in global memory (the grid is then capped to that many workgroups)
-void launch_fock_coop_C3131(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int os, int grid, double* gscratch, hipStream_t s)
+void launch_fock_coop_C3131(const Task* t, int nt, const PairBlock* b, const MolDesc* m, int os, int grid, double* gscratch, LaunchTo& q)
 {
     using D = C3131Coop;
     if (nt <= 0) return;
@@ -13,9 +13,9 @@ void launch_fock_coop_C3131(const Task* t, int nt, const PairBlock* b, const Mol
     if (D::GLOBAL_SLOTS && grid > COOP_GLOBAL_SLICES) grid = COOP_GLOBAL_SLICES;
     const size_t lds = D::GLOBAL_SLOTS ? 0 : D::LDS * sizeof(double);
     if (os)
-        hipLaunchKernelGGL((fock_coop_kernel<D, true>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch);
+        q((fock_coop_kernel<D, true>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch);
     else
-        hipLaunchKernelGGL((fock_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, s, t, nt, b, m, gscratch);
+        q((fock_coop_kernel<D>), dim3(grid), dim3(D::NT), lds, t, nt, b, m, gscratch);
 }
 
 void launch_schwarz_C3131(PairBlock blk, double* out, double* gscratch, hipStream_t s)

@@ -1,49 +1,50 @@
 // Generated by quick_amd/codegen/gen_grad.py - do not edit.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "../qf_launch.h"
 #include "../qf_types.h"
 
 namespace qf {
 
-using GradLaunch = void (*)(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
+using GradLaunch = void (*)(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
 
-void launch_grad_C0000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C0000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C1000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C1000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C1010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C1010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C1100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C1100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C1110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C1110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2121(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_lane_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2211(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2220(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2221(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
-void launch_grad_C2222(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, hipStream_t);
+void launch_grad_C0000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C0000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C1000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C1000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C1010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C1010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C1100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C1100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C1110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C1110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2000(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2010(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2100(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2110(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2121(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_lane_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2211(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2220(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2221(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
+void launch_grad_C2222(const Task*, int, const PairBlock*, const MolDesc*, int, size_t, double*, int, LaunchTo&);
 
 // nullptr: no gradient kernel for the class (f shells)
 inline GradLaunch grad_launcher(int cb, int ck)

@@ -1,123 +1,124 @@
 // Generated by quick_amd/codegen/gen_eri.py - do not edit.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "../qf_launch.h"
 #include "../qf_types.h"
 
 namespace qf {
 
 // returns nonzero when the launch is refused (FP32 on the direct kernel)
-// (tasks, ntasks, blocks, mols, fp32, os, grid, stream)
-using FockLaunch = int (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-// (groups, ngroups, tasks, blocks, mols, fp32, os, waves, lds bytes, grid, stream)
-using FockTileLaunch = void (*)(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-// (tasks, ntasks, blocks, mols, os, grid, global slots, stream)
-using FockCoopLaunch = void (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+// (tasks, ntasks, blocks, mols, fp32, os, grid, target)
+using FockLaunch = int (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+// (groups, ngroups, tasks, blocks, mols, fp32, os, waves, lds bytes, grid, target)
+using FockTileLaunch = void (*)(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+// (tasks, ntasks, blocks, mols, os, grid, global slots, target)
+using FockCoopLaunch = void (*)(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 using SchwarzLaunch = void (*)(PairBlock, double*, double*, hipStream_t);
 
-int launch_fock_C0000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C0000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
+int launch_fock_C0000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C0000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
 void launch_schwarz_C0000(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C1000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C1000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C1010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C1010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
+int launch_fock_C1000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C1000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C1010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C1010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
 void launch_schwarz_C1010(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C1100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C1100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C1110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C1110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C1111(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C1100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C1100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C1110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C1110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C1111(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C1111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C1111(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C2000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C2010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2011(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2020(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C2000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C2010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2011(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2011(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2020(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2020(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C2020(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C2100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C2110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-int launch_fock_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2111(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2120(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_tile_C2121(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2121(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C2100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C2110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+int launch_fock_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2111(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2120(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2120(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_tile_C2121(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2121(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C2121(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2200(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C2210(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_tile_C2211(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2211(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_tile_C2220(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C2220(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C2221(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C2222(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2200(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2200(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C2210(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2210(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_tile_C2211(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2211(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_tile_C2220(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C2220(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C2221(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C2222(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C2222(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C3000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3000(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C3010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3010(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C3011(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3011(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3011(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C3020(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3020(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3020(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3021(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3022(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3030(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3000(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3000(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3000(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C3010(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3010(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3010(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C3011(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3011(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3011(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C3020(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3020(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3020(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3021(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3022(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3030(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C3030(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C3100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3100(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-int launch_fock_C3110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3110(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3120(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3121(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3122(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3130(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3131(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3100(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3100(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3100(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+int launch_fock_C3110(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3110(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3110(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3111(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3120(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3121(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3122(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3130(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3131(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C3131(PairBlock, double*, double*, hipStream_t);
-int launch_fock_C3200(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, hipStream_t);
-void launch_fock_tile_C3200(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, hipStream_t);
-void launch_fock_coop_C3200(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3210(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3211(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3220(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3221(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3222(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3230(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3231(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3232(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+int launch_fock_C3200(const Task*, int, const PairBlock*, const MolDesc*, int, int, int, LaunchTo&);
+void launch_fock_tile_C3200(const TileGroup*, int, const Task*, const PairBlock*, const MolDesc*, int, int, int, size_t, int, LaunchTo&);
+void launch_fock_coop_C3200(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3210(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3211(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3220(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3221(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3222(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3230(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3231(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3232(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C3232(PairBlock, double*, double*, hipStream_t);
-void launch_fock_coop_C3300(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3310(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3311(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3320(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3321(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3322(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3330(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3331(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3332(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
-void launch_fock_coop_C3333(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, hipStream_t);
+void launch_fock_coop_C3300(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3310(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3311(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3320(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3321(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3322(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3330(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3331(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3332(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fock_coop_C3333(const Task*, int, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
 void launch_schwarz_C3333(PairBlock, double*, double*, hipStream_t);
 
 // Algorithmic FLOPs of nq quartets with np primitive quartets in class (cb|ck).

@@ -8,6 +8,7 @@
 #include <cmath>
 
 #include "gen/boys_grid.h"
+#include "qf_launch.h"
 #include "qf_types.h"
 
 namespace qf {

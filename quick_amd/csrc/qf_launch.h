@@ -1,0 +1,46 @@
+// Where a launcher puts its kernel: on a stream, as a node into a HIP graph, or
+// as new arguments into a node of an instantiated one.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace qf {
+
+struct LaunchTo {
+    hipStream_t stream = nullptr;
+    hipGraph_t graph = nullptr;             // building: the new node follows deps and becomes `node`
+    const hipGraphNode_t* deps = nullptr;
+    int ndeps = 0;
+    hipGraphExec_t exec = nullptr;          // updating: `node` of this graph takes the new arguments
+    hipGraphNode_t node = nullptr;
+    hipError_t err = hipSuccess;            // of building and updating
+
+    LaunchTo(hipStream_t s) : stream(s) {}
+    LaunchTo(hipGraph_t g, const hipGraphNode_t* after, int n) : graph(g), deps(after), ndeps(n) {}
+    LaunchTo(hipGraphExec_t x, hipGraphNode_t n) : exec(x), node(n) {}
+
+    template <class... Params, class... Args>
+    void operator()(void (*kernel)(Params...), dim3 grid, dim3 block, size_t lds, const Args&... args)
+    {
+        if (!graph && !exec)
+            hipLaunchKernelGGL(kernel, grid, block, (unsigned)lds, stream, Params(args)...);
+        else
+            node_of(kernel, grid, block, lds, Params(args)...);
+    }
+
+private:
+    template <class... Params>
+    void node_of(void (*kernel)(Params...), dim3 grid, dim3 block, size_t lds, Params... params)
+    {
+        void* list[] = {(void*)&params...};
+        hipKernelNodeParams p{};
+        p.func = (void*)kernel;
+        p.gridDim = grid;
+        p.blockDim = block;
+        p.sharedMemBytes = (unsigned)lds;
+        p.kernelParams = list;
+        err = exec ? hipGraphExecKernelNodeSetParams(exec, node, &p)
+                   : hipGraphAddKernelNode(&node, graph, ndeps ? deps : nullptr, ndeps, &p);
+    }
+};
+
+}  // namespace qf

@@ -75,6 +75,73 @@ def test_forked_build_in_a_captured_graph(warm):
         close(other, G)
 
 
+def test_replayed_builds_follow_every_change():
+    """From the second build on the class launches are replayed: other buffers,
+    a changed cutoff, grid cap or kernel choice and builds of another kind
+    between them must all show in the result."""
+    announce("streams replay")
+    from quick_amd.engine import FockEngine
+    eng, P, G = setup("gly1")
+    s = torch.cuda.current_stream().cuda_stream
+
+    def closed(density, want):
+        F = torch.zeros_like(density)
+        eng.fock2e_device(density.data_ptr(), F.data_ptr(), s)
+        torch.cuda.synchronize()
+        close(F, want)
+
+    Q = P * torch.linspace(0.5, 1.5, P.shape[0], dtype=P.dtype, device="cuda")
+    Q = 0.5 * (Q + Q.T).contiguous()
+    other = FockEngine(eng.basis, cutoff=eng.cutoff)
+    other.set_timing(True)
+    GQ = other.fock2e(Q.cpu().numpy())
+    g = other.eri_grad(P.cpu().numpy())
+    Ga, Gb = other.fock2e_os(P.cpu().numpy() / 2, Q.cpu().numpy() / 2)
+    for _ in range(3):
+        closed(P, G)
+        closed(Q, GQ)
+        assert np.abs(eng.eri_grad(P.cpu().numpy()) - g).max() <= 1e-11 * np.abs(g).max()
+        a, b = eng.fock2e_os(P.cpu().numpy() / 2, Q.cpu().numpy() / 2)
+        close(torch.from_numpy(a), Ga)
+        close(torch.from_numpy(b), Gb)
+    eng.set_persistent(64)
+    eng.set_grad_kernel(lane=False)
+    closed(P, G)
+    for _ in range(3):
+        assert np.abs(eng.eri_grad(P.cpu().numpy()) - g).max() <= 1e-11 * np.abs(g).max()
+    eng.set_cutoffs(1e-6)
+    other.set_cutoffs(1e-6)
+    loose = other.fock2e(P.cpu().numpy())
+    assert np.abs(loose - G).max() > 1e-9     # the cutoff shows
+    for _ in range(3):
+        closed(P, loose)
+    eng.close()                               # a replay may still be in flight in a user's program
+    other.close()
+
+
+@pytest.mark.parametrize("name", ["water", "gly1"])
+def test_builds_in_flight_keep_their_own_buffers(name):
+    """Many builds queued without a wait, each with its own density and Fock
+    matrix: a replay's arguments are changed while earlier ones still run."""
+    announce("streams in flight %s" % name)
+    eng, P, G = setup(name)
+    s = torch.cuda.current_stream().cuda_stream
+    scale = [1.0 + 0.25 * k for k in range(24)]
+    Ps = [P * x for x in scale]
+    Fs = [torch.zeros_like(P) for _ in scale]
+    gs = [torch.zeros(eng.basis.mol.natom, 3, dtype=P.dtype, device="cuda") for _ in scale]
+    torch.cuda.synchronize()
+    for k in range(len(scale)):
+        eng.fock2e_device(Ps[k].data_ptr(), Fs[k].data_ptr(), s)
+        eng.eri_grad_device(Ps[k].data_ptr(), gs[k].data_ptr(), s)
+    torch.cuda.synchronize()
+    one = gs[0].cpu().numpy()
+    for x, F, g in zip(scale, Fs, gs):
+        # G is linear in P up to the quartets that the density screen drops or keeps
+        assert np.abs(F.cpu().numpy() - x * G).max() <= 1e-8
+        assert np.abs(g.cpu().numpy() - x * x * one).max() <= 1e-7
+
+
 def test_forked_builds_of_several_threads():
     announce("streams threads")
     sets = [setup(n) for n in ("water", "water3", "alkane2")]
