@@ -33,7 +33,8 @@ FLAGS = [
 
 
 def sources():
-    srcs = sorted(glob.glob(os.path.join(CSRC, "gen", "eri_*.hip")))
+    srcs = sorted(glob.glob(os.path.join(CSRC, "gen", "fuse_*.hip")))   # the longest to compile first
+    srcs += sorted(glob.glob(os.path.join(CSRC, "gen", "eri_*.hip")))
     srcs += sorted(glob.glob(os.path.join(CSRC, "gen", "egrad_*.hip")))
     srcs += [os.path.join(CSRC, "engine.hip"), os.path.join(CSRC, "oei.hip"),
              os.path.join(CSRC, "quick_compat.cpp")]
@@ -48,6 +49,9 @@ def _deps(src):
         deps.append(os.path.join(CSRC, "gen", base[4:-4] + ".h"))
         deps.append(os.path.join(CSRC, "gen", "coop_" + base[4:-4] + ".h"))
         deps += [os.path.join(CSRC, "qf_md.h"), os.path.join(CSRC, "gen", "md_" + base[4:-4] + ".h")]
+    if base.startswith("fuse_"):
+        deps += [os.path.join(CSRC, "qf_fuse.h")] + glob.glob(os.path.join(CSRC, "gen", "C*.h"))
+        deps += glob.glob(os.path.join(CSRC, "gen", "coop_*.h"))
     if base.startswith("egrad_"):
         deps += [os.path.join(CSRC, "qf_grad.h"), os.path.join(CSRC, "gen", "grad_maps.h"),
                  os.path.join(CSRC, "gen", "grad_" + base[6:-4] + ".h")]

@@ -739,6 +739,61 @@ def launcher_source(name, diag, coop=False, lane=True, fp32=True, md=False):
     return "\n".join(out)
 
 
+# Launches that hold several classes (qf_fuse.h): classes of one kernel need
+# about the same registers.  Tile kernels: waves per SIMD of the budget, and the
+# classes; wave-per-quartet kernels (all within 128 registers): the classes by
+# the slots they need in LDS, those over 64 KiB in global memory apart.
+def fuse_buckets():
+    out = []
+    for w in (3, 2, 1):
+        cls = [c for c in quartet_classes() if has_lane_kernels(*c) and c not in MD_CLASSES and
+               min(3, MIN_WAVES_OVERRIDE.get(c, min_waves(*_sizes(*c)))) == w]
+        out.append(dict(name="tile%d" % w, waves=w, classes=cls, coop=False, glob=False))
+    tab = {c: coop_tables(*c) for c in COOP_CLASSES}
+    small = [c for c in quartet_classes() if c in tab and tab[c]["total"] <= 1300]
+    large = [c for c in quartet_classes() if c in tab and tab[c]["total"] > 1300 and not tab[c]["glob"]]
+    glob = [c for c in quartet_classes() if c in tab and tab[c]["glob"]]
+    for name, cls, g in (("coop_small", small, False), ("coop_large", large, False), ("coop_global", glob, True)):
+        out.append(dict(name=name, classes=cls, coop=True, glob=g,
+                        stride=max(tab[c]["total"] for c in cls)))
+    return out
+
+
+def fuse_source(bucket, ids):
+    cls, name = bucket["classes"], bucket["name"]
+    members = ",\n        ".join("FuseMember<%d, C%d%d%d%d%s>" % ((ids[c],) + c + ("Coop" if bucket["coop"] else "",))
+                                for c in cls)
+    out = ["// Generated by quick_amd/codegen/gen_eri.py - do not edit.", '#include "../qf_fuse.h"',
+           '#include "../qf_launch.h"']
+    out += ['#include "%sC%d%d%d%d.h"' % (("coop_" if bucket["coop"] else "",) + c) for c in cls]
+    out += ["", "namespace qf {", "",
+            "void launch_fuse_%s(const FusedBlock* list, int n, const TileGroup* g, const Task* t, const PairBlock* b,"
+            % name,
+            "    const MolDesc* m, int os, int waves, size_t lds, double* gscratch, LaunchTo& q)", "{"]
+    if bucket["coop"]:
+        out += ["    (void)g;", "    (void)waves;",
+                "    const int grid = %s;" % ("n > COOP_GLOBAL_SLICES ? COOP_GLOBAL_SLICES : n" if bucket["glob"] else "n")]
+        for os_ in (True, False):
+            out += ["    if (os)" if os_ else "    else",
+                    "        q((fused_coop_kernel<%s, %d,\n        %s>),"
+                    % ("true" if os_ else "false", bucket["stride"], members),
+                    "          dim3(grid), dim3(WAVE), lds, list, n, t, b, m, gscratch);"]
+    else:
+        out += ["    (void)gscratch;"]
+        for os_ in (True, False):
+            out += ["    if (os)" if os_ else "    else",
+                    "        q((fused_tile_kernel<%d, %s,\n        %s>),"
+                    % (bucket["waves"], "true" if os_ else "false", members),
+                    "          dim3(n), dim3(waves * WAVE), lds, list, g, t, b, m);"]
+    out += ["}", "", "}  // namespace qf", ""]
+    return "\n".join(out)
+
+
+def _sizes(La, Lb, Lc, Ld):
+    nacc = sum(ncart(E) for E in range(La, La + Lb + 1)) * sum(ncart(F) for F in range(Lc, Lc + Ld + 1))
+    return nacc, ncart(La) * ncart(Lb) * ncart(Lc) * ncart(Ld)
+
+
 def _write(path, text):
     """Write only when the content changes, so incremental builds stay incremental."""
     if os.path.exists(path):
@@ -852,7 +907,36 @@ def main():
     for (name, La, Lb, Lc, Ld, diag) in names:
         if diag:
             lines.append("    if (c == %d) return launch_schwarz_%s;" % (pc[(La, Lb)], name))
-    lines += ["    return nullptr;", "}", "", "}  // namespace qf", ""]
+    lines += ["    return nullptr;", "}", ""]
+    # launches that hold several classes
+    buckets = fuse_buckets()
+    ids = {(La, Lb, Lc, Ld): pc[(La, Lb)] * 16 + pc[(Lc, Ld)] for (_, La, Lb, Lc, Ld, _) in names}
+    lines += ["// (list, workgroups, groups, tasks, blocks, mols, os, waves, lds bytes, global slots, target)",
+              "using FuseLaunch = void (*)(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*,"
+              " const MolDesc*, int, int, size_t, double*, LaunchTo&);"]
+    for b in buckets:
+        _write(os.path.join(OUT, "fuse_%s.hip" % b["name"]), fuse_source(b, ids))
+        lines.append("void launch_fuse_%s(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*,"
+                     " const MolDesc*, int, int, size_t, double*, LaunchTo&);" % b["name"])
+    lines += ["", "struct FuseKernel {", "    FuseLaunch launch;", "    bool coop;          // wave-per-quartet classes",
+              "    int global;         // doubles of a workgroup's slice of the global slot buffer (0: slots in LDS)",
+              "};", "constexpr int kFuseKernels = %d;" % len(buckets),
+              "inline FuseKernel fuse_kernel(int k)", "{", "    constexpr FuseKernel all[kFuseKernels] = {"]
+    lines += ["        {launch_fuse_%s, %s, %d}," % (b["name"], "true" if b["coop"] else "false",
+                                                     b["stride"] if b["glob"] else 0) for b in buckets]
+    lines += ["    };", "    return all[k];", "}", "",
+              "// the kernel that runs a class beside others (-1: none), and the class's number in it",
+              "inline int fuse_bucket(int cb, int ck, bool coop)", "{", "    switch ((cb * 16 + ck) * 2 + (coop ? 1 : 0)) {"]
+    for k, b in enumerate(buckets):
+        for c in b["classes"]:
+            lines.append("    case %d: return %d;" % (ids[c] * 2 + (1 if b["coop"] else 0), k))
+    lines += ["    }", "    return -1;", "}", "", "// doubles of LDS a wave-per-quartet class needs (0: its slots are global)",
+              "inline int coop_lds_doubles(int cb, int ck)", "{", "    switch (cb * 16 + ck) {"]
+    for c in COOP_CLASSES:
+        t = coop_tables(*c)
+        if not t["glob"]:
+            lines.append("    case %d: return %d;" % (ids[c], t["total"]))
+    lines += ["    }", "    return 0;", "}", "", "}  // namespace qf", ""]
     _write(os.path.join(OUT, "launchers.h"), "\n".join(lines))
     from . import gen_boys, gen_grad
     _write(os.path.join(OUT, "boys_grid.h"), gen_boys.header())

@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <map>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -430,8 +431,19 @@ struct qf_engine {
         size_t gslot;    // first double of its region of the global slot buffer (classes that need one)
     };
     std::vector<Launch> launches;
-    std::vector<std::pair<int, int>> order;   // issue order: (launch index, stream 0..kSide)
-    double fork_gain = 0.0;                   // seconds the forked order saves (estimate)
+    struct Fused {           // classes of `launches` that share a launch
+        int kernel;          // qf::fuse_kernel
+        int offset, count;   // its workgroups in d_fused
+        int waves;
+        size_t lds, gslot;
+        double seconds;      // estimate
+    };
+    std::vector<Fused> fused;
+    struct Plan {
+        std::vector<std::pair<int, int>> order;   // (launch index, or ~ the index into fused; stream 0..kSide)
+        double gain = 0.0;                        // seconds the forked order saves (estimate)
+    };
+    Plan plan[3];                             // closed shell, open shell, gradient and one launch per class
     SideStreams* side = nullptr;              // taken at the first forked build
     Replay replay[3];                         // closed shell, open shell, gradient
     void drop_replays()
@@ -452,6 +464,7 @@ struct qf_engine {
     DevBuf<qf::MolDesc> d_mol;
     DevBuf<qf::Task> d_tasks;
     DevBuf<qf::TileGroup> d_groups;
+    DevBuf<qf::FusedBlock> d_fused;
     DevBuf<int> d_colf;
     DevBuf<double> d_Gt, d_Gs, d_cm, d_P;
     DevBuf<double> d_Pb, d_Pt, d_Ps, d_Fa, d_Fb;   // open-shell builds (allocated on first use)
@@ -754,46 +767,144 @@ size_t place_slots(std::vector<qf_engine::Launch>& launches)
     return total;
 }
 
-// Issue order of class launches and the stream of each: longest first, each
-// to the stream with the least time so far.  The time of a launch is taken as
-// the larger of its longest task alone and all of its work spread over the
-// GPU, plus a launch: algorithmic FLOPs of every quartet of the windows, at
-// 1.3 GFLOP/s for a wave that works through quartets one by one ((dd|dd)
-// 39 kFLOP in 34 us, (ff|ff) 340 kFLOP in 476 us) and 0.2 GFLOP/s for a lane
-// of the per-lane kernels, and at the 1.2 and 6 TFLOP/s that whole launches
-// reach.
-std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launch>& launches,
-                                              const std::vector<qf::Task>& tasks, double* gain = nullptr)
-{
-    const int n = (int)launches.size();
-    std::vector<double> t(n);
-    for (int l = 0; l < n; ++l) {
-        const auto& L = launches[l];
-        const bool wave = L.tile == 2;
-        double all = 0.0, longest = 0.0;
-        for (int x = L.offset; x < L.offset + L.count; ++x) {
-            const qf::Task& k = tasks[x];
-            const int bras = k.ke - k.kb;
-            const double one = qf::class_flops(L.cb, L.ck, 1, (unsigned long long)(k.pe - k.pb) * (k.qe - k.qb));
-            all += one * bras * k.ket_count;
-            longest = std::max(longest, one * bras * (wave ? k.ket_count : 1));
-        }
-        t[l] = 5e-6 + std::max(longest / (wave ? 1.3e9 : 0.2e9), all / (wave ? 1.2e12 : 6e12));
+// Estimated seconds of a launch: the larger of its longest task alone and all of
+// its work spread over the GPU, plus a launch.  Algorithmic FLOPs of every
+// quartet of the windows, at 1.3 GFLOP/s for a wave that works through quartets
+// one by one ((dd|dd) 39 kFLOP in 34 us, (ff|ff) 340 kFLOP in 476 us) and 0.2
+// GFLOP/s for a lane of the per-lane kernels, and at the 1.2 and 6 TFLOP/s that
+// whole launches reach.
+struct LaunchCost {
+    double all = 0.0, longest = 0.0;
+    double task(const qf_engine::Launch& L, const qf::Task& k, bool wave)
+    {
+        const int bras = k.ke - k.kb;
+        const double one = qf::class_flops(L.cb, L.ck, 1, (unsigned long long)(k.pe - k.pb) * (k.qe - k.qb));
+        const double t = one * bras * (wave ? k.ket_count / 1.3e9 : 1 / 0.2e9);
+        all += one * bras * k.ket_count / (wave ? 1.2e12 : 6e12);
+        longest = std::max(longest, t);
+        return t;
     }
-    std::vector<int> ord(n);
+    double seconds() const { return 5e-6 + std::max(longest, all); }
+};
+
+// Issue order of launches that take t seconds, and the stream of each: longest
+// first, each to the stream with the least time so far.
+qf_engine::Plan stream_order(const std::vector<std::pair<int, double>>& t)
+{
+    qf_engine::Plan p;
+    std::vector<int> ord(t.size());
     std::iota(ord.begin(), ord.end(), 0);
-    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return t[x] > t[y]; });
+    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return t[x].second > t[y].second; });
     double load[kSide + 1] = {};
-    std::vector<std::pair<int, int>> out;
     for (int l : ord) {
         int to = 0;
         for (int k = 1; k <= kSide; ++k)
             if (load[k] < load[to]) to = k;
-        load[to] += t[l];
-        out.push_back({l, to});
+        load[to] += t[l].second;
+        p.order.push_back({t[l].first, to});
+        p.gain += t[l].second;
     }
-    if (gain) *gain = std::accumulate(t.begin(), t.end(), 0.0) - *std::max_element(load, load + kSide + 1);
-    return out;
+    p.gain -= *std::max_element(load, load + kSide + 1);
+    return p;
+}
+
+qf_engine::Plan stream_order(const std::vector<qf_engine::Launch>& launches, const std::vector<qf::Task>& tasks)
+{
+    std::vector<std::pair<int, double>> t;
+    for (int l = 0; l < (int)launches.size(); ++l) {
+        const auto& L = launches[l];
+        LaunchCost c;
+        for (int x = L.offset; x < L.offset + L.count; ++x) c.task(L, tasks[x], L.tile == 2);
+        t.push_back({l, c.seconds()});
+    }
+    return stream_order(t);
+}
+
+// Molecules whose classes share launches: up to 200 functions, without d shells
+// (six classes) up to 100.  Builds in us, one launch per class and stream chain ->
+// shared launches (each with the task shapes that suit it): ethane 6-31G (30
+// functions) 151 -> 82, glycine 3-21G (55) 143 -> 102, (Gly)2 6-31G (97) 423 -> 434,
+// C12H26 6-31G (160) 1027 -> 1107; with d shells water 6-31G* (19) 134 -> 77, ethane
+// 6-31G* (42) 273 -> 153, glycine 6-31G** (100) 637 -> 394, ethane def2-TZVP (108, 55
+// classes) 1561 -> 1104, (H2O)8 6-31G* (152) 799 -> 526, its cation 1003 -> 679, (Gly)2
+// 6-31G** (175) 1411 -> 1373, (H2O)8 cc-pVDZ (200) 1065 -> 960.  Above, a launch
+// fills the GPU by itself and a bucket costs its light classes their occupancy:
+// (H2O)12 (228) 1484 -> 1513, C20H42 3-21G (264) 911 -> 1097, (H2O)16 (304) 2896 ->
+// 2993, (H2O)32 (608) 9982 -> 12755.
+bool shares_launches(const qf_engine* e)
+{
+    int lmax = 0;
+    for (int l : e->s_lmax) lmax = std::max(lmax, l);
+    return e->tile != 0 && e->nbasis <= (lmax > 1 ? 200 : 100);
+}
+
+// Plan of closed-shell (os 0) or open-shell (os 1) builds in which classes of
+// the same kernel bucket share a launch, its workgroups longest first.
+// Appends to e->fused and to `list`, their workgroups; slots: doubles of the
+// global slot buffer that the plan's shared launches need.
+qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& list, size_t& slots)
+{
+    struct Group {
+        std::vector<std::pair<double, qf::FusedBlock>> blocks;
+        std::vector<int> members;
+        LaunchCost cost;
+        size_t lds = 0;
+    };
+    std::map<std::pair<int, int>, Group> groups;   // by kernel and waves
+    std::vector<std::pair<int, double>> t;
+    for (int l = 0; l < (int)e->launches.size(); ++l) {
+        const auto& L = e->launches[l];
+        const bool alt = os && L.alt_count > 0, coop = L.tile == 2 || alt;
+        const int id = L.cb * 16 + L.ck;
+        const int kernel = L.fp32 || L.tile == 0 || (os && L.os_split) || (os && !coop && !L.os_lean)
+                               ? -1
+                               : qf::fuse_bucket(L.cb, L.ck, coop);
+        LaunchCost own;
+        const int first = alt ? L.alt_offset : L.offset, count = alt ? L.alt_count : L.count;
+        Group* g = kernel < 0 ? nullptr : &groups[{kernel, coop ? 1 : L.waves}];
+        LaunchCost& c = g ? g->cost : own;
+        if (g && !coop) {
+            const bool two = os && L.lds_os;
+            g->lds = std::max(g->lds, two ? L.lds_os : L.lds);
+            for (int x = L.goffset; x < L.goffset + L.gcount; ++x) {
+                const auto& tg = e->groups[x];
+                std::vector<double> wave(L.waves, 0.0);
+                for (int k = tg.task_begin; k < tg.task_end; ++k)
+                    wave[(k - tg.task_begin) % L.waves] += c.task(L, e->tasks[k], false);
+                g->blocks.push_back({*std::max_element(wave.begin(), wave.end()),
+                                     qf::FusedBlock{id + (two ? 256 : 0), x}});
+            }
+        } else {
+            if (g) g->lds = std::max(g->lds, sizeof(double) * qf::coop_lds_doubles(L.cb, L.ck));
+            for (int x = first; x < first + count; ++x) {
+                const double s = c.task(L, e->tasks[x], coop);
+                if (g) g->blocks.push_back({s, qf::FusedBlock{id, x}});
+            }
+        }
+        if (g)
+            g->members.push_back(l);
+        else
+            t.push_back({l, own.seconds()});
+    }
+    slots = 0;
+    for (auto& kv : groups) {
+        Group& g = kv.second;
+        std::stable_sort(g.blocks.begin(), g.blocks.end(),
+                         [](const auto& x, const auto& y) { return x.first > y.first; });
+        qf_engine::Fused f{};
+        f.kernel = kv.first.first;
+        f.waves = kv.first.second;
+        f.offset = (int)list.size();
+        f.count = (int)g.blocks.size();
+        f.lds = g.lds;
+        f.gslot = slots;
+        f.seconds = g.cost.seconds();
+        slots += (size_t)qf::fuse_kernel(f.kernel).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
+        for (const auto& x : g.blocks) list.push_back(x.second);
+        t.push_back({~(int)e->fused.size(), f.seconds});
+        e->fused.push_back(f);
+    }
+    return stream_order(t);
 }
 
 // Wave tasks, tile groups and launches of one engine, per quartet class and
@@ -802,7 +913,7 @@ std::vector<std::pair<int, int>> stream_order(const std::vector<qf_engine::Launc
 // that of the molecule whose build holds as much work (the precision split
 // goes by the engine's own size).  Index ranges are those of the output vectors.
 int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::vector<qf::TileGroup>& groups,
-               std::vector<qf_engine::Launch>& launches, qf_stats* stats)
+               std::vector<qf_engine::Launch>& launches, qf_stats* stats, bool shared = false)
 {
     const double thr_hi = e->split_thr;
     tasks.clear();
@@ -821,13 +932,19 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
     // workgroup) 1710 / 824 / 614 / 589 / 616 / 989, (H2O)8 6-31G* (152) 1808 /
     // 881 / 788 / 857 / 1015 / 1479, (Gly)2 6-31G** (175) 4526 / 2258 / 1483 /
     // 1442 / 1560 / 2021, (H2O)16 6-31G* (304) 10064 / 4669 / 2909 / 2823 / 2599 /
-    // 2931, (H2O)32 (608) 34806 / 17910 / 11420 / 11298 / 10712 / 10692.
+    // 2931, (H2O)32 (608) 34806 / 17910 / 11420 / 11298 / 10712 / 10692.  Shared
+    // launches (`shared`) have no tails of their own to shorten and take longer
+    // pieces; 1 / 2 / 3 / 4 / 6: water 113 / 72 / 91 / - / -, ethane 6-31G* (42) 217 / 151 /
+    // 255 / 303 / 436, butane 775 / 402 / 357 / 316 / 606, glycine 1116 / 548 / 401 / 393 /
+    // 436, (H2O)8 6-31G* 1753 / 865 / 587 / 580 / 526, (Gly)2 3839 / 2116 / 1478 / 1472 /
+    // 1371.
     const int piece = e->prim_piece > 0   ? e->prim_piece
                       : e->prim_piece < 0 ? 1 << 20
+                      : shared            ? (size <= 48 ? 2 : size <= 64 ? 3 : size <= 128 ? 4 : 6)
                       : size <= 48        ? 1
                       : size <= 96        ? 2
                       : size <= 160       ? 3
-                      : size <= 256       ? 4
+                      : size <= 200       ? 4
                       : size <= 400       ? 6
                                           : 12;
     for (int cb = 0; cb < kNPC; ++cb)
@@ -854,10 +971,13 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // 928 / 1180, (H2O)8 cc-pVDZ (200 functions) 1077 / 1129 / 1202 / 1242 /
                 // 1447, C20H42 3-21G (264) 1825 / 1105 / 912 / 897 / 994, (H2O)16
                 // 3703 / 2940 / 3133 / 3171 / 3142, (H2O)32 25512 / 14599 / 12000 / 11245 /
-                // 10973)
+                // 10973; shared launches, 1 / 2 / 4: ethane 6-31G* 155 / 151 / 237, glycine
+                // 393 / 442 / 593, (H2O)8 6-31G* 516 / 526 / 628, its cation 853 / 677 / 753,
+                // (Gly)2 6-31G** 1438 / 1371 / 1889)
                 int tile_tasks = ct.tpg > 0        ? ct.tpg
                                        : e->tile_tasks > 0 ? e->tile_tasks
-                                       : size <= 200       ? 2
+                                       : shared            ? (size <= 48 || size > 128 ? 2 : 1)
+                                       : size <= 256       ? 2
                                        : size <= 400       ? 4
                                                            : 16;
                 int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
@@ -904,8 +1024,11 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // (QUICK's regression inputs of 49-128 functions run their
                 // La+Lb+Lc+Ld = 4 classes faster on the tile kernel: PO4 6-31G*
                 // 15.8x -> 18.0x, PSB5 6-31G 26x -> 34x QUICK's build times;
-                // up to 48 functions and at 5 the wave-per-quartet kernel wins)
-                const int coop_lmin = size <= 48 ? 4 : size <= 128 ? 5 : 6;
+                // up to 48 functions and at 5 the wave-per-quartet kernel wins;
+                // in shared launches, with La+Lb+Lc+Ld >= 4 / 5 / 6 on it: water 72 / 79 / 97,
+                // ethane 6-31G* 211 / 155 / 151, butane 633 / 336 / 316, glycine 800 / 509 /
+                // 393, (H2O)8 6-31G* 972 / 635 / 516)
+                const int coop_lmin = shared ? (size <= 32 ? 4 : 6) : size <= 48 ? 4 : size <= 128 ? 5 : 6;
                 const bool tile_class = qf::fock_tile_launcher(cb, ck) != nullptr;
                 const bool tile_ok = tile_class && mfit >= 1;
                 // Classes whose FP64 tile kernel runs in Hermite Gaussians: above 256
@@ -1202,15 +1325,25 @@ int prepare(qf_engine* e)
     e->split_thr = e->split * ymax * ymax;
     e->stats = qf_stats{};
     for (auto& b : e->blocks) e->stats.n_pairs += (long long)b.info.size();
-    rc = make_tasks(e, e->nbasis, e->tasks, e->groups, e->launches, &e->stats);
+    rc = make_tasks(e, e->nbasis, e->tasks, e->groups, e->launches, &e->stats, shares_launches(e));
     if (rc) return rc;
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
-    e->order = stream_order(e->launches, e->tasks, &e->fork_gain);
     e->drop_replays();
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
-    const size_t gdoubles = place_slots(e->launches);
+    size_t gdoubles = place_slots(e->launches);
+    e->fused.clear();
+    e->plan[0] = e->plan[1] = e->plan[2] = stream_order(e->launches, e->tasks);
+    if (shares_launches(e)) {
+        std::vector<qf::FusedBlock> list;
+        for (int os = 0; os < 2; ++os) {
+            size_t slots = 0;
+            e->plan[os] = fuse_plan(e, os, list, slots);
+            gdoubles = std::max(gdoubles, slots);
+        }
+        QF_HIP(e->d_fused.upload(list));
+    }
     if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles));
 
     // ---- per-build buffers -------------------------------------------------
@@ -1364,7 +1497,8 @@ int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, con
 {
     Replay& r = e->replay[kind];
     const bool captured = is_capturing(s);
-    if (!captured && !r.exec && !r.failed && !e->order.empty() && ++r.uses > 1) {
+    const qf_engine::Plan& plan = e->plan[e->persist > 0 ? 2 : kind];   // a capped grid caps each class's
+    if (!captured && !r.exec && !r.failed && !plan.order.empty() && ++r.uses > 1) {
         hipGraphNode_t last[kSide + 1] = {};
         bool ok = hipGraphCreate(&r.graph, 0) == hipSuccess;
         if (ok) {
@@ -1373,7 +1507,7 @@ int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, con
             r.first = to.node;
             ok = to.err == hipSuccess;
         }
-        for (const auto& o : e->order) {
+        for (const auto& o : plan.order) {
             if (!ok) break;
             qf::LaunchTo to(r.graph, last[o.second] ? &last[o.second] : &r.first, 1);
             const int rc = issue(o.first, to);
@@ -1422,8 +1556,8 @@ int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, con
     }
     qf::LaunchTo to(s);
     open_build(open, to);
-    const bool forked = e->order.size() > 1 && (e->side || e->fork_gain > 8e-5) && side_ready(e->side, e->device, s);
-    const int rc = issue_forked(forked ? e->side : nullptr, s, e->order, [&](int li, hipStream_t q) {
+    const bool forked = plan.order.size() > 1 && (e->side || plan.gain > 8e-5) && side_ready(e->side, e->device, s);
+    const int rc = issue_forked(forked ? e->side : nullptr, s, plan.order, [&](int li, hipStream_t q) {
         qf::LaunchTo x(q);
         return issue(li, x);
     });
@@ -1525,20 +1659,37 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         const int rc = launch(L, dmol, 0, q);
         return rc ? rc : launch(L, dmol_x, 0, q);
     };
+    auto shared_launch = [&](const qf_engine::Fused& f, qf::LaunchTo& q) -> int {
+        qf::fuse_kernel(f.kernel).launch(e->d_fused.p + f.offset, f.count, e->d_groups.p, e->d_tasks.p, e->d_blocks.p,
+                                         dmol, os, f.waves, f.lds, e->d_cscratch.p + f.gslot, q);
+        return QF_OK;
+    };
     if (gb.fork && !gb.timing) {
         const int rc = issue_build(e, os, s, oa, &ca,
-                                   [&](int li, qf::LaunchTo& q) { return class_launch(e->launches[li], q); });
+                                   [&](int li, qf::LaunchTo& q) {
+                                       return li < 0 ? shared_launch(e->fused[~li], q)
+                                                     : class_launch(e->launches[li], q);
+                                   });
         if (rc) return rc;
+    } else if (!gb.timing) {
+        // one after another on s
+        qf::LaunchTo to(s);
+        open_build(oa, to);
+        for (const auto& o : e->plan[e->persist > 0 ? 2 : os].order) {
+            const int rc = o.first < 0 ? shared_launch(e->fused[~o.first], to) : class_launch(e->launches[o.first], to);
+            if (rc) return rc;
+        }
+        close_build(ca, to);
     } else {
-        // one after another on s, timed ones between events
+        // class by class between events
         qf::LaunchTo to(s);
         open_build(oa, to);
         for (size_t li = 0; li < e->launches.size(); ++li) {
             hipEvent_t eb = nullptr;
-            if (gb.timing && timing_begin(e, (int)li, s, &eb)) return QF_ERR_HIP;
+            if (timing_begin(e, (int)li, s, &eb)) return QF_ERR_HIP;
             const int rc = class_launch(e->launches[li], to);
             if (rc) return rc;
-            if (eb) QF_HIP(hipEventRecord(eb, s));
+            QF_HIP(hipEventRecord(eb, s));
         }
         close_build(ca, to);
     }
@@ -2543,7 +2694,7 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
         b->d_groups.upload(groups) != hipSuccess || b->d_moldesc.upload(md) != hipSuccess ||
         b->d_bm.upload(b->mols) != hipSuccess)
         return bail(fail(QF_ERR_HIP, "batch table upload"));
-    b->order = stream_order(b->launches, tasks);
+    b->order = stream_order(b->launches, tasks).order;
     b->side = SidePool::get().take(b->device);   // null: the batch runs on the caller's stream alone
     *out = b;
     return QF_OK;

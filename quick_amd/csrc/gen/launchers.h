@@ -328,4 +328,157 @@ inline SchwarzLaunch schwarz_launcher(int c)
     return nullptr;
 }
 
+// (list, workgroups, groups, tasks, blocks, mols, os, waves, lds bytes, global slots, target)
+using FuseLaunch = void (*)(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+void launch_fuse_tile3(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+void launch_fuse_tile2(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+void launch_fuse_tile1(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+void launch_fuse_coop_small(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+void launch_fuse_coop_large(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+void launch_fuse_coop_global(const FusedBlock*, int, const TileGroup*, const Task*, const PairBlock*, const MolDesc*, int, int, size_t, double*, LaunchTo&);
+
+struct FuseKernel {
+    FuseLaunch launch;
+    bool coop;          // wave-per-quartet classes
+    int global;         // doubles of a workgroup's slice of the global slot buffer (0: slots in LDS)
+};
+constexpr int kFuseKernels = 6;
+inline FuseKernel fuse_kernel(int k)
+{
+    constexpr FuseKernel all[kFuseKernels] = {
+        {launch_fuse_tile3, false, 0},
+        {launch_fuse_tile2, false, 0},
+        {launch_fuse_tile1, false, 0},
+        {launch_fuse_coop_small, true, 0},
+        {launch_fuse_coop_large, true, 0},
+        {launch_fuse_coop_global, true, 35734},
+    };
+    return all[k];
+}
+
+// the kernel that runs a class beside others (-1: none), and the class's number in it
+inline int fuse_bucket(int cb, int ck, bool coop)
+{
+    switch ((cb * 16 + ck) * 2 + (coop ? 1 : 0)) {
+    case 0: return 0;
+    case 32: return 0;
+    case 34: return 0;
+    case 64: return 0;
+    case 96: return 0;
+    case 128: return 0;
+    case 192: return 0;
+    case 66: return 1;
+    case 98: return 1;
+    case 160: return 1;
+    case 194: return 1;
+    case 224: return 1;
+    case 68: return 2;
+    case 100: return 2;
+    case 102: return 2;
+    case 130: return 2;
+    case 134: return 2;
+    case 162: return 2;
+    case 196: return 2;
+    case 198: return 2;
+    case 226: return 2;
+    case 256: return 2;
+    case 69: return 3;
+    case 101: return 3;
+    case 103: return 3;
+    case 133: return 3;
+    case 135: return 3;
+    case 137: return 3;
+    case 161: return 3;
+    case 163: return 3;
+    case 165: return 3;
+    case 167: return 3;
+    case 193: return 3;
+    case 195: return 3;
+    case 197: return 3;
+    case 199: return 3;
+    case 201: return 3;
+    case 205: return 3;
+    case 225: return 3;
+    case 227: return 3;
+    case 229: return 3;
+    case 231: return 3;
+    case 257: return 3;
+    case 259: return 3;
+    case 263: return 3;
+    case 289: return 3;
+    case 291: return 3;
+    case 169: return 4;
+    case 171: return 4;
+    case 203: return 4;
+    case 233: return 4;
+    case 235: return 4;
+    case 237: return 4;
+    case 239: return 4;
+    case 261: return 4;
+    case 265: return 4;
+    case 267: return 4;
+    case 269: return 4;
+    case 271: return 4;
+    case 293: return 4;
+    case 295: return 4;
+    case 297: return 4;
+    case 301: return 4;
+    case 273: return 5;
+    case 299: return 5;
+    case 303: return 5;
+    case 305: return 5;
+    case 307: return 5;
+    }
+    return -1;
+}
+
+// doubles of LDS a wave-per-quartet class needs (0: its slots are global)
+inline int coop_lds_doubles(int cb, int ck)
+{
+    switch (cb * 16 + ck) {
+    case 34: return 334;
+    case 50: return 268;
+    case 51: return 236;
+    case 66: return 574;
+    case 67: return 478;
+    case 68: return 1090;
+    case 80: return 205;
+    case 81: return 451;
+    case 82: return 1141;
+    case 83: return 820;
+    case 84: return 2176;
+    case 85: return 4210;
+    case 96: return 107;
+    case 97: return 194;
+    case 98: return 419;
+    case 99: return 367;
+    case 100: return 786;
+    case 101: return 1386;
+    case 102: return 660;
+    case 112: return 182;
+    case 113: return 354;
+    case 114: return 889;
+    case 115: return 734;
+    case 116: return 1700;
+    case 117: return 3311;
+    case 118: return 1328;
+    case 119: return 2802;
+    case 128: return 302;
+    case 129: return 686;
+    case 130: return 1774;
+    case 131: return 1262;
+    case 132: return 3406;
+    case 133: return 6622;
+    case 134: return 2189;
+    case 135: return 5582;
+    case 144: return 526;
+    case 145: return 1270;
+    case 146: return 3422;
+    case 147: return 2386;
+    case 148: return 6650;
+    case 150: return 3874;
+    }
+    return 0;
+}
+
 }  // namespace qf

@@ -350,22 +350,63 @@ __device__ __forceinline__ void coop_quartet(const Task& t, const PairBlock& bb,
 }
 
 // Slot memory of this workgroup: dynamic LDS, or its slice of the global
-// scratch buffer (gscratch holds gridDim.x slices of D::LDS doubles).
-template <class D>
+// scratch buffer (gscratch holds gridDim.x slices of STRIDE doubles).
+template <class D, int STRIDE = D::LDS>
 __device__ __forceinline__ CoopSlots<D> coop_slots(double* gscratch)
 {
     if constexpr (D::GLOBAL_SLOTS) {
-        return (QF_AS_GLOBAL double*)(gscratch + (size_t)blockIdx.x * D::LDS);
+        return (QF_AS_GLOBAL double*)(gscratch + (size_t)blockIdx.x * STRIDE);
     } else {
         extern __shared__ double qf_lds[];
         return (QF_AS_LDS double*)qf_lds;
     }
 }
 
-// One workgroup (one wave) per task of a narrow ket window: the wave
-// screens the task's quartets lane-parallel, then processes the surviving
-// quartets one after another.  FP64 throughout.  Dynamic LDS: D::LDS doubles
-// (none with GLOBAL_SLOTS).
+// One task of a narrow ket window: the wave screens the task's quartets
+// lane-parallel, then processes the surviving quartets one after another.
+// FP64 throughout.
+template <class D, bool OS, typename SP>
+__device__ __forceinline__ void coop_task(const Task t, const PairBlock* __restrict__ blocks,
+                                          const MolDesc* __restrict__ mols, SP s, const QF_AS_LDS double* boys_tab)
+{
+    const int lane = threadIdx.x % WAVE;
+    const PairBlock bb = cptr(blocks)[t.bra_block];
+    const PairBlock kb = cptr(blocks)[t.ket_block];
+    const MolDesc md = cptr(mols)[bb.mol];
+    const int ns = md.nshell;
+    const size_t roff = (size_t)(blockIdx.x % md.replicas) * md.nbasis * md.nbasis;
+    const auto G = gptr_rw(md.G + roff);
+    const auto G2 = gptr_rw(OS ? md.G2 + roff : md.G);
+    const auto cm = gptr(md.cutmat);
+    const auto bperm = cptr(bb.bperm);
+    const bool in_range = lane < t.ket_count;
+    const int jl = t.ket_start + (in_range ? lane : 0);
+    const PairInfo kl = gptr(kb.info)[jl];
+    for (int kk = t.kb; kk < t.ke; ++kk) {
+        const int i = bperm[kk];
+        const PairInfo bi = cptr(bb.info)[i];
+        const double ytest = bi.ycut * kl.ycut;
+        double dn = fmax(4.0 * cm[bi.sa * ns + bi.sb], 4.0 * cm[kl.sa * ns + kl.sb]);
+        dn = fmax(dn, cm[bi.sa * ns + kl.sb]);
+        dn = fmax(dn, cm[bi.sa * ns + kl.sa]);
+        dn = fmax(dn, cm[bi.sb * ns + kl.sa]);
+        dn = fmax(dn, cm[bi.sb * ns + kl.sb]);
+        const bool valid = in_range && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
+                           (!t.same_block || jl <= i) && (t.all_fp64 || ytest >= md.split);
+        unsigned long long mask = __ballot(valid);
+        while (mask) {
+            const int v = __builtin_ctzll(mask);
+            mask &= mask - 1;
+            const int j = t.ket_start + v;
+            const PairInfo ki = cptr(kb.info)[j];
+            const double dnv = wave_read_lane(dn, v);
+            coop_quartet<D, OS>(t, bb, i, bi, kb, j, ki, dnv, md, G, G2, s, boys_tab);
+        }
+    }
+}
+
+// One workgroup (one wave) per task.  Dynamic LDS: D::LDS doubles (none with
+// GLOBAL_SLOTS).
 template <class D, bool OS = false>
 __global__ __launch_bounds__(D::NT) void fock_coop_kernel(const Task* __restrict__ tasks, int ntasks,
                                                          const PairBlock* __restrict__ blocks,
@@ -375,43 +416,8 @@ __global__ __launch_bounds__(D::NT) void fock_coop_kernel(const Task* __restrict
     QF_BOYS_LDS_DECL;
     QF_BOYS_LDS_FILL();
     const auto s = coop_slots<D>(gscratch);
-    const int lane = threadIdx.x % WAVE;
-    for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
-        const Task t = cptr(tasks)[ti];
-        const PairBlock bb = cptr(blocks)[t.bra_block];
-        const PairBlock kb = cptr(blocks)[t.ket_block];
-        const MolDesc md = cptr(mols)[bb.mol];
-        const int ns = md.nshell;
-        const size_t roff = (size_t)(blockIdx.x % md.replicas) * md.nbasis * md.nbasis;
-        const auto G = gptr_rw(md.G + roff);
-        const auto G2 = gptr_rw(OS ? md.G2 + roff : md.G);
-        const auto cm = gptr(md.cutmat);
-        const auto bperm = cptr(bb.bperm);
-        const bool in_range = lane < t.ket_count;
-        const int jl = t.ket_start + (in_range ? lane : 0);
-        const PairInfo kl = gptr(kb.info)[jl];
-        for (int kk = t.kb; kk < t.ke; ++kk) {
-            const int i = bperm[kk];
-            const PairInfo bi = cptr(bb.info)[i];
-            const double ytest = bi.ycut * kl.ycut;
-            double dn = fmax(4.0 * cm[bi.sa * ns + bi.sb], 4.0 * cm[kl.sa * ns + kl.sb]);
-            dn = fmax(dn, cm[bi.sa * ns + kl.sb]);
-            dn = fmax(dn, cm[bi.sa * ns + kl.sa]);
-            dn = fmax(dn, cm[bi.sb * ns + kl.sa]);
-            dn = fmax(dn, cm[bi.sb * ns + kl.sb]);
-            const bool valid = in_range && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
-                               (!t.same_block || jl <= i) && (t.all_fp64 || ytest >= md.split);
-            unsigned long long mask = __ballot(valid);
-            while (mask) {
-                const int v = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                const int j = t.ket_start + v;
-                const PairInfo ki = cptr(kb.info)[j];
-                const double dnv = wave_read_lane(dn, v);
-                coop_quartet<D, OS>(t, bb, i, bi, kb, j, ki, dnv, md, G, G2, s, QF_BOYS_LDS_PTR);
-            }
-        }
-    }
+    for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x)
+        coop_task<D, OS>(cptr(tasks)[ti], blocks, mols, s, QF_BOYS_LDS_PTR);
 }
 
 // Schwarz diagonal of a class (La Lb | La Lb) on the wave-per-quartet node

@@ -921,13 +921,51 @@ __device__ __forceinline__ void tile_flush(QF_AS_LDS double* lds, int nk, int nt
 // (na + nbra*nb) * ncol * (k2 ? 2 : 1) + nbra*na*nb doubles.  OS: the
 // second exchange terms go to a second LDS tile (k2 = 1) or straight to
 // G2 (k2 = 0, where two tiles do not fit).
+// One group of the tile kernel (a workgroup's work).
+template <class C, typename R, bool OS, bool LEAN>
+__device__ __forceinline__ void fock_tile_group(const TileGroup g, const Task* __restrict__ tasks,
+                                                const PairBlock* __restrict__ blocks,
+                                                const MolDesc* __restrict__ mols, int k2, QF_AS_LDS double* lds,
+                                                const QF_AS_LDS double* boys_tab, const QF_AS_LDS float* boys_grid)
+{
+    constexpr int na = ncart(C::La), nb = ncart(C::Lb);
+    const int nw = blockDim.x / WAVE;
+    const Task t0 = cptr(tasks)[g.task_begin];
+    const PairBlock bb = cptr(blocks)[t0.bra_block];
+    const PairBlock kb = cptr(blocks)[t0.ket_block];
+    const MolDesc md = cptr(mols)[bb.mol];
+    const int n = md.nbasis;
+    const int nrow = na + g.nbra * nb, ncol = kb.ncol;
+    const int ntile = nrow * ncol, njab = g.nbra * na * nb;
+    const bool two = OS && k2;
+    const int nk = two ? 2 * ntile : ntile;
+    for (int x = threadIdx.x; x < nk + njab; x += blockDim.x) lds[x] = 0.0;
+    __syncthreads();
+
+    const size_t roff = (size_t)(blockIdx.x % md.replicas) * n * n;
+    const auto G = gptr_rw(md.G + roff);
+    const auto G2 = gptr_rw(OS ? md.G2 + roff : md.G);
+    const TileRef tr{lds, two ? lds + ntile : nullptr, lds + nk, ncol, g.chunk_kb, boys_tab, boys_grid};
+    // the wave index through readfirstlane: the compiler cannot prove
+    // threadIdx.x / 64 wave-uniform, and would otherwise keep the task,
+    // its loop bounds and the bra primitive data in vector registers
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
+    for (int ti = g.task_begin + wave; ti < g.task_end; ti += nw) {
+        const Task t = cptr(tasks)[wave_uniform(ti)];
+        fock_task<C, R, true, OS, LEAN>(t, bb, kb, md, G, G2, tr);
+    }
+    __syncthreads();
+
+    tile_flush<na, nb>(lds, nk, ntile, njab, ncol, g, bb, kb, md, G, G2);
+    __syncthreads();   // the next group reuses the tile
+}
+
 template <class C, typename R, bool OS = false, bool LEAN = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(WAVE, 4 * WAVE),
                           amdgpu_waves_per_eu((OS && !LEAN) ? C::MIN_WAVES_OS : C::MIN_WAVES)))
 void fock_tile_kernel(const TileGroup* __restrict__ groups, int ngroups, const Task* __restrict__ tasks,
                       const PairBlock* __restrict__ blocks, const MolDesc* __restrict__ mols, int k2)
 {
-    constexpr int na = ncart(C::La), nb = ncart(C::Lb);
     constexpr bool kF32 = sizeof(R) == 4;
     extern __shared__ double qf_lds[];
     // FP32 kernels: the FP32 Boys grid in LDS (6 KB; global-memory gathers
@@ -937,40 +975,9 @@ void fock_tile_kernel(const TileGroup* __restrict__ groups, int ngroups, const T
         for (int x = threadIdx.x; x < kBoysGridN * kBoysGridM; x += blockDim.x) qf_boys_grid[x] = kBoysGrid[x];
     QF_BOYS_LDS_DECL;
     QF_BOYS_LDS_FILL();
-    QF_AS_LDS double* lds = (QF_AS_LDS double*)qf_lds;
-    const int nw = blockDim.x / WAVE;
-    for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x) {
-        const TileGroup g = cptr(groups)[gi];
-        const Task t0 = cptr(tasks)[g.task_begin];
-        const PairBlock bb = cptr(blocks)[t0.bra_block];
-        const PairBlock kb = cptr(blocks)[t0.ket_block];
-        const MolDesc md = cptr(mols)[bb.mol];
-        const int n = md.nbasis;
-        const int nrow = na + g.nbra * nb, ncol = kb.ncol;
-        const int ntile = nrow * ncol, njab = g.nbra * na * nb;
-        const bool two = OS && k2;
-        const int nk = two ? 2 * ntile : ntile;
-        for (int x = threadIdx.x; x < nk + njab; x += blockDim.x) lds[x] = 0.0;
-        __syncthreads();
-
-        const size_t roff = (size_t)(blockIdx.x % md.replicas) * n * n;
-        const auto G = gptr_rw(md.G + roff);
-        const auto G2 = gptr_rw(OS ? md.G2 + roff : md.G);
-        const TileRef tr{lds, two ? lds + ntile : nullptr, lds + nk, ncol, g.chunk_kb, QF_BOYS_LDS_PTR,
-                         (const QF_AS_LDS float*)qf_boys_grid};
-        // the wave index through readfirstlane: the compiler cannot prove
-        // threadIdx.x / 64 wave-uniform, and would otherwise keep the task,
-        // its loop bounds and the bra primitive data in vector registers
-        const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE));
-        for (int ti = g.task_begin + wave; ti < g.task_end; ti += nw) {
-            const Task t = cptr(tasks)[wave_uniform(ti)];
-            fock_task<C, R, true, OS, LEAN>(t, bb, kb, md, G, G2, tr);
-        }
-        __syncthreads();
-
-        tile_flush<na, nb>(lds, nk, ntile, njab, ncol, g, bb, kb, md, G, G2);
-        __syncthreads();   // the next group reuses the tile
-    }
+    for (int gi = blockIdx.x; gi < ngroups; gi += gridDim.x)
+        fock_tile_group<C, R, OS, LEAN>(cptr(groups)[gi], tasks, blocks, mols, k2, (QF_AS_LDS double*)qf_lds,
+                                        QF_BOYS_LDS_PTR, (const QF_AS_LDS float*)qf_boys_grid);
 }
 
 // ---------------------------------------------------------------------------

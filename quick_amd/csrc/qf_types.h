@@ -82,4 +82,11 @@ struct TileGroup {
     int chunk_kb, nbra;
 };
 
+// A workgroup of a launch that holds several classes: the group (tile classes)
+// or task (wave-per-quartet classes) it runs.
+struct FusedBlock {
+    int cls;     // class: bra pair class * 16 + ket pair class; + 256: open shell with a second LDS tile
+    int index;   // into the groups or tasks
+};
+
 }  // namespace qf
