@@ -50,7 +50,9 @@ def _deps(src):
         deps.append(os.path.join(CSRC, "gen", "coop_" + base[4:-4] + ".h"))
         deps += [os.path.join(CSRC, "qf_md.h"), os.path.join(CSRC, "gen", "md_" + base[4:-4] + ".h")]
     if base.startswith("fuse_"):
-        deps += [os.path.join(CSRC, "qf_fuse.h")] + glob.glob(os.path.join(CSRC, "gen", "C*.h"))
+        deps += [os.path.join(CSRC, "qf_fuse.h"), os.path.join(CSRC, "qf_gfuse.h"), os.path.join(CSRC, "qf_grad.h"),
+                 os.path.join(CSRC, "gen", "grad_maps.h")]
+        deps += glob.glob(os.path.join(CSRC, "gen", "C*.h")) + glob.glob(os.path.join(CSRC, "gen", "grad_C*.h"))
         deps += glob.glob(os.path.join(CSRC, "gen", "coop_*.h"))
     if base.startswith("egrad_"):
         deps += [os.path.join(CSRC, "qf_grad.h"), os.path.join(CSRC, "gen", "grad_maps.h"),

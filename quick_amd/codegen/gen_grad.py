@@ -358,6 +358,43 @@ def launcher_source(name, g, lane):
         "}", ""] + extra + ["}  // namespace qf", ""])
 
 
+# Launches that hold several classes (qf_gfuse.h): per-lane classes by the waves
+# per SIMD their registers allow, the others by where their slots are.
+def fuse_buckets():
+    waves = {(0, 0, 0, 0): 3, (1, 0, 0, 0): 3, (1, 0, 1, 0): 2, (1, 1, 0, 0): 2, (2, 0, 0, 0): 2, (2, 1, 0, 0): 2}
+    out = []
+    for w in (3, 2, 1):
+        out.append(dict(name="grad_lane%d" % w, waves=w, coop=False, glob=False,
+                        classes=[c for c in grad_classes() if has_lane_grad(*c) and waves.get(c, 1) == w]))
+    for glob in (False, True):
+        cls = [c for c in grad_classes() if not has_lane_grad(*c) and grad_tables(*c)["glob"] == glob]
+        out.append(dict(name="grad_coop_global" if glob else "grad_coop", classes=cls, coop=True, glob=glob,
+                        stride=max(grad_tables(*c)["total"] for c in cls)))
+    return out
+
+
+def fuse_source(b, pc):
+    members = ",\n        ".join("FuseMember<%d, C%d%d%d%d%s>" % ((pc[c[:2]] * 16 + pc[c[2:]],) + c +
+                                                                 ("Grad" if b["coop"] else "GradMd",))
+                                for c in b["classes"])
+    out = ["// Generated by quick_amd/codegen/gen_grad.py - do not edit.", '#include "../qf_gfuse.h"',
+           '#include "../qf_launch.h"']
+    out += ['#include "grad_C%d%d%d%d.h"' % c for c in b["classes"]]
+    out += ["", "namespace qf {", "", "// slots: doubles of LDS slots (wave-per-quartet classes); tile: doubles of the gradient",
+            "void launch_fuse_%s(const FusedBlock* list, int n, const Task* t, const PairBlock* b, const MolDesc* m,"
+            % b["name"], "    int slots, int tile, double* gscratch, LaunchTo& q)", "{"]
+    if b["coop"]:
+        out += ["    const int grid = %s;" % ("n > COOP_GLOBAL_SLICES ? COOP_GLOBAL_SLICES : n" if b["glob"] else "n"),
+                "    q((fused_grad_coop_kernel<%d,\n        %s>)," % (b["stride"], members),
+                "      dim3(grid), dim3(WAVE), (slots + tile) * sizeof(double), list, n, t, b, m, gscratch, slots, tile);"]
+    else:
+        out += ["    (void)slots;", "    (void)gscratch;",
+                "    q((fused_grad_md_kernel<%d,\n        %s>)," % (b["waves"], members),
+                "      dim3(n), dim3(WAVE), tile * sizeof(double), list, t, b, m, tile);"]
+    out += ["}", "", "}  // namespace qf", ""]
+    return "\n".join(out)
+
+
 def main(outdir, write):
     pc = {pcl: k for k, pcl in enumerate(PAIR_CLASSES)}
     names = []
@@ -411,7 +448,29 @@ def main(outdir, write):
     for (name, La, Lb, Lc, Ld, t) in names:
         lines.append("    if (cb == %d && ck == %d) return double(np) * %d.0 + double(nq) * %d.0;"
                      % (pc[(La, Lb)], pc[(Lc, Ld)], t["prim_flop"], t["quartet_flop"]))
-    lines += ["    return 0.0;", "}", "", "}  // namespace qf", ""]
+    lines += ["    return 0.0;", "}", "",
+              "// (list, workgroups, tasks, blocks, mols, slot doubles in LDS, gradient doubles, global slots, target)",
+              "using GradFuseLaunch = void (*)(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int,"
+              " double*, LaunchTo&);"]
+    buckets = fuse_buckets()
+    for b in buckets:
+        write("fuse_%s.hip" % b["name"], fuse_source(b, pc))
+        lines.append("void launch_fuse_%s(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int,"
+                     " double*, LaunchTo&);" % b["name"])
+    lines += ["", "struct GradFuseKernel {", "    GradFuseLaunch launch;", "    bool coop;          // wave-per-quartet classes",
+              "    int global;         // doubles of a workgroup's slice of the global slot buffer (0: slots in LDS)",
+              "};", "constexpr int kGradFuseKernels = %d;" % len(buckets),
+              "inline GradFuseKernel grad_fuse_kernel(int k)", "{",
+              "    constexpr GradFuseKernel all[kGradFuseKernels] = {"]
+    lines += ["        {launch_fuse_%s, %s, %d}," % (b["name"], "true" if b["coop"] else "false",
+                                                     b["stride"] if b["glob"] else 0) for b in buckets]
+    lines += ["    };", "    return all[k];", "}", "",
+              "// the kernel that runs a class's gradient beside others (-1: none)",
+              "inline int grad_fuse_bucket(int cb, int ck)", "{", "    switch (cb * 16 + ck) {"]
+    for k, b in enumerate(buckets):
+        for c in b["classes"]:
+            lines.append("    case %d: return %d;" % (pc[c[:2]] * 16 + pc[c[2:]], k))
+    lines += ["    }", "    return -1;", "}", "", "}  // namespace qf", ""]
     write("grad_launchers.h", "\n".join(lines))
     write("grad_maps.h", "\n".join([
         "// Generated by quick_amd/codegen/gen_grad.py - do not edit.", "#pragma once", "", "namespace qf {", "",

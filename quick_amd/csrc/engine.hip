@@ -439,11 +439,12 @@ struct qf_engine {
         double seconds;      // estimate
     };
     std::vector<Fused> fused;
+    size_t grad_slots = 0;   // doubles of the global slot buffer that the gradient's shared launches need
     struct Plan {
         std::vector<std::pair<int, int>> order;   // (launch index, or ~ the index into fused; stream 0..kSide)
         double gain = 0.0;                        // seconds the forked order saves (estimate)
     };
-    Plan plan[3];                             // closed shell, open shell, gradient and one launch per class
+    Plan plan[4];                             // closed shell, open shell, gradient; one launch per class
     SideStreams* side = nullptr;              // taken at the first forked build
     Replay replay[3];                         // closed shell, open shell, gradient
     void drop_replays()
@@ -838,6 +839,19 @@ bool shares_launches(const qf_engine* e)
     return e->tile != 0 && e->nbasis <= (lmax > 1 ? 200 : 100);
 }
 
+// The plan of a build or gradient (kind 2): one launch per class where the grid
+// is capped (qf_set_persistent caps each class's) or a gradient kernel was chosen.
+const qf_engine::Plan& plan_of(const qf_engine* e, int kind)
+{
+    bool plain = e->persist > 0;
+    if (kind == 2 && !plain) {
+        plain = !e->grad_lane;
+        for (const auto& row : e->ctune)
+            for (const auto& c : row) plain = plain || c.grad >= 0;
+    }
+    return e->plan[plain ? 3 : kind];
+}
+
 // Plan of closed-shell (os 0) or open-shell (os 1) builds in which classes of
 // the same kernel bucket share a launch, its workgroups longest first.
 // Appends to e->fused and to `list`, their workgroups; slots: doubles of the
@@ -907,11 +921,50 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
     return stream_order(t);
 }
 
+// The same for gradients (water 6-31G*, host to host: 291 -> 168 us).
+qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, size_t& slots)
+{
+    std::vector<std::vector<std::pair<double, qf::FusedBlock>>> blocks(qf::kGradFuseKernels);
+    std::vector<LaunchCost> cost(qf::kGradFuseKernels);
+    std::vector<size_t> lds(qf::kGradFuseKernels, 0);
+    std::vector<std::pair<int, double>> t;
+    slots = 0;
+    for (const auto& L : e->launches) {
+        const int k = qf::grad_fuse_bucket(L.cb, L.ck);
+        if (k < 0) return e->plan[3];   // an f class: gradients are refused
+        const bool alt = L.alt_count > 0, coop = qf::grad_fuse_kernel(k).coop;
+        if (coop) lds[k] = std::max(lds[k], sizeof(double) * qf::grad_lds_doubles(L.cb, L.ck));
+        const int first = alt ? L.alt_offset : L.offset, count = alt ? L.alt_count : L.count;
+        for (int x = first; x < first + count; ++x)
+            blocks[k].push_back({cost[k].task(L, e->tasks[x], coop),
+                                 qf::FusedBlock{L.cb * 16 + L.ck + (L.fp32 ? 256 : 0), x}});
+    }
+    for (int k = 0; k < qf::kGradFuseKernels; ++k) {
+        if (blocks[k].empty()) continue;
+        std::stable_sort(blocks[k].begin(), blocks[k].end(),
+                         [](const auto& x, const auto& y) { return x.first > y.first; });
+        qf_engine::Fused f{};
+        f.kernel = k;
+        f.waves = 1;
+        f.offset = (int)list.size();
+        f.count = (int)blocks[k].size();
+        f.lds = lds[k];
+        f.gslot = slots;
+        f.seconds = cost[k].seconds();
+        slots += (size_t)qf::grad_fuse_kernel(k).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
+        for (const auto& x : blocks[k]) list.push_back(x.second);
+        t.push_back({~(int)e->fused.size(), f.seconds});
+        e->fused.push_back(f);
+    }
+    return stream_order(t);
+}
+
 // Wave tasks, tile groups and launches of one engine, per quartet class and
 // precision.  `size` stands for the number of basis functions in the rules
 // that choose launch shapes: the engine's own, or for an engine in a batch
 // that of the molecule whose build holds as much work (the precision split
-// goes by the engine's own size).  Index ranges are those of the output vectors.
+// goes by the engine's own size); shared: tile and wave-per-quartet
+// classes share launches.  Index ranges are those of the output vectors.
 int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::vector<qf::TileGroup>& groups,
                std::vector<qf_engine::Launch>& launches, qf_stats* stats, bool shared = false)
 {
@@ -1334,7 +1387,8 @@ int prepare(qf_engine* e)
     // node-program slots in global memory
     size_t gdoubles = place_slots(e->launches);
     e->fused.clear();
-    e->plan[0] = e->plan[1] = e->plan[2] = stream_order(e->launches, e->tasks);
+    e->grad_slots = 0;
+    e->plan[0] = e->plan[1] = e->plan[2] = e->plan[3] = stream_order(e->launches, e->tasks);
     if (shares_launches(e)) {
         std::vector<qf::FusedBlock> list;
         for (int os = 0; os < 2; ++os) {
@@ -1342,6 +1396,7 @@ int prepare(qf_engine* e)
             e->plan[os] = fuse_plan(e, os, list, slots);
             gdoubles = std::max(gdoubles, slots);
         }
+        e->plan[2] = grad_fuse_plan(e, list, e->grad_slots);
         QF_HIP(e->d_fused.upload(list));
     }
     if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles));
@@ -1497,7 +1552,7 @@ int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, con
 {
     Replay& r = e->replay[kind];
     const bool captured = is_capturing(s);
-    const qf_engine::Plan& plan = e->plan[e->persist > 0 ? 2 : kind];   // a capped grid caps each class's
+    const qf_engine::Plan& plan = plan_of(e, kind);
     if (!captured && !r.exec && !r.failed && !plan.order.empty() && ++r.uses > 1) {
         hipGraphNode_t last[kSide + 1] = {};
         bool ok = hipGraphCreate(&r.graph, 0) == hipSuccess;
@@ -1675,7 +1730,7 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         // one after another on s
         qf::LaunchTo to(s);
         open_build(oa, to);
-        for (const auto& o : e->plan[e->persist > 0 ? 2 : os].order) {
+        for (const auto& o : plan_of(e, os).order) {
             const int rc = o.first < 0 ? shared_launch(e->fused[~o.first], to) : class_launch(e->launches[o.first], to);
             if (rc) return rc;
         }
@@ -1947,6 +2002,7 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
             gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) *
                         std::min(std::max(L.count, L.alt_count), qf::COOP_GLOBAL_SLICES);
     }
+    gdoubles = std::max(gdoubles, e->grad_slots);
     if (gdoubles && e->d_gscratch.n < gdoubles) {
         e->replay[2].drop();   // it holds the old buffer
         QF_HIP(e->d_gscratch.resize(gdoubles));
@@ -1978,6 +2034,14 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     oa.nshell = e->nshell;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
     auto launch = [&](int li, qf::LaunchTo& q) -> int {
+        if (li < 0) {
+            const qf_engine::Fused& f = e->fused[~li];
+            qf::grad_fuse_kernel(f.kernel).launch(e->d_fused.p + f.offset, f.count, e->d_tasks.p, e->d_blocks.p, dmol,
+                                                  (int)(f.lds / sizeof(double)),
+                                                  f.lds + tile_bytes <= kGradLdsMax ? 3 * e->natom : 0,
+                                                  e->d_gscratch.p + f.gslot, q);
+            return QF_OK;
+        }
         const auto& L = e->launches[li];
         const qf::GradLaunch lane = lane_kernel(L);
         const size_t slots = lane ? 0 : (size_t)qf::grad_lds_doubles(L.cb, L.ck) * sizeof(double);

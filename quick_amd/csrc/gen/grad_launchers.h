@@ -156,4 +156,59 @@ inline double grad_class_flops(int cb, int ck, unsigned long long nq, unsigned l
     return 0.0;
 }
 
+// (list, workgroups, tasks, blocks, mols, slot doubles in LDS, gradient doubles, global slots, target)
+using GradFuseLaunch = void (*)(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fuse_grad_lane3(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fuse_grad_lane2(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fuse_grad_lane1(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fuse_grad_coop(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+void launch_fuse_grad_coop_global(const FusedBlock*, int, const Task*, const PairBlock*, const MolDesc*, int, int, double*, LaunchTo&);
+
+struct GradFuseKernel {
+    GradFuseLaunch launch;
+    bool coop;          // wave-per-quartet classes
+    int global;         // doubles of a workgroup's slice of the global slot buffer (0: slots in LDS)
+};
+constexpr int kGradFuseKernels = 5;
+inline GradFuseKernel grad_fuse_kernel(int k)
+{
+    constexpr GradFuseKernel all[kGradFuseKernels] = {
+        {launch_fuse_grad_lane3, false, 0},
+        {launch_fuse_grad_lane2, false, 0},
+        {launch_fuse_grad_lane1, false, 0},
+        {launch_fuse_grad_coop, true, 0},
+        {launch_fuse_grad_coop_global, true, 25290},
+    };
+    return all[k];
+}
+
+// the kernel that runs a class's gradient beside others (-1: none)
+inline int grad_fuse_bucket(int cb, int ck)
+{
+    switch (cb * 16 + ck) {
+    case 0: return 0;
+    case 16: return 0;
+    case 17: return 1;
+    case 32: return 1;
+    case 48: return 1;
+    case 64: return 1;
+    case 33: return 2;
+    case 34: return 2;
+    case 49: return 2;
+    case 50: return 2;
+    case 51: return 2;
+    case 65: return 2;
+    case 66: return 2;
+    case 67: return 2;
+    case 80: return 2;
+    case 81: return 2;
+    case 68: return 3;
+    case 82: return 3;
+    case 83: return 3;
+    case 84: return 4;
+    case 85: return 4;
+    }
+    return -1;
+}
+
 }  // namespace qf

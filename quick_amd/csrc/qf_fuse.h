@@ -19,7 +19,8 @@ struct FuseMember {
     using type = C;
 };
 
-constexpr int kFuseTwoTiles = 256;
+constexpr int kFuseTwoTiles = 256;   // FusedBlock::cls of a Fock launch: open shell with a second LDS tile
+constexpr int kFuseFp32 = 256;       // ... of a gradient launch: the task is of the FP32 half of its class
 
 // Tile classes; W: waves per SIMD the register budget of all of them targets.
 template <int W, bool OS, class... M>

@@ -190,6 +190,81 @@ __device__ __forceinline__ void grad_quartet(const Task& t, const PairBlock& bb,
     __syncthreads();   // the next quartet reuses the slots
 }
 
+// The workgroup's gradient, from LDS to md.grad.
+__device__ __forceinline__ void grad_flush(const MolDesc* m, QF_AS_LDS double* gt, int tile)
+{
+    __syncthreads();
+    if (tile && m) {
+        const MolDesc md = *m;
+        for (int x = threadIdx.x % WAVE; x < tile; x += WAVE)
+            if (gt[x] != 0.0) atomic_add(gptr_rw(md.grad) + x, gt[x]);
+    }
+}
+
+// One task of the wave-per-quartet gradient: sums to the workgroup's gradient
+// gt (tile doubles), or straight to md.grad (tile 0).
+template <class D, typename SP>
+__device__ __forceinline__ void grad_coop_task(const Task t, const PairBlock* __restrict__ blocks,
+                                               const MolDesc* __restrict__ mols, SP s, QF_AS_LDS double* gt, int tile,
+                                               int fp32, const QF_AS_LDS double* boys_tab)
+{
+    const int lane = threadIdx.x % WAVE;
+    const PairBlock bb = cptr(blocks)[t.bra_block];
+    const PairBlock kb = cptr(blocks)[t.ket_block];
+    const MolDesc md = cptr(mols)[bb.mol];
+    const int ns = md.nshell;
+    const auto cm = gptr(md.cutmat);
+    const auto sat = gptr(md.shell_atom);
+    const auto bperm = cptr(bb.bperm);
+    const bool in_range = lane < t.ket_count;
+    const int jl = t.ket_start + (in_range ? lane : 0);
+    const PairInfo kl = gptr(kb.info)[jl];
+    const int atC = sat[kl.sa], atD = sat[kl.sb];
+    for (int kk = t.kb; kk < t.ke; ++kk) {
+        const int i = bperm[kk];
+        const PairInfo bi = cptr(bb.info)[i];
+        const int atA = sat[bi.sa], atB = sat[bi.sb];
+        const double ytest = bi.ycut * kl.ycut;
+        double dn = fmax(4.0 * cm[bi.sa * ns + bi.sb], 4.0 * cm[kl.sa * ns + kl.sb]);
+        dn = fmax(dn, cm[bi.sa * ns + kl.sb]);
+        dn = fmax(dn, cm[bi.sa * ns + kl.sa]);
+        dn = fmax(dn, cm[bi.sb * ns + kl.sa]);
+        dn = fmax(dn, cm[bi.sb * ns + kl.sb]);
+        const bool one_atom = atA == atB && atA == atC && atA == atD;
+        // the two precision halves of a split class share boundary windows: each
+        // launch keeps its own side of md.split, as the Fock kernels do
+        const bool half = fp32 ? (ytest < md.split) : (t.all_fp64 || ytest >= md.split);
+        const bool valid = in_range && !one_atom && half && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
+                           (!t.same_block || jl <= i);
+        unsigned long long mask = __ballot(valid);
+        while (mask) {
+            const int v = __builtin_ctzll(mask);
+            mask &= mask - 1;
+            const int j = t.ket_start + v;
+            const PairInfo ki = cptr(kb.info)[j];
+            const double dnv = __shfl(dn, v, WAVE);
+            const int atCv = __shfl(atC, v, WAVE), atDv = __shfl(atD, v, WAVE);
+            double g[9];
+            grad_quartet<D>(t, bb, i, bi, kb, j, ki, dnv, md, s, boys_tab, g);
+            // lanes 0-11: A, B, C, D x y z
+            if (lane < 12) {
+                const int which = lane / 3, dir = lane % 3;
+                double val;
+                if (which < 3) {
+                    val = g[3 * which + dir];
+                } else {
+                    val = -(g[dir] + g[3 + dir] + g[6 + dir]);
+                }
+                const int at = which == 0 ? atA : which == 1 ? atB : which == 2 ? atCv : atDv;
+                if (tile)
+                    lds_add(gt + 3 * at + dir, val);
+                else
+                    atomic_add(gptr_rw(md.grad) + 3 * at + dir, val);
+            }
+        }
+    }
+}
+
 // One workgroup (one wave) per task, as fock_coop_kernel, with QUICK's
 // gradient screen in md.cutoff; fp32 = 1 for the tasks of a Fock launch that
 // holds the FP32 half of a split class (the gradient itself is FP64).  Dynamic LDS: the slots (unless they are
@@ -207,74 +282,15 @@ __global__ __launch_bounds__(D::NT) void grad_coop_kernel(const Task* __restrict
     extern __shared__ double qf_lds[];
     const auto s = coop_slots<D>(gscratch);
     QF_AS_LDS double* gt = (QF_AS_LDS double*)qf_lds + (D::GLOBAL_SLOTS ? 0 : D::LDS);
-    const int lane = threadIdx.x % WAVE;
-    for (int x = lane; x < tile; x += WAVE) gt[x] = 0.0;
+    for (int x = threadIdx.x; x < tile; x += WAVE) gt[x] = 0.0;
     __syncthreads();
     const MolDesc* md_last = nullptr;
     for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
         const Task t = cptr(tasks)[ti];
-        const PairBlock bb = cptr(blocks)[t.bra_block];
-        const PairBlock kb = cptr(blocks)[t.ket_block];
-        const MolDesc md = cptr(mols)[bb.mol];
-        md_last = mols + bb.mol;
-        const int ns = md.nshell;
-        const auto cm = gptr(md.cutmat);
-        const auto sat = gptr(md.shell_atom);
-        const auto bperm = cptr(bb.bperm);
-        const bool in_range = lane < t.ket_count;
-        const int jl = t.ket_start + (in_range ? lane : 0);
-        const PairInfo kl = gptr(kb.info)[jl];
-        const int atC = sat[kl.sa], atD = sat[kl.sb];
-        for (int kk = t.kb; kk < t.ke; ++kk) {
-            const int i = bperm[kk];
-            const PairInfo bi = cptr(bb.info)[i];
-            const int atA = sat[bi.sa], atB = sat[bi.sb];
-            const double ytest = bi.ycut * kl.ycut;
-            double dn = fmax(4.0 * cm[bi.sa * ns + bi.sb], 4.0 * cm[kl.sa * ns + kl.sb]);
-            dn = fmax(dn, cm[bi.sa * ns + kl.sb]);
-            dn = fmax(dn, cm[bi.sa * ns + kl.sa]);
-            dn = fmax(dn, cm[bi.sb * ns + kl.sa]);
-            dn = fmax(dn, cm[bi.sb * ns + kl.sb]);
-            const bool one_atom = atA == atB && atA == atC && atA == atD;
-            // the two precision halves of a split class share boundary windows: each
-            // launch keeps its own side of md.split, as the Fock kernels do
-            const bool half = fp32 ? (ytest < md.split) : (t.all_fp64 || ytest >= md.split);
-            const bool valid = in_range && !one_atom && half && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
-                               (!t.same_block || jl <= i);
-            unsigned long long mask = __ballot(valid);
-            while (mask) {
-                const int v = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                const int j = t.ket_start + v;
-                const PairInfo ki = cptr(kb.info)[j];
-                const double dnv = __shfl(dn, v, WAVE);
-                const int atCv = __shfl(atC, v, WAVE), atDv = __shfl(atD, v, WAVE);
-                double g[9];
-                grad_quartet<D>(t, bb, i, bi, kb, j, ki, dnv, md, s, QF_BOYS_LDS_PTR, g);
-                // lanes 0-11: A, B, C, D x y z
-                if (lane < 12) {
-                    const int which = lane / 3, dir = lane % 3;
-                    double val;
-                    if (which < 3) {
-                        val = g[3 * which + dir];
-                    } else {
-                        val = -(g[dir] + g[3 + dir] + g[6 + dir]);
-                    }
-                    const int at = which == 0 ? atA : which == 1 ? atB : which == 2 ? atCv : atDv;
-                    if (tile)
-                        lds_add(gt + 3 * at + dir, val);
-                    else
-                        atomic_add(gptr_rw(md.grad) + 3 * at + dir, val);
-                }
-            }
-        }
+        md_last = mols + cptr(blocks)[t.bra_block].mol;
+        grad_coop_task<D>(t, blocks, mols, s, gt, tile, fp32, QF_BOYS_LDS_PTR);
     }
-    __syncthreads();
-    if (tile && md_last) {
-        const MolDesc md = *md_last;
-        for (int x = lane; x < tile; x += WAVE)
-            if (gt[x] != 0.0) atomic_add(gptr_rw(md.grad) + x, gt[x]);
-    }
+    grad_flush(md_last, gt, tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -300,186 +316,193 @@ __global__ __launch_bounds__(D::NT) void grad_coop_kernel(const Task* __restrict
 // cutprim.
 // ---------------------------------------------------------------------------
 template <class C>
+__device__ __forceinline__ void grad_md_task(const Task t, const PairBlock* __restrict__ blocks,
+                                             const MolDesc* __restrict__ mols, QF_AS_LDS double* bra,
+                                             QF_AS_LDS double* gt, int tile, int fp32,
+                                             const QF_AS_LDS double* boys_tab)
+{
+    constexpr int nb = ncart(C::Lb), nc = ncart(C::Lc), nd = ncart(C::Ld);
+    const int lane = threadIdx.x % WAVE;
+    const auto index = gptr(C::index());
+    const PairBlock bb = cptr(blocks)[t.bra_block];
+    const PairBlock kb = cptr(blocks)[t.ket_block];
+    const MolDesc md = cptr(mols)[bb.mol];
+    const int n = md.nbasis, ns = md.nshell;
+    const auto grad = gptr_rw(md.grad);
+    const auto cm = gptr(md.cutmat);
+    const auto sat = gptr(md.shell_atom);
+    const auto P = gptr(md.P);
+    const auto Pu = cptr(md.P);
+    const auto bperm = cptr(bb.bperm);
+    const auto bp = cptr(bb.prim);     // bra data, the same in every lane: scalar loads
+    const auto kp = gptr(kb.prim);
+    const int bn = bb.n, bK = bb.K, kn = kb.n, kK = kb.K;
+    const bool in_range = lane < t.ket_count;
+    const int j = t.ket_start + (in_range ? lane : 0);
+    const PairInfo ki = gptr(kb.info)[j];
+    const int atC = sat[ki.sa], atD = sat[ki.sb];
+    const double hh = 0.5 * md.hyb;
+    double gA[3] = {0.0, 0.0, 0.0}, gC[3] = {0.0, 0.0, 0.0}, gD[3] = {0.0, 0.0, 0.0};
+    int atA = 0;
+    // density block of the ket pair (the same for every bra), scaled as C::prim takes it
+    double Dcd[nc * nd];
+#pragma unroll
+    for (int x = 0; x < nc * nd; ++x)
+        Dcd[x] = P[(ki.fa + x / nd) * n + ki.fb + x % nd] * (2.0 * kCons[C::Lc][x / nd] * kCons[C::Ld][x % nd]);
+    for (int kk0 = t.kb; kk0 < t.ke; ++kk0) {
+        const int kk = wave_uniform(kk0);
+        const int i = bperm[kk];
+        const PairInfo bi = cptr(bb.info)[i];
+        atA = sat[bi.sa];
+        const int atB = sat[bi.sb];
+        const double ytest = bi.ycut * ki.ycut;
+        double dn = fmax(4.0 * cm[bi.sa * ns + bi.sb], 4.0 * cm[ki.sa * ns + ki.sb]);
+        dn = fmax(dn, cm[bi.sa * ns + ki.sb]);
+        dn = fmax(dn, cm[bi.sa * ns + ki.sa]);
+        dn = fmax(dn, cm[bi.sb * ns + ki.sa]);
+        dn = fmax(dn, cm[bi.sb * ns + ki.sb]);
+        const bool one_atom = atA == atB && atA == atC && atA == atD;
+        // the two precision halves of a split class share boundary windows: each
+        // launch keeps its own side of md.split, as the Fock kernels do
+        const bool half = fp32 ? (ytest < md.split) : (t.all_fp64 || ytest >= md.split);
+        const bool valid = in_range && !one_atom && half && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
+                           (!t.same_block || j <= i);
+        if (!__any(valid)) continue;
+        double Dbc[nb * nc], Dbd[nb * nd];
+#pragma unroll
+        for (int x = 0; x < nb * nc; ++x)
+            Dbc[x] = P[(bi.fb + x / nc) * n + ki.fa + x % nc] * (hh * (kCons[C::Lb][x / nc] * kCons[C::Lc][x % nc]));
+#pragma unroll
+        for (int x = 0; x < nb * nd; ++x)
+            Dbd[x] = P[(bi.fb + x / nd) * n + ki.fb + x % nd] * (hh * (kCons[C::Lb][x / nd] * kCons[C::Ld][x % nd]));
+        // QUICK's CPU gradient evaluates FmT with NABCD + 2 (eri_grad.fh:104-106)
+        const int maxm = bi.qfs + ki.qfs + 2;
+        double g[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) g[k] = 0.0;
+        for (int ip0 = t.pb; ip0 < t.pe; ++ip0) {
+            const int ip = wave_uniform(ip0);
+            const double cb = dn * bp[(PF_CUT * bK + ip) * bn + i];
+            if (!__any(valid && cb * kp[(PF_CUT * kK + t.qb) * kn + j] > md.primlim)) break;
+            const double zb = bp[(PF_ZETA * bK + ip) * bn + i];
+            const double hb = bp[(PF_OOZ2 * bK + ip) * bn + i];
+            const double ab = bp[(PF_ALPHA * bK + ip) * bn + i];
+            const double Pb[3] = {bp[(PF_PX * bK + ip) * bn + i], bp[(PF_PY * bK + ip) * bn + i],
+                                  bp[(PF_PZ * bK + ip) * bn + i]};
+            const double Kb = bp[(PF_KC * bK + ip) * bn + i];
+            const double wa = 2.0 * hb * ab, wb = 2.0 * hb * (zb - ab);   // alpha/p, beta/p
+            if constexpr (C::NE > 0) {
+                __syncthreads();   // the previous primitive's table has been read
+                const int dir = lane % 3;
+                const double PA = dir == 0 ? Pb[0] - bi.A[0] : dir == 1 ? Pb[1] - bi.A[1] : Pb[2] - bi.A[2];
+                const double AB = dir == 0 ? bi.AB[0] : dir == 1 ? bi.AB[1] : bi.AB[2];
+                if (lane < 3) C::bra1d(PA, PA + AB, hb, -wb, wa, bra + lane * C::N1);
+                __syncthreads();
+#pragma unroll
+                for (int x0 = 0; x0 < C::NE; x0 += WAVE) {
+                    const int x = x0 + lane;
+                    const unsigned id = index[x < C::NE ? x : 0];
+                    const double v = bra[id & 255] * bra[C::N1 + ((id >> 8) & 255)] * bra[2 * C::N1 + (id >> 16)];
+                    if (x < C::NE) bra[3 * C::N1 + x] = v;
+                }
+                __syncthreads();
+            }
+            const double mu2 = -2.0 * wa * (zb - ab);    // -2 alpha beta / p
+            for (int jp0 = t.qb; jp0 < t.qe; ++jp0) {
+                const int jp = wave_uniform(jp0);
+                const size_t ko = (size_t)jp * kn + j, kf = (size_t)kK * kn;
+                const bool act = valid && cb * kp[PF_CUT * kf + ko] > md.primlim;
+                if (!__any(act)) break;
+                if (act) {
+                    const double zk = kp[PF_ZETA * kf + ko], hk = kp[PF_OOZ2 * kf + ko];
+                    const double gk = kp[PF_ALPHA * kf + ko], Kk = kp[PF_KC * kf + ko];
+                    const double Qk[3] = {kp[PF_PX * kf + ko], kp[PF_PY * kf + ko], kp[PF_PZ * kf + ko]};
+                    const double QC[3] = {Qk[0] - ki.A[0], Qk[1] - ki.A[1], Qk[2] - ki.A[2]};
+                    const double QD[3] = {QC[0] + ki.AB[0], QC[1] + ki.AB[1], QC[2] + ki.AB[2]};
+                    const double PQ[3] = {Pb[0] - Qk[0], Pb[1] - Qk[1], Pb[2] - Qk[2]};
+                    const double rs = qf_rsqrt(zb + zk);
+                    const double al = zb * zk * (rs * rs);
+                    const double rpq = PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2];
+                    double F[C::L + 1];
+                    boys_quick<C::L, const QF_AS_LDS double*, 4>(rpq * al, maxm, F, boys_tab);
+                    const double wc = 2.0 * hk * gk, wd = 2.0 * hk * (zk - gk);   // gamma/q, delta/q
+                    double W, gP[3], gR[3], gS[3];
+                    // the product table and the a-b block are the same for every ket
+                    // primitive: hoisted, they would be hundreds of registers
+                    int eo = 3 * C::N1, po = bi.fa * n + bi.fb;
+                    QF_OPAQUE(eo);
+                    QF_OPAQUE_S(po);
+                    C::prim(F, Kb * Kk * rs, -2.0 * al, PQ, QC, QD, hk, -wd, wc, bra + eo, Pu + po, P, n, bi.fa * n + ki.fa, bi.fa * n + ki.fb, Dcd, Dbc, Dbd, W,
+                            gP, gR, gS);
+                    const double nu2 = -2.0 * wc * (zk - gk);
+#pragma unroll
+                    for (int x = 0; x < 3; ++x) {
+                        const double r = fma(mu2 * bi.AB[x], W, gR[x]), s = fma(nu2 * ki.AB[x], W, gS[x]);
+                        g[x] += fma(wa, gP[x], r);
+                        g[3 + x] += fma(wb, gP[x], -r);
+                        g[6 + x] += fma(-wc, gP[x], s);
+                    }
+                }
+            }
+        }
+        const double sdeg = 0.25 * (bi.qa != bi.qb ? 2.0 : 1.0) * (ki.qa != ki.qb ? 2.0 : 1.0) *
+                            (bi.id != ki.id ? 2.0 : 1.0);
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            const double a = sdeg * g[x], bs = sdeg * g[3 + x], c = sdeg * g[6 + x];
+            gA[x] += a;
+            gC[x] += c;
+            gD[x] -= a + bs + c;
+            const double b = wave_sum_all_active(bs);
+            if (lane == 0) {
+                if (tile)
+                    lds_add(gt + 3 * atB + x, b);
+                else if (b != 0.0)
+                    atomic_add(grad + 3 * atB + x, b);
+            }
+        }
+    }
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        const double a = wave_sum_all_active(gA[x]);
+        if (tile) {
+            if (lane == 0) lds_add(gt + 3 * atA + x, a);
+            if (in_range) {
+                lds_add(gt + 3 * atC + x, gC[x]);
+                lds_add(gt + 3 * atD + x, gD[x]);
+            }
+        } else {
+            if (lane == 0 && a != 0.0) atomic_add(grad + 3 * atA + x, a);
+            if (in_range && gC[x] != 0.0) atomic_add(grad + 3 * atC + x, gC[x]);
+            if (in_range && gD[x] != 0.0) atomic_add(grad + 3 * atD + x, gD[x]);
+        }
+    }
+}
+
+// doubles of grad_md_task's bra: 1D coefficients of x, y, z of the bra primitive,
+// then the products C::prim reads
+template <class C>
+constexpr int kGradBra = 3 * C::N1 + (C::NE > 0 ? C::NE : 1);
+
+template <class C>
 __global__ __attribute__((amdgpu_flat_work_group_size(WAVE, WAVE), amdgpu_waves_per_eu(C::MIN_WAVES)))
 void grad_md_kernel(const Task* __restrict__ tasks, int ntasks, const PairBlock* __restrict__ blocks,
                     const MolDesc* __restrict__ mols, int tile, int fp32)
 {
-    constexpr int nb = ncart(C::Lb), nc = ncart(C::Lc), nd = ncart(C::Ld);
     QF_BOYS_LDS_DECL;
     QF_BOYS_LDS_FILL();
-    // bra primitive: 1D coefficients of x, y, z, then the products C::prim reads
-    __shared__ double qf_bra[3 * C::N1 + (C::NE > 0 ? C::NE : 1)];
-    QF_AS_LDS double* bra = (QF_AS_LDS double*)qf_bra;
+    __shared__ double qf_bra[kGradBra<C>];
     extern __shared__ double qf_lds[];
     QF_AS_LDS double* gt = (QF_AS_LDS double*)qf_lds;
-    const int lane = threadIdx.x % WAVE;
-    for (int x = lane; x < tile; x += WAVE) gt[x] = 0.0;
+    for (int x = threadIdx.x; x < tile; x += WAVE) gt[x] = 0.0;
     __syncthreads();
-    const auto index = gptr(C::index());
     const MolDesc* md_last = nullptr;
     for (int ti = blockIdx.x; ti < ntasks; ti += gridDim.x) {
         const Task t = cptr(tasks)[ti];
-        const PairBlock bb = cptr(blocks)[t.bra_block];
-        const PairBlock kb = cptr(blocks)[t.ket_block];
-        const MolDesc md = cptr(mols)[bb.mol];
-        md_last = mols + bb.mol;
-        const int n = md.nbasis, ns = md.nshell;
-        const auto grad = gptr_rw(md.grad);
-        const auto cm = gptr(md.cutmat);
-        const auto sat = gptr(md.shell_atom);
-        const auto P = gptr(md.P);
-        const auto Pu = cptr(md.P);
-        const auto bperm = cptr(bb.bperm);
-        const auto bp = cptr(bb.prim);     // bra data, the same in every lane: scalar loads
-        const auto kp = gptr(kb.prim);
-        const int bn = bb.n, bK = bb.K, kn = kb.n, kK = kb.K;
-        const bool in_range = lane < t.ket_count;
-        const int j = t.ket_start + (in_range ? lane : 0);
-        const PairInfo ki = gptr(kb.info)[j];
-        const int atC = sat[ki.sa], atD = sat[ki.sb];
-        const double hh = 0.5 * md.hyb;
-        double gA[3] = {0.0, 0.0, 0.0}, gC[3] = {0.0, 0.0, 0.0}, gD[3] = {0.0, 0.0, 0.0};
-        int atA = 0;
-        // density block of the ket pair (the same for every bra), scaled as C::prim takes it
-        double Dcd[nc * nd];
-#pragma unroll
-        for (int x = 0; x < nc * nd; ++x)
-            Dcd[x] = P[(ki.fa + x / nd) * n + ki.fb + x % nd] * (2.0 * kCons[C::Lc][x / nd] * kCons[C::Ld][x % nd]);
-        for (int kk0 = t.kb; kk0 < t.ke; ++kk0) {
-            const int kk = wave_uniform(kk0);
-            const int i = bperm[kk];
-            const PairInfo bi = cptr(bb.info)[i];
-            atA = sat[bi.sa];
-            const int atB = sat[bi.sb];
-            const double ytest = bi.ycut * ki.ycut;
-            double dn = fmax(4.0 * cm[bi.sa * ns + bi.sb], 4.0 * cm[ki.sa * ns + ki.sb]);
-            dn = fmax(dn, cm[bi.sa * ns + ki.sb]);
-            dn = fmax(dn, cm[bi.sa * ns + ki.sa]);
-            dn = fmax(dn, cm[bi.sb * ns + ki.sa]);
-            dn = fmax(dn, cm[bi.sb * ns + ki.sb]);
-            const bool one_atom = atA == atB && atA == atC && atA == atD;
-            // the two precision halves of a split class share boundary windows: each
-            // launch keeps its own side of md.split, as the Fock kernels do
-            const bool half = fp32 ? (ytest < md.split) : (t.all_fp64 || ytest >= md.split);
-            const bool valid = in_range && !one_atom && half && (ytest > md.cutoff) && (ytest * dn > md.cutoff) &&
-                               (!t.same_block || j <= i);
-            if (!__any(valid)) continue;
-            double Dbc[nb * nc], Dbd[nb * nd];
-#pragma unroll
-            for (int x = 0; x < nb * nc; ++x)
-                Dbc[x] = P[(bi.fb + x / nc) * n + ki.fa + x % nc] * (hh * (kCons[C::Lb][x / nc] * kCons[C::Lc][x % nc]));
-#pragma unroll
-            for (int x = 0; x < nb * nd; ++x)
-                Dbd[x] = P[(bi.fb + x / nd) * n + ki.fb + x % nd] * (hh * (kCons[C::Lb][x / nd] * kCons[C::Ld][x % nd]));
-            // QUICK's CPU gradient evaluates FmT with NABCD + 2 (eri_grad.fh:104-106)
-            const int maxm = bi.qfs + ki.qfs + 2;
-            double g[9];
-#pragma unroll
-            for (int k = 0; k < 9; ++k) g[k] = 0.0;
-            for (int ip0 = t.pb; ip0 < t.pe; ++ip0) {
-                const int ip = wave_uniform(ip0);
-                const double cb = dn * bp[(PF_CUT * bK + ip) * bn + i];
-                if (!__any(valid && cb * kp[(PF_CUT * kK + t.qb) * kn + j] > md.primlim)) break;
-                const double zb = bp[(PF_ZETA * bK + ip) * bn + i];
-                const double hb = bp[(PF_OOZ2 * bK + ip) * bn + i];
-                const double ab = bp[(PF_ALPHA * bK + ip) * bn + i];
-                const double Pb[3] = {bp[(PF_PX * bK + ip) * bn + i], bp[(PF_PY * bK + ip) * bn + i],
-                                      bp[(PF_PZ * bK + ip) * bn + i]};
-                const double Kb = bp[(PF_KC * bK + ip) * bn + i];
-                const double wa = 2.0 * hb * ab, wb = 2.0 * hb * (zb - ab);   // alpha/p, beta/p
-                if constexpr (C::NE > 0) {
-                    __syncthreads();   // the previous primitive's table has been read
-                    const int dir = lane % 3;
-                    const double PA = dir == 0 ? Pb[0] - bi.A[0] : dir == 1 ? Pb[1] - bi.A[1] : Pb[2] - bi.A[2];
-                    const double AB = dir == 0 ? bi.AB[0] : dir == 1 ? bi.AB[1] : bi.AB[2];
-                    if (lane < 3) C::bra1d(PA, PA + AB, hb, -wb, wa, bra + lane * C::N1);
-                    __syncthreads();
-#pragma unroll
-                    for (int x0 = 0; x0 < C::NE; x0 += WAVE) {
-                        const int x = x0 + lane;
-                        const unsigned id = index[x < C::NE ? x : 0];
-                        const double v = bra[id & 255] * bra[C::N1 + ((id >> 8) & 255)] * bra[2 * C::N1 + (id >> 16)];
-                        if (x < C::NE) bra[3 * C::N1 + x] = v;
-                    }
-                    __syncthreads();
-                }
-                const double mu2 = -2.0 * wa * (zb - ab);    // -2 alpha beta / p
-                for (int jp0 = t.qb; jp0 < t.qe; ++jp0) {
-                    const int jp = wave_uniform(jp0);
-                    const size_t ko = (size_t)jp * kn + j, kf = (size_t)kK * kn;
-                    const bool act = valid && cb * kp[PF_CUT * kf + ko] > md.primlim;
-                    if (!__any(act)) break;
-                    if (act) {
-                        const double zk = kp[PF_ZETA * kf + ko], hk = kp[PF_OOZ2 * kf + ko];
-                        const double gk = kp[PF_ALPHA * kf + ko], Kk = kp[PF_KC * kf + ko];
-                        const double Qk[3] = {kp[PF_PX * kf + ko], kp[PF_PY * kf + ko], kp[PF_PZ * kf + ko]};
-                        const double QC[3] = {Qk[0] - ki.A[0], Qk[1] - ki.A[1], Qk[2] - ki.A[2]};
-                        const double QD[3] = {QC[0] + ki.AB[0], QC[1] + ki.AB[1], QC[2] + ki.AB[2]};
-                        const double PQ[3] = {Pb[0] - Qk[0], Pb[1] - Qk[1], Pb[2] - Qk[2]};
-                        const double rs = qf_rsqrt(zb + zk);
-                        const double al = zb * zk * (rs * rs);
-                        const double rpq = PQ[0] * PQ[0] + PQ[1] * PQ[1] + PQ[2] * PQ[2];
-                        double F[C::L + 1];
-                        boys_quick<C::L, const QF_AS_LDS double*, 4>(rpq * al, maxm, F, QF_BOYS_LDS_PTR);
-                        const double wc = 2.0 * hk * gk, wd = 2.0 * hk * (zk - gk);   // gamma/q, delta/q
-                        double W, gP[3], gR[3], gS[3];
-                        // the product table and the a-b block are the same for every ket
-                        // primitive: hoisted, they would be hundreds of registers
-                        int eo = 3 * C::N1, po = bi.fa * n + bi.fb;
-                        QF_OPAQUE(eo);
-                        QF_OPAQUE_S(po);
-                        C::prim(F, Kb * Kk * rs, -2.0 * al, PQ, QC, QD, hk, -wd, wc, bra + eo, Pu + po, P, n, bi.fa * n + ki.fa, bi.fa * n + ki.fb, Dcd, Dbc, Dbd, W,
-                                gP, gR, gS);
-                        const double nu2 = -2.0 * wc * (zk - gk);
-#pragma unroll
-                        for (int x = 0; x < 3; ++x) {
-                            const double r = fma(mu2 * bi.AB[x], W, gR[x]), s = fma(nu2 * ki.AB[x], W, gS[x]);
-                            g[x] += fma(wa, gP[x], r);
-                            g[3 + x] += fma(wb, gP[x], -r);
-                            g[6 + x] += fma(-wc, gP[x], s);
-                        }
-                    }
-                }
-            }
-            const double sdeg = 0.25 * (bi.qa != bi.qb ? 2.0 : 1.0) * (ki.qa != ki.qb ? 2.0 : 1.0) *
-                                (bi.id != ki.id ? 2.0 : 1.0);
-#pragma unroll
-            for (int x = 0; x < 3; ++x) {
-                const double a = sdeg * g[x], bs = sdeg * g[3 + x], c = sdeg * g[6 + x];
-                gA[x] += a;
-                gC[x] += c;
-                gD[x] -= a + bs + c;
-                const double b = wave_sum_all_active(bs);
-                if (lane == 0) {
-                    if (tile)
-                        lds_add(gt + 3 * atB + x, b);
-                    else if (b != 0.0)
-                        atomic_add(grad + 3 * atB + x, b);
-                }
-            }
-        }
-#pragma unroll
-        for (int x = 0; x < 3; ++x) {
-            const double a = wave_sum_all_active(gA[x]);
-            if (tile) {
-                if (lane == 0) lds_add(gt + 3 * atA + x, a);
-                if (in_range) {
-                    lds_add(gt + 3 * atC + x, gC[x]);
-                    lds_add(gt + 3 * atD + x, gD[x]);
-                }
-            } else {
-                if (lane == 0 && a != 0.0) atomic_add(grad + 3 * atA + x, a);
-                if (in_range && gC[x] != 0.0) atomic_add(grad + 3 * atC + x, gC[x]);
-                if (in_range && gD[x] != 0.0) atomic_add(grad + 3 * atD + x, gD[x]);
-            }
-        }
+        md_last = mols + cptr(blocks)[t.bra_block].mol;
+        grad_md_task<C>(t, blocks, mols, (QF_AS_LDS double*)qf_bra, gt, tile, fp32, QF_BOYS_LDS_PTR);
     }
-    __syncthreads();
-    if (tile && md_last) {
-        const MolDesc md = *md_last;
-        for (int x = lane; x < tile; x += WAVE)
-            if (gt[x] != 0.0) atomic_add(gptr_rw(md.grad) + x, gt[x]);
-    }
+    grad_flush(md_last, gt, tile);
 }
 
 }  // namespace qf

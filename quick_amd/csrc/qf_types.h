@@ -85,7 +85,7 @@ struct TileGroup {
 // A workgroup of a launch that holds several classes: the group (tile classes)
 // or task (wave-per-quartet classes) it runs.
 struct FusedBlock {
-    int cls;     // class: bra pair class * 16 + ket pair class; + 256: open shell with a second LDS tile
+    int cls;     // class: bra pair class * 16 + ket pair class, and a flag of the kernel (+ 256)
     int index;   // into the groups or tasks
 };
 

@@ -9,7 +9,7 @@ import pytest
 
 from quick_amd import basis as B
 from quick_amd import molecules as M
-from quick_amd.codegen import gen_eri
+from quick_amd.codegen import gen_eri, gen_grad
 from quick_amd.engine import FockEngine
 
 TOL = 2e-11
@@ -59,4 +59,35 @@ def test_shared_launches(mol, basis, precision):
         assert np.abs(G - one).max() < TOL * max(1.0, np.abs(one).max())
         assert np.abs(Ga - two[0]).max() < TOL * max(1.0, np.abs(two[0]).max())
         assert np.abs(Gb - two[1]).max() < TOL * max(1.0, np.abs(two[1]).max())
+    eng.close()
+
+
+def test_every_gradient_class_has_one_place():
+    buckets = gen_grad.fuse_buckets()
+    cls = [c for b in buckets for c in b["classes"]]
+    assert len(set(cls)) == len(cls) and set(cls) == set(gen_grad.grad_classes())
+    for b in buckets:
+        for c in b["classes"]:
+            assert b["coop"] != gen_grad.has_lane_grad(*c)
+            t = gen_grad.grad_tables(*c)
+            assert not b["coop"] or (t["glob"] == b["glob"] and t["total"] <= b["stride"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mol, basis", [("water", "STO-3G"), ("water", "6-31G*"), ("ethane", "6-31G*"),
+                                        ("alkane4", "6-31G*"), ("waters8", "6-31G*")])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_shared_gradient_launches(mol, basis, precision):
+    m = {"water": M.water, "ethane": lambda: M.alkane(2), "alkane4": lambda: M.alkane(4),
+         "waters8": lambda: M.water_cluster(8)}[mol]()
+    bs = B.build_basis(m, basis)
+    P = _density(bs.nbasis, np.random.default_rng(bs.nbasis), 0.3)
+    eng = FockEngine(bs, cutoff=1e-11, precision=precision)
+    shared = [eng.eri_grad(P) for _ in range(3)]
+    eng.set_timing(True)
+    one = eng.eri_grad(P)
+    eng.set_timing(False)
+    # as above, with the contributions of up to 1e6 quartets to an atom
+    for g in shared:
+        assert np.abs(g - one).max() < 50 * TOL * max(1.0, np.abs(one).max())
     eng.close()
