@@ -885,12 +885,19 @@ size_t place_slots(std::vector<qf_engine::Launch>& launches)
 // whole launches reach.
 struct LaunchCost {
     double all = 0.0, longest = 0.0;
-    double task(const qf_engine::Launch& L, const qf::Task& k, bool wave)
+    double quartet = 0.0, prim = 0.0;   // FLOPs of the launch that is being added
+    bool wave = false;                  // ... and whether it runs a quartet per wave
+    void launch(const qf_engine::Launch& L, bool per_wave)
     {
-        const int bras = k.ke - k.kb;
-        const double one = qf::class_flops(L.cb, L.ck, 1, (unsigned long long)(k.pe - k.pb) * (k.qe - k.qb));
-        const double t = one * bras * (wave ? k.ket_count / 1.3e9 : 1 / 0.2e9);
-        all += one * bras * k.ket_count / (wave ? 1.2e12 : 6e12);
+        quartet = qf::class_flops(L.cb, L.ck, 1, 0);
+        prim = qf::class_flops(L.cb, L.ck, 0, 1);
+        wave = per_wave;
+    }
+    double task(const qf::Task& k)
+    {
+        const double one = (quartet + prim * ((k.pe - k.pb) * (k.qe - k.qb))) * (k.ke - k.kb);
+        const double t = one * (wave ? k.ket_count / 1.3e9 : 1 / 0.2e9);
+        all += one * k.ket_count * (wave ? 1 / 1.2e12 : 1 / 6e12);
         longest = std::max(longest, t);
         return t;
     }
@@ -924,7 +931,8 @@ qf_engine::Plan stream_order(const std::vector<qf_engine::Launch>& launches, con
     for (int l = 0; l < (int)launches.size(); ++l) {
         const auto& L = launches[l];
         LaunchCost c;
-        for (int x = L.offset; x < L.offset + L.count; ++x) c.task(L, tasks[x], L.tile == 2);
+        c.launch(L, L.tile == 2);
+        for (int x = L.offset; x < L.offset + L.count; ++x) c.task(tasks[x]);
         t.push_back({l, c.seconds()});
     }
     return stream_order(t);
@@ -961,6 +969,30 @@ const qf_engine::Plan& plan_of(const qf_engine* e, int kind)
     return e->plan[plain ? 3 : kind];
 }
 
+// Workgroups of a shared launch and their estimated seconds.
+struct FusedList {
+    std::vector<qf::FusedBlock> blocks;
+    std::vector<unsigned short> key;   // exponent and two mantissa bits of the time: steps of at most 25 %
+    void add(double t, int cls, int index)
+    {
+        uint64_t u;
+        std::memcpy(&u, &t, sizeof(u));
+        blocks.push_back(qf::FusedBlock{cls, index});
+        key.push_back((unsigned short)((u >> 50) & 8191));
+    }
+    // appends them to `out`, longest first (a counting sort: a comparison sort of
+    // the 30000 workgroups of a molecule would take longer than its build)
+    void append(std::vector<qf::FusedBlock>& out) const
+    {
+        std::vector<int> at(8193, 0);
+        for (unsigned short k : key) ++at[8192 - k];
+        for (int k = 1; k <= 8192; ++k) at[k] += at[k - 1];
+        const size_t base = out.size();
+        out.resize(base + blocks.size());
+        for (size_t x = blocks.size(); x-- > 0;) out[base + --at[8192 - key[x]]] = blocks[x];
+    }
+};
+
 // Plan of closed-shell (os 0) or open-shell (os 1) builds in which classes of
 // the same kernel bucket share a launch, its workgroups longest first.
 // Appends to e->fused and to `list`, their workgroups; slots: doubles of the
@@ -968,8 +1000,7 @@ const qf_engine::Plan& plan_of(const qf_engine* e, int kind)
 qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& list, size_t& slots)
 {
     struct Group {
-        std::vector<std::pair<double, qf::FusedBlock>> blocks;
-        std::vector<int> members;
+        FusedList list;
         LaunchCost cost;
         size_t lds = 0;
     };
@@ -986,44 +1017,39 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
         const int first = alt ? L.alt_offset : L.offset, count = alt ? L.alt_count : L.count;
         Group* g = kernel < 0 ? nullptr : &groups[{kernel, coop ? 1 : L.waves}];
         LaunchCost& c = g ? g->cost : own;
+        c.launch(L, coop);
         if (g && !coop) {
             const bool two = os && L.lds_os;
             g->lds = std::max(g->lds, two ? L.lds_os : L.lds);
             for (int x = L.goffset; x < L.goffset + L.gcount; ++x) {
                 const auto& tg = e->groups[x];
-                std::vector<double> wave(L.waves, 0.0);
+                double wave[4] = {};
                 for (int k = tg.task_begin; k < tg.task_end; ++k)
-                    wave[(k - tg.task_begin) % L.waves] += c.task(L, e->tasks[k], false);
-                g->blocks.push_back({*std::max_element(wave.begin(), wave.end()),
-                                     qf::FusedBlock{id + (two ? 256 : 0), x}});
+                    wave[(k - tg.task_begin) % L.waves] += c.task(e->tasks[k]);
+                g->list.add(*std::max_element(wave, wave + 4), id + (two ? 256 : 0), x);
             }
         } else {
             if (g) g->lds = std::max(g->lds, sizeof(double) * qf::coop_lds_doubles(L.cb, L.ck));
             for (int x = first; x < first + count; ++x) {
-                const double s = c.task(L, e->tasks[x], coop);
-                if (g) g->blocks.push_back({s, qf::FusedBlock{id, x}});
+                const double s = c.task(e->tasks[x]);
+                if (g) g->list.add(s, id, x);
             }
         }
-        if (g)
-            g->members.push_back(l);
-        else
-            t.push_back({l, own.seconds()});
+        if (!g) t.push_back({l, own.seconds()});
     }
     slots = 0;
     for (auto& kv : groups) {
         Group& g = kv.second;
-        std::stable_sort(g.blocks.begin(), g.blocks.end(),
-                         [](const auto& x, const auto& y) { return x.first > y.first; });
         qf_engine::Fused f{};
         f.kernel = kv.first.first;
         f.waves = kv.first.second;
         f.offset = (int)list.size();
-        f.count = (int)g.blocks.size();
+        f.count = (int)g.list.blocks.size();
         f.lds = g.lds;
         f.gslot = slots;
         f.seconds = g.cost.seconds();
         slots += (size_t)qf::fuse_kernel(f.kernel).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
-        for (const auto& x : g.blocks) list.push_back(x.second);
+        g.list.append(list);
         t.push_back({~(int)e->fused.size(), f.seconds});
         e->fused.push_back(f);
     }
@@ -1033,7 +1059,7 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
 // The same for gradients (water 6-31G*, host to host: 291 -> 168 us).
 qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, size_t& slots)
 {
-    std::vector<std::vector<std::pair<double, qf::FusedBlock>>> blocks(qf::kGradFuseKernels);
+    std::vector<FusedList> lists(qf::kGradFuseKernels);
     std::vector<LaunchCost> cost(qf::kGradFuseKernels);
     std::vector<size_t> lds(qf::kGradFuseKernels, 0);
     std::vector<std::pair<int, double>> t;
@@ -1044,24 +1070,22 @@ qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, 
         const bool alt = L.alt_count > 0, coop = qf::grad_fuse_kernel(k).coop;
         if (coop) lds[k] = std::max(lds[k], sizeof(double) * qf::grad_lds_doubles(L.cb, L.ck));
         const int first = alt ? L.alt_offset : L.offset, count = alt ? L.alt_count : L.count;
+        cost[k].launch(L, coop);
         for (int x = first; x < first + count; ++x)
-            blocks[k].push_back({cost[k].task(L, e->tasks[x], coop),
-                                 qf::FusedBlock{L.cb * 16 + L.ck + (L.fp32 ? 256 : 0), x}});
+            lists[k].add(cost[k].task(e->tasks[x]), L.cb * 16 + L.ck + (L.fp32 ? 256 : 0), x);
     }
     for (int k = 0; k < qf::kGradFuseKernels; ++k) {
-        if (blocks[k].empty()) continue;
-        std::stable_sort(blocks[k].begin(), blocks[k].end(),
-                         [](const auto& x, const auto& y) { return x.first > y.first; });
+        if (lists[k].blocks.empty()) continue;
         qf_engine::Fused f{};
         f.kernel = k;
         f.waves = 1;
         f.offset = (int)list.size();
-        f.count = (int)blocks[k].size();
+        f.count = (int)lists[k].blocks.size();
         f.lds = lds[k];
         f.gslot = slots;
         f.seconds = cost[k].seconds();
         slots += (size_t)qf::grad_fuse_kernel(k).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
-        for (const auto& x : blocks[k]) list.push_back(x.second);
+        lists[k].append(list);
         t.push_back({~(int)e->fused.size(), f.seconds});
         e->fused.push_back(f);
     }
