@@ -232,7 +232,7 @@ class FockEngine:
         L.check(self.lib.qf_set_tuning(self.h, int(replicas), 1 if shuffle else 0), "qf_set_tuning")
 
     def set_tile(self, enable=True, waves=4, tasks_per_group=0, lds_bytes=64 * 1024):
-        """LDS-tile digestion on/off; tasks_per_group 0: 2 up to 200 functions, 4 up to 400, 16 above."""
+        """LDS-tile digestion on/off; tasks_per_group 0: 1 or 2 up to 256 functions, 4 up to 400, 16 above."""
         L.check(self.lib.qf_set_tile(self.h, 1 if enable else 0, int(waves), int(tasks_per_group), int(lds_bytes)),
                 "qf_set_tile")
 
