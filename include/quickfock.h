@@ -234,10 +234,10 @@ int qf_set_tuning(qf_engine *e, int replicas, int shuffle);
  * enable = 1 accumulates J_ab and all exchange terms of a bra chunk in a
  * workgroup-shared tile and adds it to G once, instead of one FP64 atomic
  * per quartet.  waves: waves per workgroup (1..4); tasks_per_group: tasks
- * one workgroup takes (0, the default: 2 up to 200 basis functions, 4 up to 400, 16
- * above); lds_bytes: tile budget (1 KiB..64 KiB).  Classes
+ * one workgroup takes (0, the default: 1 or 2 up to 256 basis functions, 4 up to
+ * 400, 16 above); lds_bytes: tile budget (1 KiB..64 KiB).  Classes
  * whose tile does not fit fall back to direct atomics.  With enable = 1 the
- * d-heavy classes (La+Lb+Lc+Ld >= 6; >= 5 up to 128 basis functions, >= 4 up to 48)
+ * d-heavy classes (La+Lb+Lc+Ld >= 6; >= 4 up to 32 basis functions)
  * default to the wave-per-quartet kernel;
  * enable = 0 runs every class without a qf_set_class_tuning entry on the
  * per-lane direct-atomic kernels. */
@@ -259,8 +259,8 @@ int qf_set_persistent(qf_engine *e, int max_workgroups);
 /* Primitive pieces (no QUICK counterpart: a launch-shape choice).  Each task
  * sums at most `piece` bra and `piece` ket primitive pairs of its quartets, so
  * the most contracted quartets of a small molecule are spread over several
- * waves; the pieces add up to the same Fock matrix.  piece = 0: automatic (1
- * up to 48 basis functions, 2 up to 96, 3 up to 160, 4 up to 256, 6 up to 400, 12 above); piece < 0:
+ * waves; the pieces add up to the same Fock matrix.  piece = 0: automatic,
+ * chosen by the number of basis functions, 1 to 4 up to 128, 4 or 6 up to 400, 12 above; piece < 0:
  * never split. */
 int qf_set_prim_split(qf_engine *e, int piece);
 /* Per-class primitive piece size (class indices as qf_set_class_tuning):

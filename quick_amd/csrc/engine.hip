@@ -511,7 +511,7 @@ struct qf_engine {
     int shuffle = 1;         // permute tasks inside a launch (decorrelates atomic targets)
     int tile = 1;            // accumulate exchange terms in LDS tiles (fock_tile_kernel)
     int tile_waves = 4;      // max waves per tile workgroup
-    int tile_tasks = 0;      // max tasks per tile workgroup (0: 2 up to 200 functions, 4 up to 400, 16 above)
+    int tile_tasks = 0;      // max tasks per tile workgroup (0: 1 or 2 up to 256 functions, 4 up to 400, 16 above)
     int lds_budget = 64 * 1024;
     int persist = 0;         // grid cap of the class launches (0: one workgroup per task / group)
     int prim_piece = 0;      // primitive pairs per task piece: 0 auto, < 0 never split
@@ -1201,7 +1201,7 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // wave-per-quartet kernel (FP64 launches of classes that have one)
                 // wave-per-quartet kernel: where the class tuning asks for it, and by
                 // default (unless qf_set_tile turned the shared-memory kernels off)
-                // for the d-heavy classes (La+Lb+Lc+Ld >= 6; >= 5 up to 128 functions and >= 4 up to 48,
+                // for the d-heavy classes (La+Lb+Lc+Ld >= 6; in launches of one class >= 5 up to 128 functions and >= 4 up to 48,
                 // where few waves run and latency decides), whose per-lane
                 // kernels spill several KB per lane: one such quartet alone on a
                 // lane costs milliseconds, which dominates the build of a small
