@@ -90,6 +90,66 @@ def test_open_shell_f_shells_match_oracle(name, basis):
         assert ea <= FOCK_TOL and eb <= FOCK_TOL
 
 
+def _replays_match(eng, Pa, Pb, Ga_ref, Gb_ref):
+    """The first build of an engine is issued launch by launch, the later ones
+    are replayed from a graph; the last has the spins exchanged."""
+    for k in range(4):
+        Ga, Gb = eng.fock2e_os(*((Pa, Pb) if k < 3 else (Pb, Pa)))
+        if k == 3:
+            Ga, Gb = Gb, Ga
+        ea, eb = float(np.max(np.abs(Ga - Ga_ref))), float(np.max(np.abs(Gb - Gb_ref)))
+        assert ea <= FOCK_TOL and eb <= FOCK_TOL, (k, ea, eb)
+
+
+@pytest.mark.parametrize("mode", ["register", "direct", "coop", "two-pass", "two-pass-direct"])
+def test_open_shell_replays_match_oracle(mode):
+    announce(f"open-shell replays water3+ 6-31G* {mode}")
+    mol = molecule("water3+")
+    orc = oracle_for(mol, "6-31G*")
+    Pa, Pb = seeded_spin_densities_for(orc, mol, 2)
+    Ga_ref, Gb_ref, _ = orc.fock2e_os(Pa, Pb, cutoff=1e-12, threads=4)
+    eng = _engine(product_basis(mol, "6-31G*"), cutoff=1e-12)
+    _set_mode(eng, mode)
+    _replays_match(eng, Pa, Pb, Ga_ref, Gb_ref)
+
+
+@pytest.mark.parametrize("form", [0, 1])
+def test_open_shell_f_shell_replays_match_oracle(form):
+    """Classes with their slots in global memory, also in the two-pass form."""
+    announce(f"open-shell replays f shells form {form}")
+    mol = molecule("water+")
+    orc = oracle_for(mol, "cc-pVTZ")
+    Pa, Pb = seeded_spin_densities_for(orc, mol, 2)
+    Ga_ref, Gb_ref, _ = orc.fock2e_os(Pa, Pb, cutoff=1e-11, threads=4)
+    eng = _engine(product_basis(mol, "cc-pVTZ"), cutoff=1e-11)
+    for cb in range(10):
+        for ck in range(cb + 1):
+            eng.set_class_os(cb, ck, form)
+    _replays_match(eng, Pa, Pb, Ga_ref, Gb_ref)
+
+
+def test_open_shell_replays_of_a_tuned_engine():
+    """Above 256 functions with the committed open-shell table ((dd|ps) in two
+    passes): replayed builds equal the timed build, whose launches run one after
+    another.  Same terms, other order of the sums: 1e-12 of the largest element."""
+    announce("open-shell replays water16+ 6-31G* tuned")
+    from quick_amd import autotune
+    mol = molecule("water16+")
+    eng = _engine(product_basis(mol, "6-31G*"), cutoff=1e-10)
+    table = autotune.load_table("gfx950|single|fp64|n>256|h2o32+")
+    assert any(len(c) > 5 and c[5] == 1 for c in table.values())
+    autotune.apply_table(eng, table)
+    rng = np.random.default_rng(5)
+    Pa, Pb = (0.05 * (lambda x: x + x.T)(rng.standard_normal((eng.n, eng.n))) for _ in range(2))
+    eng.set_timing(True)
+    Ga_ref, Gb_ref = eng.fock2e_os(Pa, Pb)
+    eng.set_timing(False)
+    tol = 1e-12 * max(1.0, float(np.max(np.abs(Ga_ref))), float(np.max(np.abs(Gb_ref))))
+    for _ in range(3):
+        Ga, Gb = eng.fock2e_os(Pa, Pb)
+        assert np.max(np.abs(Ga - Ga_ref)) <= tol and np.max(np.abs(Gb - Gb_ref)) <= tol
+
+
 def test_open_shell_closed_shell_limit():
     """Pa = Pb = P/2 gives Ga = Gb = the closed-shell G(P)."""
     announce("open-shell closed-shell limit water3 6-31G*")

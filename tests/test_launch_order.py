@@ -1,0 +1,85 @@
+"""Order and buffers of a build's launches, on the CPU: the library runs over
+mock_hip.cpp, which records every launch with the launches it waits for.
+
+A build is right for every timing if each class kernel starts after the
+opening kernel (which clears the accumulators and writes the descriptors), has
+ended when the closing kernel sums them, and shares its slice of the global
+slot buffer with no kernel that may run at the same time."""
+import pytest
+
+from tests import mock_hip
+
+
+@pytest.fixture(scope="module")
+def mock(tmp_path_factory):
+    return mock_hip.build(tmp_path_factory.mktemp("mock_hip"))
+
+
+BUILD = """
+import ctypes, numpy as np
+from quick_amd import molecules as M
+mock = start()
+
+def check(ops, closing=True):
+    opens = [i for i, o in enumerate(ops) if "k_open" in o.name]
+    assert len(opens) == 1, [o.name for o in ops]
+    classes = [i for i, o in enumerate(ops) if any(k in o.name for k in ("fock_", "fused_", "grad_"))]
+    assert classes
+    for i in classes:
+        assert opens[0] in ops[i].before, ("not after the opening kernel", ops[i].name)
+    if closing:
+        close = [i for i, o in enumerate(ops) if "k_close" in o.name]
+        assert len(close) == 1
+        for i in classes:
+            assert i in ops[close[0]].before, ("not complete at the closing kernel", ops[i].name)
+    regions = []
+    for i in classes:
+        d = slice_doubles(ops[i].name)
+        if d:
+            a = ops[i].slots
+            regions.append((i, a, a + 8 * d * ops[i].grid))
+    for x, (i, a, b) in enumerate(regions):
+        for j, c, d in regions[:x]:
+            if j not in ops[i].before and i not in ops[j].before:
+                assert b <= c or d <= a, ("two kernels share slots", ops[i].name[:40], ops[j].name[:40])
+    return len(classes), len(regions)
+
+def builds(e, kind, count=3, closing=True):
+    n = e.n
+    P, Q, F, H = (np.zeros((n, n)) for _ in range(4))
+    p = lambda x: x.ctypes.data
+    counts = []
+    for _ in range(count):
+        mock.mock_clear()
+        if kind == "fock": e.fock2e_device(p(P), p(F))
+        if kind == "os": e.fock2e_os_device(p(P), p(Q), p(F), p(H))
+        if kind == "grad": e.eri_grad_device(p(P), p(F))
+        ops = launches(mock)
+        last = {int(x) for x in mock.mock_stream(None).decode().split()}
+        done = last.union(*(ops[i].before for i in last))
+        # the accumulator of zeros is filled once per engine, outside the build's graph
+        assert done == set(range(len(ops))), "a launch is not ordered before the caller's next one"
+        counts.append(check(ops, closing))
+    return counts
+"""
+
+MOLECULES = [("M.water()", "6-31G*"), ("M.alkane(2)", "6-31G"), ("M.water()", "cc-pVTZ"), ("M.polyglycine(1)", "6-31G**"),
+             ("M.alkane(18)", "6-31G*")]     # the last one above 256 functions
+
+
+@pytest.mark.parametrize("form", [-1, 0, 1, 2])
+@pytest.mark.parametrize("mol,basis", MOLECULES)
+def test_open_shell_builds(mock, mol, basis, form):
+    """Every open-shell form, the first build and the replayed ones: a class in
+    the two-pass form issues two kernels, one after the other."""
+    out = mock_hip.run(mock, BUILD + f"""
+e = engine({mol}, "{basis}", prepare=False)
+for cb in range(10):
+    for ck in range(cb + 1):
+        e.set_class_os(cb, ck, {form})
+e.prepare()
+c = builds(e, "os")
+assert len(set(c)) == 1, c       # a replay issues what the first build issued
+print(c)
+""")
+    print(out)
