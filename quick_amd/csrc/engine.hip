@@ -866,13 +866,17 @@ int prefix_count(const std::vector<qf::PairInfo>& kets, double yi, double thr, b
 // Regions of the global slot buffer, one per launch whose node programs keep
 // their slots there (launches on different streams run at the same time), of
 // one slice per workgroup of its grid.  Returns the doubles needed in all.
+size_t slot_doubles(const qf_engine::Launch& L)
+{
+    return L.tile == 2 ? (size_t)qf::coop_global_doubles(L.cb, L.ck) * std::min(L.count, qf::COOP_GLOBAL_SLICES) : 0;
+}
+
 size_t place_slots(std::vector<qf_engine::Launch>& launches)
 {
     size_t total = 0;
     for (auto& L : launches) {
         L.gslot = total;
-        if (L.tile == 2)
-            total += (size_t)qf::coop_global_doubles(L.cb, L.ck) * std::min(L.count, qf::COOP_GLOBAL_SLICES);
+        total += slot_doubles(L);
     }
     return total;
 }
@@ -996,7 +1000,7 @@ struct FusedList {
 // Plan of closed-shell (os 0) or open-shell (os 1) builds in which classes of
 // the same kernel bucket share a launch, its workgroups longest first.
 // Appends to e->fused and to `list`, their workgroups; slots: doubles of the
-// global slot buffer that the plan's shared launches need.
+// global slot buffer that the plan needs.
 qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& list, size_t& slots)
 {
     struct Group {
@@ -1005,6 +1009,7 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
         size_t lds = 0;
     };
     std::map<std::pair<int, int>, Group> groups;   // by kernel and waves
+    slots = 0;
     std::vector<std::pair<int, double>> t;
     for (int l = 0; l < (int)e->launches.size(); ++l) {
         const auto& L = e->launches[l];
@@ -1035,9 +1040,12 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
                 if (g) g->list.add(s, id, x);
             }
         }
-        if (!g) t.push_back({l, own.seconds()});
+        if (!g) {
+            t.push_back({l, own.seconds()});
+            // shared launches run beside this one: their regions follow its own
+            if (slot_doubles(L)) slots = std::max(slots, L.gslot + slot_doubles(L));
+        }
     }
-    slots = 0;
     for (auto& kv : groups) {
         Group& g = kv.second;
         qf_engine::Fused f{};

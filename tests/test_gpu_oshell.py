@@ -113,9 +113,10 @@ def test_open_shell_replays_match_oracle(mode):
     _replays_match(eng, Pa, Pb, Ga_ref, Gb_ref)
 
 
-@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("form", [0, 1, "(ff|ff) and (fd|fd) in two passes"])
 def test_open_shell_f_shell_replays_match_oracle(form):
-    """Classes with their slots in global memory, also in the two-pass form."""
+    """Classes with their slots in global memory, also in the two-pass form and
+    in that form beside others that share a launch."""
     announce(f"open-shell replays f shells form {form}")
     mol = molecule("water+")
     orc = oracle_for(mol, "cc-pVTZ")
@@ -124,7 +125,7 @@ def test_open_shell_f_shell_replays_match_oracle(form):
     eng = _engine(product_basis(mol, "cc-pVTZ"), cutoff=1e-11)
     for cb in range(10):
         for ck in range(cb + 1):
-            eng.set_class_os(cb, ck, form)
+            eng.set_class_os(cb, ck, form if isinstance(form, int) else 1 if cb == ck and cb >= 8 else -1)
     _replays_match(eng, Pa, Pb, Ga_ref, Gb_ref)
 
 

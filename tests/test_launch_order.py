@@ -83,3 +83,38 @@ assert len(set(c)) == 1, c       # a replay issues what the first build issued
 print(c)
 """)
     print(out)
+
+
+@pytest.mark.parametrize("two_pass", [[(9, 9)], [(8, 8)], [(9, 5), (9, 7)], [(9, 8), (8, 8), (5, 5)], []])
+def test_slot_regions_of_shared_and_own_launches(mock, two_pass):
+    """Classes with global slots, some in the two-pass form (a launch of their
+    own), the others in a shared launch beside them."""
+    mock_hip.run(mock, BUILD + f"""
+e = engine(M.alkane(2), "def2-TZVP", prepare=False)
+for cb, ck in {two_pass}:
+    e.set_class_os(cb, ck, 1)
+e.prepare()
+c = builds(e, "os")
+assert len(set(c)) == 1 and c[0][1] >= 1, c
+""")
+
+
+@pytest.mark.parametrize("mol,basis", MOLECULES)
+@pytest.mark.parametrize("kind", ["fock", "os", "grad"])
+def test_builds_of_every_kind(mock, mol, basis, kind):
+    """Default forms, then a capped grid (one launch per class), then the timed path."""
+    if kind == "grad" and "TZ" in basis:
+        pytest.skip("no gradient of f shells")
+    mock_hip.run(mock, BUILD + f"""
+e = engine({mol}, "{basis}")
+closing = {kind!r} != "grad"
+assert len(set(builds(e, {kind!r}, closing=closing))) == 1
+e.set_persistent(64)
+assert len(set(builds(e, {kind!r}, closing=closing))) == 1
+e.set_persistent(0)
+if {kind!r} == "grad":
+    e.set_grad_kernel(lane=False)
+    assert len(set(builds(e, "grad", closing=False))) == 1
+e.set_timing(True)
+builds(e, {kind!r}, closing=closing)
+""")
