@@ -1631,8 +1631,9 @@ struct GBufs {
 
 // Issues the launches of `order` with issue(launch index, stream): forked
 // from s over the side streams and joined again, or all on s where there are
-// none.  After a failed launch the streams are joined all the same, so that a
-// capture of s stays whole.
+// none.  After a failed launch or event call every side stream that took part is
+// joined all the same, so that a capture of s stays whole and what follows on s
+// waits for the launches that were made; the first error is returned.
 template <class F>
 int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<int, int>>& order, F&& issue)
 {
@@ -1642,6 +1643,10 @@ int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<i
             if ((rc = issue(o.first, s))) return rc;
         return rc;
     }
+    auto ok = [&](hipError_t err, const char* call) {
+        if (err != hipSuccess && rc == QF_OK) rc = fail(QF_ERR_HIP, std::string(call) + ": " + hipGetErrorString(err));
+        return err == hipSuccess;
+    };
     bool used[kSide] = {};
     QF_HIP(hipEventRecord(side->fork, s));
     for (const auto& o : order) {
@@ -1649,17 +1654,15 @@ int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<i
         if (o.second > 0) {
             q = side->s[o.second - 1];
             if (!used[o.second - 1]) {
-                QF_HIP(hipStreamWaitEvent(q, side->fork, 0));
+                if (!ok(hipStreamWaitEvent(q, side->fork, 0), "hipStreamWaitEvent(fork)")) break;
                 used[o.second - 1] = true;
             }
         }
         if ((rc = issue(o.first, q))) break;
     }
     for (int k = 0; k < kSide; ++k)
-        if (used[k]) {
-            QF_HIP(hipEventRecord(side->done[k], side->s[k]));
-            QF_HIP(hipStreamWaitEvent(s, side->done[k], 0));
-        }
+        if (used[k] && ok(hipEventRecord(side->done[k], side->s[k]), "hipEventRecord(done)"))
+            ok(hipStreamWaitEvent(s, side->done[k], 0), "hipStreamWaitEvent(done)");
     return rc;
 }
 

@@ -118,3 +118,43 @@ if {kind!r} == "grad":
 e.set_timing(True)
 builds(e, {kind!r}, closing=closing)
 """)
+
+
+@pytest.mark.parametrize("call,fork_calls", [("hipStreamWaitEvent", 3), ("hipEventRecord", 1)])
+def test_side_streams_are_joined_after_a_failure(mock, call, fork_calls):
+    """A failing event call in the middle of a forked build (here under capture,
+    where builds are issued launch by launch) is reported, and every launch that
+    was made, except those behind a join that fails itself, is ordered before the
+    caller's next one."""
+    mock_hip.run(mock, BUILD + f"""
+from quick_amd._lib import QuickFockError
+e = engine(M.polyglycine(2), "6-31G**")
+n = e.n
+P, F = np.zeros((n, n)), np.zeros((n, n))
+build = lambda: e.fock2e_device(P.ctypes.data, F.ctypes.data)
+build()                                   # takes side streams
+mock.mock_capture(None, 1)
+mock.mock_clear()
+build()
+assert any(len(o.deps) > 1 for o in launches(mock)), "the captured build is not forked"
+check(launches(mock))
+for k in range(20):
+    mock.mock_clear()
+    mock.mock_fail(b"{call}", k)
+    try:
+        build()
+    except QuickFockError as x:
+        assert "mock" in str(x) and "{call}" in str(x), x
+    else:
+        assert k >= 4, k                  # the build makes fewer such calls
+        break
+    ops = launches(mock)
+    last = {{int(x) for x in mock.mock_stream(None).decode().split()}}
+    done = last.union(*(ops[i].before for i in last)) if last else set()
+    lost = set(range(len(ops))) - done
+    heads = [i for i in lost if not any(i in ops[j].before for j in lost)]
+    assert len(heads) <= (1 if k >= {fork_calls} else 0), (k, [ops[i].name[:40] for i in heads])
+    mock.mock_fail(b"", -1)
+    mock.hipGetLastError()
+    build()                               # the engine still builds
+""")
