@@ -163,8 +163,9 @@ public:
         }
         SideStreams* ss = new SideStreams();
         if (ss->create(device)) return ss;
+        (void)hipGetLastError();   // not an error of the build, which ends by asking for the last one
         delete ss;
-        return nullptr;   // the caller runs on its own stream alone
+        return nullptr;            // the caller runs on its own stream alone
     }
     void give(SideStreams* ss)
     {

@@ -231,7 +231,7 @@ MOCK hipError_t hipMalloc(void** p, size_t n)
     return hipSuccess;
 }
 MOCK hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
-MOCK hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+MOCK hipError_t hipHostMalloc(void** p, size_t n, unsigned) { MAY_FAIL; return hipMalloc(p, n); }
 MOCK hipError_t hipHostFree(void* p) { return hipFree(p); }
 MOCK hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { MAY_FAIL; std::memcpy(to, from, n); return hipSuccess; }
 MOCK hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(to, from, n, k); }

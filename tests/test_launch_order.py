@@ -158,3 +158,22 @@ for k in range(20):
     mock.hipGetLastError()
     build()                               # the engine still builds
 """)
+
+
+@pytest.mark.parametrize("call", ["hipStreamCreateWithFlags", "hipEventCreateWithFlags", "hipGraphCreate",
+                                  "hipGraphAddKernelNode", "hipGraphInstantiate", "hipHostMalloc"])
+@pytest.mark.parametrize("after", [0, 1, 2])
+def test_builds_go_on_without_streams_graphs_and_pinned_memory(mock, call, after):
+    """What only makes a build faster may fail: the build is issued without it."""
+    mock_hip.run(mock, BUILD + f"""
+e = engine(M.polyglycine(2), "6-31G**")
+mock.mock_fail(b"{call}", {after})
+builds(e, "fock", 4)
+mock.mock_fail(b"{call}", {after})
+builds(e, "os", 4)
+mock.mock_fail(b"{call}", {after})
+builds(e, "grad", 4, closing=False)
+P = np.zeros((e.n, e.n))
+mock.mock_fail(b"{call}", 0)
+e.fock2e(P), e.fock2e_os(P, P), e.eri_grad(P)
+""")
