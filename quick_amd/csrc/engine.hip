@@ -32,6 +32,9 @@ thread_local std::string g_err;
 
 int fail(int code, const std::string& msg)
 {
+    // a failed HIP call is reported here: the next call of this library, which asks
+    // for the runtime's last error, is not to report it again
+    if (code == QF_ERR_HIP || code == QF_ERR_MEMORY) (void)hipGetLastError();
     g_err = msg;
     return code;
 }
@@ -1645,8 +1648,9 @@ int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<i
         return rc;
     }
     auto ok = [&](hipError_t err, const char* call) {
-        if (err != hipSuccess && rc == QF_OK) rc = fail(QF_ERR_HIP, std::string(call) + ": " + hipGetErrorString(err));
-        return err == hipSuccess;
+        if (err == hipSuccess) return true;
+        if (rc == QF_OK) rc = fail(QF_ERR_HIP, std::string(call) + ": " + hipGetErrorString(err));
+        return false;
     };
     bool used[kSide] = {};
     QF_HIP(hipEventRecord(side->fork, s));

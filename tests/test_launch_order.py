@@ -177,3 +177,20 @@ P = np.zeros((e.n, e.n))
 mock.mock_fail(b"{call}", 0)
 e.fock2e(P), e.fock2e_os(P, P), e.eri_grad(P)
 """)
+
+
+def test_a_reported_error_is_reported_once(mock):
+    mock_hip.run(mock, BUILD + """
+from quick_amd._lib import QuickFockError
+e = engine(M.water(), "6-31G*")
+P = np.zeros((e.n, e.n))
+for call in (b"hipLaunchKernel", b"hipStreamSynchronize", b"hipMemcpy"):
+    mock.mock_fail(call, 0)
+    try:
+        e.fock2e(P, cutmatrix=np.ones((len(e.basis.shells),) * 2))
+    except QuickFockError:
+        pass
+    else:
+        assert 0, call
+    e.fock2e(P)
+""")
