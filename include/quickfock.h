@@ -247,7 +247,9 @@ int qf_set_tile(qf_engine *e, int enable, int waves, int tasks_per_group, int ld
  * class (cb|ck), pair classes 0..9 = ss, ps, pp, ds, dp, dd, fs, fp, fd, ff
  * with ck <= cb: tile (-1 engine default, 0 direct atomics, 1 LDS tile, 2
  * one quartet per wave with the recursions in LDS - d-heavy classes; others
- * use the tile), waves per tile workgroup, tasks per tile workgroup (with
+ * use the tile; 1 on a class with La+Lb+Lc+Ld >= 6: (dd|ds), (dd|pp) and
+ * (dp|dp) take the tile above 256 basis functions, else and the other classes
+ * 2), waves per tile workgroup, tasks per tile workgroup (with
  * tile = 2: kets per task, 1..64, default 1 up to 256 basis functions and 2
  * above) and bras per task (0: default). */
 int qf_set_class_tuning(qf_engine *e, int cb, int ck, int tile, int waves, int tasks_per_group,

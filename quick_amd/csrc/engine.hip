@@ -1237,13 +1237,19 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // not change: 48 molecules 16.0 -> 16.9), with two waves,
                 // four tasks of one bra a workgroup ((dp|pp), (H2O)32: 10.5 ms against
                 // 10.7 with the other classes' shapes).
+                // A class without another tile kernel takes this one with tile = 1 on the
+                // same condition, else the wave-per-quartet kernel, as saved tables
+                // mean it: tile = 1 for these three, wave per quartet -> Hermite, water
+                // 0.12 -> 0.24 ms, glycine 0.42 -> 0.96, (H2O)8 6-31G* 0.63 -> 1.36, (H2O)12
+                // 1.41 -> 2.32, 256 batched molecules in mixed precision 68.0 -> 71.6, but
+                // (H2O)16 (304) 2.83 -> 2.80.
                 const bool md = !fp32 && tile_ok && qf::fock_tile_is_md(cb, ck);
                 const bool md_shape = md && e->nbasis > 256 && ct.tile < 0 && e->tile != 0;
                 if (md_shape && ct.mmax == 0) mmax = 1;
                 if (md_shape && ct.tpg == 0 && e->tile_tasks == 0) tile_tasks = 4;
                 if (md_shape && ct.waves == 0) tile_waves = std::min(tile_waves, 2);
                 const bool want_coop = ct.tile == 2   ? true
-                                       : ct.tile == 1 ? !lane_class && !tile_ok
+                                       : ct.tile == 1 ? !lane_class && !(tile_ok && e->nbasis > 256)
                                        : ct.tile == 0 || e->tile == 0 ? !lane_class
                                        : md_shape ? false
                                                   : Lsum >= coop_lmin || (!lane_class && !tile_ok);

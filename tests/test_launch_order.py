@@ -194,3 +194,36 @@ for call in (b"hipLaunchKernel", b"hipStreamSynchronize", b"hipMemcpy"):
         assert 0, call
     e.fock2e(P)
 """)
+
+
+def test_hermite_only_classes_take_the_tile_above_256_functions(mock):
+    """(dd|ds), (dd|pp) and (dp|dp) have no other LDS-tile kernel than the Hermite
+    one, which is slower up to 256 functions and in batches of such molecules:
+    there tile = 1, as in saved tables, keeps them on the wave-per-quartet kernel."""
+    mock_hip.run(mock, BUILD + """
+from quick_amd.engine import FockBatch
+only = ("C2220", "C2211", "C2121")
+def setup(n, tile):
+    e = engine(M.alkane(n), "6-31G*", prepare=False)
+    for cb in range(10):
+        for ck in range(cb + 1):
+            e.set_class_tuning(cb, ck, tile)
+    e.prepare()
+    assert (e.n > 256) == (n > 13)
+    return e
+def hermite():
+    names = [o.name for o in launches(mock) if "fock_md_kernel" in o.name]
+    return {c for c in only if any(c in x for x in names)}
+for n, tile, want in ((1, 1, 0), (4, 1, 0), (13, 1, 0), (13, -1, 0), (14, 1, 3), (14, -1, 3), (14, 2, 0)):
+    e = setup(n, tile)
+    builds(e, "fock", 2)
+    assert len(hermite()) == want, (n, tile, hermite())
+    builds(e, "os", 2)
+    assert not hermite()
+    mock.mock_clear()
+    b = FockBatch([e])
+    b.build()
+    assert len(hermite()) == want, (n, tile, hermite())
+    b.close()
+    e.close()
+""")
