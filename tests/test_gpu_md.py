@@ -50,3 +50,25 @@ def test_md_defaults_above_256_functions(precision):
     for x, y in zip(a.fock2e_os(P / 2, Q / 2), b.fock2e_os(P / 2, Q / 2)):
         close(x, y)
     close(a.eri_grad(P), b.eri_grad(P))
+
+
+@pytest.mark.parametrize("name,basis,copies", [("water", "6-31G*", 14), ("water", "cc-pVDZ", 11), ("LiF", "cc-pVDZ", 9)])
+@pytest.mark.parametrize("shape", [(1, 1, 2, 1, 0), (1, 4, 16, 4, -1), (1, 2, 4, 2, 1)])
+def test_md_tile_kernels_above_256_functions_match_the_oracle(name, basis, copies, shape):
+    """Copies so far apart that the quartets are those of the pairs of single
+    molecules: short ket windows in every class."""
+    announce("md copies %s %s %s" % (name, basis, shape))
+    from quick_amd.basis import Molecule
+    from quick_amd.engine import FockEngine
+    one = molecule(name)
+    mol = Molecule(list(one.symbols) * copies,
+                   np.concatenate([one.xyz + np.array([20.0 * k, 3.0 * (k % 2), 0.0]) for k in range(copies)]))
+    orc = oracle_for(mol, basis)
+    P, _ = seeded_density_for(orc, mol)
+    bs = product_basis(mol, basis)
+    assert bs.nbasis > 256
+    e = FockEngine(bs, cutoff=1e-10)
+    for cb, ck in MD:
+        e.set_class_tuning(cb, ck, *shape[:4])
+        e.set_class_piece(cb, ck, shape[4])
+    assert np.abs(e.fock2e(P) - orc.fock2e(P, cutoff=1e-10)[0]).max() <= 1e-10
