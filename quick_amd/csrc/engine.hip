@@ -539,11 +539,13 @@ struct qf_engine {
         size_t lds_os;   // open-shell pass with a second exchange tile (0: it does not fit)
         int os_split;    // open-shell builds run this class as two closed-shell passes
         int os_lean;     // ... or, on the tile kernel, in the fused lean form
-        int alt_offset, alt_count;   // wave-per-quartet tasks of a class whose tile kernel is closed-shell Fock
-                                     // only: open-shell builds and gradients run these (alt_count 0: none)
+        int closed_only;             // the tile kernel has no open-shell and no gradient form: these run the
+                                     // class on the wave-per-quartet kernels,
+        int alt_offset, alt_count;   // with tasks of their own in d_alt (count 0: not made, the tile tasks serve)
         size_t gslot;    // first double of its region of the global slot buffer (classes that need one)
     };
     std::vector<Launch> launches;
+    bool alt_made = false;   // the tasks in d_alt are those of `launches`
     struct Fused {           // classes of `launches` that share a launch
         int kernel;          // qf::fuse_kernel
         int offset, count;   // its workgroups in d_fused
@@ -577,6 +579,7 @@ struct qf_engine {
     DevBuf<qf::PairBlock> d_blocks;
     DevBuf<qf::MolDesc> d_mol;
     DevBuf<qf::Task> d_tasks;
+    DevBuf<qf::Task> d_alt;
     DevBuf<qf::TileGroup> d_groups;
     DevBuf<qf::FusedBlock> d_fused;
     DevBuf<int> d_colf;
@@ -1017,13 +1020,12 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
     std::vector<std::pair<int, double>> t;
     for (int l = 0; l < (int)e->launches.size(); ++l) {
         const auto& L = e->launches[l];
-        const bool alt = os && L.alt_count > 0, coop = L.tile == 2 || alt;
+        const bool coop = L.tile == 2;
         const int id = L.cb * 16 + L.ck;
         const int kernel = L.fp32 || L.tile == 0 || (os && L.os_split) || (os && !coop && !L.os_lean)
                                ? -1
                                : qf::fuse_bucket(L.cb, L.ck, coop);
         LaunchCost own;
-        const int first = alt ? L.alt_offset : L.offset, count = alt ? L.alt_count : L.count;
         Group* g = kernel < 0 ? nullptr : &groups[{kernel, coop ? 1 : L.waves}];
         LaunchCost& c = g ? g->cost : own;
         c.launch(L, coop);
@@ -1039,7 +1041,7 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
             }
         } else {
             if (g) g->lds = std::max(g->lds, sizeof(double) * qf::coop_lds_doubles(L.cb, L.ck));
-            for (int x = first; x < first + count; ++x) {
+            for (int x = L.offset; x < L.offset + L.count; ++x) {
                 const double s = c.task(e->tasks[x]);
                 if (g) g->list.add(s, id, x);
             }
@@ -1079,11 +1081,10 @@ qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, 
     for (const auto& L : e->launches) {
         const int k = qf::grad_fuse_bucket(L.cb, L.ck);
         if (k < 0) return e->plan[3];   // an f class: gradients are refused
-        const bool alt = L.alt_count > 0, coop = qf::grad_fuse_kernel(k).coop;
+        const bool coop = qf::grad_fuse_kernel(k).coop;
         if (coop) lds[k] = std::max(lds[k], sizeof(double) * qf::grad_lds_doubles(L.cb, L.ck));
-        const int first = alt ? L.alt_offset : L.offset, count = alt ? L.alt_count : L.count;
         cost[k].launch(L, coop);
-        for (int x = first; x < first + count; ++x)
+        for (int x = L.offset; x < L.offset + L.count; ++x)
             lists[k].add(cost[k].task(e->tasks[x]), L.cb * 16 + L.ck + (L.fp32 ? 256 : 0), x);
     }
     for (int k = 0; k < qf::kGradFuseKernels; ++k) {
@@ -1104,6 +1105,66 @@ qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, 
     return stream_order(t);
 }
 
+// Primitive pieces: a wave's lanes each run the whole primitive loop of
+// one quartet, so the most contracted quartets set the tail of a launch
+// (and, for small molecules with few waves, its whole time).  The
+// primitive pairs of a task are therefore cut into pieces: a small molecule
+// has too few quartets to fill the GPU and takes one primitive pair per
+// piece, a large one only cuts the longest loops (e.g. 36 -> 3 x 12), since
+// every piece repeats the screen, the HRR and the digestion.  Builds in us
+// with pieces of 1 / 2 / 3 / 4 / 6 / 12, launches over four streams:
+// water 6-31G* (19 functions) 143 / 184 / 284 / 291 / 396 / 731, butane 6-31G* (80)
+// 835 / 521 / 776 / 805 / 1361 / 1793, glycine 6-31G** (100, two tasks a
+// workgroup) 1710 / 824 / 614 / 589 / 616 / 989, (H2O)8 6-31G* (152) 1808 /
+// 881 / 788 / 857 / 1015 / 1479, (Gly)2 6-31G** (175) 4526 / 2258 / 1483 /
+// 1442 / 1560 / 2021, (H2O)16 6-31G* (304) 10064 / 4669 / 2909 / 2823 / 2599 /
+// 2931, (H2O)32 (608) 34806 / 17910 / 11420 / 11298 / 10712 / 10692.  Shared
+// launches (`shared`) have no tails of their own to shorten and take longer
+// pieces; 1 / 2 / 3 / 4 / 6: water 113 / 72 / 91 / - / -, ethane 6-31G* (42) 217 / 151 /
+// 255 / 303 / 436, butane 775 / 402 / 357 / 316 / 606, glycine 1116 / 548 / 401 / 393 /
+// 436, (H2O)8 6-31G* 1753 / 865 / 587 / 580 / 526, (Gly)2 3839 / 2116 / 1478 / 1472 /
+// 1371.
+int prim_piece(const qf_engine* e, int size, bool shared)
+{
+    return e->prim_piece > 0   ? e->prim_piece
+           : e->prim_piece < 0 ? 1 << 20
+           : shared            ? (size <= 48 ? 2 : size <= 64 ? 3 : size <= 128 ? 4 : 6)
+           : size <= 48        ? 1
+           : size <= 96        ? 2
+           : size <= 160       ? 3
+           : size <= 200       ? 4
+           : size <= 400       ? 6
+                               : 12;
+}
+
+// Kets per task of the wave-per-quartet kernels (builds in us with windows of 1 / 2 / 4 / 8 / 16: (H2O)16 2828 / 2846 /
+// 2853 / 2953 / 2987, (H2O)32 10701 / 10658 / 10663 / 11389 / 11136, (Gly)6
+// 6-31G** 11829 / 11813 / 12198 / 12191 / 13524)
+int coop_window(int size) { return size <= 256 ? 1 : kCoopWindow; }
+
+// A task as tasks of at most `piece` bra and ket primitive pairs each.
+void push_pieces(qf::Task t, int Kb, int Kk, int piece, std::vector<qf::Task>& out)
+{
+    const int nb = (Kb + piece - 1) / piece, nk = (Kk + piece - 1) / piece;
+    const int sb = (Kb + nb - 1) / nb, sk = (Kk + nk - 1) / nk;
+    for (int pb = 0; pb < Kb; pb += sb)
+        for (int qb = 0; qb < Kk; qb += sk) {
+            t.pb = pb;
+            t.pe = std::min(Kb, pb + sb);
+            t.qb = qb;
+            t.qe = std::min(Kk, qb + sk);
+            out.push_back(t);
+        }
+}
+
+// Work of a task: bras x kets x primitive pairs (bra and ket); without the
+// primitive factor the longest-first order misjudges the contracted classes (13 %
+// of the (H2O)32 build).
+long long task_work(const qf::Task& x)
+{
+    return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
+}
+
 // Wave tasks, tile groups and launches of one engine, per quartet class and
 // precision.  `size` stands for the number of basis functions in the rules
 // that choose launch shapes: the engine's own, or for an engine in a batch
@@ -1117,34 +1178,7 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
     tasks.clear();
     groups.clear();
     launches.clear();
-    // Primitive pieces: a wave's lanes each run the whole primitive loop of
-    // one quartet, so the most contracted quartets set the tail of a launch
-    // (and, for small molecules with few waves, its whole time).  The
-    // primitive pairs of a task are therefore cut into pieces: a small molecule
-    // has too few quartets to fill the GPU and takes one primitive pair per
-    // piece, a large one only cuts the longest loops (e.g. 36 -> 3 x 12), since
-    // every piece repeats the screen, the HRR and the digestion.  Builds in us
-    // with pieces of 1 / 2 / 3 / 4 / 6 / 12, launches over four streams:
-    // water 6-31G* (19 functions) 143 / 184 / 284 / 291 / 396 / 731, butane 6-31G* (80)
-    // 835 / 521 / 776 / 805 / 1361 / 1793, glycine 6-31G** (100, two tasks a
-    // workgroup) 1710 / 824 / 614 / 589 / 616 / 989, (H2O)8 6-31G* (152) 1808 /
-    // 881 / 788 / 857 / 1015 / 1479, (Gly)2 6-31G** (175) 4526 / 2258 / 1483 /
-    // 1442 / 1560 / 2021, (H2O)16 6-31G* (304) 10064 / 4669 / 2909 / 2823 / 2599 /
-    // 2931, (H2O)32 (608) 34806 / 17910 / 11420 / 11298 / 10712 / 10692.  Shared
-    // launches (`shared`) have no tails of their own to shorten and take longer
-    // pieces; 1 / 2 / 3 / 4 / 6: water 113 / 72 / 91 / - / -, ethane 6-31G* (42) 217 / 151 /
-    // 255 / 303 / 436, butane 775 / 402 / 357 / 316 / 606, glycine 1116 / 548 / 401 / 393 /
-    // 436, (H2O)8 6-31G* 1753 / 865 / 587 / 580 / 526, (Gly)2 3839 / 2116 / 1478 / 1472 /
-    // 1371.
-    const int piece = e->prim_piece > 0   ? e->prim_piece
-                      : e->prim_piece < 0 ? 1 << 20
-                      : shared            ? (size <= 48 ? 2 : size <= 64 ? 3 : size <= 128 ? 4 : 6)
-                      : size <= 48        ? 1
-                      : size <= 96        ? 2
-                      : size <= 160       ? 3
-                      : size <= 200       ? 4
-                      : size <= 400       ? 6
-                                          : 12;
+    const int piece = prim_piece(e, size, shared);
     for (int cb = 0; cb < kNPC; ++cb)
         for (int ck = 0; ck <= cb; ++ck)
             for (int fp32 = 0; fp32 < 2; ++fp32) {
@@ -1261,117 +1295,89 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 // wave-per-quartet kernel a window (the class tuning's
                 // tasks_per_group): small windows give more workgroups to
                 // classes with few quartets
-                // (builds in us with windows of 1 / 2 / 4 / 8 / 16: (H2O)16 2828 / 2846 /
-                // 2853 / 2953 / 2987, (H2O)32 10701 / 10658 / 10663 / 11389 / 11136, (Gly)6
-                // 6-31G** 11829 / 11813 / 12198 / 12191 / 13524)
-                const int coop_win = size <= 256 ? 1 : kCoopWindow;
-                const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_win) : qf::WAVE;
+                const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_window(size)) : qf::WAVE;
+                const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
                 size_t lds = 0, lds_os = 0;
                 long long group_tasks = 0;
-                // tasks of this launch (and its tile groups), or with alt the
-                // wave-per-quartet tasks of the same quartets
-                auto emit = [&](int win, int mmax, bool alt) {
-                    for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
-                        const HostBlock& B = e->blocks[bbk];
-                        if (B.cls != cb) continue;
-                        for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
-                            const HostBlock& Kb = e->blocks[kbk];
-                            if (Kb.cls != ck) continue;
-                            if (cb == ck && kbk > bbk) continue;
-                            const bool same = (cb == ck && kbk == bbk);
-                            std::vector<std::pair<int, int>> chunks;
-                            for (const auto& g : B.groups)
-                                for (int c0 = g.first; c0 < g.second; c0 += mmax)
-                                    chunks.push_back({c0, std::min(g.second, c0 + mmax)});
-                            for (const auto& g : chunks) {
-                                // per bra of the group: ket range [lo, hi) of this precision
-                                const int M = g.second - g.first;
-                                std::vector<int> lo(M), hi(M);
-                                int nmax = 0;
-                                for (int k = 0; k < M; ++k) {
-                                    const int i = B.bperm[g.first + k];
-                                    const double yi = B.info[i].ycut;
-                                    int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
-                                    if (same) n = std::min(n, i + 1);
-                                    if (!fp32 && stats && !alt) stats->n_quartets_bound += n;
-                                    int n64 = n;
-                                    if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
-                                    lo[k] = fp32 ? n64 : 0;
-                                    hi[k] = fp32 ? n : n64;
-                                    nmax = std::max(nmax, hi[k]);
-                                }
-                                const int chunk_first = (int)tasks.size();
-                                for (int s0 = 0; s0 < nmax; s0 += win) {
-                                    int kb = -1, ke = -1;
-                                    for (int k = 0; k < M; ++k)
-                                        if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
-                                            if (kb < 0) kb = k;
-                                            ke = k + 1;
-                                        }
-                                    if (kb < 0) continue;
-                                    qf::Task t{};
-                                    t.bra_block = (int)bbk;
-                                    t.kb = g.first + kb;
-                                    t.ke = g.first + ke;
-                                    t.ket_block = (int)kbk;
-                                    t.ket_start = s0;
-                                    t.ket_count = std::min(win, nmax - s0);
-                                    t.same_block = same ? 1 : 0;
-                                    t.all_fp64 = split_class ? 0 : 1;
-                                    // highly contracted pairs: spread the primitive
-                                    // pairs of the window over several tasks
-                                    const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
-                                    const int nbp = (B.K + cpiece - 1) / cpiece, nkp = (Kb.K + cpiece - 1) / cpiece;
-                                    const int sb = (B.K + nbp - 1) / nbp, sk = (Kb.K + nkp - 1) / nkp;
-                                    for (int pbi = 0; pbi < B.K; pbi += sb)
-                                        for (int qbi = 0; qbi < Kb.K; qbi += sk) {
-                                            t.pb = pbi;
-                                            t.pe = std::min(B.K, pbi + sb);
-                                            t.qb = qbi;
-                                            t.qe = std::min(Kb.K, qbi + sk);
-                                            tasks.push_back(t);
-                                        }
-                                }
-                                if (!tile || alt) continue;
-                                // workgroups of the chunk: consecutive runs of its tasks
-                                const int chunk_end = (int)tasks.size();
-                                for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
-                                    qf::TileGroup tg{};
-                                    tg.task_begin = t0;
-                                    tg.task_end = std::min(chunk_end, t0 + tile_tasks);
-                                    tg.chunk_kb = g.first;
-                                    tg.nbra = M;
-                                    groups.push_back(tg);
-                                    group_tasks += tg.task_end - tg.task_begin;
-                                }
-                                if (chunk_end > chunk_first) {
-                                    const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
-                                    lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
-                                    lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
-                                }
+                for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
+                    const HostBlock& B = e->blocks[bbk];
+                    if (B.cls != cb) continue;
+                    for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
+                        const HostBlock& Kb = e->blocks[kbk];
+                        if (Kb.cls != ck) continue;
+                        if (cb == ck && kbk > bbk) continue;
+                        const bool same = (cb == ck && kbk == bbk);
+                        std::vector<std::pair<int, int>> chunks;
+                        for (const auto& g : B.groups)
+                            for (int c0 = g.first; c0 < g.second; c0 += mmax)
+                                chunks.push_back({c0, std::min(g.second, c0 + mmax)});
+                        for (const auto& g : chunks) {
+                            // per bra of the group: ket range [lo, hi) of this precision
+                            const int M = g.second - g.first;
+                            std::vector<int> lo(M), hi(M);
+                            int nmax = 0;
+                            for (int k = 0; k < M; ++k) {
+                                const int i = B.bperm[g.first + k];
+                                const double yi = B.info[i].ycut;
+                                int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
+                                if (same) n = std::min(n, i + 1);
+                                if (!fp32 && stats) stats->n_quartets_bound += n;
+                                int n64 = n;
+                                if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
+                                lo[k] = fp32 ? n64 : 0;
+                                hi[k] = fp32 ? n : n64;
+                                nmax = std::max(nmax, hi[k]);
+                            }
+                            const int chunk_first = (int)tasks.size();
+                            for (int s0 = 0; s0 < nmax; s0 += win) {
+                                int kb = -1, ke = -1;
+                                for (int k = 0; k < M; ++k)
+                                    if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
+                                        if (kb < 0) kb = k;
+                                        ke = k + 1;
+                                    }
+                                if (kb < 0) continue;
+                                qf::Task t{};
+                                t.bra_block = (int)bbk;
+                                t.kb = g.first + kb;
+                                t.ke = g.first + ke;
+                                t.ket_block = (int)kbk;
+                                t.ket_start = s0;
+                                t.ket_count = std::min(win, nmax - s0);
+                                t.same_block = same ? 1 : 0;
+                                t.all_fp64 = split_class ? 0 : 1;
+                                // highly contracted pairs: spread the primitive
+                                // pairs of the window over several tasks
+                                push_pieces(t, B.K, Kb.K, cpiece, tasks);
+                            }
+                            if (!tile) continue;
+                            // workgroups of the chunk: consecutive runs of its tasks
+                            const int chunk_end = (int)tasks.size();
+                            for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
+                                qf::TileGroup tg{};
+                                tg.task_begin = t0;
+                                tg.task_end = std::min(chunk_end, t0 + tile_tasks);
+                                tg.chunk_kb = g.first;
+                                tg.nbra = M;
+                                groups.push_back(tg);
+                                group_tasks += tg.task_end - tg.task_begin;
+                            }
+                            if (chunk_end > chunk_first) {
+                                const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
+                                lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
+                                lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
                             }
                         }
                     }
-                };
-                emit(win, mmax, false);
+                }
                 const int count = (int)tasks.size() - offset;
                 const int gcount = (int)groups.size() - goffset;
-                // open-shell builds and gradients of a class whose tile kernel has neither
-                const int alt_offset = (int)tasks.size();
-                if (tile && !fp32 && !lane_class && stats) emit(coop_win, 1, true);
-                const int alt_count = (int)tasks.size() - alt_offset;
-                // work of a task: bras x kets x primitive pairs (bra and ket);
-                // without the primitive factor the longest-first order misjudges
-                // the contracted classes (13 % of the (H2O)32 build)
-                auto cost = [](const qf::Task& x) {
-                    return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
-                };
                 if (tile && gcount > 0) {
                     // longest workgroups first so the launch ends evenly
                     std::vector<long long> gc(gcount, 0);
                     for (int q = 0; q < gcount; ++q) {
                         const auto& tg = groups[goffset + q];
-                        for (int x = tg.task_begin; x < tg.task_end; ++x) gc[q] += cost(tasks[x]);
+                        for (int x = tg.task_begin; x < tg.task_end; ++x) gc[q] += task_work(tasks[x]);
                     }
                     std::vector<int> ord(gcount);
                     std::iota(ord.begin(), ord.end(), 0);
@@ -1391,14 +1397,11 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                         std::swap(tasks[offset + q], tasks[offset + r]);
                     }
                     std::stable_sort(tasks.begin() + offset, tasks.end(),
-                                     [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
+                                     [](const qf::Task& x, const qf::Task& y) { return task_work(x) > task_work(y); });
                 }
-                std::stable_sort(tasks.begin() + alt_offset, tasks.end(),
-                                 [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
                 if (count > 0) {
                     qf_engine::Launch L{};
-                    L.alt_offset = alt_offset;
-                    L.alt_count = alt_count;
+                    L.closed_only = tile && !fp32 && !lane_class;
                     L.cb = cb;
                     L.ck = ck;
                     L.fp32 = fp32;
@@ -1441,6 +1444,69 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
         }
     }
     return QF_OK;
+}
+
+// Wave-per-quartet tasks of the closed_only classes, at the first open-shell build
+// or gradient since a prepare: a closed-shell program never runs them (made by
+// prepare they took it from 24 to 50 ms for (Gly)10 6-31G**).  Not under capture,
+// where nothing can be uploaded: until then those kernels run the tile tasks,
+// whose windows of 64 kets leave longer tails.
+int make_alt_tasks(qf_engine* e, hipStream_t s)
+{
+    if (e->alt_made) return QF_OK;
+    bool any = false;
+    for (const auto& L : e->launches) any = any || L.closed_only;
+    if (any && is_capturing(s)) return QF_OK;
+    std::vector<qf::Task> tasks;
+    for (auto& L : e->launches) {
+        if (!L.closed_only) continue;
+        const int ct = e->ctune[L.cb][L.ck].piece;
+        const int piece = ct > 0 ? ct : ct < 0 ? 1 << 20 : prim_piece(e, e->nbasis, shares_launches(e));
+        const int win = coop_window(e->nbasis);
+        L.alt_offset = (int)tasks.size();
+        for (int bb = 0; bb < (int)e->blocks.size(); ++bb)
+            for (int kb = 0; kb < (int)e->blocks.size(); ++kb) {
+                const HostBlock &B = e->blocks[bb], &K = e->blocks[kb];
+                if (B.cls != L.cb || K.cls != L.ck || (L.cb == L.ck && kb > bb)) continue;
+                for (int x = 0; x < (int)B.bperm.size(); ++x) {
+                    const int i = B.bperm[x];
+                    int n = prefix_count(K.info, B.info[i].ycut, e->list_cutoff(), true);
+                    if (bb == kb) n = std::min(n, i + 1);
+                    for (int k0 = 0; k0 < n; k0 += win) {
+                        qf::Task t{};
+                        t.bra_block = bb;
+                        t.kb = x;
+                        t.ke = x + 1;
+                        t.ket_block = kb;
+                        t.ket_start = k0;
+                        t.ket_count = std::min(win, n - k0);
+                        t.same_block = bb == kb;
+                        t.all_fp64 = 1;
+                        push_pieces(t, B.K, K.K, piece, tasks);
+                    }
+                }
+            }
+        L.alt_count = (int)tasks.size() - L.alt_offset;
+        std::stable_sort(tasks.begin() + L.alt_offset, tasks.end(),
+                         [](const qf::Task& x, const qf::Task& y) { return task_work(x) > task_work(y); });
+    }
+    const hipError_t err = e->d_alt.upload(tasks);
+    if (err != hipSuccess)
+        for (auto& L : e->launches) L.alt_count = 0;
+    QF_HIP(err);
+    e->alt_made = true;
+    return QF_OK;
+}
+
+// Tasks of a class for its wave-per-quartet kernels.
+struct WaveTasks {
+    const qf::Task* p;
+    int count;
+};
+WaveTasks wave_tasks(const qf_engine* e, const qf_engine::Launch& L)
+{
+    if (L.alt_count > 0) return {e->d_alt.p + L.alt_offset, L.alt_count};
+    return {e->d_tasks.p + L.offset, L.count};
 }
 
 int prepare(qf_engine* e)
@@ -1533,6 +1599,7 @@ int prepare(qf_engine* e)
     if (rc) return rc;
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
+    e->alt_made = false;
     e->drop_replays();
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
@@ -1851,11 +1918,11 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     ca.n = n;
     // one class launch with descriptor m on stream q; los: its open-shell form
     auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, qf::LaunchTo& q) -> int {
-        const bool alt = los && L.alt_count > 0;
-        if (L.tile == 2 || alt) {
+        if (L.tile == 2 || (los && L.closed_only)) {
             qf::FockCoopLaunch fc = qf::fock_coop_launcher(L.cb, L.ck);
             if (!fc) return fail(QF_ERR_ARG, "no wave-per-quartet kernel for class");
-            fc(e->d_tasks.p + (alt ? L.alt_offset : L.offset), alt ? L.alt_count : L.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p + L.gslot, q);
+            const WaveTasks w = wave_tasks(e, L);
+            fc(w.p, w.count, e->d_blocks.p, m, los, e->persist, e->d_cscratch.p + L.gslot, q);
         } else if (L.tile) {
             qf::FockTileLaunch ft = qf::fock_tile_launcher(L.cb, L.ck);
             if (!ft) return fail(QF_ERR_ARG, "no tile kernel for class");
@@ -1947,6 +2014,7 @@ int build_os(qf_engine* e, const double* dPa, const double* dPb, double* dFa, do
 {
     if (!e->prepared) return fail(QF_ERR_STATE, "qf_prepare has not been called");
     const int n2 = e->nbasis * e->nbasis;
+    if (int rc = make_alt_tasks(e, s)) return rc;
     QF_HIP(e->d_Pt.resize(n2));
     QF_HIP(e->d_Ps.resize(n2));
     double* cm_out = dcm ? nullptr : e->d_cm.p;
@@ -2169,15 +2237,17 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
         const int gm = e->ctune[L.cb][L.ck].grad;
         return (gm >= 0 ? gm == 1 : e->grad_lane) ? qf::grad_lane_launcher(L.cb, L.ck) : nullptr;
     };
+    for (const auto& L : e->launches)
+        if (!qf::grad_launcher(L.cb, L.ck))
+            return fail(QF_ERR_ARG, "ERI gradients cover shells up to d; this basis has f shells");
+    if (int rc = make_alt_tasks(e, s)) return rc;
     size_t gdoubles = 0;
     std::vector<size_t> gslot;   // per launch: its region of the global slot buffer
     for (const auto& L : e->launches) {
-        if (!qf::grad_launcher(L.cb, L.ck))
-            return fail(QF_ERR_ARG, "ERI gradients cover shells up to d; this basis has f shells");
         gslot.push_back(gdoubles);
         if (!lane_kernel(L))
             gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) *
-                        std::min(std::max(L.count, L.alt_count), qf::COOP_GLOBAL_SLICES);
+                        std::min(wave_tasks(e, L).count, qf::COOP_GLOBAL_SLICES);
     }
     gdoubles = std::max(gdoubles, e->grad_slots);
     if (gdoubles && e->d_gscratch.n < gdoubles) {
@@ -2231,12 +2301,10 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
         const size_t tile = slots + tile_bytes <= kGradLdsMax ? tile_bytes : 0;
         // one workgroup per task unless the engine caps the grid (qf_set_persistent):
         // the hardware then hands out tasks as workgroups finish
-        const bool alt = L.alt_count > 0;
-        const int count = alt ? L.alt_count : L.count;
-        const int grid = e->persist > 0 ? std::min(count, e->persist) : count;
-        (lane ? lane : qf::grad_launcher(L.cb, L.ck))(e->d_tasks.p + (alt ? L.alt_offset : L.offset), count,
-                                                      e->d_blocks.p, dmol, grid,
-                                                      tile, e->d_gscratch.p + gslot[li], L.fp32, q);
+        const WaveTasks w = wave_tasks(e, L);
+        const int grid = e->persist > 0 ? std::min(w.count, e->persist) : w.count;
+        (lane ? lane : qf::grad_launcher(L.cb, L.ck))(w.p, w.count, e->d_blocks.p, dmol, grid, tile,
+                                                      e->d_gscratch.p + gslot[li], L.fp32, q);
         return QF_OK;
     };
     if (!e->timing) {

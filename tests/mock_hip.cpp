@@ -41,6 +41,7 @@ std::string text;
 hipError_t last_error = hipSuccess;
 std::string fail_name;
 int fail_after = -1;
+long long uploaded = 0;    // bytes copied to the device
 
 // true where the test asked this call to fail
 bool fails(const char* fn)
@@ -84,7 +85,8 @@ struct Call {
 MOCK void mock_clear() { ops.clear(); stream_last.clear(); event_at.clear(); }
 MOCK void mock_fail(const char* fn, int after) { fail_name = fn; fail_after = after; }
 MOCK void mock_capture(void* s, int on) { on ? (void)capturing.insert(s) : (void)capturing.erase(s); }
-MOCK int mock_kernel_count() { return (int)ops.size(); }
+MOCK long long mock_uploaded() { return uploaded; }
+MOCK void mock_upload_reset() { uploaded = 0; }
 // one line per launch: index, name, grid, slot buffer (0: none), indices it waits for
 MOCK const char* mock_log()
 {
@@ -233,7 +235,13 @@ MOCK hipError_t hipMalloc(void** p, size_t n)
 MOCK hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
 MOCK hipError_t hipHostMalloc(void** p, size_t n, unsigned) { MAY_FAIL; return hipMalloc(p, n); }
 MOCK hipError_t hipHostFree(void* p) { return hipFree(p); }
-MOCK hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { MAY_FAIL; std::memcpy(to, from, n); return hipSuccess; }
+MOCK hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind kind)
+{
+    MAY_FAIL;
+    std::memcpy(to, from, n);
+    if (kind == hipMemcpyHostToDevice) uploaded += n;
+    return hipSuccess;
+}
 MOCK hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(to, from, n, k); }
 MOCK hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
 MOCK hipError_t hipGetSymbolAddress(void** p, const void*)

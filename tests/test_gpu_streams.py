@@ -170,3 +170,45 @@ def test_forked_builds_of_several_threads():
     assert not errors
     for F, (_, _, G) in zip(out, sets):
         close(F, G)
+
+
+@pytest.mark.parametrize("name,basis", [("water16", "6-31G*"), ("water3", "6-31G*")])
+def test_first_open_shell_build_and_gradient_under_capture(name, basis):
+    """What an open-shell build or a gradient needs beyond a closed-shell build is
+    made at the first of them; under capture nothing can be, and the kernels run
+    what prepare made (16 waters: the tile tasks of the Hermite-only classes)."""
+    announce("streams first call under capture %s" % name)
+    eng, P, _ = setup(name, basis, cutoff=1e-10)
+    Q = (0.3 * P).contiguous()
+    s = torch.cuda.Stream()
+    Fa, Fb = torch.zeros_like(P), torch.zeros_like(P)
+    g = torch.zeros(eng.basis.mol.natom, 3, dtype=P.dtype, device="cuda")
+
+    def calls():
+        for x in (Fa, Fb, g):
+            x.zero_()
+        eng.fock2e_os_device(P.data_ptr(), Q.data_ptr(), Fa.data_ptr(), Fb.data_ptr(), s.cuda_stream)
+        eng.eri_grad_device(P.data_ptr(), g.data_ptr(), s.cuda_stream)
+
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        for _ in range(3):              # allocates the buffers of both kinds
+            calls()
+    s.synchronize()
+    want = [x.cpu().numpy() for x in (Fa, Fb, g)]
+    eng.set_cutoffs(1e-10)
+    eng.prepare()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(graph, stream=s):
+            calls()
+    for k in range(4):                  # eager calls between the replays
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, w in zip((Fa, Fb, g), want):
+            assert np.abs(x.cpu().numpy() - w).max() <= 1e-11 * max(1.0, np.abs(w).max())
+        with torch.cuda.stream(s):
+            calls()
+        s.synchronize()
+        for x, w in zip((Fa, Fb, g), want):
+            assert np.abs(x.cpu().numpy() - w).max() <= 1e-11 * max(1.0, np.abs(w).max())

@@ -227,3 +227,39 @@ for n, tile, want in ((1, 1, 0), (4, 1, 0), (13, 1, 0), (13, -1, 0), (14, 1, 3),
     b.close()
     e.close()
 """)
+
+
+def test_tasks_that_only_some_calls_need_are_made_by_those_calls(mock):
+    """Above 256 functions the wave-per-quartet tasks of the Hermite-only classes
+    are made at the first open-shell build or gradient: prepare uploads none, a
+    call under capture before that runs the tile tasks, and all cover the same
+    quartets."""
+    mock_hip.run(mock, BUILD + """
+def grids(kind):
+    out = {}
+    for o in launches(mock):
+        for c in ("C2220", "C2211", "C2121"):
+            if c + ("Grad" if kind == "grad" else "Coop") in o.name: out[c] = o.grid
+    return out
+for kind in ("os", "grad"):
+    e = engine(M.alkane(14), "6-31G*", prepare=False)
+    mock.mock_upload_reset()
+    e.prepare()
+    first = mock.mock_uploaded()
+    builds(e, "fock", 3)
+    assert mock.mock_uploaded() == first, "a closed-shell build uploads nothing"
+    mock.mock_capture(None, 1)
+    builds(e, kind, 1, closing=kind == "os")
+    captured = grids(kind)
+    assert mock.mock_uploaded() == first
+    mock.mock_capture(None, 0)
+    builds(e, kind, 3, closing=kind == "os")
+    own = grids(kind)
+    assert len(own) == 3 and captured.keys() == own.keys()
+    assert all(own[c] > captured[c] for c in own), (own, captured)
+    made = mock.mock_uploaded()
+    assert made > first
+    builds(e, "grad" if kind == "os" else "os", 2, closing=kind == "grad")
+    assert mock.mock_uploaded() == made, "made twice"
+    e.close()
+""")
