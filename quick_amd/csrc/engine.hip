@@ -548,16 +548,17 @@ struct qf_engine {
     bool alt_made = false;   // the tasks in d_alt are those of `launches`
     struct Fused {           // classes of `launches` that share a launch
         int kernel;          // qf::fuse_kernel
-        int offset, count;   // its workgroups in d_fused
+        int offset, count;   // its workgroups in the plan's d_fused
         int waves;
         size_t lds, gslot;
         double seconds;      // estimate
     };
-    std::vector<Fused> fused;
-    size_t grad_slots = 0;   // doubles of the global slot buffer that the gradient's shared launches need
     struct Plan {
+        bool made = false;
         std::vector<std::pair<int, int>> order;   // (launch index, or ~ the index into fused; stream 0..kSide)
         double gain = 0.0;                        // seconds the forked order saves (estimate)
+        std::vector<Fused> fused;
+        DevBuf<qf::FusedBlock> d_fused;
     };
     Plan plan[4];                             // closed shell, open shell, gradient; one launch per class
     SideStreams* side = nullptr;              // taken at the first forked build
@@ -581,7 +582,6 @@ struct qf_engine {
     DevBuf<qf::Task> d_tasks;
     DevBuf<qf::Task> d_alt;
     DevBuf<qf::TileGroup> d_groups;
-    DevBuf<qf::FusedBlock> d_fused;
     DevBuf<int> d_colf;
     DevBuf<double> d_Gt, d_Gs, d_cm, d_P;
     DevBuf<double> d_Pb, d_Pt, d_Ps, d_Fa, d_Fb;   // open-shell builds (allocated on first use)
@@ -917,9 +917,10 @@ struct LaunchCost {
 
 // Issue order of launches that take t seconds, and the stream of each: longest
 // first, each to the stream with the least time so far.
-qf_engine::Plan stream_order(const std::vector<std::pair<int, double>>& t)
+void stream_order(const std::vector<std::pair<int, double>>& t, qf_engine::Plan& p)
 {
-    qf_engine::Plan p;
+    p.order.clear();
+    p.gain = 0.0;
     std::vector<int> ord(t.size());
     std::iota(ord.begin(), ord.end(), 0);
     std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return t[x].second > t[y].second; });
@@ -933,10 +934,10 @@ qf_engine::Plan stream_order(const std::vector<std::pair<int, double>>& t)
         p.gain += t[l].second;
     }
     p.gain -= *std::max_element(load, load + kSide + 1);
-    return p;
 }
 
-qf_engine::Plan stream_order(const std::vector<qf_engine::Launch>& launches, const std::vector<qf::Task>& tasks)
+void stream_order(const std::vector<qf_engine::Launch>& launches, const std::vector<qf::Task>& tasks,
+                  qf_engine::Plan& p)
 {
     std::vector<std::pair<int, double>> t;
     for (int l = 0; l < (int)launches.size(); ++l) {
@@ -946,7 +947,7 @@ qf_engine::Plan stream_order(const std::vector<qf_engine::Launch>& launches, con
         for (int x = L.offset; x < L.offset + L.count; ++x) c.task(tasks[x]);
         t.push_back({l, c.seconds()});
     }
-    return stream_order(t);
+    stream_order(t, p);
 }
 
 // Molecules whose classes share launches: up to 200 functions, without d shells
@@ -965,19 +966,6 @@ bool shares_launches(const qf_engine* e)
     int lmax = 0;
     for (int l : e->s_lmax) lmax = std::max(lmax, l);
     return e->tile != 0 && e->nbasis <= (lmax > 1 ? 200 : 100);
-}
-
-// The plan of a build or gradient (kind 2): one launch per class where the grid
-// is capped (qf_set_persistent caps each class's) or a gradient kernel was chosen.
-const qf_engine::Plan& plan_of(const qf_engine* e, int kind)
-{
-    bool plain = e->persist > 0;
-    if (kind == 2 && !plain) {
-        plain = !e->grad_lane;
-        for (const auto& row : e->ctune)
-            for (const auto& c : row) plain = plain || c.grad >= 0;
-    }
-    return e->plan[plain ? 3 : kind];
 }
 
 // Workgroups of a shared launch and their estimated seconds.
@@ -1004,11 +992,20 @@ struct FusedList {
     }
 };
 
+// The kernel that runs a class of closed-shell (os 0) or open-shell (os 1) builds
+// beside others (-1: the class has a launch of its own).
+int shared_kernel(const qf_engine::Launch& L, int os)
+{
+    const bool coop = L.tile == 2;
+    if (L.fp32 || L.tile == 0 || (os && L.os_split) || (os && !coop && !L.os_lean)) return -1;
+    return qf::fuse_bucket(L.cb, L.ck, coop);
+}
+
 // Plan of closed-shell (os 0) or open-shell (os 1) builds in which classes of
-// the same kernel bucket share a launch, its workgroups longest first.
-// Appends to e->fused and to `list`, their workgroups; slots: doubles of the
-// global slot buffer that the plan needs.
-qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& list, size_t& slots)
+// the same kernel bucket share a launch, its workgroups (appended to `list`)
+// longest first.  Launches run side by side: the regions of the shared ones in
+// the global slot buffer follow those of the plan's own launches (shared_slots).
+void fuse_plan(const qf_engine* e, int os, qf_engine::Plan& p, std::vector<qf::FusedBlock>& list)
 {
     struct Group {
         FusedList list;
@@ -1016,15 +1013,13 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
         size_t lds = 0;
     };
     std::map<std::pair<int, int>, Group> groups;   // by kernel and waves
-    slots = 0;
+    size_t slots = 0;
     std::vector<std::pair<int, double>> t;
     for (int l = 0; l < (int)e->launches.size(); ++l) {
         const auto& L = e->launches[l];
         const bool coop = L.tile == 2;
         const int id = L.cb * 16 + L.ck;
-        const int kernel = L.fp32 || L.tile == 0 || (os && L.os_split) || (os && !coop && !L.os_lean)
-                               ? -1
-                               : qf::fuse_bucket(L.cb, L.ck, coop);
+        const int kernel = shared_kernel(L, os);
         LaunchCost own;
         Group* g = kernel < 0 ? nullptr : &groups[{kernel, coop ? 1 : L.waves}];
         LaunchCost& c = g ? g->cost : own;
@@ -1048,7 +1043,6 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
         }
         if (!g) {
             t.push_back({l, own.seconds()});
-            // shared launches run beside this one: their regions follow its own
             if (slot_doubles(L)) slots = std::max(slots, L.gslot + slot_doubles(L));
         }
     }
@@ -1064,23 +1058,41 @@ qf_engine::Plan fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& lis
         f.seconds = g.cost.seconds();
         slots += (size_t)qf::fuse_kernel(f.kernel).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
         g.list.append(list);
-        t.push_back({~(int)e->fused.size(), f.seconds});
-        e->fused.push_back(f);
+        t.push_back({~(int)p.fused.size(), f.seconds});
+        p.fused.push_back(f);
     }
-    return stream_order(t);
+    stream_order(t, p);
 }
 
-// The same for gradients (water 6-31G*, host to host: 291 -> 168 us).
-qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, size_t& slots)
+// Doubles of the global slot buffer that fuse_plan's launches need, without the
+// plan: the buffer is never resized between prepares (graphs hold it).
+size_t shared_slots(const qf_engine* e, int os)
+{
+    size_t own = 0;
+    int count[qf::kFuseKernels] = {};
+    for (const auto& L : e->launches) {
+        const int k = shared_kernel(L, os);
+        if (k >= 0)
+            count[k] += L.count;
+        else if (slot_doubles(L))
+            own = std::max(own, L.gslot + slot_doubles(L));
+    }
+    for (int k = 0; k < qf::kFuseKernels; ++k)
+        own += (size_t)qf::fuse_kernel(k).global * std::min(count[k], qf::COOP_GLOBAL_SLICES);
+    return own;
+}
+
+// The same for gradients (water 6-31G*, host to host: 291 -> 168 us).  Every class
+// of the engine has a gradient kernel (grad_pass).
+void grad_fuse_plan(const qf_engine* e, qf_engine::Plan& p, std::vector<qf::FusedBlock>& list)
 {
     std::vector<FusedList> lists(qf::kGradFuseKernels);
     std::vector<LaunchCost> cost(qf::kGradFuseKernels);
     std::vector<size_t> lds(qf::kGradFuseKernels, 0);
     std::vector<std::pair<int, double>> t;
-    slots = 0;
+    size_t slots = 0;
     for (const auto& L : e->launches) {
         const int k = qf::grad_fuse_bucket(L.cb, L.ck);
-        if (k < 0) return e->plan[3];   // an f class: gradients are refused
         const bool coop = qf::grad_fuse_kernel(k).coop;
         if (coop) lds[k] = std::max(lds[k], sizeof(double) * qf::grad_lds_doubles(L.cb, L.ck));
         cost[k].launch(L, coop);
@@ -1099,10 +1111,62 @@ qf_engine::Plan grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list, 
         f.seconds = cost[k].seconds();
         slots += (size_t)qf::grad_fuse_kernel(k).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
         lists[k].append(list);
-        t.push_back({~(int)e->fused.size(), f.seconds});
-        e->fused.push_back(f);
+        t.push_back({~(int)p.fused.size(), f.seconds});
+        p.fused.push_back(f);
     }
-    return stream_order(t);
+    stream_order(t, p);
+}
+
+size_t grad_shared_slots(const qf_engine* e)
+{
+    size_t sum = 0;
+    int count[qf::kGradFuseKernels] = {};
+    for (const auto& L : e->launches) count[qf::grad_fuse_bucket(L.cb, L.ck)] += L.count;
+    for (int k = 0; k < qf::kGradFuseKernels; ++k)
+        sum += (size_t)qf::grad_fuse_kernel(k).global * std::min(count[k], qf::COOP_GLOBAL_SLICES);
+    return sum;
+}
+
+// Plan of a kind of build in shared launches: closed shell (0), open shell (1) or
+// gradient (2); or of any kind with one launch per class (3).
+int make_plan(qf_engine* e, int kind)
+{
+    qf_engine::Plan& p = e->plan[kind];
+    if (p.made) return QF_OK;
+    p.fused.clear();
+    if (kind == 3) {
+        stream_order(e->launches, e->tasks, p);
+    } else {
+        std::vector<qf::FusedBlock> list;
+        if (kind == 2)
+            grad_fuse_plan(e, p, list);
+        else
+            fuse_plan(e, kind, p, list);
+        QF_HIP(p.d_fused.upload(list));
+    }
+    p.made = true;
+    return QF_OK;
+}
+
+// The plan of a build on s.  One launch per class above the sizes of
+// shares_launches, where the grid is capped (qf_set_persistent caps each class's)
+// and where a gradient kernel was chosen.  The plan of the closed shell is made by
+// prepare, the others at the first call: a closed-shell program never uses them
+// (prepare of water 6-31G* 0.48 -> 0.35 ms, (H2O)8 cc-pVDZ 4.2 -> 3.4).  Under
+// capture, where nothing can be uploaded, a first open-shell build or gradient has
+// one launch per class.
+int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
+{
+    bool plain = e->persist > 0 || !shares_launches(e);
+    if (kind == 2 && !plain) {
+        plain = !e->grad_lane;
+        for (const auto& row : e->ctune)
+            for (const auto& c : row) plain = plain || c.grad >= 0;
+    }
+    if (!plain && !e->plan[kind].made && is_capturing(s)) plain = true;
+    if (plain) kind = 3;
+    *out = &e->plan[kind];
+    return make_plan(e, kind);
 }
 
 // Primitive pieces: a wave's lanes each run the whole primitive loop of
@@ -1604,20 +1668,10 @@ int prepare(qf_engine* e)
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
     size_t gdoubles = place_slots(e->launches);
-    e->fused.clear();
-    e->grad_slots = 0;
-    e->plan[0] = e->plan[1] = e->plan[2] = e->plan[3] = stream_order(e->launches, e->tasks);
-    if (shares_launches(e)) {
-        std::vector<qf::FusedBlock> list;
-        for (int os = 0; os < 2; ++os) {
-            size_t slots = 0;
-            e->plan[os] = fuse_plan(e, os, list, slots);
-            gdoubles = std::max(gdoubles, slots);
-        }
-        e->plan[2] = grad_fuse_plan(e, list, e->grad_slots);
-        QF_HIP(e->d_fused.upload(list));
-    }
+    if (shares_launches(e)) gdoubles = std::max({gdoubles, shared_slots(e, 0), shared_slots(e, 1)});
     if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles));
+    for (auto& p : e->plan) p.made = false;
+    if ((rc = make_plan(e, shares_launches(e) ? 0 : 3))) return rc;
 
     // ---- per-build buffers -------------------------------------------------
     const size_t n2 = (size_t)e->nbasis * e->nbasis;
@@ -1773,11 +1827,11 @@ int timing_begin(qf_engine* e, int li, hipStream_t s, hipEvent_t* stop)
 // 670, ethane def2-TZVP 4482 / 2498 / 1568.  A build under capture is issued
 // launch by launch.
 template <class F>
-int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, const CloseArgs* close, F&& issue)
+int issue_build(qf_engine* e, int kind, const qf_engine::Plan& plan, hipStream_t s, const OpenArgs& open,
+                const CloseArgs* close, F&& issue)
 {
     Replay& r = e->replay[kind];
     const bool captured = is_capturing(s);
-    const qf_engine::Plan& plan = plan_of(e, kind);
     if (!captured && !r.exec && !r.failed && !plan.order.empty() && ++r.uses > 1) {
         hipGraphNode_t last[kSide + 1] = {};
         bool ok = hipGraphCreate(&r.graph, 0) == hipSuccess;
@@ -1916,6 +1970,9 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     ca.H2 = gb.H2;
     ca.replicas = gb.replicas;
     ca.n = n;
+    const qf_engine::Plan* plan = nullptr;
+    if (!gb.timing)
+        if (int rc = plan_of(e, os, s, &plan)) return rc;
     // one class launch with descriptor m on stream q; los: its open-shell form
     auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, qf::LaunchTo& q) -> int {
         if (L.tile == 2 || (los && L.closed_only)) {
@@ -1944,14 +2001,14 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         return rc ? rc : launch(L, dmol_x, 0, q);
     };
     auto shared_launch = [&](const qf_engine::Fused& f, qf::LaunchTo& q) -> int {
-        qf::fuse_kernel(f.kernel).launch(e->d_fused.p + f.offset, f.count, e->d_groups.p, e->d_tasks.p, e->d_blocks.p,
+        qf::fuse_kernel(f.kernel).launch(plan->d_fused.p + f.offset, f.count, e->d_groups.p, e->d_tasks.p, e->d_blocks.p,
                                          dmol, os, f.waves, f.lds, e->d_cscratch.p + f.gslot, q);
         return QF_OK;
     };
     if (gb.fork && !gb.timing) {
-        const int rc = issue_build(e, os, s, oa, &ca,
+        const int rc = issue_build(e, os, *plan, s, oa, &ca,
                                    [&](int li, qf::LaunchTo& q) {
-                                       return li < 0 ? shared_launch(e->fused[~li], q)
+                                       return li < 0 ? shared_launch(plan->fused[~li], q)
                                                      : class_launch(e->launches[li], q);
                                    });
         if (rc) return rc;
@@ -1959,8 +2016,8 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         // one after another on s
         qf::LaunchTo to(s);
         open_build(oa, to);
-        for (const auto& o : plan_of(e, os).order) {
-            const int rc = o.first < 0 ? shared_launch(e->fused[~o.first], to) : class_launch(e->launches[o.first], to);
+        for (const auto& o : plan->order) {
+            const int rc = o.first < 0 ? shared_launch(plan->fused[~o.first], to) : class_launch(e->launches[o.first], to);
             if (rc) return rc;
         }
         close_build(ca, to);
@@ -2249,7 +2306,7 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
             gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) *
                         std::min(wave_tasks(e, L).count, qf::COOP_GLOBAL_SLICES);
     }
-    gdoubles = std::max(gdoubles, e->grad_slots);
+    if (shares_launches(e)) gdoubles = std::max(gdoubles, grad_shared_slots(e));
     if (gdoubles && e->d_gscratch.n < gdoubles) {
         e->replay[2].drop();   // it holds the old buffer
         QF_HIP(e->d_gscratch.resize(gdoubles));
@@ -2286,10 +2343,11 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     oa.n = e->nbasis;
     oa.nshell = e->nshell;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
+    const qf_engine::Plan* plan = nullptr;
     auto launch = [&](int li, qf::LaunchTo& q) -> int {
         if (li < 0) {
-            const qf_engine::Fused& f = e->fused[~li];
-            qf::grad_fuse_kernel(f.kernel).launch(e->d_fused.p + f.offset, f.count, e->d_tasks.p, e->d_blocks.p, dmol,
+            const qf_engine::Fused& f = plan->fused[~li];
+            qf::grad_fuse_kernel(f.kernel).launch(plan->d_fused.p + f.offset, f.count, e->d_tasks.p, e->d_blocks.p, dmol,
                                                   (int)(f.lds / sizeof(double)),
                                                   f.lds + tile_bytes <= kGradLdsMax ? 3 * e->natom : 0,
                                                   e->d_gscratch.p + f.gslot, q);
@@ -2308,7 +2366,8 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
         return QF_OK;
     };
     if (!e->timing) {
-        const int rc = issue_build(e, 2, s, oa, nullptr, launch);
+        if (int rc = plan_of(e, 2, s, &plan)) return rc;
+        const int rc = issue_build(e, 2, *plan, s, oa, nullptr, launch);
         if (rc) return rc;
     } else {
         qf::LaunchTo to(s);
@@ -3050,7 +3109,9 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
         b->d_groups.upload(groups) != hipSuccess || b->d_moldesc.upload(md) != hipSuccess ||
         b->d_bm.upload(b->mols) != hipSuccess)
         return bail(fail(QF_ERR_HIP, "batch table upload"));
-    b->order = stream_order(b->launches, tasks).order;
+    qf_engine::Plan order;
+    stream_order(b->launches, tasks, order);
+    b->order = std::move(order.order);
     b->side = SidePool::get().take(b->device);   // null: the batch runs on the caller's stream alone
     *out = b;
     return QF_OK;

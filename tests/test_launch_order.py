@@ -263,3 +263,45 @@ for kind in ("os", "grad"):
     assert mock.mock_uploaded() == made, "made twice"
     e.close()
 """)
+
+
+@pytest.mark.parametrize("mol,basis", [("M.polyglycine(1)", "6-31G**"), ("M.alkane(2)", "6-31G"),
+                                       ("M.alkane(2)", "def2-TZVP")])
+def test_plans_that_only_some_calls_need_are_made_by_those_calls(mock, mol, basis):
+    """Up to 200 functions the shared launches of open-shell builds and gradients
+    are planned at the first of them; under capture before that they have one
+    launch per class.  The slots of a closed-shell graph stay where they are."""
+    mock_hip.run(mock, BUILD + f"""
+kinds = ["os"] if "TZ" in "{basis}" else ["os", "grad"]
+for kind in kinds:
+    e = engine({mol}, "{basis}", prepare=False)
+    mock.mock_upload_reset()
+    e.prepare()
+    first = mock.mock_uploaded()
+    builds(e, "fock", 3)
+    slots = [o.slots for o in launches(mock)]
+    closing = kind == "os"
+    mock.mock_capture(None, 1)
+    (captured, _), = builds(e, kind, 1, closing=closing)
+    assert mock.mock_uploaded() == first and not any("fused_" in o.name for o in launches(mock))
+    mock.mock_capture(None, 0)
+    own = builds(e, kind, 3, closing=closing)
+    assert len(set(own)) == 1 and own[0][0] < captured and any("fused_" in o.name for o in launches(mock))
+    made = mock.mock_uploaded()
+    assert made > first
+    mock.mock_capture(None, 1)
+    builds(e, kind, 1, closing=closing)
+    mock.mock_capture(None, 0)
+    assert any("fused_" in o.name for o in launches(mock)) and mock.mock_uploaded() == made
+    builds(e, "fock", 1)
+    assert [o.slots for o in launches(mock)] == slots
+    # a capped grid at prepare still leaves the plan of shared launches ready
+    e.set_persistent(64)
+    e.set_cutoffs(1e-9)
+    e.prepare()
+    e.set_persistent(0)
+    made = mock.mock_uploaded()
+    builds(e, "fock", 2)
+    assert any("fused_" in o.name for o in launches(mock)) and mock.mock_uploaded() == made
+    e.close()
+""")
