@@ -17,6 +17,7 @@
 #include <cstring>
 #include <mutex>
 #include <map>
+#include <memory>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -855,19 +856,21 @@ int compute_schwarz(qf_engine* e)
     return QF_OK;
 }
 
-// Upper bound of kets j (sorted by ycut desc) with ycut_i*ycut_j > thr.
-int prefix_count(const std::vector<qf::PairInfo>& kets, double yi, double thr, bool strict)
+// For every bra the number of kets with ycut_i*ycut_j > thr (>= where not strict):
+// both sorted by ycut descending, so one walk finds them all.
+void prefix_counts(const std::vector<qf::PairInfo>& bras, const std::vector<qf::PairInfo>& kets, double thr, bool strict,
+                   std::vector<int>& out)
 {
-    int lo = 0, hi = (int)kets.size();
-    while (lo < hi) {
-        const int mid = (lo + hi) / 2;
-        const double y = yi * kets[mid].ycut;
-        if (strict ? (y > thr) : (y >= thr))
-            lo = mid + 1;
-        else
-            hi = mid;
+    out.resize(bras.size());
+    int n = (int)kets.size();
+    for (size_t i = 0; i < bras.size(); ++i) {
+        while (n > 0) {
+            const double y = bras[i].ycut * kets[n - 1].ycut;
+            if (strict ? (y > thr) : (y >= thr)) break;
+            --n;
+        }
+        out[i] = n;
     }
-    return lo;
 }
 
 // Regions of the global slot buffer, one per launch whose node programs keep
@@ -1207,7 +1210,8 @@ int prim_piece(const qf_engine* e, int size, bool shared)
 int coop_window(int size) { return size <= 256 ? 1 : kCoopWindow; }
 
 // A task as tasks of at most `piece` bra and ket primitive pairs each.
-void push_pieces(qf::Task t, int Kb, int Kk, int piece, std::vector<qf::Task>& out)
+template <class F>
+void each_piece(qf::Task& t, int Kb, int Kk, int piece, F&& f)
 {
     const int nb = (Kb + piece - 1) / piece, nk = (Kk + piece - 1) / piece;
     const int sb = (Kb + nb - 1) / nb, sk = (Kk + nk - 1) / nk;
@@ -1217,7 +1221,7 @@ void push_pieces(qf::Task t, int Kb, int Kk, int piece, std::vector<qf::Task>& o
             t.pe = std::min(Kb, pb + sb);
             t.qb = qb;
             t.qe = std::min(Kk, qb + sk);
-            out.push_back(t);
+            f(t);
         }
 }
 
@@ -1227,6 +1231,56 @@ void push_pieces(qf::Task t, int Kb, int Kk, int piece, std::vector<qf::Task>& o
 long long task_work(const qf::Task& x)
 {
     return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
+}
+
+// Indices in order of descending work, equal ones in their order, so that a launch
+// ends evenly: by counting, digit by digit.  A comparison sort of the tasks
+// themselves was a fifth of prepare.
+std::vector<int> longest_first(const std::vector<long long>& work)
+{
+    const size_t n = work.size();
+    std::vector<int> ord(n);
+    std::iota(ord.begin(), ord.end(), 0);
+    if (n < 512) {
+        std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return work[x] > work[y]; });
+        return ord;
+    }
+    const long long top = *std::max_element(work.begin(), work.end());
+    constexpr int kBits = 11;
+    constexpr long long kDigit = (1 << kBits) - 1;
+    std::vector<int> next(n);
+    for (int shift = 0; shift < 62 && (top >> shift) > 0; shift += kBits) {
+        int at[kDigit + 2] = {};
+        for (size_t k = 0; k < n; ++k) ++at[kDigit - ((work[k] >> shift) & kDigit) + 1];
+        for (int d = 0; d <= kDigit; ++d) at[d + 1] += at[d];
+        for (size_t k = 0; k < n; ++k) next[at[kDigit - ((work[ord[k]] >> shift) & kDigit)]++] = ord[k];
+        ord.swap(next);
+    }
+    return ord;
+}
+
+template <class T>
+void longest_first(T* p, const std::vector<long long>& work)
+{
+    const std::vector<int> ord = longest_first(work);
+    const std::vector<T> was(p, p + ord.size());
+    for (size_t k = 0; k < ord.size(); ++k) p[k] = was[ord[k]];
+}
+
+void longest_first(std::vector<qf::Task>& tasks, size_t first)
+{
+    std::vector<long long> work(tasks.size() - first);
+    for (size_t x = 0; x < work.size(); ++x) work[x] = task_work(tasks[first + x]);
+    longest_first(tasks.data() + first, work);
+}
+
+// Tile groups of `groups` from `first` on, by the work of their tasks.
+void longest_first(std::vector<qf::TileGroup>& groups, size_t first, const std::vector<qf::Task>& tasks)
+{
+    std::vector<long long> work(groups.size() - first, 0);
+    for (size_t q = 0; q < work.size(); ++q)
+        for (int x = groups[first + q].task_begin; x < groups[first + q].task_end; ++x) work[q] += task_work(tasks[x]);
+    longest_first(groups.data() + first, work);
 }
 
 // Wave tasks, tile groups and launches of one engine, per quartet class and
@@ -1240,9 +1294,12 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
 {
     const double thr_hi = e->split_thr;
     tasks.clear();
+    if (tasks.capacity() < 32768) tasks.reserve(32768);   // most molecules': growing touches every page twice
     groups.clear();
     launches.clear();
     const int piece = prim_piece(e, size, shared);
+    std::vector<std::pair<int, int>> chunks;   // bra chunks of a block
+    std::vector<int> nall, nhigh, lo, hi;      // kets of each bra of a block, of each of a chunk
     for (int cb = 0; cb < kNPC; ++cb)
         for (int ck = 0; ck <= cb; ++ck)
             for (int fp32 = 0; fp32 < 2; ++fp32) {
@@ -1371,23 +1428,23 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                         if (Kb.cls != ck) continue;
                         if (cb == ck && kbk > bbk) continue;
                         const bool same = (cb == ck && kbk == bbk);
-                        std::vector<std::pair<int, int>> chunks;
+                        prefix_counts(B.info, Kb.info, e->list_cutoff(), true, nall);
+                        if (split_class) prefix_counts(B.info, Kb.info, thr_hi, false, nhigh);
+                        chunks.clear();
                         for (const auto& g : B.groups)
                             for (int c0 = g.first; c0 < g.second; c0 += mmax)
                                 chunks.push_back({c0, std::min(g.second, c0 + mmax)});
                         for (const auto& g : chunks) {
                             // per bra of the group: ket range [lo, hi) of this precision
                             const int M = g.second - g.first;
-                            std::vector<int> lo(M), hi(M);
+                            lo.resize(M);
+                            hi.resize(M);
                             int nmax = 0;
                             for (int k = 0; k < M; ++k) {
                                 const int i = B.bperm[g.first + k];
-                                const double yi = B.info[i].ycut;
-                                int n = prefix_count(Kb.info, yi, e->list_cutoff(), true);
-                                if (same) n = std::min(n, i + 1);
+                                const int n = same ? std::min(nall[i], i + 1) : nall[i];
                                 if (!fp32 && stats) stats->n_quartets_bound += n;
-                                int n64 = n;
-                                if (split_class) n64 = std::min(n, prefix_count(Kb.info, yi, thr_hi, false));
+                                const int n64 = split_class ? std::min(n, nhigh[i]) : n;
                                 lo[k] = fp32 ? n64 : 0;
                                 hi[k] = fp32 ? n : n64;
                                 nmax = std::max(nmax, hi[k]);
@@ -1412,7 +1469,7 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                                 t.all_fp64 = split_class ? 0 : 1;
                                 // highly contracted pairs: spread the primitive
                                 // pairs of the window over several tasks
-                                push_pieces(t, B.K, Kb.K, cpiece, tasks);
+                                each_piece(t, B.K, Kb.K, cpiece, [&](const qf::Task& x) { tasks.push_back(x); });
                             }
                             if (!tile) continue;
                             // workgroups of the chunk: consecutive runs of its tasks
@@ -1436,22 +1493,11 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                 }
                 const int count = (int)tasks.size() - offset;
                 const int gcount = (int)groups.size() - goffset;
+                // longest first, unless the caller orders (a batch, over its molecules)
                 if (tile && gcount > 0) {
-                    // longest workgroups first so the launch ends evenly
-                    std::vector<long long> gc(gcount, 0);
-                    for (int q = 0; q < gcount; ++q) {
-                        const auto& tg = groups[goffset + q];
-                        for (int x = tg.task_begin; x < tg.task_end; ++x) gc[q] += task_work(tasks[x]);
-                    }
-                    std::vector<int> ord(gcount);
-                    std::iota(ord.begin(), ord.end(), 0);
-                    std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return gc[x] > gc[y]; });
-                    std::vector<qf::TileGroup> sorted(gcount);
-                    for (int q = 0; q < gcount; ++q) sorted[q] = groups[goffset + ord[q]];
-                    std::copy(sorted.begin(), sorted.end(), groups.begin() + goffset);
+                    if (stats) longest_first(groups, goffset, tasks);
                 } else if (e->shuffle && count > 1) {
-                    // deterministic permutation (concurrent waves then hit different
-                    // kets), then longest tasks first so the launch ends evenly
+                    // deterministic permutation first: concurrent waves then hit different kets
                     uint64_t st = 0x9E3779B97F4A7C15ull ^ (uint64_t)(cb * 12 + ck * 2 + fp32);
                     for (int q = count - 1; q > 0; --q) {
                         st ^= st << 13;
@@ -1460,8 +1506,7 @@ int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::
                         const int r = (int)(st % (uint64_t)(q + 1));
                         std::swap(tasks[offset + q], tasks[offset + r]);
                     }
-                    std::stable_sort(tasks.begin() + offset, tasks.end(),
-                                     [](const qf::Task& x, const qf::Task& y) { return task_work(x) > task_work(y); });
+                    if (stats) longest_first(tasks, offset);
                 }
                 if (count > 0) {
                     qf_engine::Launch L{};
@@ -1521,40 +1566,60 @@ int make_alt_tasks(qf_engine* e, hipStream_t s)
     bool any = false;
     for (const auto& L : e->launches) any = any || L.closed_only;
     if (any && is_capturing(s)) return QF_OK;
-    std::vector<qf::Task> tasks;
-    for (auto& L : e->launches) {
-        if (!L.closed_only) continue;
+    std::vector<int> nall;
+    auto each_task = [&](const qf_engine::Launch& L, auto&& f) {
         const int ct = e->ctune[L.cb][L.ck].piece;
         const int piece = ct > 0 ? ct : ct < 0 ? 1 << 20 : prim_piece(e, e->nbasis, shares_launches(e));
         const int win = coop_window(e->nbasis);
-        L.alt_offset = (int)tasks.size();
         for (int bb = 0; bb < (int)e->blocks.size(); ++bb)
             for (int kb = 0; kb < (int)e->blocks.size(); ++kb) {
                 const HostBlock &B = e->blocks[bb], &K = e->blocks[kb];
                 if (B.cls != L.cb || K.cls != L.ck || (L.cb == L.ck && kb > bb)) continue;
+                prefix_counts(B.info, K.info, e->list_cutoff(), true, nall);
+                qf::Task t{};
+                t.bra_block = bb;
+                t.ket_block = kb;
+                t.same_block = bb == kb;
+                t.all_fp64 = 1;
                 for (int x = 0; x < (int)B.bperm.size(); ++x) {
                     const int i = B.bperm[x];
-                    int n = prefix_count(K.info, B.info[i].ycut, e->list_cutoff(), true);
-                    if (bb == kb) n = std::min(n, i + 1);
+                    const int n = bb == kb ? std::min(nall[i], i + 1) : nall[i];
+                    t.kb = x;
+                    t.ke = x + 1;
                     for (int k0 = 0; k0 < n; k0 += win) {
-                        qf::Task t{};
-                        t.bra_block = bb;
-                        t.kb = x;
-                        t.ke = x + 1;
-                        t.ket_block = kb;
                         t.ket_start = k0;
                         t.ket_count = std::min(win, n - k0);
-                        t.same_block = bb == kb;
-                        t.all_fp64 = 1;
-                        push_pieces(t, B.K, K.K, piece, tasks);
+                        each_piece(t, B.K, K.K, piece, f);
                     }
                 }
             }
-        L.alt_count = (int)tasks.size() - L.alt_offset;
-        std::stable_sort(tasks.begin() + L.alt_offset, tasks.end(),
-                         [](const qf::Task& x, const qf::Task& y) { return task_work(x) > task_work(y); });
+    };
+    // first the work of every task, then each task straight to its place (0.7 million
+    // tasks, 32 MB, for (Gly)10: new pages are most of the time)
+    std::vector<std::vector<int>> place(e->launches.size());
+    std::vector<long long> work;
+    size_t total = 0;
+    for (size_t l = 0; l < e->launches.size(); ++l) {
+        auto& L = e->launches[l];
+        if (!L.closed_only) continue;
+        work.clear();
+        each_task(L, [&](const qf::Task& t) { work.push_back(task_work(t)); });
+        const std::vector<int> ord = longest_first(work);
+        place[l].resize(ord.size());
+        for (size_t k = 0; k < ord.size(); ++k) place[l][ord[k]] = (int)(total + k);
+        L.alt_offset = (int)total;
+        L.alt_count = (int)ord.size();
+        total += ord.size();
     }
-    const hipError_t err = e->d_alt.upload(tasks);
+    std::unique_ptr<qf::Task[]> tasks(new qf::Task[total]);
+    for (size_t l = 0; l < e->launches.size(); ++l) {
+        if (place[l].empty()) continue;
+        size_t k = 0;
+        each_task(e->launches[l], [&](const qf::Task& t) { tasks[place[l][k++]] = t; });
+    }
+    hipError_t err = e->d_alt.resize(total);
+    if (err == hipSuccess && total)
+        err = hipMemcpy(e->d_alt.p, tasks.get(), total * sizeof(qf::Task), hipMemcpyHostToDevice);
     if (err != hipSuccess)
         for (auto& L : e->launches) L.alt_count = 0;
     QF_HIP(err);
@@ -3027,10 +3092,6 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
     }
     std::vector<qf::Task> tasks;
     std::vector<qf::TileGroup> groups;
-    // work of a task: bras x kets x primitive pairs (bra and ket)
-    auto cost = [](const qf::Task& x) {
-        return (long long)(x.ke - x.kb) * x.ket_count * (x.pe - x.pb) * (x.qe - x.qb);
-    };
     // The molecules of a batch fill the GPU together, so their launch shapes are
     // those of the one molecule with as much work: quartets grow about as the
     // cube of the functions.  (With each molecule's own shapes, primitive pieces
@@ -3045,10 +3106,17 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
         std::vector<qf_engine::Launch> launches;
     };
     std::vector<EngineTasks> et(count);
+    size_t ntasks = 0, ngroups = 0;
+    std::vector<qf::Task> scratch;   // kept over the engines: what grows touches new pages
     for (int i = 0; i < count; ++i) {
-        rc = make_tasks(b->engs[i], size, et[i].tasks, et[i].groups, et[i].launches, nullptr);
+        rc = make_tasks(b->engs[i], size, scratch, et[i].groups, et[i].launches, nullptr);
         if (rc) return bail(rc);
+        et[i].tasks.assign(scratch.begin(), scratch.end());
+        ntasks += et[i].tasks.size();
+        ngroups += et[i].groups.size();
     }
+    tasks.reserve(ntasks);
+    groups.reserve(ngroups);
     for (int cb = 0; cb < kNPC; ++cb)
         for (int ck = 0; ck <= cb; ++ck)
             for (int fp32 = 0; fp32 < 2; ++fp32)
@@ -3085,21 +3153,10 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
                     C.count = (int)tasks.size() - C.offset;
                     C.gcount = (int)groups.size() - C.goffset;
                     if (C.count == 0) continue;
-                    if (tile == 1) {
-                        std::vector<long long> gc(C.gcount, 0);
-                        for (int q = 0; q < C.gcount; ++q)
-                            for (int x = groups[C.goffset + q].task_begin; x < groups[C.goffset + q].task_end; ++x)
-                                gc[q] += cost(tasks[x]);
-                        std::vector<int> ord(C.gcount);
-                        std::iota(ord.begin(), ord.end(), 0);
-                        std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return gc[x] > gc[y]; });
-                        std::vector<qf::TileGroup> sorted(C.gcount);
-                        for (int q = 0; q < C.gcount; ++q) sorted[q] = groups[C.goffset + ord[q]];
-                        std::copy(sorted.begin(), sorted.end(), groups.begin() + C.goffset);
-                    } else {
-                        std::stable_sort(tasks.begin() + C.offset, tasks.end(),
-                                         [&](const qf::Task& x, const qf::Task& y) { return cost(x) > cost(y); });
-                    }
+                    if (tile == 1)
+                        longest_first(groups, C.goffset, tasks);
+                    else
+                        longest_first(tasks, C.offset);
                     b->launches.push_back(C);
                 }
     const size_t gdoubles = place_slots(b->launches);
