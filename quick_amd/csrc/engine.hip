@@ -588,10 +588,12 @@ struct qf_engine {
     DevBuf<double> d_Pb, d_Pt, d_Ps, d_Fa, d_Fb;   // open-shell builds (allocated on first use)
     DevBuf<double> d_Gt2;                           // their second exchange accumulators (replicas x n^2)
     DevBuf<double> d_zero;                          // nbasis^2 zeros: Coulomb density of an exchange-only pass
-    DevBuf<int> d_f0, d_f1;
+    DevBuf<int> d_shells;        // per shell: first and last function, atom (nshell each)
+    const int* shell_f0() const { return d_shells.p; }
+    const int* shell_f1() const { return d_shells.p + nshell; }
+    const int* shell_at() const { return d_shells.p + 2 * nshell; }
     DevBuf<unsigned long long> d_counts;
     DevBuf<double> d_cscratch;   // global slots of the wave-per-quartet classes that need them
-    DevBuf<int> d_shell_atom;    // original shell -> atom (gradient)
     DevBuf<double> d_gscratch;   // global slots of the gradient classes that need them (on first use)
     DevBuf<double> d_grad;       // gradient of the host entry point (on first use)
     bool grad_built = false;     // a gradient has run since the last prepare() (counts need it) ...
@@ -1283,275 +1285,308 @@ void longest_first(std::vector<qf::TileGroup>& groups, size_t first, const std::
     longest_first(groups.data() + first, work);
 }
 
-// Wave tasks, tile groups and launches of one engine, per quartet class and
-// precision.  `size` stands for the number of basis functions in the rules
-// that choose launch shapes: the engine's own, or for an engine in a batch
-// that of the molecule whose build holds as much work (the precision split
-// goes by the engine's own size); shared: tile and wave-per-quartet
-// classes share launches.  Index ranges are those of the output vectors.
-int make_tasks(const qf_engine* e, int size, std::vector<qf::Task>& tasks, std::vector<qf::TileGroup>& groups,
-               std::vector<qf_engine::Launch>& launches, qf_stats* stats, bool shared = false)
+// How a quartet class runs: the shape of its launch for one precision.
+struct ClassShape {
+    bool runs = false;       // (the FP32 half of a class that is not split does not)
+    int kind;                // 0 direct atomics, 1 LDS tile, 2 one quartet per wave
+    bool split, closed_only;
+    int mmax, win, piece;    // bras and kets a task, primitive pairs a piece
+    int tile_tasks, tile_waves;
+};
+
+// `size` stands for the number of basis functions in the rules that choose launch
+// shapes: the engine's own, or for an engine in a batch that of the molecule whose
+// build holds as much work (the precision split goes by the engine's own size);
+// shared: tile and wave-per-quartet classes share launches.
+int class_shape(const qf_engine* e, int cb, int ck, int fp32, int size, bool shared, ClassShape& out)
 {
-    const double thr_hi = e->split_thr;
-    tasks.clear();
-    if (tasks.capacity() < 32768) tasks.reserve(32768);   // most molecules': growing touches every page twice
-    groups.clear();
-    launches.clear();
-    const int piece = prim_piece(e, size, shared);
+    out.runs = false;
+    const int na = ncart(kClassL[cb][0]), nb = ncart(kClassL[cb][1]);
+    // bras per task: long loops for cheap classes (more register
+    // accumulation, fewer atomics), short ones for expensive classes
+    // (enough waves to fill 256 CUs)
+    const int ni = na * nb * ncart(kClassL[ck][0]) * ncart(kClassL[ck][1]);
+    const qf_engine::ClassTune& ct = e->ctune[cb][ck];
+    int mmax = ni <= 10 ? 16 : ni <= 36 ? 8 : ni <= 108 ? 4 : ni <= 324 ? 2 : 1;
+    // up to 32 functions at most 2 bras per task: more, shorter
+    // tasks for launches that hold few (QUICK's regression inputs
+    // up to 32 functions, geometric mean 16.3x -> 17.8x QUICK's
+    // saved build times; no gain above)
+    if (size <= 32) mmax = std::min(mmax, 2);
+    if (ct.mmax > 0) mmax = ct.mmax;
+    // tasks per tile workgroup: few for small molecules, whose launches
+    // hold few tasks (builds in us with 1 / 2 / 4 / 8 / 16: glycine
+    // 6-31G** 633 / 633 / 814 / 992 / 992, (H2O)8 6-31G* 924 / 885 / 975 /
+    // 928 / 1180, (H2O)8 cc-pVDZ (200 functions) 1077 / 1129 / 1202 / 1242 /
+    // 1447, C20H42 3-21G (264) 1825 / 1105 / 912 / 897 / 994, (H2O)16
+    // 3703 / 2940 / 3133 / 3171 / 3142, (H2O)32 25512 / 14599 / 12000 / 11245 /
+    // 10973; shared launches, 1 / 2 / 4: ethane 6-31G* 155 / 151 / 237, glycine
+    // 393 / 442 / 593, (H2O)8 6-31G* 516 / 526 / 628, its cation 853 / 677 / 753,
+    // (Gly)2 6-31G** 1438 / 1371 / 1889)
+    int tile_tasks = ct.tpg > 0        ? ct.tpg
+                           : e->tile_tasks > 0 ? e->tile_tasks
+                           : shared            ? (size <= 48 || size > 128 ? 2 : 1)
+                           : size <= 256       ? 2
+                           : size <= 400       ? 4
+                                               : 16;
+    int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
+    // LDS tile: (na + m*nb) x ncol exchange terms + m*na*nb Coulomb terms
+    int maxcol = 0;
+    for (const auto& Kb : e->blocks)
+        if (Kb.cls == ck) maxcol = std::max(maxcol, (int)Kb.colf.size());
+    const long long room = e->lds_budget / 8 - (long long)na * maxcol;
+    const long long mfit = room > 0 ? room / ((long long)nb * maxcol + na * nb) : 0;
+    // Mixed precision splits a class only where its FP32 half can run
+    // through the LDS-tile kernel: the direct-atomic FP32 kernels of
+    // (dp|dp) gave wrong Fock matrices on gfx950 and the (dd|dp) one
+    // non-finite values, while CPU builds of the same code are right.
+    // (dd|dp) and (dd|dd) stay FP64 (their FP32 forms spill several KB
+    // per lane: little to gain).
+    // classes without per-lane kernels (La+Lb+Lc+Ld >= 6) run every
+    // quartet in FP64 on the wave-per-quartet kernel
+    const bool lane_class = qf::fock_launcher(cb, ck) != nullptr;
+    // Classes with La+Lb+Lc+Ld >= split_lmin are split (qf_set_split_classes).
+    // FP32 quartets compute their Boys function, exponents and
+    // recursions in FP32, which shortens the primitive loop (the
+    // FP64 Boys function is most of a light class's work) and halves
+    // the registers of the spilling d classes.
+    const int Lsum_s = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
+    // By default every class above 256 functions, and only the
+    // classes with La+Lb+Lc+Ld >= 5 below: a small molecule's
+    // light classes hold too few quartets for the second launch
+    // to pay (256 batched molecules: 1389 builds/s splitting all,
+    // FP64 1432).
+    const int lmin = e->split_lmin >= 0 ? e->split_lmin : e->nbasis <= 256 ? 5 : 0;
+    const bool f_class = std::max(kClassL[cb][0], kClassL[ck][0]) == 3;   // f classes stay FP64
+    const bool split_class = e->prec == QF_PREC_MIXED && mfit >= 1 && lane_class && !f_class &&
+                             (ct.split >= 0 ? ct.split == 1 : Lsum_s >= lmin);
+    if (fp32 && !split_class) return QF_OK;
+    // wave-per-quartet kernel (FP64 launches of classes that have one)
+    // wave-per-quartet kernel: where the class tuning asks for it, and by
+    // default (unless qf_set_tile turned the shared-memory kernels off)
+    // for the d-heavy classes (La+Lb+Lc+Ld >= 6; in launches of one class >= 5 up to 128 functions and >= 4 up to 48,
+    // where few waves run and latency decides), whose per-lane
+    // kernels spill several KB per lane: one such quartet alone on a
+    // lane costs milliseconds, which dominates the build of a small
+    // molecule
+    const int Lsum = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
+    // (QUICK's regression inputs of 49-128 functions run their
+    // La+Lb+Lc+Ld = 4 classes faster on the tile kernel: PO4 6-31G*
+    // 15.8x -> 18.0x, PSB5 6-31G 26x -> 34x QUICK's build times;
+    // up to 48 functions and at 5 the wave-per-quartet kernel wins;
+    // in shared launches, with La+Lb+Lc+Ld >= 4 / 5 / 6 on it: water 72 / 79 / 97,
+    // ethane 6-31G* 211 / 155 / 151, butane 633 / 336 / 316, glycine 800 / 509 /
+    // 393, (H2O)8 6-31G* 972 / 635 / 516)
+    const int coop_lmin = shared ? (size <= 32 ? 4 : 6) : size <= 48 ? 4 : size <= 128 ? 5 : 6;
+    const bool tile_class = qf::fock_tile_launcher(cb, ck) != nullptr;
+    const bool tile_ok = tile_class && mfit >= 1;
+    // Classes whose FP64 tile kernel runs in Hermite Gaussians: above 256
+    // functions it takes over from the wave-per-quartet kernel ((dd|ds),
+    // (dd|pp) and (dp|dp) together: (H2O)32 10.65 -> 10.2 ms a build, (Gly)10
+    // mixed 29.4 -> 26.0; below, too few quartets fill its waves: glycine
+    // 6-31G** 0.63 -> 0.93, (H2O)8 cc-pVDZ 1.08 -> 1.26, which a batch does
+    // not change: 48 molecules 16.0 -> 16.9), with two waves,
+    // four tasks of one bra a workgroup ((dp|pp), (H2O)32: 10.5 ms against
+    // 10.7 with the other classes' shapes).
+    // A class without another tile kernel takes this one with tile = 1 on the
+    // same condition, else the wave-per-quartet kernel, as saved tables
+    // mean it: tile = 1 for these three, wave per quartet -> Hermite, water
+    // 0.12 -> 0.24 ms, glycine 0.42 -> 0.96, (H2O)8 6-31G* 0.63 -> 1.36, (H2O)12
+    // 1.41 -> 2.32, 256 batched molecules in mixed precision 68.0 -> 71.6, but
+    // (H2O)16 (304) 2.83 -> 2.80.
+    const bool md = !fp32 && tile_ok && qf::fock_tile_is_md(cb, ck);
+    const bool md_shape = md && e->nbasis > 256 && ct.tile < 0 && e->tile != 0;
+    if (md_shape && ct.mmax == 0) mmax = 1;
+    if (md_shape && ct.tpg == 0 && e->tile_tasks == 0) tile_tasks = 4;
+    if (md_shape && ct.waves == 0) tile_waves = std::min(tile_waves, 2);
+    const bool want_coop = ct.tile == 2   ? true
+                           : ct.tile == 1 ? !lane_class && !(tile_ok && e->nbasis > 256)
+                           : ct.tile == 0 || e->tile == 0 ? !lane_class
+                           : md_shape ? false
+                                      : Lsum >= coop_lmin || (!lane_class && !tile_ok);
+    const bool coop = !fp32 && want_coop && qf::fock_coop_launcher(cb, ck) != nullptr;
+    if (!coop && !lane_class && !tile_ok) return fail(QF_ERR_STATE, "class has no kernel for its launch");
+    const bool tile = !coop && tile_ok && (fp32 || !lane_class || (ct.tile >= 0 ? ct.tile != 0 : e->tile != 0));
+    if (tile) mmax = (int)std::min<long long>(mmax, mfit);
+    // kets per task: a full wave for the per-lane kernels; for the
+    // wave-per-quartet kernel a window (the class tuning's
+    // tasks_per_group): small windows give more workgroups to
+    // classes with few quartets
+    out.win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_window(size)) : qf::WAVE;
+    out.piece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : prim_piece(e, size, shared);
+    out.runs = true;
+    out.kind = coop ? 2 : tile ? 1 : 0;
+    out.split = split_class;
+    out.closed_only = tile && !fp32 && !lane_class;
+    out.mmax = mmax;
+    out.tile_tasks = tile_tasks;
+    out.tile_waves = tile_waves;
+    return QF_OK;
+}
+
+// Buffers of class_tasks, kept over its calls.
+struct TaskScratch {
     std::vector<std::pair<int, int>> chunks;   // bra chunks of a block
     std::vector<int> nall, nhigh, lo, hi;      // kets of each bra of a block, of each of a chunk
-    for (int cb = 0; cb < kNPC; ++cb)
-        for (int ck = 0; ck <= cb; ++ck)
-            for (int fp32 = 0; fp32 < 2; ++fp32) {
-                const int offset = (int)tasks.size();
-                const int goffset = (int)groups.size();
-                const int na = ncart(kClassL[cb][0]), nb = ncart(kClassL[cb][1]);
-                // bras per task: long loops for cheap classes (more register
-                // accumulation, fewer atomics), short ones for expensive classes
-                // (enough waves to fill 256 CUs)
-                const int ni = na * nb * ncart(kClassL[ck][0]) * ncart(kClassL[ck][1]);
-                const qf_engine::ClassTune& ct = e->ctune[cb][ck];
-                int mmax = ni <= 10 ? 16 : ni <= 36 ? 8 : ni <= 108 ? 4 : ni <= 324 ? 2 : 1;
-                // up to 32 functions at most 2 bras per task: more, shorter
-                // tasks for launches that hold few (QUICK's regression inputs
-                // up to 32 functions, geometric mean 16.3x -> 17.8x QUICK's
-                // saved build times; no gain above)
-                if (size <= 32) mmax = std::min(mmax, 2);
-                if (ct.mmax > 0) mmax = ct.mmax;
-                // tasks per tile workgroup: few for small molecules, whose launches
-                // hold few tasks (builds in us with 1 / 2 / 4 / 8 / 16: glycine
-                // 6-31G** 633 / 633 / 814 / 992 / 992, (H2O)8 6-31G* 924 / 885 / 975 /
-                // 928 / 1180, (H2O)8 cc-pVDZ (200 functions) 1077 / 1129 / 1202 / 1242 /
-                // 1447, C20H42 3-21G (264) 1825 / 1105 / 912 / 897 / 994, (H2O)16
-                // 3703 / 2940 / 3133 / 3171 / 3142, (H2O)32 25512 / 14599 / 12000 / 11245 /
-                // 10973; shared launches, 1 / 2 / 4: ethane 6-31G* 155 / 151 / 237, glycine
-                // 393 / 442 / 593, (H2O)8 6-31G* 516 / 526 / 628, its cation 853 / 677 / 753,
-                // (Gly)2 6-31G** 1438 / 1371 / 1889)
-                int tile_tasks = ct.tpg > 0        ? ct.tpg
-                                       : e->tile_tasks > 0 ? e->tile_tasks
-                                       : shared            ? (size <= 48 || size > 128 ? 2 : 1)
-                                       : size <= 256       ? 2
-                                       : size <= 400       ? 4
-                                                           : 16;
-                int tile_waves = ct.waves > 0 ? ct.waves : e->tile_waves;
-                // LDS tile: (na + m*nb) x ncol exchange terms + m*na*nb Coulomb terms
-                int maxcol = 0;
-                for (const auto& Kb : e->blocks)
-                    if (Kb.cls == ck) maxcol = std::max(maxcol, (int)Kb.colf.size());
-                const long long room = e->lds_budget / 8 - (long long)na * maxcol;
-                const long long mfit = room > 0 ? room / ((long long)nb * maxcol + na * nb) : 0;
-                // Mixed precision splits a class only where its FP32 half can run
-                // through the LDS-tile kernel: the direct-atomic FP32 kernels of
-                // (dp|dp) gave wrong Fock matrices on gfx950 and the (dd|dp) one
-                // non-finite values, while CPU builds of the same code are right.
-                // (dd|dp) and (dd|dd) stay FP64 (their FP32 forms spill several KB
-                // per lane: little to gain).
-                // classes without per-lane kernels (La+Lb+Lc+Ld >= 6) run every
-                // quartet in FP64 on the wave-per-quartet kernel
-                const bool lane_class = qf::fock_launcher(cb, ck) != nullptr;
-                // Classes with La+Lb+Lc+Ld >= split_lmin are split (qf_set_split_classes).
-                // FP32 quartets compute their Boys function, exponents and
-                // recursions in FP32, which shortens the primitive loop (the
-                // FP64 Boys function is most of a light class's work) and halves
-                // the registers of the spilling d classes.
-                const int Lsum_s = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
-                // By default every class above 256 functions, and only the
-                // classes with La+Lb+Lc+Ld >= 5 below: a small molecule's
-                // light classes hold too few quartets for the second launch
-                // to pay (256 batched molecules: 1389 builds/s splitting all,
-                // FP64 1432).
-                const int lmin = e->split_lmin >= 0 ? e->split_lmin : e->nbasis <= 256 ? 5 : 0;
-                const bool f_class = std::max(kClassL[cb][0], kClassL[ck][0]) == 3;   // f classes stay FP64
-                const bool split_class = e->prec == QF_PREC_MIXED && mfit >= 1 && lane_class && !f_class &&
-                                         (ct.split >= 0 ? ct.split == 1 : Lsum_s >= lmin);
-                if (fp32 && !split_class) continue;
-                // wave-per-quartet kernel (FP64 launches of classes that have one)
-                // wave-per-quartet kernel: where the class tuning asks for it, and by
-                // default (unless qf_set_tile turned the shared-memory kernels off)
-                // for the d-heavy classes (La+Lb+Lc+Ld >= 6; in launches of one class >= 5 up to 128 functions and >= 4 up to 48,
-                // where few waves run and latency decides), whose per-lane
-                // kernels spill several KB per lane: one such quartet alone on a
-                // lane costs milliseconds, which dominates the build of a small
-                // molecule
-                const int Lsum = kClassL[cb][0] + kClassL[cb][1] + kClassL[ck][0] + kClassL[ck][1];
-                // (QUICK's regression inputs of 49-128 functions run their
-                // La+Lb+Lc+Ld = 4 classes faster on the tile kernel: PO4 6-31G*
-                // 15.8x -> 18.0x, PSB5 6-31G 26x -> 34x QUICK's build times;
-                // up to 48 functions and at 5 the wave-per-quartet kernel wins;
-                // in shared launches, with La+Lb+Lc+Ld >= 4 / 5 / 6 on it: water 72 / 79 / 97,
-                // ethane 6-31G* 211 / 155 / 151, butane 633 / 336 / 316, glycine 800 / 509 /
-                // 393, (H2O)8 6-31G* 972 / 635 / 516)
-                const int coop_lmin = shared ? (size <= 32 ? 4 : 6) : size <= 48 ? 4 : size <= 128 ? 5 : 6;
-                const bool tile_class = qf::fock_tile_launcher(cb, ck) != nullptr;
-                const bool tile_ok = tile_class && mfit >= 1;
-                // Classes whose FP64 tile kernel runs in Hermite Gaussians: above 256
-                // functions it takes over from the wave-per-quartet kernel ((dd|ds),
-                // (dd|pp) and (dp|dp) together: (H2O)32 10.65 -> 10.2 ms a build, (Gly)10
-                // mixed 29.4 -> 26.0; below, too few quartets fill its waves: glycine
-                // 6-31G** 0.63 -> 0.93, (H2O)8 cc-pVDZ 1.08 -> 1.26, which a batch does
-                // not change: 48 molecules 16.0 -> 16.9), with two waves,
-                // four tasks of one bra a workgroup ((dp|pp), (H2O)32: 10.5 ms against
-                // 10.7 with the other classes' shapes).
-                // A class without another tile kernel takes this one with tile = 1 on the
-                // same condition, else the wave-per-quartet kernel, as saved tables
-                // mean it: tile = 1 for these three, wave per quartet -> Hermite, water
-                // 0.12 -> 0.24 ms, glycine 0.42 -> 0.96, (H2O)8 6-31G* 0.63 -> 1.36, (H2O)12
-                // 1.41 -> 2.32, 256 batched molecules in mixed precision 68.0 -> 71.6, but
-                // (H2O)16 (304) 2.83 -> 2.80.
-                const bool md = !fp32 && tile_ok && qf::fock_tile_is_md(cb, ck);
-                const bool md_shape = md && e->nbasis > 256 && ct.tile < 0 && e->tile != 0;
-                if (md_shape && ct.mmax == 0) mmax = 1;
-                if (md_shape && ct.tpg == 0 && e->tile_tasks == 0) tile_tasks = 4;
-                if (md_shape && ct.waves == 0) tile_waves = std::min(tile_waves, 2);
-                const bool want_coop = ct.tile == 2   ? true
-                                       : ct.tile == 1 ? !lane_class && !(tile_ok && e->nbasis > 256)
-                                       : ct.tile == 0 || e->tile == 0 ? !lane_class
-                                       : md_shape ? false
-                                                  : Lsum >= coop_lmin || (!lane_class && !tile_ok);
-                const bool coop = !fp32 && want_coop && qf::fock_coop_launcher(cb, ck) != nullptr;
-                if (!coop && !lane_class && !tile_ok) return fail(QF_ERR_STATE, "class has no kernel for its launch");
-                const bool tile = !coop && tile_ok && (fp32 || !lane_class || (ct.tile >= 0 ? ct.tile != 0 : e->tile != 0));
-                if (tile) mmax = (int)std::min<long long>(mmax, mfit);
-                // kets per task: a full wave for the per-lane kernels; for the
-                // wave-per-quartet kernel a window (the class tuning's
-                // tasks_per_group): small windows give more workgroups to
-                // classes with few quartets
-                const int win = coop ? (ct.tpg > 0 ? std::min(ct.tpg, qf::WAVE) : coop_window(size)) : qf::WAVE;
-                const int cpiece = ct.piece > 0 ? ct.piece : ct.piece < 0 ? 1 << 20 : piece;
-                size_t lds = 0, lds_os = 0;
-                long long group_tasks = 0;
-                for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
-                    const HostBlock& B = e->blocks[bbk];
-                    if (B.cls != cb) continue;
-                    for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
-                        const HostBlock& Kb = e->blocks[kbk];
-                        if (Kb.cls != ck) continue;
-                        if (cb == ck && kbk > bbk) continue;
-                        const bool same = (cb == ck && kbk == bbk);
-                        prefix_counts(B.info, Kb.info, e->list_cutoff(), true, nall);
-                        if (split_class) prefix_counts(B.info, Kb.info, thr_hi, false, nhigh);
-                        chunks.clear();
-                        for (const auto& g : B.groups)
-                            for (int c0 = g.first; c0 < g.second; c0 += mmax)
-                                chunks.push_back({c0, std::min(g.second, c0 + mmax)});
-                        for (const auto& g : chunks) {
-                            // per bra of the group: ket range [lo, hi) of this precision
-                            const int M = g.second - g.first;
-                            lo.resize(M);
-                            hi.resize(M);
-                            int nmax = 0;
-                            for (int k = 0; k < M; ++k) {
-                                const int i = B.bperm[g.first + k];
-                                const int n = same ? std::min(nall[i], i + 1) : nall[i];
-                                if (!fp32 && stats) stats->n_quartets_bound += n;
-                                const int n64 = split_class ? std::min(n, nhigh[i]) : n;
-                                lo[k] = fp32 ? n64 : 0;
-                                hi[k] = fp32 ? n : n64;
-                                nmax = std::max(nmax, hi[k]);
-                            }
-                            const int chunk_first = (int)tasks.size();
-                            for (int s0 = 0; s0 < nmax; s0 += win) {
-                                int kb = -1, ke = -1;
-                                for (int k = 0; k < M; ++k)
-                                    if (lo[k] < hi[k] && lo[k] < s0 + win && hi[k] > s0) {
-                                        if (kb < 0) kb = k;
-                                        ke = k + 1;
-                                    }
-                                if (kb < 0) continue;
-                                qf::Task t{};
-                                t.bra_block = (int)bbk;
-                                t.kb = g.first + kb;
-                                t.ke = g.first + ke;
-                                t.ket_block = (int)kbk;
-                                t.ket_start = s0;
-                                t.ket_count = std::min(win, nmax - s0);
-                                t.same_block = same ? 1 : 0;
-                                t.all_fp64 = split_class ? 0 : 1;
-                                // highly contracted pairs: spread the primitive
-                                // pairs of the window over several tasks
-                                each_piece(t, B.K, Kb.K, cpiece, [&](const qf::Task& x) { tasks.push_back(x); });
-                            }
-                            if (!tile) continue;
-                            // workgroups of the chunk: consecutive runs of its tasks
-                            const int chunk_end = (int)tasks.size();
-                            for (int t0 = chunk_first; t0 < chunk_end; t0 += tile_tasks) {
-                                qf::TileGroup tg{};
-                                tg.task_begin = t0;
-                                tg.task_end = std::min(chunk_end, t0 + tile_tasks);
-                                tg.chunk_kb = g.first;
-                                tg.nbra = M;
-                                groups.push_back(tg);
-                                group_tasks += tg.task_end - tg.task_begin;
-                            }
-                            if (chunk_end > chunk_first) {
-                                const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
-                                lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
-                                lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
-                            }
+};
+
+// Appends the wave tasks and tile groups of one class, precision and engine, whose
+// blocks are numbered from `base`; the launch's index ranges are those of the
+// vectors (count 0: it has none).  order: longest first (a batch orders over its
+// molecules itself).
+int class_tasks(const qf_engine* e, int cb, int ck, int fp32, const ClassShape& sh, int base, TaskScratch& sc,
+                std::vector<qf::Task>& tasks, std::vector<qf::TileGroup>& groups, qf_stats* stats, bool order,
+                qf_engine::Launch& L)
+{
+    const int offset = (int)tasks.size(), goffset = (int)groups.size();
+    const int na = ncart(kClassL[cb][0]), nb = ncart(kClassL[cb][1]);
+    const qf_engine::ClassTune& ct = e->ctune[cb][ck];
+    size_t lds = 0, lds_os = 0;
+    long long group_tasks = 0;
+    for (size_t bbk = 0; bbk < e->blocks.size(); ++bbk) {
+        const HostBlock& B = e->blocks[bbk];
+        if (B.cls != cb) continue;
+        for (size_t kbk = 0; kbk < e->blocks.size(); ++kbk) {
+            const HostBlock& Kb = e->blocks[kbk];
+            if (Kb.cls != ck) continue;
+            if (cb == ck && kbk > bbk) continue;
+            const bool same = (cb == ck && kbk == bbk);
+            prefix_counts(B.info, Kb.info, e->list_cutoff(), true, sc.nall);
+            if (sh.split) prefix_counts(B.info, Kb.info, e->split_thr, false, sc.nhigh);
+            sc.chunks.clear();
+            for (const auto& g : B.groups)
+                for (int c0 = g.first; c0 < g.second; c0 += sh.mmax)
+                    sc.chunks.push_back({c0, std::min(g.second, c0 + sh.mmax)});
+            for (const auto& g : sc.chunks) {
+                // per bra of the group: ket range [lo, hi) of this precision
+                const int M = g.second - g.first;
+                sc.lo.resize(M);
+                sc.hi.resize(M);
+                int nmax = 0;
+                for (int k = 0; k < M; ++k) {
+                    const int i = B.bperm[g.first + k];
+                    const int n = same ? std::min(sc.nall[i], i + 1) : sc.nall[i];
+                    if (!fp32 && stats) stats->n_quartets_bound += n;
+                    const int n64 = sh.split ? std::min(n, sc.nhigh[i]) : n;
+                    sc.lo[k] = fp32 ? n64 : 0;
+                    sc.hi[k] = fp32 ? n : n64;
+                    nmax = std::max(nmax, sc.hi[k]);
+                }
+                const int chunk_first = (int)tasks.size();
+                for (int s0 = 0; s0 < nmax; s0 += sh.win) {
+                    int kb = -1, ke = -1;
+                    for (int k = 0; k < M; ++k)
+                        if (sc.lo[k] < sc.hi[k] && sc.lo[k] < s0 + sh.win && sc.hi[k] > s0) {
+                            if (kb < 0) kb = k;
+                            ke = k + 1;
                         }
-                    }
+                    if (kb < 0) continue;
+                    qf::Task t{};
+                    t.bra_block = base + (int)bbk;
+                    t.kb = g.first + kb;
+                    t.ke = g.first + ke;
+                    t.ket_block = base + (int)kbk;
+                    t.ket_start = s0;
+                    t.ket_count = std::min(sh.win, nmax - s0);
+                    t.same_block = same ? 1 : 0;
+                    t.all_fp64 = sh.split ? 0 : 1;
+                    // highly contracted pairs: spread the primitive
+                    // pairs of the window over several tasks
+                    each_piece(t, B.K, Kb.K, sh.piece, [&](const qf::Task& x) { tasks.push_back(x); });
                 }
-                const int count = (int)tasks.size() - offset;
-                const int gcount = (int)groups.size() - goffset;
-                // longest first, unless the caller orders (a batch, over its molecules)
-                if (tile && gcount > 0) {
-                    if (stats) longest_first(groups, goffset, tasks);
-                } else if (e->shuffle && count > 1) {
-                    // deterministic permutation first: concurrent waves then hit different kets
-                    uint64_t st = 0x9E3779B97F4A7C15ull ^ (uint64_t)(cb * 12 + ck * 2 + fp32);
-                    for (int q = count - 1; q > 0; --q) {
-                        st ^= st << 13;
-                        st ^= st >> 7;
-                        st ^= st << 17;
-                        const int r = (int)(st % (uint64_t)(q + 1));
-                        std::swap(tasks[offset + q], tasks[offset + r]);
-                    }
-                    if (stats) longest_first(tasks, offset);
+                if (sh.kind != 1) continue;
+                // workgroups of the chunk: consecutive runs of its tasks
+                const int chunk_end = (int)tasks.size();
+                for (int t0 = chunk_first; t0 < chunk_end; t0 += sh.tile_tasks) {
+                    qf::TileGroup tg{};
+                    tg.task_begin = t0;
+                    tg.task_end = std::min(chunk_end, t0 + sh.tile_tasks);
+                    tg.chunk_kb = g.first;
+                    tg.nbra = M;
+                    groups.push_back(tg);
+                    group_tasks += tg.task_end - tg.task_begin;
                 }
-                if (count > 0) {
-                    qf_engine::Launch L{};
-                    L.closed_only = tile && !fp32 && !lane_class;
-                    L.cb = cb;
-                    L.ck = ck;
-                    L.fp32 = fp32;
-                    L.offset = offset;
-                    L.count = count;
-                    L.tile = coop ? 2 : (tile && gcount > 0) ? 1 : 0;
-                    L.goffset = goffset;
-                    L.gcount = gcount;
-                    L.waves = gcount > 0 ? (int)std::min<long long>(tile_waves,
-                                                                  std::max<long long>(1, (group_tasks + gcount - 1) / gcount))
-                                         : 1;
-                    L.lds = lds;
-                    L.lds_os = lds_os <= kMaxTileLds ? lds_os : 0;
-                    L.os_split = ct.os == 1;
-                    L.os_lean = ct.os == 2 || ct.os < 0;
-                    launches.push_back(L);
+                if (chunk_end > chunk_first) {
+                    const size_t kt = (size_t)(na + M * nb) * Kb.colf.size();
+                    lds = std::max(lds, sizeof(double) * (kt + (size_t)M * na * nb));
+                    lds_os = std::max(lds_os, sizeof(double) * (2 * kt + (size_t)M * na * nb));
                 }
-                if (stats) (fp32 ? stats->n_tasks_fp32 : stats->n_tasks_fp64) += count;
-            }
-    // every tile workgroup must stay inside its chunk and its LDS allocation
-    for (const auto& L : launches) {
-        if (L.tile != 1) continue;
-        const int na = ncart(kClassL[L.cb][0]), nb = ncart(kClassL[L.cb][1]);
-        for (int q = L.goffset; q < L.goffset + L.gcount; ++q) {
-            const qf::TileGroup& g = groups[q];
-            if (g.task_begin < L.offset || g.task_end > L.offset + L.count || g.task_begin >= g.task_end)
-                return fail(QF_ERR_STATE, "tile group outside its launch");
-            const qf::Task& t0 = tasks[g.task_begin];
-            const size_t need = sizeof(double) * ((size_t)(na + g.nbra * nb) * e->blocks[t0.ket_block].colf.size() +
-                                                  (size_t)g.nbra * na * nb);
-            if (need > L.lds) return fail(QF_ERR_STATE, "tile group exceeds its LDS allocation");
-            if (L.lds_os && 2 * need - sizeof(double) * (size_t)g.nbra * na * nb > L.lds_os)
-                return fail(QF_ERR_STATE, "tile group exceeds its open-shell LDS allocation");
-            for (int x = g.task_begin; x < g.task_end; ++x) {
-                const qf::Task& t = tasks[x];
-                if (t.bra_block != t0.bra_block || t.ket_block != t0.ket_block || t.kb < g.chunk_kb ||
-                    t.ke > g.chunk_kb + g.nbra || t.kb >= t.ke)
-                    return fail(QF_ERR_STATE, "tile group mixes chunks");
             }
         }
     }
+    const int count = (int)tasks.size() - offset;
+    const int gcount = (int)groups.size() - goffset;
+    if (sh.kind == 1) {
+        if (order) longest_first(groups, goffset, tasks);
+    } else if (e->shuffle && count > 1) {
+        // deterministic permutation first: concurrent waves then hit different kets
+        uint64_t st = 0x9E3779B97F4A7C15ull ^ (uint64_t)(cb * 12 + ck * 2 + fp32);
+        for (int q = count - 1; q > 0; --q) {
+            st ^= st << 13;
+            st ^= st >> 7;
+            st ^= st << 17;
+            const int r = (int)(st % (uint64_t)(q + 1));
+            std::swap(tasks[offset + q], tasks[offset + r]);
+        }
+        if (order) longest_first(tasks, offset);
+    }
+    L = qf_engine::Launch{};
+    L.closed_only = sh.closed_only;
+    L.cb = cb;
+    L.ck = ck;
+    L.fp32 = fp32;
+    L.offset = offset;
+    L.count = count;
+    L.tile = sh.kind;
+    L.goffset = goffset;
+    L.gcount = gcount;
+    L.waves = gcount > 0 ? (int)std::min<long long>(sh.tile_waves,
+                                                    std::max<long long>(1, (group_tasks + gcount - 1) / gcount))
+                         : 1;
+    L.lds = lds;
+    L.lds_os = lds_os <= kMaxTileLds ? lds_os : 0;
+    L.os_split = ct.os == 1;
+    L.os_lean = ct.os == 2 || ct.os < 0;
+    if (stats) (fp32 ? stats->n_tasks_fp32 : stats->n_tasks_fp64) += count;
+    // every tile workgroup must stay inside its chunk and its LDS allocation
+    for (int q = goffset; q < goffset + gcount; ++q) {
+        const qf::TileGroup& g = groups[q];
+        if (g.task_begin < offset || g.task_end > offset + count || g.task_begin >= g.task_end)
+            return fail(QF_ERR_STATE, "tile group outside its launch");
+        const qf::Task& t0 = tasks[g.task_begin];
+        const size_t need = sizeof(double) * ((size_t)(na + g.nbra * nb) * e->blocks[t0.ket_block - base].colf.size() +
+                                              (size_t)g.nbra * na * nb);
+        if (need > L.lds) return fail(QF_ERR_STATE, "tile group exceeds its LDS allocation");
+        if (L.lds_os && 2 * need - sizeof(double) * (size_t)g.nbra * na * nb > L.lds_os)
+            return fail(QF_ERR_STATE, "tile group exceeds its open-shell LDS allocation");
+        for (int x = g.task_begin; x < g.task_end; ++x) {
+            const qf::Task& t = tasks[x];
+            if (t.bra_block != t0.bra_block || t.ket_block != t0.ket_block || t.kb < g.chunk_kb ||
+                t.ke > g.chunk_kb + g.nbra || t.kb >= t.ke)
+                return fail(QF_ERR_STATE, "tile group mixes chunks");
+        }
+    }
+    return QF_OK;
+}
+
+// Tasks, tile groups and launches of the engine, per quartet class and precision.
+int make_tasks(qf_engine* e)
+{
+    e->tasks.clear();
+    e->groups.clear();
+    e->launches.clear();
+    TaskScratch sc;
+    for (int cb = 0; cb < kNPC; ++cb)
+        for (int ck = 0; ck <= cb; ++ck)
+            for (int fp32 = 0; fp32 < 2; ++fp32) {
+                ClassShape sh;
+                qf_engine::Launch L;
+                int rc = class_shape(e, cb, ck, fp32, e->nbasis, shares_launches(e), sh);
+                if (rc == QF_OK && sh.runs)
+                    rc = class_tasks(e, cb, ck, fp32, sh, 0, sc, e->tasks, e->groups, &e->stats, true, L);
+                if (rc) return rc;
+                if (sh.runs && L.count > 0) e->launches.push_back(L);
+            }
     return QF_OK;
 }
 
@@ -1724,7 +1759,7 @@ int prepare(qf_engine* e)
     e->split_thr = e->split * ymax * ymax;
     e->stats = qf_stats{};
     for (auto& b : e->blocks) e->stats.n_pairs += (long long)b.info.size();
-    rc = make_tasks(e, e->nbasis, e->tasks, e->groups, e->launches, &e->stats, shares_launches(e));
+    rc = make_tasks(e);
     if (rc) return rc;
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
@@ -1744,17 +1779,16 @@ int prepare(qf_engine* e)
     QF_HIP(e->d_Gs.resize(n2));
     QF_HIP(e->d_P.resize(n2));
     QF_HIP(e->d_cm.resize((size_t)e->nshell * e->nshell));
-    std::vector<int> f0(e->nshell), f1(e->nshell);
-    for (int s = 0; s < e->nshell; ++s) {
+    std::vector<int> shells(3 * (size_t)e->nshell);
+    for (int k = 0; k < e->nshell; ++k) {
         int nf = 0;
-        for (int L = e->s_lmin[s]; L <= e->s_lmax[s]; ++L) nf += ncart(L);
-        f0[s] = e->s_fstart[s];
-        f1[s] = e->s_fstart[s] + nf - 1;
+        for (int L = e->s_lmin[k]; L <= e->s_lmax[k]; ++L) nf += ncart(L);
+        shells[k] = e->s_fstart[k];
+        shells[e->nshell + k] = e->s_fstart[k] + nf - 1;
+        shells[2 * e->nshell + k] = e->s_atom[k];
     }
-    QF_HIP(e->d_f0.upload(f0));
-    QF_HIP(e->d_f1.upload(f1));
+    QF_HIP(e->d_shells.upload(shells));
     QF_HIP(e->d_mol.resize(4));   // slots: build / open-shell pass 1, open-shell pass 2, no-alloc build, gradient
-    QF_HIP(e->d_shell_atom.upload(e->s_atom));
     QF_HIP(e->d_counts.resize(2 * std::max<size_t>(1, e->launches.size())));
     e->stats.device_bytes = (long long)(e->d_info.bytes() + e->d_prim.bytes() + e->d_tasks.bytes() +
                                         e->d_Gt.bytes() * 3 + e->d_cm.bytes() + e->d_blocks.bytes());
@@ -2021,8 +2055,8 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     oa.G2 = os ? gb.Gt2 : nullptr;
     oa.ng = (size_t)n * n * gb.replicas;
     oa.cm = cm_out;
-    oa.f0 = e->d_f0.p;
-    oa.f1 = e->d_f1.p;
+    oa.f0 = e->shell_f0();
+    oa.f1 = e->shell_f1();
     oa.n = n;
     oa.nshell = ns;
     CloseArgs ca{};
@@ -2389,7 +2423,7 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     md.split = (e->prec == QF_PREC_MIXED) ? e->split_thr : 0.0;   // only separates the launches' halves
     md.replicas = 1;
     md.natom = e->natom;
-    md.shell_atom = e->d_shell_atom.p;
+    md.shell_atom = e->shell_at();
     md.grad = dgrad;
     qf::MolDesc* dmol = e->d_mol.p + 3;
     OpenArgs oa{};
@@ -2403,8 +2437,8 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
         oa.ng = (size_t)3 * e->natom;
     }
     oa.cm = cm_out;
-    oa.f0 = e->d_f0.p;
-    oa.f1 = e->d_f1.p;
+    oa.f0 = e->shell_f0();
+    oa.f1 = e->shell_f1();
     oa.n = e->nbasis;
     oa.nshell = e->nshell;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
@@ -3084,8 +3118,8 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
         bm.Gt = m.G;
         bm.Gs = b->d_Gs.p + poff[i];
         bm.cm = b->d_cm.p + cmoff[i];
-        bm.f0 = e->d_f0.p;
-        bm.f1 = e->d_f1.p;
+        bm.f0 = e->shell_f0();
+        bm.f1 = e->shell_f1();
         bm.n = e->nbasis;
         bm.ns = e->nshell;
         b->mols.push_back(bm);
@@ -3100,27 +3134,21 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
     double cube = 0.0;
     for (const qf_engine* e : b->engs) cube += std::pow((double)e->nbasis, 3.0);
     const int size = (int)std::cbrt(cube);
-    struct EngineTasks {
-        std::vector<qf::Task> tasks;
-        std::vector<qf::TileGroup> groups;
-        std::vector<qf_engine::Launch> launches;
-    };
-    std::vector<EngineTasks> et(count);
-    size_t ntasks = 0, ngroups = 0;
-    std::vector<qf::Task> scratch;   // kept over the engines: what grows touches new pages
-    for (int i = 0; i < count; ++i) {
-        rc = make_tasks(b->engs[i], size, scratch, et[i].groups, et[i].launches, nullptr);
-        if (rc) return bail(rc);
-        et[i].tasks.assign(scratch.begin(), scratch.end());
-        ntasks += et[i].tasks.size();
-        ngroups += et[i].groups.size();
-    }
-    tasks.reserve(ntasks);
-    groups.reserve(ngroups);
+    std::vector<ClassShape> shapes(count);
+    TaskScratch sc;
+    // room for the usual number (pieces and windows differ from the engines' own):
+    // growing would touch every page twice, what is not used is never touched
+    size_t expect = 0;
+    for (const qf_engine* e : b->engs) expect += e->tasks.size();
+    tasks.reserve(4 * expect);
+    groups.reserve(4 * expect);
     for (int cb = 0; cb < kNPC; ++cb)
         for (int ck = 0; ck <= cb; ++ck)
             for (int fp32 = 0; fp32 < 2; ++fp32)
                 for (int tile = 0; tile < 3; ++tile) {
+                    if (tile == 0)
+                        for (int i = 0; i < count; ++i)
+                            if ((rc = class_shape(b->engs[i], cb, ck, fp32, size, false, shapes[i]))) return bail(rc);
                     qf_engine::Launch C{};
                     C.cb = cb;
                     C.ck = ck;
@@ -3130,25 +3158,13 @@ int qf_batch_create_ext(qf_engine* const* engines, int count, int replicas, cons
                     C.goffset = (int)groups.size();
                     C.waves = 1;
                     for (int i = 0; i < count; ++i) {
-                        const EngineTasks* e = &et[i];
-                        for (const auto& L : e->launches) {
-                            if (L.cb != cb || L.ck != ck || L.fp32 != fp32 || L.tile != tile) continue;
-                            const int tbase = (int)tasks.size();
-                            for (int x = L.offset; x < L.offset + L.count; ++x) {
-                                qf::Task t = e->tasks[x];
-                                t.bra_block += boff[i];
-                                t.ket_block += boff[i];
-                                tasks.push_back(t);
-                            }
-                            for (int q = L.goffset; q < L.goffset + L.gcount; ++q) {
-                                qf::TileGroup g = e->groups[q];
-                                g.task_begin += tbase - L.offset;
-                                g.task_end += tbase - L.offset;
-                                groups.push_back(g);
-                            }
-                            C.lds = std::max(C.lds, L.lds);
-                            C.waves = std::max(C.waves, L.waves);
-                        }
+                        if (!shapes[i].runs || shapes[i].kind != tile) continue;
+                        qf_engine::Launch L;
+                        if ((rc = class_tasks(b->engs[i], cb, ck, fp32, shapes[i], boff[i], sc, tasks, groups, nullptr,
+                                              false, L)))
+                            return bail(rc);
+                        C.lds = std::max(C.lds, L.lds);
+                        C.waves = std::max(C.waves, L.waves);
                     }
                     C.count = (int)tasks.size() - C.offset;
                     C.gcount = (int)groups.size() - C.goffset;
