@@ -1,24 +1,32 @@
 """Per-class launch-shape autotuner for the Fock build.
 
-Every class launch of a build is timed with HIP events (launches run one
+Every class launch of a build is timed with HIP events (timed launches run one
 after another on one stream, so a class's time does not depend on the shape
 chosen for the others).  Each candidate shape is applied to all classes at
 once, a few builds are timed, and each (bra|ket) class then keeps the
 candidate that was fastest for it.  Works on a FockEngine (one molecule) or
 on a list of engines that are built as a FockBatch.
+
+A build as a program runs it is another thing than the sum of its launches: they
+overlap on four queues, and up to 200 functions classes share launches, with
+default shapes that were chosen for that.  The last step therefore compares whole
+builds and returns to the engine's defaults where those are not slower.
 """
 from __future__ import annotations
 
 import json
 import os
+import time
 
 import numpy as np
 
 # (digestion, waves, tasks_per_group, bras_per_task); digestion 0 direct
 # atomics, 1 LDS tile, 2 wave per quartet (classes without that kernel use
 # the tile; for it tasks_per_group is the ket window); 0 elsewhere = engine
-# default
+# default; digestion -1: the engine's default for the class
+DEFAULT = (-1, 0, 0, 0)
 CANDIDATES = [
+    DEFAULT,
     (0, 0, 0, 0), (0, 0, 0, 1), (0, 0, 0, 2), (0, 0, 0, 4),
     (1, 4, 16, 0), (1, 4, 8, 0), (1, 2, 8, 0), (1, 1, 4, 0), (1, 4, 32, 0),
     (1, 4, 16, 2), (1, 4, 16, 4), (1, 4, 32, 2), (1, 4, 32, 4),
@@ -43,6 +51,26 @@ def _class_times(build, launches, read_timing, set_timing, builds):
     return out
 
 
+def whole_time(build, samples=3, seconds=0.02):
+    """Seconds of an untimed build, or None without a GPU: the smallest average
+    over runs of builds that take ``seconds`` each.  The first builds after a
+    change of settings, which are issued launch by launch, are not counted."""
+    import torch
+    if not torch.cuda.is_available():
+        return None
+
+    def run(n):
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+        for _ in range(n):
+            build()
+        torch.cuda.synchronize()
+        return (time.perf_counter() - t0) / n
+    run(3)
+    n = max(2, min(200, int(seconds / run(1))))
+    return min(run(n) for _ in range(samples))
+
+
 NPC = 10    # pair classes s..f
 
 
@@ -53,7 +81,7 @@ def _class_index(name):
 
 
 def autotune(engines, stream, builds=2, candidates=CANDIDATES, batch_kw=None, make_density=None, densities=None,
-             pieces=PIECES, build=None, os_modes=None, split_modes=None):
+             pieces=PIECES, build=None, os_modes=None, split_modes=None, whole=whole_time):
     """Choose a launch shape per class, then a primitive piece size per class.
     ``engines``: one FockEngine or a list (tuned as one FockBatch).  Single
     engine: ``make_density(0)`` returns the device pointer (int) of the
@@ -66,7 +94,10 @@ def autotune(engines, stream, builds=2, candidates=CANDIDATES, batch_kw=None, ma
     appended to the candidate.  ``split_modes`` (e.g. (0, 1) for mixed
     engines): a last pass choosing per class between FP64 only and the
     precision split, timed over both halves; the candidate then carries
-    (..., piece, open-shell form or -1, split mode)."""
+    (..., piece, open-shell form or -1, split mode).  At the end ``whole(build)``
+    times whole builds with the settings found and with the engine's defaults; the
+    defaults are kept where they are not slower (``whole`` may return None: no
+    comparison)."""
     from .engine import FockBatch
     single = not isinstance(engines, (list, tuple))
     engs = [engines] if single else list(engines)
@@ -168,6 +199,29 @@ def autotune(engines, stream, builds=2, candidates=CANDIDATES, batch_kw=None, ma
             cand = tuple(cand) + ((-1,) if len(cand) < 6 else ())
             chosen[name] = (cand + (best,), stotal(best))
         autotune.last_split_times = stimes
+
+    def whole_build():
+        if single:
+            e = engs[0]
+            P = None if build is not None else make_density(0)
+            return whole(build if build is not None else lambda: e.fock2e_device(P, 0, stream))
+        b = FockBatch(engs, **dict(batch_kw or {}, graph=True))
+        for i, P in enumerate(densities):
+            b.set_density(i, P)
+        t = whole(lambda: b.build(stream))
+        b.close()
+        return t
+
+    found = whole_build()
+    if found is not None:
+        default = {name: (tuple(DEFAULT) + (0, -1, -1)[:len(cand) - 4], times.get(DEFAULT, {}).get((name, False)))
+                   for name, (cand, _) in chosen.items()}
+        apply_table(engs, {name: cand for name, (cand, _) in default.items()})
+        base = whole_build()
+        autotune.last_whole_times = {"found": found, "default": base}
+        if base <= found:
+            return default
+        apply_table(engs, {name: cand for name, (cand, _) in chosen.items()})
     return chosen
 
 
@@ -179,11 +233,13 @@ def autotune(engines, stream, builds=2, candidates=CANDIDATES, batch_kw=None, ma
 TABLE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning", "autotune.json")
 
 
-def tune_grad(engine, grad_call, calls=2):
+def tune_grad(engine, grad_call, calls=2, whole=whole_time):
     """Chooses each class's gradient kernel (per-lane or wave-per-quartet)
     from event-timed gradient calls of both kinds: ``grad_call()`` runs one
     gradient on the engine's stream.  Leaves the faster kernel set per class
-    and returns {class name: (mode, ms)}."""
+    and returns {class name: (mode, ms)}; where whole gradients are not slower
+    with the engine's defaults (up to 200 functions the classes then share
+    launches), those are kept: mode -1."""
     names = sorted({nm for nm, _, _ in engine.launches()})
     times = {}
     for mode in (1, 0):
@@ -198,6 +254,14 @@ def tune_grad(engine, grad_call, calls=2):
         engine.set_grad_class(*_class_index(nm), best)
         chosen[nm] = (best, tot[best])
     tune_grad.last_times = times
+    found = whole(grad_call)
+    if found is not None:
+        for nm in names:
+            engine.set_grad_class(*_class_index(nm), -1)
+        if whole(grad_call) <= found:
+            return {nm: (-1, chosen[nm][1]) for nm in names}
+        for nm in names:
+            engine.set_grad_class(*_class_index(nm), chosen[nm][0])
     return chosen
 
 

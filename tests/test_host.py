@@ -230,3 +230,48 @@ def test_tune_grad_keeps_the_faster_kernel_per_class():
     chosen = A.tune_grad(e, e.build, calls=2)
     assert chosen["(ss|ss)"][0] == 1 and chosen["(ps|ss)"][0] == 0
     assert e.grad[(0, 0)] == 1 and e.grad[(1, 0)] == 0
+
+
+@pytest.mark.parametrize("found,default", [(1.0, 0.5), (1.0, 1.0), (0.5, 1.0)])
+def test_autotune_returns_to_the_defaults_where_whole_builds_are_not_slower(found, default):
+    from quick_amd import autotune as A
+    e = _MockEngine()
+    seen = []
+
+    def whole(build):
+        build()
+        seen.append(dict(e.tune))
+        return default if all(t == A.DEFAULT for t in e.tune.values()) else found
+
+    chosen = A.autotune(e, 0, builds=1, candidates=[(1, 4, 8, 0), (2, 0, 0, 1)], pieces=[0, 8, -1], build=e.build,
+                        os_modes=(0, 1, 2), split_modes=(0, 1), whole=whole)
+    assert len(seen) == 2
+    if default <= found:
+        want = {(0, 0): (-1, 0, 0, 0, 0, -1, -1), (1, 0): (-1, 0, 0, 0, 0, -1, -1)}
+    else:
+        want = {(0, 0): (1, 4, 8, 0, 8, 2, 0), (1, 0): (2, 0, 0, 1, -1, 1, 1)}
+    for k, nm in e.NAMES.items():
+        assert chosen[nm][0] == want[k]
+        assert e.tune[k] + (e.piece[k], e.os[k], e.split[k]) == want[k]
+
+
+@pytest.mark.parametrize("found,default", [(1.0, 0.5), (0.5, 1.0)])
+def test_tune_grad_returns_to_the_defaults_where_whole_gradients_are_not_slower(found, default):
+    from quick_amd import autotune as A
+
+    class G(_MockEngine):
+        def __init__(self):
+            super().__init__()
+            self.grad = {k: -1 for k in self.NAMES}
+
+        def set_grad_class(self, cb, ck, mode):
+            self.grad[(cb, ck)] = mode
+
+        def cost(self, k, fp32):
+            return {(0, 0): {1: 1.0, 0: 3.0}, (1, 0): {1: 2.0, 0: 1.5}}[k][self.grad[k]]
+
+    e = G()
+    whole = lambda call: default if set(e.grad.values()) == {-1} else found
+    chosen = A.tune_grad(e, e.build, calls=2, whole=whole)
+    want = {(0, 0): -1, (1, 0): -1} if default <= found else {(0, 0): 1, (1, 0): 0}
+    assert e.grad == want and {k: chosen[nm][0] for k, nm in e.NAMES.items()} == want
