@@ -696,7 +696,8 @@ def launcher_source(name, diag, coop=False, lane=True, fp32=True, md=False):
                  " g, ng, t, b, m, 0);" % name])
         out += ["}", ""]
     elif md:
-        out += ["// closed shell, FP64 only (an open-shell build runs the class in two passes)",
+        out += ["// closed shell, FP64 only: an open-shell build runs the wave-per-quartet kernel",
+                "// instead, unless the class is asked for in two closed-shell passes",
                 "void launch_fock_tile_%s(const TileGroup* g, int ng, const Task* t, const PairBlock* b,"
                 " const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, LaunchTo& q)" % name, "{",
                 "    if (ng <= 0) return;",

@@ -4,7 +4,8 @@
 
 namespace qf {
 
-// closed shell, FP64 only (an open-shell build runs the class in two passes)
+// closed shell, FP64 only: an open-shell build runs the wave-per-quartet kernel
+// instead, unless the class is asked for in two closed-shell passes
 void launch_fock_tile_C2211(const TileGroup* g, int ng, const Task* t, const PairBlock* b, const MolDesc* m, int fp32, int os, int waves, size_t lds, int grid, LaunchTo& q)
 {
     if (ng <= 0) return;
