@@ -1157,7 +1157,7 @@ int make_plan(qf_engine* e, int kind)
 // shares_launches, where the grid is capped (qf_set_persistent caps each class's)
 // and where a gradient kernel was chosen.  The plan of the closed shell is made by
 // prepare, the others at the first call: a closed-shell program never uses them
-// (prepare of water 6-31G* 0.48 -> 0.35 ms, (H2O)8 cc-pVDZ 4.2 -> 3.4).  Under
+// (prepare of water 6-31G* 496 -> 418 us, (H2O)8 cc-pVDZ 4226 -> 3717).  Under
 // capture, where nothing can be uploaded, a first open-shell build or gradient has
 // one launch per class.
 int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
@@ -1192,7 +1192,13 @@ int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
 // pieces; 1 / 2 / 3 / 4 / 6: water 113 / 72 / 91 / - / -, ethane 6-31G* (42) 217 / 151 /
 // 255 / 303 / 436, butane 775 / 402 / 357 / 316 / 606, glycine 1116 / 548 / 401 / 393 /
 // 436, (H2O)8 6-31G* 1753 / 865 / 587 / 580 / 526, (Gly)2 3839 / 2116 / 1478 / 1472 /
-// 1371.
+// 1371.  Up to 200 functions the other sizes therefore serve batches (by their
+// summed size) and qf_set_tile(0) only, and rest on the single builds above.
+// Batches, pieces of 1 / 2 / 3: two molecules 6-31G (size 19) 202 / 104 / 119, 6-31G*
+// (26) 287 / 218 / 240, four molecules 3-21G (37) 106 / 130 / 149, three 6-31G* (41)
+// 351 / 309 / 417, five 6-31G* (69) 812 / 484 / 529, eight 6-31G (79) 1308 / 543 /
+// 394, eight 6-31G* (114) 2180 / 1117 / 896; water 6-31G* without tiles 278 / 210 / -.
+// At sizes up to 48 pieces of 2 would serve all of these better but 3-21G.
 int prim_piece(const qf_engine* e, int size, bool shared)
 {
     return e->prim_piece > 0   ? e->prim_piece
@@ -1322,7 +1328,12 @@ int class_shape(const qf_engine* e, int cb, int ck, int fp32, int size, bool sha
     // 3703 / 2940 / 3133 / 3171 / 3142, (H2O)32 25512 / 14599 / 12000 / 11245 /
     // 10973; shared launches, 1 / 2 / 4: ethane 6-31G* 155 / 151 / 237, glycine
     // 393 / 442 / 593, (H2O)8 6-31G* 516 / 526 / 628, its cation 853 / 677 / 753,
-    // (Gly)2 6-31G** 1438 / 1371 / 1889)
+    // (Gly)2 6-31G** 1438 / 1371 / 1889; between, (H2O)3 6-31G* (57) 275 / 270 / 470,
+    // (H2O)4 (76) 327 / 494 / 575, butane (80) 348 / 343 / 581, (H2O)5 (95) 363 / 386 /
+    // 577, C5H12 (99) 481 / 497 / 913, (H2O)6 (114) 428 / 425 / 700, C6H14 (118) 617 /
+    // 648 / 980; batches, 1 / 2 / 4 / 8: two molecules 6-31G* (size 26) 385 / 296 / 252 /
+    // 273, five (69) 477 / 474 / 515 / 591, twelve (186) 1971 / 2202 / 2651 / 2517, 24 (272)
+    // 4396 / 4963 / 6236 / 6061: the line at 256 is the single molecules')
     int tile_tasks = ct.tpg > 0        ? ct.tpg
                            : e->tile_tasks > 0 ? e->tile_tasks
                            : shared            ? (size <= 48 || size > 128 ? 2 : 1)
@@ -1376,7 +1387,7 @@ int class_shape(const qf_engine* e, int cb, int ck, int fp32, int size, bool sha
     // up to 48 functions and at 5 the wave-per-quartet kernel wins;
     // in shared launches, with La+Lb+Lc+Ld >= 4 / 5 / 6 on it: water 72 / 79 / 97,
     // ethane 6-31G* 211 / 155 / 151, butane 633 / 336 / 316, glycine 800 / 509 /
-    // 393, (H2O)8 6-31G* 972 / 635 / 516)
+    // 393, (H2O)8 6-31G* 972 / 635 / 516; small batches were not measured)
     const int coop_lmin = shared ? (size <= 32 ? 4 : 6) : size <= 48 ? 4 : size <= 128 ? 5 : 6;
     const bool tile_class = qf::fock_tile_launcher(cb, ck) != nullptr;
     const bool tile_ok = tile_class && mfit >= 1;
