@@ -562,6 +562,8 @@ struct qf_engine {
         DevBuf<qf::FusedBlock> d_fused;
     };
     Plan plan[4];                             // closed shell, open shell, gradient; one launch per class
+    bool shared = false;                      // up to the sizes of shares_launches
+    size_t grad_slots = 0;                    // doubles of global slots of the gradient's shared launches
     SideStreams* side = nullptr;              // taken at the first forked build
     Replay replay[3];                         // closed shell, open shell, gradient
     void drop_replays()
@@ -1126,7 +1128,11 @@ size_t grad_shared_slots(const qf_engine* e)
 {
     size_t sum = 0;
     int count[qf::kGradFuseKernels] = {};
-    for (const auto& L : e->launches) count[qf::grad_fuse_bucket(L.cb, L.ck)] += L.count;
+    for (const auto& L : e->launches) {
+        const int k = qf::grad_fuse_bucket(L.cb, L.ck);
+        if (k < 0) return 0;   // an f class: gradients are refused
+        count[k] += L.count;
+    }
     for (int k = 0; k < qf::kGradFuseKernels; ++k)
         sum += (size_t)qf::grad_fuse_kernel(k).global * std::min(count[k], qf::COOP_GLOBAL_SLICES);
     return sum;
@@ -1162,7 +1168,7 @@ int make_plan(qf_engine* e, int kind)
 // one launch per class.
 int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
 {
-    bool plain = e->persist > 0 || !shares_launches(e);
+    bool plain = e->persist > 0 || !e->shared;
     if (kind == 2 && !plain) {
         plain = !e->grad_lane;
         for (const auto& row : e->ctune)
@@ -1583,6 +1589,7 @@ int class_tasks(const qf_engine* e, int cb, int ck, int fp32, const ClassShape& 
 // Tasks, tile groups and launches of the engine, per quartet class and precision.
 int make_tasks(qf_engine* e)
 {
+    e->shared = shares_launches(e);
     e->tasks.clear();
     e->groups.clear();
     e->launches.clear();
@@ -1592,7 +1599,7 @@ int make_tasks(qf_engine* e)
             for (int fp32 = 0; fp32 < 2; ++fp32) {
                 ClassShape sh;
                 qf_engine::Launch L;
-                int rc = class_shape(e, cb, ck, fp32, e->nbasis, shares_launches(e), sh);
+                int rc = class_shape(e, cb, ck, fp32, e->nbasis, e->shared, sh);
                 if (rc == QF_OK && sh.runs)
                     rc = class_tasks(e, cb, ck, fp32, sh, 0, sc, e->tasks, e->groups, &e->stats, true, L);
                 if (rc) return rc;
@@ -1615,7 +1622,7 @@ int make_alt_tasks(qf_engine* e, hipStream_t s)
     std::vector<int> nall;
     auto each_task = [&](const qf_engine::Launch& L, auto&& f) {
         const int ct = e->ctune[L.cb][L.ck].piece;
-        const int piece = ct > 0 ? ct : ct < 0 ? 1 << 20 : prim_piece(e, e->nbasis, shares_launches(e));
+        const int piece = ct > 0 ? ct : ct < 0 ? 1 << 20 : prim_piece(e, e->nbasis, e->shared);
         const int win = coop_window(e->nbasis);
         for (int bb = 0; bb < (int)e->blocks.size(); ++bb)
             for (int kb = 0; kb < (int)e->blocks.size(); ++kb) {
@@ -1779,10 +1786,11 @@ int prepare(qf_engine* e)
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
     size_t gdoubles = place_slots(e->launches);
-    if (shares_launches(e)) gdoubles = std::max({gdoubles, shared_slots(e, 0), shared_slots(e, 1)});
+    if (e->shared) gdoubles = std::max({gdoubles, shared_slots(e, 0), shared_slots(e, 1)});
+    e->grad_slots = e->shared ? grad_shared_slots(e) : 0;
     if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles));
     for (auto& p : e->plan) p.made = false;
-    if ((rc = make_plan(e, shares_launches(e) ? 0 : 3))) return rc;
+    if ((rc = make_plan(e, e->shared ? 0 : 3))) return rc;
 
     // ---- per-build buffers -------------------------------------------------
     const size_t n2 = (size_t)e->nbasis * e->nbasis;
@@ -2416,7 +2424,7 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
             gdoubles += (size_t)qf::grad_global_doubles(L.cb, L.ck) *
                         std::min(wave_tasks(e, L).count, qf::COOP_GLOBAL_SLICES);
     }
-    if (shares_launches(e)) gdoubles = std::max(gdoubles, grad_shared_slots(e));
+    gdoubles = std::max(gdoubles, e->grad_slots);
     if (gdoubles && e->d_gscratch.n < gdoubles) {
         e->replay[2].drop();   // it holds the old buffer
         QF_HIP(e->d_gscratch.resize(gdoubles));
