@@ -202,6 +202,30 @@ bool is_capturing(hipStream_t s)
     return st != hipStreamCaptureStatusNone;
 }
 
+// Id of the capture that s takes part in, 0 for none.
+unsigned long long capture_of(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(s, &st, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return ~0ull;
+    }
+    return st == hipStreamCaptureStatusNone ? 0 : id;
+}
+
+// Whether work on s may be forked onto the side streams: those that took part in a
+// capture belong to it until it ends, and can serve no other stream.
+bool side_free(const SideStreams& side, hipStream_t s)
+{
+    const unsigned long long of = capture_of(s);
+    for (hipStream_t q : side.s) {
+        const unsigned long long id = capture_of(q);
+        if (id != 0 && id != of) return false;
+    }
+    return true;
+}
+
 // Makes sure `side` has its streams, unless s is being captured (creating
 // streams is no work for a capture; without them everything runs on s).
 bool side_ready(SideStreams*& side, int device, hipStream_t s)
@@ -1887,7 +1911,7 @@ template <class F>
 int issue_forked(SideStreams* side, hipStream_t s, const std::vector<std::pair<int, int>>& order, F&& issue)
 {
     int rc = QF_OK;
-    if (!side) {
+    if (!side || !side_free(*side, s)) {
         for (const auto& o : order)
             if ((rc = issue(o.first, s))) return rc;
         return rc;

@@ -36,7 +36,9 @@ std::map<const void*, std::string> names;
 std::vector<Op> ops;
 std::map<void*, std::set<int>> stream_last;   // what the next operation of a stream waits for
 std::map<void*, std::set<int>> event_at;
-std::set<void*> capturing;
+std::map<void*, int> capturing;                // id of the capture a stream takes part in
+std::map<void*, int> event_capture;
+std::vector<void*> streams;                    // created and not destroyed
 std::string text;
 hipError_t last_error = hipSuccess;
 std::string fail_name;
@@ -84,7 +86,17 @@ struct Call {
 // ---- the test's side
 MOCK void mock_clear() { ops.clear(); stream_last.clear(); event_at.clear(); }
 MOCK void mock_fail(const char* fn, int after) { fail_name = fn; fail_after = after; }
-MOCK void mock_capture(void* s, int on) { on ? (void)capturing.insert(s) : (void)capturing.erase(s); }
+// begins capture `id` on a stream, or (0) ends the one it takes part in
+MOCK void mock_capture(void* s, int id)
+{
+    if (id) {
+        capturing[s] = id;
+        return;
+    }
+    const int was = capturing.count(s) ? capturing[s] : 0;
+    for (auto it = capturing.begin(); it != capturing.end();) it = it->second == was ? capturing.erase(it) : ++it;
+}
+MOCK int mock_streams() { return (int)streams.size(); }
 MOCK long long mock_uploaded() { return uploaded; }
 MOCK void mock_upload_reset() { uploaded = 0; }
 // one line per launch: index, name, grid, slot buffer (0: none), indices it waits for
@@ -146,13 +158,26 @@ MOCK hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned)
 {
     MAY_FAIL;
     *s = (hipStream_t) new char;
+    streams.push_back(*s);
     return hipSuccess;
 }
-MOCK hipError_t hipStreamDestroy(hipStream_t s) { delete (char*)s; return hipSuccess; }
+MOCK hipError_t hipStreamDestroy(hipStream_t s)
+{
+    for (size_t k = 0; k < streams.size(); ++k)
+        if (streams[k] == s) streams.erase(streams.begin() + k--);
+    delete (char*)s;
+    return hipSuccess;
+}
 MOCK hipError_t hipStreamSynchronize(hipStream_t) { MAY_FAIL; return hipSuccess; }
 MOCK hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st)
 {
     *st = capturing.count(s) ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+MOCK hipError_t hipStreamGetCaptureInfo(hipStream_t s, hipStreamCaptureStatus* st, unsigned long long* id)
+{
+    hipStreamIsCapturing(s, st);
+    if (id) *id = capturing.count(s) ? capturing[s] : 0;
     return hipSuccess;
 }
 MOCK hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
@@ -171,11 +196,17 @@ MOCK hipError_t hipEventRecord(hipEvent_t e, hipStream_t s)
 {
     MAY_FAIL;
     event_at[e] = stream_last[s];
+    event_capture[e] = capturing.count(s) ? capturing[s] : 0;
     return hipSuccess;
 }
 MOCK hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
 {
     MAY_FAIL;
+    // a stream outside takes part in a capture by its first wait; one of another capture, or a
+    // captured one that waits for work outside it, is an error
+    const int mine = capturing.count(s) ? capturing[s] : 0, theirs = event_capture[e];
+    if (mine && mine != theirs) return last_error = hipErrorStreamCaptureIsolation;
+    if (theirs) capturing[s] = theirs;
     stream_last[s].insert(event_at[e].begin(), event_at[e].end());
     return hipSuccess;
 }

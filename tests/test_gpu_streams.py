@@ -212,3 +212,32 @@ def test_first_open_shell_build_and_gradient_under_capture(name, basis):
         s.synchronize()
         for x, w in zip((Fa, Fb, g), want):
             assert np.abs(x.cpu().numpy() - w).max() <= 1e-11 * max(1.0, np.abs(w).max())
+
+
+def test_batch_build_beside_a_capture_of_the_batch():
+    """While a capture holds the batch's side streams, a build on another stream
+    goes without them and disturbs neither."""
+    announce("streams batch beside capture")
+    from quick_amd.engine import FockBatch
+    sets = [setup(n) for n in ("water", "water3")]
+    b = FockBatch([e for e, _, _ in sets])
+    for i, (_, P, _) in enumerate(sets):
+        b.set_density(i, P.cpu().numpy())
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    b.build(s.cuda_stream)
+    torch.cuda.synchronize()
+    b.clear_fock(t.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
+            b.build(s.cuda_stream)
+            b.build(t.cuda_stream)
+    torch.cuda.synchronize()
+    for k in range(3):                  # the build on t, then each replay
+        for i, (_, _, G) in enumerate(sets):
+            F = b.get(i, g=False, f=True)[1]
+            assert np.abs(F - (k + 1) * G).max() <= 1e-11 * max(1.0, np.abs(G).max())
+        g.replay()
+        torch.cuda.synchronize()
+    b.close()

@@ -305,3 +305,41 @@ for kind in kinds:
     assert any("fused_" in o.name for o in launches(mock)) and mock.mock_uploaded() == made
     e.close()
 """)
+
+
+@pytest.mark.parametrize("what", ["engine", "batch"])
+def test_builds_beside_a_capture_of_the_same_engine(mock, what):
+    """The side streams of an engine or batch that took part in a capture belong to
+    it until it ends: a build on another stream meanwhile, captured or not, goes
+    without them."""
+    mock_hip.run(mock, BUILD + f"""
+from quick_amd.engine import FockBatch
+e = engine(M.polyglycine(2), "6-31G**")
+n = e.n
+P, F = np.zeros((n, n)), np.zeros((n, n))
+if {what!r} == "batch":
+    b = FockBatch([e])
+    build = lambda s: b.build(s)
+else:
+    build = lambda s: e.fock2e_device(P.ctypes.data, F.ctypes.data, s)
+one, two, three = 1 << 20, 2 << 20, 3 << 20     # three streams of the caller
+build(one)
+assert mock.mock_streams() == 3
+def issue(s, name):
+    mock.mock_clear()
+    build(s)
+    ops = launches(mock)
+    assert {{int(x) for x in mock.mock_stream(s).decode().split()}}
+    forked = any(len(o.deps) > 1 for o in ops)
+    return forked
+mock.mock_capture(one, 1)
+assert issue(one, "captured")                    # forks
+e.set_persistent(0)                              # no graph to replay: issued launch by launch
+assert not issue(two, "beside it")
+mock.mock_capture(three, 2)
+assert not issue(three, "another capture beside it")
+mock.mock_capture(one, 0)
+mock.mock_capture(three, 0)
+e.set_persistent(0)
+assert issue(two, "after it")
+""")
