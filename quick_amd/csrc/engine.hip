@@ -456,6 +456,7 @@ struct Replay {
             (void)hipGraphExecDestroy(exec);
         }
         if (graph) (void)hipGraphDestroy(graph);
+        (void)hipGetLastError();
         exec = nullptr;
         graph = nullptr;
         uses = 0;
@@ -1187,9 +1188,9 @@ int make_plan(qf_engine* e, int kind)
 // shares_launches, where the grid is capped (qf_set_persistent caps each class's)
 // and where a gradient kernel was chosen.  The plan of the closed shell is made by
 // prepare, the others at the first call: a closed-shell program never uses them
-// (prepare of water 6-31G* 496 -> 418 us, (H2O)8 cc-pVDZ 4226 -> 3717).  Under
-// capture, where nothing can be uploaded, a first open-shell build or gradient has
-// one launch per class.
+// (prepare of water 6-31G* 496 -> 418 us, (H2O)8 cc-pVDZ 4226 -> 3717).  Where the
+// plan cannot be uploaded, as under capture or while another stream is captured, a
+// first open-shell build or gradient has one launch per class.
 int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
 {
     bool plain = e->persist > 0 || !e->shared;
@@ -1198,7 +1199,7 @@ int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
         for (const auto& row : e->ctune)
             for (const auto& c : row) plain = plain || c.grad >= 0;
     }
-    if (!plain && !e->plan[kind].made && is_capturing(s)) plain = true;
+    if (!plain && !e->plan[kind].made) plain = is_capturing(s) || make_plan(e, kind) != QF_OK;
     if (plain) kind = 3;
     *out = &e->plan[kind];
     return make_plan(e, kind);
@@ -1634,15 +1635,16 @@ int make_tasks(qf_engine* e)
 
 // Wave-per-quartet tasks of the closed_only classes, at the first open-shell build
 // or gradient since a prepare: a closed-shell program never runs them (made by
-// prepare they took it from 24 to 50 ms for (Gly)10 6-31G**).  Not under capture,
-// where nothing can be uploaded: until then those kernels run the tile tasks,
-// whose windows of 64 kets leave longer tails.
-int make_alt_tasks(qf_engine* e, hipStream_t s)
+// prepare they took it from 24 to 50 ms for (Gly)10 6-31G**).  Where they cannot be
+// uploaded, as under capture or while another stream is captured, those kernels run
+// the tile tasks, whose windows of 64 kets leave longer tails, and the next call
+// tries again.
+void make_alt_tasks(qf_engine* e, hipStream_t s)
 {
-    if (e->alt_made) return QF_OK;
+    if (e->alt_made) return;
     bool any = false;
     for (const auto& L : e->launches) any = any || L.closed_only;
-    if (any && is_capturing(s)) return QF_OK;
+    if (any && is_capturing(s)) return;
     std::vector<int> nall;
     auto each_task = [&](const qf_engine::Launch& L, auto&& f) {
         const int ct = e->ctune[L.cb][L.ck].piece;
@@ -1697,11 +1699,10 @@ int make_alt_tasks(qf_engine* e, hipStream_t s)
     hipError_t err = e->d_alt.resize(total);
     if (err == hipSuccess && total)
         err = hipMemcpy(e->d_alt.p, tasks.get(), total * sizeof(qf::Task), hipMemcpyHostToDevice);
-    if (err != hipSuccess)
-        for (auto& L : e->launches) L.alt_count = 0;
-    QF_HIP(err);
-    e->alt_made = true;
-    return QF_OK;
+    e->alt_made = err == hipSuccess;
+    if (e->alt_made) return;
+    (void)hipGetLastError();
+    for (auto& L : e->launches) L.alt_count = 0;
 }
 
 // Tasks of a class for its wave-per-quartet kernels.
@@ -2213,7 +2214,7 @@ int build_os(qf_engine* e, const double* dPa, const double* dPb, double* dFa, do
 {
     if (!e->prepared) return fail(QF_ERR_STATE, "qf_prepare has not been called");
     const int n2 = e->nbasis * e->nbasis;
-    if (int rc = make_alt_tasks(e, s)) return rc;
+    make_alt_tasks(e, s);
     QF_HIP(e->d_Pt.resize(n2));
     QF_HIP(e->d_Ps.resize(n2));
     double* cm_out = dcm ? nullptr : e->d_cm.p;
@@ -2439,7 +2440,7 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     for (const auto& L : e->launches)
         if (!qf::grad_launcher(L.cb, L.ck))
             return fail(QF_ERR_ARG, "ERI gradients cover shells up to d; this basis has f shells");
-    if (int rc = make_alt_tasks(e, s)) return rc;
+    make_alt_tasks(e, s);
     size_t gdoubles = 0;
     std::vector<size_t> gslot;   // per launch: its region of the global slot buffer
     for (const auto& L : e->launches) {

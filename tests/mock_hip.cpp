@@ -42,7 +42,7 @@ std::vector<void*> streams;                    // created and not destroyed
 std::string text;
 hipError_t last_error = hipSuccess;
 std::string fail_name;
-int fail_after = -1;
+int fail_after = -1, failed = 0;
 long long uploaded = 0;    // bytes copied to the device
 
 // true where the test asked this call to fail
@@ -50,6 +50,7 @@ bool fails(const char* fn)
 {
     if (fail_after < 0 || fail_name != fn) return false;
     if (fail_after-- > 0) return false;
+    ++failed;
     last_error = hipErrorInvalidValue;
     return true;
 }
@@ -85,7 +86,14 @@ struct Call {
 
 // ---- the test's side
 MOCK void mock_clear() { ops.clear(); stream_last.clear(); event_at.clear(); }
-MOCK void mock_fail(const char* fn, int after) { fail_name = fn; fail_after = after; }
+// makes the call after `after` more of its name fail; how many have since
+MOCK void mock_fail(const char* fn, int after)
+{
+    fail_name = fn;
+    fail_after = after;
+    failed = 0;
+}
+MOCK int mock_failed() { return failed; }
 // begins capture `id` on a stream, or (0) ends the one it takes part in
 MOCK void mock_capture(void* s, int id)
 {

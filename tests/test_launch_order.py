@@ -343,3 +343,28 @@ mock.mock_capture(three, 0)
 e.set_persistent(0)
 assert issue(two, "after it")
 """)
+
+
+@pytest.mark.parametrize("mol", ["M.polyglycine(1)", "M.alkane(14)"])
+@pytest.mark.parametrize("kind", ["os", "grad"])
+@pytest.mark.parametrize("call", ["hipMemcpy", "hipMalloc"])
+def test_a_first_build_goes_on_where_its_own_tables_cannot_be_uploaded(mock, mol, kind, call):
+    """As while another stream of the thread is captured: the build runs what prepare
+    made, and the next one tries again."""
+    mock_hip.run(mock, BUILD + f"""
+e = engine({mol}, "6-31G*")
+closing = {kind!r} == "os"
+own = builds(e, {kind!r}, 2, closing=closing) and [(o.name, o.grid) for o in launches(mock)]
+# other tables than the ones that were made: a larger buffer is needed
+e.set_cutoffs(1e-14)
+e.prepare()
+mock.mock_fail(b"{call}", 0)
+builds(e, {kind!r}, 1, closing=closing)
+plain = [(o.name, o.grid) for o in launches(mock)]
+assert mock.mock_failed() == 1, "the call that was to fail was not made"
+mock.mock_fail(b"", -1)
+builds(e, {kind!r}, 3, closing=closing)
+again = [(o.name, o.grid) for o in launches(mock)]
+assert plain != again
+assert sorted(n for n, _ in own) == sorted(n for n, _ in again)
+""")
