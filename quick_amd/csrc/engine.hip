@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <map>
 #include <memory>
@@ -566,29 +567,25 @@ struct qf_engine {
         int os_split;    // open-shell builds run this class as two closed-shell passes
         int os_lean;     // ... or, on the tile kernel, in the fused lean form
         int closed_only;             // the tile kernel has no open-shell and no gradient form: these run the
-                                     // class on the wave-per-quartet kernels,
-        int alt_offset, alt_count;   // with tasks of their own in d_alt (count 0: not made, the tile tasks serve)
+        int alt_offset, alt_count;   // class on the wave-per-quartet kernels, with tasks of their own in d_alt
         size_t gslot;    // first double of its region of the global slot buffer (classes that need one)
     };
     std::vector<Launch> launches;
-    bool alt_made = false;   // the tasks in d_alt are those of `launches`
     struct Fused {           // classes of `launches` that share a launch
         int kernel;          // qf::fuse_kernel
-        int offset, count;   // its workgroups in the plan's d_fused
+        int offset, count;   // its workgroups in d_fused
         int waves;
         size_t lds, gslot;
         double seconds;      // estimate
     };
+    std::vector<Fused> fused;
     struct Plan {
-        bool made = false;
         std::vector<std::pair<int, int>> order;   // (launch index, or ~ the index into fused; stream 0..kSide)
         double gain = 0.0;                        // seconds the forked order saves (estimate)
-        std::vector<Fused> fused;
-        DevBuf<qf::FusedBlock> d_fused;
     };
     Plan plan[4];                             // closed shell, open shell, gradient; one launch per class
     bool shared = false;                      // up to the sizes of shares_launches
-    size_t grad_slots = 0;                    // doubles of global slots of the gradient's shared launches
+    size_t grad_slots = 0;                    // doubles of global slots that the gradient's shared launches need
     SideStreams* side = nullptr;              // taken at the first forked build
     Replay replay[3];                         // closed shell, open shell, gradient
     void drop_replays()
@@ -610,6 +607,7 @@ struct qf_engine {
     DevBuf<qf::Task> d_tasks;
     DevBuf<qf::Task> d_alt;
     DevBuf<qf::TileGroup> d_groups;
+    DevBuf<qf::FusedBlock> d_fused;
     DevBuf<int> d_colf;
     DevBuf<double> d_Gt, d_Gs, d_cm, d_P;
     DevBuf<double> d_Pb, d_Pt, d_Ps, d_Fa, d_Fb;   // open-shell builds (allocated on first use)
@@ -1034,10 +1032,11 @@ int shared_kernel(const qf_engine::Launch& L, int os)
 }
 
 // Plan of closed-shell (os 0) or open-shell (os 1) builds in which classes of
-// the same kernel bucket share a launch, its workgroups (appended to `list`)
-// longest first.  Launches run side by side: the regions of the shared ones in
-// the global slot buffer follow those of the plan's own launches (shared_slots).
-void fuse_plan(const qf_engine* e, int os, qf_engine::Plan& p, std::vector<qf::FusedBlock>& list)
+// the same kernel bucket share a launch, its workgroups longest first.
+// Appends to e->fused and to `list`, their workgroups.  Launches run side by side:
+// the regions of the shared ones in the global slot buffer follow those of the
+// plan's own launches.  Returns the doubles of the buffer that the plan needs.
+size_t fuse_plan(qf_engine* e, int os, std::vector<qf::FusedBlock>& list)
 {
     struct Group {
         FusedList list;
@@ -1090,33 +1089,15 @@ void fuse_plan(const qf_engine* e, int os, qf_engine::Plan& p, std::vector<qf::F
         f.seconds = g.cost.seconds();
         slots += (size_t)qf::fuse_kernel(f.kernel).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
         g.list.append(list);
-        t.push_back({~(int)p.fused.size(), f.seconds});
-        p.fused.push_back(f);
+        t.push_back({~(int)e->fused.size(), f.seconds});
+        e->fused.push_back(f);
     }
-    stream_order(t, p);
+    stream_order(t, e->plan[os]);
+    return slots;
 }
 
-// Doubles of the global slot buffer that fuse_plan's launches need, without the
-// plan: the buffer is never resized between prepares (graphs hold it).
-size_t shared_slots(const qf_engine* e, int os)
-{
-    size_t own = 0;
-    int count[qf::kFuseKernels] = {};
-    for (const auto& L : e->launches) {
-        const int k = shared_kernel(L, os);
-        if (k >= 0)
-            count[k] += L.count;
-        else if (slot_doubles(L))
-            own = std::max(own, L.gslot + slot_doubles(L));
-    }
-    for (int k = 0; k < qf::kFuseKernels; ++k)
-        own += (size_t)qf::fuse_kernel(k).global * std::min(count[k], qf::COOP_GLOBAL_SLICES);
-    return own;
-}
-
-// The same for gradients (water 6-31G*, host to host: 291 -> 168 us).  Every class
-// of the engine has a gradient kernel (grad_pass).
-void grad_fuse_plan(const qf_engine* e, qf_engine::Plan& p, std::vector<qf::FusedBlock>& list)
+// The same for gradients (water 6-31G*, host to host: 291 -> 168 us).
+size_t grad_fuse_plan(qf_engine* e, std::vector<qf::FusedBlock>& list)
 {
     std::vector<FusedList> lists(qf::kGradFuseKernels);
     std::vector<LaunchCost> cost(qf::kGradFuseKernels);
@@ -1125,6 +1106,7 @@ void grad_fuse_plan(const qf_engine* e, qf_engine::Plan& p, std::vector<qf::Fuse
     size_t slots = 0;
     for (const auto& L : e->launches) {
         const int k = qf::grad_fuse_bucket(L.cb, L.ck);
+        if (k < 0) return 0;   // an f class: gradients are refused
         const bool coop = qf::grad_fuse_kernel(k).coop;
         if (coop) lds[k] = std::max(lds[k], sizeof(double) * qf::grad_lds_doubles(L.cb, L.ck));
         cost[k].launch(L, coop);
@@ -1143,55 +1125,17 @@ void grad_fuse_plan(const qf_engine* e, qf_engine::Plan& p, std::vector<qf::Fuse
         f.seconds = cost[k].seconds();
         slots += (size_t)qf::grad_fuse_kernel(k).global * std::min(f.count, qf::COOP_GLOBAL_SLICES);
         lists[k].append(list);
-        t.push_back({~(int)p.fused.size(), f.seconds});
-        p.fused.push_back(f);
+        t.push_back({~(int)e->fused.size(), f.seconds});
+        e->fused.push_back(f);
     }
-    stream_order(t, p);
+    stream_order(t, e->plan[2]);
+    return slots;
 }
 
-size_t grad_shared_slots(const qf_engine* e)
-{
-    size_t sum = 0;
-    int count[qf::kGradFuseKernels] = {};
-    for (const auto& L : e->launches) {
-        const int k = qf::grad_fuse_bucket(L.cb, L.ck);
-        if (k < 0) return 0;   // an f class: gradients are refused
-        count[k] += L.count;
-    }
-    for (int k = 0; k < qf::kGradFuseKernels; ++k)
-        sum += (size_t)qf::grad_fuse_kernel(k).global * std::min(count[k], qf::COOP_GLOBAL_SLICES);
-    return sum;
-}
-
-// Plan of a kind of build in shared launches: closed shell (0), open shell (1) or
-// gradient (2); or of any kind with one launch per class (3).
-int make_plan(qf_engine* e, int kind)
-{
-    qf_engine::Plan& p = e->plan[kind];
-    if (p.made) return QF_OK;
-    p.fused.clear();
-    if (kind == 3) {
-        stream_order(e->launches, e->tasks, p);
-    } else {
-        std::vector<qf::FusedBlock> list;
-        if (kind == 2)
-            grad_fuse_plan(e, p, list);
-        else
-            fuse_plan(e, kind, p, list);
-        QF_HIP(p.d_fused.upload(list));
-    }
-    p.made = true;
-    return QF_OK;
-}
-
-// The plan of a build on s.  One launch per class above the sizes of
-// shares_launches, where the grid is capped (qf_set_persistent caps each class's)
-// and where a gradient kernel was chosen.  The plan of the closed shell is made by
-// prepare, the others at the first call: a closed-shell program never uses them
-// (prepare of water 6-31G* 496 -> 418 us, (H2O)8 cc-pVDZ 4226 -> 3717).  Where the
-// plan cannot be uploaded, as under capture or while another stream is captured, a
-// first open-shell build or gradient has one launch per class.
-int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
+// The plan of a build or gradient (kind 2): one launch per class above the sizes of
+// shares_launches, where the grid is capped (qf_set_persistent caps each class's) and
+// where a gradient kernel was chosen.
+const qf_engine::Plan& plan_of(const qf_engine* e, int kind)
 {
     bool plain = e->persist > 0 || !e->shared;
     if (kind == 2 && !plain) {
@@ -1199,10 +1143,7 @@ int plan_of(qf_engine* e, int kind, hipStream_t s, const qf_engine::Plan** out)
         for (const auto& row : e->ctune)
             for (const auto& c : row) plain = plain || c.grad >= 0;
     }
-    if (!plain && !e->plan[kind].made) plain = is_capturing(s) || make_plan(e, kind) != QF_OK;
-    if (plain) kind = 3;
-    *out = &e->plan[kind];
-    return make_plan(e, kind);
+    return e->plan[plain ? 3 : kind];
 }
 
 // Primitive pieces: a wave's lanes each run the whole primitive loop of
@@ -1633,76 +1574,85 @@ int make_tasks(qf_engine* e)
     return QF_OK;
 }
 
-// Wave-per-quartet tasks of the closed_only classes, at the first open-shell build
-// or gradient since a prepare: a closed-shell program never runs them (made by
-// prepare they took it from 24 to 50 ms for (Gly)10 6-31G**).  Where they cannot be
-// uploaded, as under capture or while another stream is captured, those kernels run
-// the tile tasks, whose windows of 64 kets leave longer tails, and the next call
-// tries again.
-void make_alt_tasks(qf_engine* e, hipStream_t s)
+// Wave-per-quartet tasks of the closed_only classes, longest first, for open-shell
+// builds and gradients.  Every bra alone: its kets make windows of one length and a
+// shorter one, so the number of tasks of each amount of work is known beforehand and
+// every task goes straight to its place.  Made like the other tasks and sorted, they
+// were half of prepare for (Gly)10 6-31G** (0.7 million, 32 MB: 24 -> 50 ms, now 18).
+int make_alt_tasks(qf_engine* e)
 {
-    if (e->alt_made) return;
-    bool any = false;
-    for (const auto& L : e->launches) any = any || L.closed_only;
-    if (any && is_capturing(s)) return;
+    const int win = coop_window(e->nbasis);
     std::vector<int> nall;
-    auto each_task = [&](const qf_engine::Launch& L, auto&& f) {
-        const int ct = e->ctune[L.cb][L.ck].piece;
-        const int piece = ct > 0 ? ct : ct < 0 ? 1 << 20 : prim_piece(e, e->nbasis, e->shared);
-        const int win = coop_window(e->nbasis);
+    std::vector<long long> windows(win + 1);   // of a pair of blocks, by length
+    // f(blocks, task with the fields that all tasks of the blocks share, kets of each bra in nall)
+    auto each_pair = [&](const qf_engine::Launch& L, auto&& f) {
         for (int bb = 0; bb < (int)e->blocks.size(); ++bb)
             for (int kb = 0; kb < (int)e->blocks.size(); ++kb) {
                 const HostBlock &B = e->blocks[bb], &K = e->blocks[kb];
                 if (B.cls != L.cb || K.cls != L.ck || (L.cb == L.ck && kb > bb)) continue;
                 prefix_counts(B.info, K.info, e->list_cutoff(), true, nall);
+                if (bb == kb)
+                    for (size_t i = 0; i < nall.size(); ++i) nall[i] = std::min(nall[i], (int)i + 1);
                 qf::Task t{};
                 t.bra_block = bb;
+                t.ke = 1;
                 t.ket_block = kb;
                 t.same_block = bb == kb;
                 t.all_fp64 = 1;
-                for (int x = 0; x < (int)B.bperm.size(); ++x) {
-                    const int i = B.bperm[x];
-                    const int n = bb == kb ? std::min(nall[i], i + 1) : nall[i];
-                    t.kb = x;
-                    t.ke = x + 1;
-                    for (int k0 = 0; k0 < n; k0 += win) {
-                        t.ket_start = k0;
-                        t.ket_count = std::min(win, n - k0);
-                        each_piece(t, B.K, K.K, piece, f);
-                    }
-                }
+                f(B, K, t);
             }
     };
-    // first the work of every task, then each task straight to its place (0.7 million
-    // tasks, 32 MB, for (Gly)10: new pages are most of the time)
-    std::vector<std::vector<int>> place(e->launches.size());
-    std::vector<long long> work;
-    size_t total = 0;
+    auto piece_of = [&](const qf_engine::Launch& L) {
+        const int ct = e->ctune[L.cb][L.ck].piece;
+        return ct > 0 ? ct : ct < 0 ? 1 << 20 : prim_piece(e, e->nbasis, e->shared);
+    };
+    // tasks of each amount of work, the largest first, then the place of the next one
+    std::vector<std::map<long long, int, std::greater<long long>>> place(e->launches.size());
+    int total = 0;
     for (size_t l = 0; l < e->launches.size(); ++l) {
         auto& L = e->launches[l];
         if (!L.closed_only) continue;
-        work.clear();
-        each_task(L, [&](const qf::Task& t) { work.push_back(task_work(t)); });
-        const std::vector<int> ord = longest_first(work);
-        place[l].resize(ord.size());
-        for (size_t k = 0; k < ord.size(); ++k) place[l][ord[k]] = (int)(total + k);
-        L.alt_offset = (int)total;
-        L.alt_count = (int)ord.size();
-        total += ord.size();
+        each_pair(L, [&](const HostBlock& B, const HostBlock& K, qf::Task t) {
+            std::fill(windows.begin(), windows.end(), 0);
+            for (int n : nall) {
+                windows[win] += n / win;
+                ++windows[n % win];
+            }
+            for (t.ket_count = 1; t.ket_count <= win; ++t.ket_count)
+                if (const int n = (int)windows[t.ket_count])
+                    each_piece(t, B.K, K.K, piece_of(L), [&](const qf::Task& x) { place[l][task_work(x)] += n; });
+        });
+        L.alt_offset = total;
+        for (auto& w : place[l]) {
+            const int n = w.second;
+            w.second = total;
+            total += n;
+        }
+        L.alt_count = total - L.alt_offset;
     }
     std::unique_ptr<qf::Task[]> tasks(new qf::Task[total]);
-    for (size_t l = 0; l < e->launches.size(); ++l) {
-        if (place[l].empty()) continue;
-        size_t k = 0;
-        each_task(e->launches[l], [&](const qf::Task& t) { tasks[place[l][k++]] = t; });
-    }
-    hipError_t err = e->d_alt.resize(total);
-    if (err == hipSuccess && total)
-        err = hipMemcpy(e->d_alt.p, tasks.get(), total * sizeof(qf::Task), hipMemcpyHostToDevice);
-    e->alt_made = err == hipSuccess;
-    if (e->alt_made) return;
-    (void)hipGetLastError();
-    for (auto& L : e->launches) L.alt_count = 0;
+    std::vector<std::vector<std::pair<qf::Task, int*>>> pieces(win + 1);   // of a window, by its length
+    for (size_t l = 0; l < e->launches.size(); ++l)
+        if (e->launches[l].closed_only)
+            each_pair(e->launches[l], [&](const HostBlock& B, const HostBlock& K, qf::Task t) {
+                for (t.ket_count = 1; t.ket_count <= win; ++t.ket_count) {
+                    pieces[t.ket_count].clear();
+                    each_piece(t, B.K, K.K, piece_of(e->launches[l]),
+                               [&](const qf::Task& x) { pieces[t.ket_count].push_back({x, &place[l][task_work(x)]}); });
+                }
+                for (int x = 0; x < (int)B.bperm.size(); ++x)
+                    for (int k0 = 0, n = nall[B.bperm[x]]; k0 < n; k0 += win)
+                        for (auto& p : pieces[std::min(win, n - k0)]) {
+                            qf::Task& to = tasks[(*p.second)++];
+                            to = p.first;
+                            to.kb = x;
+                            to.ke = x + 1;
+                            to.ket_start = k0;
+                        }
+            });
+    QF_HIP(e->d_alt.resize(total));
+    if (total) QF_HIP(hipMemcpy(e->d_alt.p, tasks.get(), total * sizeof(qf::Task), hipMemcpyHostToDevice));
+    return QF_OK;
 }
 
 // Tasks of a class for its wave-per-quartet kernels.
@@ -1712,7 +1662,7 @@ struct WaveTasks {
 };
 WaveTasks wave_tasks(const qf_engine* e, const qf_engine::Launch& L)
 {
-    if (L.alt_count > 0) return {e->d_alt.p + L.alt_offset, L.alt_count};
+    if (L.closed_only) return {e->d_alt.p + L.alt_offset, L.alt_count};
     return {e->d_tasks.p + L.offset, L.count};
 }
 
@@ -1806,16 +1756,21 @@ int prepare(qf_engine* e)
     if (rc) return rc;
     QF_HIP(e->d_tasks.upload(e->tasks));
     QF_HIP(e->d_groups.upload(e->groups));
-    e->alt_made = false;
+    if ((rc = make_alt_tasks(e))) return rc;
     e->drop_replays();
     // global slot buffer of the wave-per-quartet classes that keep their
     // node-program slots in global memory
     size_t gdoubles = place_slots(e->launches);
-    if (e->shared) gdoubles = std::max({gdoubles, shared_slots(e, 0), shared_slots(e, 1)});
-    e->grad_slots = e->shared ? grad_shared_slots(e) : 0;
+    e->fused.clear();
+    e->grad_slots = 0;
+    stream_order(e->launches, e->tasks, e->plan[3]);
+    if (e->shared) {
+        std::vector<qf::FusedBlock> list;
+        for (int os = 0; os < 2; ++os) gdoubles = std::max(gdoubles, fuse_plan(e, os, list));
+        e->grad_slots = grad_fuse_plan(e, list);
+        QF_HIP(e->d_fused.upload(list));
+    }
     if (gdoubles) QF_HIP(e->d_cscratch.resize(gdoubles));
-    for (auto& p : e->plan) p.made = false;
-    if ((rc = make_plan(e, e->shared ? 0 : 3))) return rc;
 
     // ---- per-build buffers -------------------------------------------------
     const size_t n2 = (size_t)e->nbasis * e->nbasis;
@@ -1970,11 +1925,11 @@ int timing_begin(qf_engine* e, int li, hipStream_t s, hipEvent_t* stop)
 // 670, ethane def2-TZVP 4482 / 2498 / 1568.  A build under capture is issued
 // launch by launch.
 template <class F>
-int issue_build(qf_engine* e, int kind, const qf_engine::Plan& plan, hipStream_t s, const OpenArgs& open,
-                const CloseArgs* close, F&& issue)
+int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, const CloseArgs* close, F&& issue)
 {
     Replay& r = e->replay[kind];
     const bool captured = is_capturing(s);
+    const qf_engine::Plan& plan = plan_of(e, kind);
     if (!captured && !r.exec && !r.failed && !plan.order.empty() && ++r.uses > 1) {
         hipGraphNode_t last[kSide + 1] = {};
         bool ok = hipGraphCreate(&r.graph, 0) == hipSuccess;
@@ -2113,9 +2068,6 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
     ca.H2 = gb.H2;
     ca.replicas = gb.replicas;
     ca.n = n;
-    const qf_engine::Plan* plan = nullptr;
-    if (!gb.timing)
-        if (int rc = plan_of(e, os, s, &plan)) return rc;
     // one class launch with descriptor m on stream q; los: its open-shell form
     auto launch = [&](const qf_engine::Launch& L, qf::MolDesc* m, int los, qf::LaunchTo& q) -> int {
         if (L.tile == 2 || (los && L.closed_only)) {
@@ -2144,14 +2096,14 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         return rc ? rc : launch(L, dmol_x, 0, q);
     };
     auto shared_launch = [&](const qf_engine::Fused& f, qf::LaunchTo& q) -> int {
-        qf::fuse_kernel(f.kernel).launch(plan->d_fused.p + f.offset, f.count, e->d_groups.p, e->d_tasks.p, e->d_blocks.p,
+        qf::fuse_kernel(f.kernel).launch(e->d_fused.p + f.offset, f.count, e->d_groups.p, e->d_tasks.p, e->d_blocks.p,
                                          dmol, os, f.waves, f.lds, e->d_cscratch.p + f.gslot, q);
         return QF_OK;
     };
     if (gb.fork && !gb.timing) {
-        const int rc = issue_build(e, os, *plan, s, oa, &ca,
+        const int rc = issue_build(e, os, s, oa, &ca,
                                    [&](int li, qf::LaunchTo& q) {
-                                       return li < 0 ? shared_launch(plan->fused[~li], q)
+                                       return li < 0 ? shared_launch(e->fused[~li], q)
                                                      : class_launch(e->launches[li], q);
                                    });
         if (rc) return rc;
@@ -2159,8 +2111,8 @@ int build_pass(qf_engine* e, const double* dP, const double* dcm, double* dF, in
         // one after another on s
         qf::LaunchTo to(s);
         open_build(oa, to);
-        for (const auto& o : plan->order) {
-            const int rc = o.first < 0 ? shared_launch(plan->fused[~o.first], to) : class_launch(e->launches[o.first], to);
+        for (const auto& o : plan_of(e, os).order) {
+            const int rc = o.first < 0 ? shared_launch(e->fused[~o.first], to) : class_launch(e->launches[o.first], to);
             if (rc) return rc;
         }
         close_build(ca, to);
@@ -2214,7 +2166,6 @@ int build_os(qf_engine* e, const double* dPa, const double* dPb, double* dFa, do
 {
     if (!e->prepared) return fail(QF_ERR_STATE, "qf_prepare has not been called");
     const int n2 = e->nbasis * e->nbasis;
-    make_alt_tasks(e, s);
     QF_HIP(e->d_Pt.resize(n2));
     QF_HIP(e->d_Ps.resize(n2));
     double* cm_out = dcm ? nullptr : e->d_cm.p;
@@ -2440,7 +2391,6 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     for (const auto& L : e->launches)
         if (!qf::grad_launcher(L.cb, L.ck))
             return fail(QF_ERR_ARG, "ERI gradients cover shells up to d; this basis has f shells");
-    make_alt_tasks(e, s);
     size_t gdoubles = 0;
     std::vector<size_t> gslot;   // per launch: its region of the global slot buffer
     for (const auto& L : e->launches) {
@@ -2486,11 +2436,10 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
     oa.n = e->nbasis;
     oa.nshell = e->nshell;
     const size_t tile_bytes = (size_t)3 * e->natom * sizeof(double);
-    const qf_engine::Plan* plan = nullptr;
     auto launch = [&](int li, qf::LaunchTo& q) -> int {
         if (li < 0) {
-            const qf_engine::Fused& f = plan->fused[~li];
-            qf::grad_fuse_kernel(f.kernel).launch(plan->d_fused.p + f.offset, f.count, e->d_tasks.p, e->d_blocks.p, dmol,
+            const qf_engine::Fused& f = e->fused[~li];
+            qf::grad_fuse_kernel(f.kernel).launch(e->d_fused.p + f.offset, f.count, e->d_tasks.p, e->d_blocks.p, dmol,
                                                   (int)(f.lds / sizeof(double)),
                                                   f.lds + tile_bytes <= kGradLdsMax ? 3 * e->natom : 0,
                                                   e->d_gscratch.p + f.gslot, q);
@@ -2509,8 +2458,7 @@ int grad_pass(qf_engine* e, const double* dP, const double* dcm, double* cm_out,
         return QF_OK;
     };
     if (!e->timing) {
-        if (int rc = plan_of(e, 2, s, &plan)) return rc;
-        const int rc = issue_build(e, 2, *plan, s, oa, nullptr, launch);
+        const int rc = issue_build(e, 2, s, oa, nullptr, launch);
         if (rc) return rc;
     } else {
         qf::LaunchTo to(s);

@@ -43,7 +43,6 @@ std::string text;
 hipError_t last_error = hipSuccess;
 std::string fail_name;
 int fail_after = -1, failed = 0;
-long long uploaded = 0;    // bytes copied to the device
 
 // true where the test asked this call to fail
 bool fails(const char* fn)
@@ -105,8 +104,6 @@ MOCK void mock_capture(void* s, int id)
     for (auto it = capturing.begin(); it != capturing.end();) it = it->second == was ? capturing.erase(it) : ++it;
 }
 MOCK int mock_streams() { return (int)streams.size(); }
-MOCK long long mock_uploaded() { return uploaded; }
-MOCK void mock_upload_reset() { uploaded = 0; }
 // one line per launch: index, name, grid, slot buffer (0: none), indices it waits for
 MOCK const char* mock_log()
 {
@@ -274,13 +271,7 @@ MOCK hipError_t hipMalloc(void** p, size_t n)
 MOCK hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
 MOCK hipError_t hipHostMalloc(void** p, size_t n, unsigned) { MAY_FAIL; return hipMalloc(p, n); }
 MOCK hipError_t hipHostFree(void* p) { return hipFree(p); }
-MOCK hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind kind)
-{
-    MAY_FAIL;
-    std::memcpy(to, from, n);
-    if (kind == hipMemcpyHostToDevice) uploaded += n;
-    return hipSuccess;
-}
+MOCK hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { MAY_FAIL; std::memcpy(to, from, n); return hipSuccess; }
 MOCK hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(to, from, n, k); }
 MOCK hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }
 MOCK hipError_t hipGetSymbolAddress(void** p, const void*)
@@ -294,7 +285,7 @@ MOCK hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 MOCK hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 MOCK hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 0; return hipSuccess; }
 MOCK hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) { std::memset(p, 0, sizeof *p); return hipSuccess; }
-MOCK hipError_t hipDeviceSynchronize() { return hipSuccess; }
+MOCK hipError_t hipDeviceSynchronize() { MAY_FAIL; return hipSuccess; }
 MOCK const char* hipGetErrorString(hipError_t) { return "mock"; }
 MOCK hipError_t hipGetLastError()
 {

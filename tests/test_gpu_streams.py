@@ -174,9 +174,9 @@ def test_forked_builds_of_several_threads():
 
 @pytest.mark.parametrize("name,basis", [("water16", "6-31G*"), ("water3", "6-31G*")])
 def test_first_open_shell_build_and_gradient_under_capture(name, basis):
-    """What an open-shell build or a gradient needs beyond a closed-shell build is
-    made at the first of them; under capture nothing can be, and the kernels run
-    what prepare made (16 waters: the tile tasks of the Hermite-only classes)."""
+    """The first calls after a prepare, which has made everything they need, under
+    capture and, on another stream, beside it (where an allocation or a synchronous
+    copy would end the capture)."""
     announce("streams first call under capture %s" % name)
     eng, P, _ = setup(name, basis, cutoff=1e-10)
     Q = (0.3 * P).contiguous()
@@ -212,6 +212,22 @@ def test_first_open_shell_build_and_gradient_under_capture(name, basis):
         s.synchronize()
         for x, w in zip((Fa, Fb, g), want):
             assert np.abs(x.cpu().numpy() - w).max() <= 1e-11 * max(1.0, np.abs(w).max())
+    eng.set_cutoffs(1e-10)
+    eng.prepare()
+    beside = torch.cuda.CUDAGraph()
+    t = torch.cuda.Stream()
+    for x in (Fa, Fb, g):
+        x.zero_()
+    F = torch.zeros_like(P)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(beside, stream=s):
+            eng.fock2e_device(P.data_ptr(), F.data_ptr(), s.cuda_stream)
+            eng.fock2e_os_device(P.data_ptr(), Q.data_ptr(), Fa.data_ptr(), Fb.data_ptr(), t.cuda_stream)
+            eng.eri_grad_device(P.data_ptr(), g.data_ptr(), t.cuda_stream)
+    torch.cuda.synchronize()
+    for x, w in zip((Fa, Fb, g), want):
+        assert np.abs(x.cpu().numpy() - w).max() <= 1e-11 * max(1.0, np.abs(w).max())
 
 
 def test_batch_build_beside_a_capture_of_the_batch():

@@ -229,84 +229,6 @@ for n, tile, want in ((1, 1, 0), (4, 1, 0), (13, 1, 0), (13, -1, 0), (14, 1, 3),
 """)
 
 
-def test_tasks_that_only_some_calls_need_are_made_by_those_calls(mock):
-    """Above 256 functions the wave-per-quartet tasks of the Hermite-only classes
-    are made at the first open-shell build or gradient: prepare uploads none, a
-    call under capture before that runs the tile tasks, and all cover the same
-    quartets."""
-    mock_hip.run(mock, BUILD + """
-def grids(kind):
-    out = {}
-    for o in launches(mock):
-        for c in ("C2220", "C2211", "C2121"):
-            if c + ("Grad" if kind == "grad" else "Coop") in o.name: out[c] = o.grid
-    return out
-for kind in ("os", "grad"):
-    e = engine(M.alkane(14), "6-31G*", prepare=False)
-    mock.mock_upload_reset()
-    e.prepare()
-    first = mock.mock_uploaded()
-    builds(e, "fock", 3)
-    assert mock.mock_uploaded() == first, "a closed-shell build uploads nothing"
-    mock.mock_capture(None, 1)
-    builds(e, kind, 1, closing=kind == "os")
-    captured = grids(kind)
-    assert mock.mock_uploaded() == first
-    mock.mock_capture(None, 0)
-    builds(e, kind, 3, closing=kind == "os")
-    own = grids(kind)
-    assert len(own) == 3 and captured.keys() == own.keys()
-    assert all(own[c] > captured[c] for c in own), (own, captured)
-    made = mock.mock_uploaded()
-    assert made > first
-    builds(e, "grad" if kind == "os" else "os", 2, closing=kind == "grad")
-    assert mock.mock_uploaded() == made, "made twice"
-    e.close()
-""")
-
-
-@pytest.mark.parametrize("mol,basis", [("M.polyglycine(1)", "6-31G**"), ("M.alkane(2)", "6-31G"),
-                                       ("M.alkane(2)", "def2-TZVP")])
-def test_plans_that_only_some_calls_need_are_made_by_those_calls(mock, mol, basis):
-    """Up to 200 functions the shared launches of open-shell builds and gradients
-    are planned at the first of them; under capture before that they have one
-    launch per class.  The slots of a closed-shell graph stay where they are."""
-    mock_hip.run(mock, BUILD + f"""
-kinds = ["os"] if "TZ" in "{basis}" else ["os", "grad"]
-for kind in kinds:
-    e = engine({mol}, "{basis}", prepare=False)
-    mock.mock_upload_reset()
-    e.prepare()
-    first = mock.mock_uploaded()
-    builds(e, "fock", 3)
-    slots = [o.slots for o in launches(mock)]
-    closing = kind == "os"
-    mock.mock_capture(None, 1)
-    (captured, _), = builds(e, kind, 1, closing=closing)
-    assert mock.mock_uploaded() == first and not any("fused_" in o.name for o in launches(mock))
-    mock.mock_capture(None, 0)
-    own = builds(e, kind, 3, closing=closing)
-    assert len(set(own)) == 1 and own[0][0] < captured and any("fused_" in o.name for o in launches(mock))
-    made = mock.mock_uploaded()
-    assert made > first
-    mock.mock_capture(None, 1)
-    builds(e, kind, 1, closing=closing)
-    mock.mock_capture(None, 0)
-    assert any("fused_" in o.name for o in launches(mock)) and mock.mock_uploaded() == made
-    builds(e, "fock", 1)
-    assert [o.slots for o in launches(mock)] == slots
-    # a capped grid at prepare still leaves the plan of shared launches ready
-    e.set_persistent(64)
-    e.set_cutoffs(1e-9)
-    e.prepare()
-    e.set_persistent(0)
-    made = mock.mock_uploaded()
-    builds(e, "fock", 2)
-    assert any("fused_" in o.name for o in launches(mock)) and mock.mock_uploaded() == made
-    e.close()
-""")
-
-
 @pytest.mark.parametrize("what", ["engine", "batch"])
 def test_builds_beside_a_capture_of_the_same_engine(mock, what):
     """The side streams of an engine or batch that took part in a capture belong to
@@ -345,26 +267,30 @@ assert issue(two, "after it")
 """)
 
 
-@pytest.mark.parametrize("mol", ["M.polyglycine(1)", "M.alkane(14)"])
-@pytest.mark.parametrize("kind", ["os", "grad"])
-@pytest.mark.parametrize("call", ["hipMemcpy", "hipMalloc"])
-def test_a_first_build_goes_on_where_its_own_tables_cannot_be_uploaded(mock, mol, kind, call):
-    """As while another stream of the thread is captured: the build runs what prepare
-    made, and the next one tries again."""
+@pytest.mark.parametrize("mol,basis", [("M.polyglycine(1)", "6-31G**"), ("M.alkane(2)", "def2-TZVP"),
+                                       ("M.alkane(14)", "6-31G*")])
+def test_builds_need_nothing_but_what_prepare_made(mock, mol, basis):
+    """While any stream of the process is captured the runtime refuses allocations
+    and synchronous copies (and the capture is lost): a first build of any kind after
+    a prepare makes neither, under capture or beside one, and issues the launches
+    that later ones do."""
     mock_hip.run(mock, BUILD + f"""
-e = engine({mol}, "6-31G*")
-closing = {kind!r} == "os"
-own = builds(e, {kind!r}, 2, closing=closing) and [(o.name, o.grid) for o in launches(mock)]
-# other tables than the ones that were made: a larger buffer is needed
-e.set_cutoffs(1e-14)
-e.prepare()
-mock.mock_fail(b"{call}", 0)
-builds(e, {kind!r}, 1, closing=closing)
-plain = [(o.name, o.grid) for o in launches(mock)]
-assert mock.mock_failed() == 1, "the call that was to fail was not made"
-mock.mock_fail(b"", -1)
-builds(e, {kind!r}, 3, closing=closing)
-again = [(o.name, o.grid) for o in launches(mock)]
-assert plain != again
-assert sorted(n for n, _ in own) == sorted(n for n, _ in again)
+kinds = ["fock", "os"] + ([] if "TZ" in "{basis}" else ["grad"])
+e = engine({mol}, "{basis}")
+for kind in kinds:
+    builds(e, kind, 3, closing=kind != "grad")     # the buffers of its kind are allocated once
+want = {{}}
+for captured in (0, 1):
+    e.set_cutoffs(1e-12)
+    e.prepare()
+    for kind in kinds:
+        mock.mock_capture(None, captured)
+        for call in (b"hipMalloc", b"hipMemcpy", b"hipHostMalloc", b"hipStreamSynchronize", b"hipDeviceSynchronize"):
+            mock.mock_fail(call, 0)
+            builds(e, kind, 1, closing=kind != "grad")
+            assert mock.mock_failed() == 0, call
+            names = sorted(o.name for o in launches(mock))
+            assert want.setdefault(kind, names) == names
+        mock.mock_fail(b"", -1)
+        mock.mock_capture(None, 0)
 """)
