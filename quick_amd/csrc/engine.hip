@@ -450,18 +450,37 @@ struct Replay {
     CloseArgs close{};
     int uses = 0;           // builds of this kind since the last prepare
     bool failed = false;    // could not be built: the launches stay eager
-    void drop()
+    std::vector<std::pair<hipGraph_t, hipGraphExec_t>> old;   // put aside, may still run
+    // Puts the graph aside without a wait: a setter may be called while a stream is
+    // captured, and a wait would end the capture.  Bounded: builds outside a capture
+    // give what was put aside back (sweep).
+    void retire()
     {
-        if (exec) {
-            (void)hipDeviceSynchronize();   // a replay may still run
-            (void)hipGraphExecDestroy(exec);
-        }
-        if (graph) (void)hipGraphDestroy(graph);
-        (void)hipGetLastError();
+        if (old.size() >= 16) sweep();
+        if (exec)
+            old.push_back({graph, exec});
+        else if (graph)
+            (void)hipGraphDestroy(graph);
         exec = nullptr;
         graph = nullptr;
         uses = 0;
         failed = false;
+    }
+    void sweep()
+    {
+        if (old.empty()) return;
+        (void)hipDeviceSynchronize();   // they may still run
+        for (auto& x : old) {
+            (void)hipGraphExecDestroy(x.second);
+            (void)hipGraphDestroy(x.first);
+        }
+        old.clear();
+        (void)hipGetLastError();
+    }
+    void drop()
+    {
+        retire();
+        sweep();
     }
 };
 
@@ -1930,6 +1949,7 @@ int issue_build(qf_engine* e, int kind, hipStream_t s, const OpenArgs& open, con
     Replay& r = e->replay[kind];
     const bool captured = is_capturing(s);
     const qf_engine::Plan& plan = plan_of(e, kind);
+    if (!captured && r.old.size() >= 4) r.sweep();
     if (!captured && !r.exec && !r.failed && !plan.order.empty() && ++r.uses > 1) {
         hipGraphNode_t last[kSide + 1] = {};
         bool ok = hipGraphCreate(&r.graph, 0) == hipSuccess;
@@ -2488,7 +2508,7 @@ int qf_set_grad_kernel(qf_engine* e, int lane)
 {
     if (!e) return fail(QF_ERR_ARG, "engine is NULL");
     e->grad_lane = lane != 0;
-    e->replay[2].drop();
+    e->replay[2].retire();
     return QF_OK;
 }
 
@@ -2498,7 +2518,7 @@ int qf_set_grad_class(qf_engine* e, int cb, int ck, int mode)
     if (cb < 0 || cb >= kNPC || ck < 0 || ck > cb) return fail(QF_ERR_ARG, "class index out of range");
     if (mode < -1 || mode > 1) return fail(QF_ERR_ARG, "mode must be -1, 0 (wave-per-quartet) or 1 (per-lane)");
     e->ctune[cb][ck].grad = mode;
-    e->replay[2].drop();
+    e->replay[2].retire();
     return QF_OK;
 }
 
@@ -2839,7 +2859,7 @@ int qf_set_persistent(qf_engine* e, int max_workgroups)
 {
     if (!e || max_workgroups < 0) return fail(QF_ERR_ARG, "max_workgroups must be >= 0");
     e->persist = max_workgroups;
-    e->drop_replays();
+    for (auto& r : e->replay) r.retire();
     return QF_OK;
 }
 

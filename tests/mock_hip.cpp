@@ -40,6 +40,7 @@ std::map<void*, int> capturing;                // id of the capture a stream tak
 std::map<void*, int> event_capture;
 std::vector<void*> streams;                    // created and not destroyed
 std::string text;
+int execs = 0;             // instantiated graphs
 hipError_t last_error = hipSuccess;
 std::string fail_name;
 int fail_after = -1, failed = 0;
@@ -93,6 +94,7 @@ MOCK void mock_fail(const char* fn, int after)
     failed = 0;
 }
 MOCK int mock_failed() { return failed; }
+MOCK int mock_execs() { return execs; }
 // begins capture `id` on a stream, or (0) ends the one it takes part in
 MOCK void mock_capture(void* s, int id)
 {
@@ -234,9 +236,15 @@ MOCK hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNod
 {
     MAY_FAIL;
     *e = (hipGraphExec_t) new Graph(*(Graph*)g);
+    ++execs;
     return hipSuccess;
 }
-MOCK hipError_t hipGraphExecDestroy(hipGraphExec_t e) { delete (Graph*)e; return hipSuccess; }
+MOCK hipError_t hipGraphExecDestroy(hipGraphExec_t e)
+{
+    delete (Graph*)e;
+    --execs;
+    return hipSuccess;
+}
 MOCK hipError_t hipGraphExecKernelNodeSetParams(hipGraphExec_t e, hipGraphNode_t n, const hipKernelNodeParams* p)
 {
     MAY_FAIL;

@@ -257,3 +257,44 @@ def test_batch_build_beside_a_capture_of_the_batch():
         g.replay()
         torch.cuda.synchronize()
     b.close()
+
+
+def test_setters_inside_a_capture():
+    """A changed gradient kernel and grid cap inside a capture, after replayed calls."""
+    announce("streams setters inside a capture")
+    eng, P, G = setup("water3")
+    s = torch.cuda.Stream()
+    F = torch.zeros_like(P)
+    g = torch.zeros(eng.basis.mol.natom, 3, dtype=P.dtype, device="cuda")
+
+    def calls():
+        F.zero_()
+        g.zero_()
+        eng.fock2e_device(P.data_ptr(), F.data_ptr(), s.cuda_stream)
+        eng.eri_grad_device(P.data_ptr(), g.data_ptr(), s.cuda_stream)
+
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        eng.set_grad_kernel(lane=False)
+        calls()                         # the buffers of both kernels
+        eng.set_grad_kernel(lane=True)
+        for _ in range(3):
+            calls()
+    s.synchronize()
+    want = g.cpu().numpy()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        with torch.cuda.graph(graph, stream=s):
+            eng.set_persistent(64)
+            eng.set_grad_kernel(lane=False)
+            calls()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        close(F, G)
+        assert np.abs(g.cpu().numpy() - want).max() <= 1e-11 * np.abs(want).max()
+        with torch.cuda.stream(s):
+            calls()
+        s.synchronize()
+        close(F, G)
+        assert np.abs(g.cpu().numpy() - want).max() <= 1e-11 * np.abs(want).max()

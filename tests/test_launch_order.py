@@ -294,3 +294,36 @@ for captured in (0, 1):
         mock.mock_fail(b"", -1)
         mock.mock_capture(None, 0)
 """)
+
+
+def test_setters_between_captured_calls_do_not_wait(mock):
+    """Grid cap and gradient kernel may change inside a capture: replays that hold the
+    old choice are put aside without a wait (which would end the capture) and
+    given back later."""
+    mock_hip.run(mock, BUILD + """
+e = engine(M.polyglycine(1), "6-31G**")
+for kind in ("fock", "os", "grad"):
+    builds(e, kind, 3, closing=kind != "grad")
+assert mock.mock_execs() == 3
+for k in range(40):
+    mock.mock_fail(b"hipDeviceSynchronize", 0)
+    mock.mock_capture(None, 1)
+    if k % 2: e.set_persistent(64 if k % 4 == 1 else 0)
+    else: e.set_grad_kernel(k % 4 == 0)
+    if k % 5 == 0: e.set_grad_class(1, 0, k % 2)
+    for kind in ("fock", "os", "grad"):
+        builds(e, kind, 1, closing=kind != "grad")
+    mock.mock_capture(None, 0)
+    assert mock.mock_failed() == 0
+    mock.mock_fail(b"", -1)
+    for kind in ("fock", "os", "grad"):
+        builds(e, kind, 2, closing=kind != "grad")
+    assert mock.mock_execs() <= 3 + 16
+e.set_cutoffs(1e-11)
+e.prepare()
+assert mock.mock_execs() == 0
+builds(e, "fock", 2)
+e.set_persistent(8)
+e.close()
+assert mock.mock_execs() == 0
+""")
