@@ -1808,7 +1808,7 @@ int prepare(qf_engine* e)
     QF_HIP(e->d_shells.upload(shells));
     QF_HIP(e->d_mol.resize(4));   // slots: build / open-shell pass 1, open-shell pass 2, no-alloc build, gradient
     QF_HIP(e->d_counts.resize(2 * std::max<size_t>(1, e->launches.size())));
-    e->stats.device_bytes = (long long)(e->d_info.bytes() + e->d_prim.bytes() + e->d_tasks.bytes() +
+    e->stats.device_bytes = (long long)(e->d_info.bytes() + e->d_prim.bytes() + e->d_tasks.bytes() + e->d_alt.bytes() +
                                         e->d_Gt.bytes() * 3 + e->d_cm.bytes() + e->d_blocks.bytes());
     // launch indices recorded for timing refer to the old launch list
     e->ev_used = 0;
