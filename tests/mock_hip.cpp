@@ -270,15 +270,23 @@ MOCK hipError_t hipGraphLaunch(hipGraphExec_t e, hipStream_t s)
 }
 
 // ---- memory, device, errors
+std::map<void*, size_t> device;   // allocations not yet freed
 MOCK hipError_t hipMalloc(void** p, size_t n)
 {
     MAY_FAIL;
     *p = std::malloc(n ? n : 1);
+    device[*p] = n;
     return hipSuccess;
 }
-MOCK hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
-MOCK hipError_t hipHostMalloc(void** p, size_t n, unsigned) { MAY_FAIL; return hipMalloc(p, n); }
-MOCK hipError_t hipHostFree(void* p) { return hipFree(p); }
+MOCK hipError_t hipFree(void* p) { device.erase(p); std::free(p); return hipSuccess; }
+MOCK long long mock_bytes()
+{
+    long long n = 0;
+    for (auto& d : device) n += (long long)d.second;
+    return n;
+}
+MOCK hipError_t hipHostMalloc(void** p, size_t n, unsigned) { MAY_FAIL; *p = std::malloc(n ? n : 1); return hipSuccess; }
+MOCK hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
 MOCK hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind) { MAY_FAIL; std::memcpy(to, from, n); return hipSuccess; }
 MOCK hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(to, from, n, k); }
 MOCK hipError_t hipMemset(void* p, int v, size_t n) { std::memset(p, v, n); return hipSuccess; }

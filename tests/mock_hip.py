@@ -36,6 +36,7 @@ def start():
     sys.modules["torch"] = None            # it would bring the real runtime
     mock = ctypes.CDLL(os.environ["MOCK_HIP"], ctypes.RTLD_GLOBAL)
     mock.mock_log.restype = mock.mock_stream.restype = ctypes.c_char_p
+    mock.mock_bytes.restype = ctypes.c_longlong
     mock.mock_stream.argtypes = [ctypes.c_void_p]
     mock.mock_capture.argtypes = [ctypes.c_void_p, ctypes.c_int]
     return mock

@@ -327,3 +327,23 @@ e.set_persistent(8)
 e.close()
 assert mock.mock_execs() == 0
 """)
+
+
+def test_device_bytes_counts_every_task_table(mock):
+    """stats()["device_bytes"] follows what is allocated, whether or not classes
+    have a second table of wave-per-quartet tasks."""
+    mock_hip.run(mock, BUILD + """
+held = []
+for tile in (-1, 2):
+    e = engine(M.water_cluster(16), "6-31G*", prepare=False)
+    for c in ((4, 2), (4, 4), (5, 2), (5, 3)):
+        e.set_class_tuning(*c, tile)
+    before = mock.mock_bytes()
+    e.prepare()
+    held.append((mock.mock_bytes() - before, e.stats()["device_bytes"]))
+    e.close()
+(a, x), (b, y) = held
+# buffers that the figure leaves out (descriptors, counters, shell maps) differ by
+# 43 KB between the two engines; the second table holds 2 MB
+assert abs((x - y) - (a - b)) < 200000, held
+""")
